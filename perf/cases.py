@@ -68,11 +68,13 @@ def _log_int(rng, lo, hi):
 
 def draw(rng):
     kind = rng.choice(["view", "train", "batch", "march_view", "march_train", "march_f64", "raster"])
-    n_max = dict(view=3_000_000, train=1_000_000, batch=250_000, march_view=200_000, march_train=60_000, march_f64=3_000, raster=200_000)[kind]
+    n_max = dict(view=3_000_000, train=1_000_000, batch=250_000, march_view=200_000, march_train=60_000, march_f64=1_500, raster=200_000)[kind]
     n_min = dict(batch=20_000, march_f64=300).get(kind, 300)
-    w_max, h_max = dict(march_view=(1024, 1024), march_train=(512, 384), march_f64=(96, 80), raster=(1024, 1024)).get(kind, (1920, 1080))
+    w_max, h_max = dict(march_view=(1024, 1024), march_train=(512, 384), march_f64=(83, 67), raster=(1024, 1024)).get(kind, (1920, 1080))
     n = _log_int(rng, n_min, n_max)
     extent = 1.0 if n < 6_000 else 5.0
+    if extent == 1.0 and kind in ("march_view", "march_train", "raster"):
+        w_max, h_max = 211, 157  # a compact scene is dense: every ray meets hundreds of Gaussians
     degree = rng.choice([0, 1, 2, 3, 3])
     width, height = _log_int(rng, 32, w_max), _log_int(rng, 32, h_max)
     if kind == "batch":
