@@ -22,6 +22,7 @@
 // back instead of recomputing sections and bins: only the adjoint walks
 // remain, which makes the backward cost about as much as the forward.
 #include <algorithm>
+#include <utility>
 
 #include "host_common.h"
 #include "march_device.h"
@@ -161,33 +162,87 @@ __global__ __launch_bounds__(kPreThreads) void k_march_preprocess(int64_t n, Mar
     mass_out[i] = mass;
 }
 
+// A Gaussian of the tile's list in LDS: what the passes read at one address for
+// the whole wave, with the per-Gaussian parts of the ray restriction (centre
+// relative to the camera, normalisation) computed once when it is staged
+// instead of by every pixel of every pass.
 template <class S>
-struct Staged {
+struct alignas(16) Staged {
+    S A[6];   // inverse filtered covariance
+    S m[3];   // mu - o
     S mu[3];
-    S A[6];
-    S rgb[3];
+    S norm3;  // sqrt(det A) / sqrt((2 pi)^3)
     S mass;
+    S rgb[3];
     S depth;
     uint32_t id;
 };
 
+// Where along any ray of the tile a staged Gaussian can matter: outside
+// [lo, hi] it holds neither a sample section nor a bin mass of 1e-5.  One
+// float pair per list entry, read by one lane each.
+struct Reach1d {
+    float lo, hi;
+};
+
 template <class S>
-__device__ __forceinline__ void stage_gaussian(Staged<S>* dst, uint32_t id, const S* means, const S* inv_cov, const S* rgb, const S* mass,
-    const S* depths)
+__device__ __forceinline__ Ray1d<S> intersect_staged(const Staged<S>& g, const S* o, const S* d)
 {
-    dst->mu[0] = means[3 * id];
-    dst->mu[1] = means[3 * id + 1];
-    dst->mu[2] = means[3 * id + 2];
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-        dst->A[k] = inv_cov[6 * id + k];
-    dst->rgb[0] = rgb[3 * id];
-    dst->rgb[1] = rgb[3 * id + 1];
-    dst->rgb[2] = rgb[3 * id + 2];
-    dst->mass = mass[id];
-    dst->depth = depths[id];
-    dst->id = id;
+    return intersect_ray_pre(g.mu, g.A, g.m, g.norm3, o, d);
 }
+
+// The window of a Gaussian over the tile's rays.  A point x d of the ray lies
+// at A-distance^2 E + z^2 from the centre mu (E: of the ray's nearest point, z:
+// standard deviations along the ray), so |x d - m| <= K sqrt(lambda) for every
+// point with E + z^2 <= K^2, lambda the largest eigenvalue of A^-1 (bounded by
+// the Frobenius norm), m = mu - o; as long as x >= 0 that bounds x by
+// |m| +- K sqrt(lambda).  The mass on the ray is at most M exp(-E / 2) with
+// M = mass norm3 sqrt(2 pi lambda), and a section or a bin of the Gaussian
+// needs
+//   mass on the ray >= 1/255 and z <= 3:   E + z^2 <= 2 ln M + 2 ln 255 + 9
+//   z within far_radius' cut:              E + z^2 <= 2 ln M + 2 ln 55556, or
+//                                          + 5.5^2 - 2 ln 2 when M can exceed 2
+// Rounding is covered by the widened K and an absolute term; where it could
+// not be (ill-conditioned A), for M >= 10 (never cut) and for rays that may
+// point away from the Gaussian, the window is the whole axis.
+template <class S>
+__device__ __forceinline__ Reach1d ray_window(const Staged<S>& g, S detA, const float* dc, float dev)
+{
+    const float inf = __builtin_inff();
+    const Reach1d all { -inf, inf };
+    const float a0 = float(g.A[0]), a1 = float(g.A[1]), a2 = float(g.A[2]), a3 = float(g.A[3]), a4 = float(g.A[4]), a5 = float(g.A[5]);
+    const float det = float(detA);
+    if (!(a0 > 0.f && a0 * a3 - a1 * a1 > 0.f && det > 0.f))
+        return all;
+    const float id = 1.f / det;
+    const float c0 = (a3 * a5 - a4 * a4) * id, c1 = (a2 * a4 - a1 * a5) * id, c2 = (a1 * a4 - a2 * a3) * id, c3 = (a0 * a5 - a2 * a2) * id,
+                c4 = (a2 * a1 - a0 * a4) * id, c5 = (a0 * a3 - a1 * a1) * id;
+    const float lam = sqrtf(c0 * c0 + c3 * c3 + c5 * c5 + 2.f * (c1 * c1 + c2 * c2 + c4 * c4));
+    const float tr = a0 + a3 + a5;
+    const float cond = tr * lam;
+    const float m0 = float(g.m[0]), m1 = float(g.m[1]), m2 = float(g.m[2]);
+    const float len = sqrtf(m0 * m0 + m1 * m1 + m2 * m2);
+    const float M = float(g.mass) * float(g.norm3) * sqrtf(float(2 * kPi) * lam);
+    if (!(cond < 1e4f) || !(1e-6f * len * sqrtf(tr) < 0.02f) || !(M < 9.9f) || !(m0 * dc[0] + m1 * dc[1] + m2 * dc[2] > 1.01f * dev * len + 1e-6f * len))
+        return all;
+    if (M < 0.0039f)
+        return Reach1d { inf, -inf }; // under 1/255 on every ray
+    const float K2 = 2.f * logf(M) + (M > 1.9f ? 29.f : 22.f);
+    const float half = (1.02f * sqrtf(fmaxf(K2, 0.f)) + 0.1f) * sqrtf(lam) + 1e-6f * cond * len;
+    return Reach1d { len - half, len + half };
+}
+
+// the direction the tile's rays deviate from by at most dev
+struct TileAxis {
+    float dc[3];
+    float dev;
+};
+
+template <class S>
+struct MarchData;
+
+template <class S>
+__device__ __forceinline__ void stage_gaussian(Staged<S>* dst, Reach1d* win, uint32_t id, const MarchData<S>& md, const S* o, const TileAxis& ax);
 
 struct MarchControl {
     int max_large_steps;
@@ -227,6 +282,30 @@ struct Replay {
 
 constexpr uint32_t kReplayNotKept = 0xffffffffu;
 
+template <class S>
+__device__ __forceinline__ void stage_gaussian(Staged<S>* dst, Reach1d* win, uint32_t id, const MarchData<S>& md, const S* o, const TileAxis& ax)
+{
+    Staged<S> g;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        g.mu[k] = md.means[3 * id + k];
+        g.rgb[k] = md.rgb[3 * id + k];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+        g.A[k] = md.inv_cov[6 * id + k];
+    g.mass = md.mass[id];
+    g.depth = md.depths[id];
+    g.id = id;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        g.m[k] = g.mu[k] - o[k];
+    const S detA = sym3_det(g.A);
+    g.norm3 = ray_norm3(detA);
+    *win = ray_window(g, detA, ax.dc, ax.dev);
+    *dst = g;
+}
+
 template <int NT>
 __host__ __device__ constexpr int64_t replay_record_elems()
 {
@@ -247,6 +326,16 @@ __device__ __forceinline__ void store4<float>(float* p, float a, float b, float 
 {
     *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
 }
+
+// A copy the compiler does not trace back: a 16-byte store needs four
+// consecutive registers, and without it the bins would be held that way (and
+// copied) through the whole deposit loop.
+__device__ __forceinline__ float detached(float v)
+{
+    asm("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ double detached(double v) { return v; }
 
 template <class S>
 __device__ __forceinline__ void load4(const S* p, S* v)
@@ -274,32 +363,82 @@ __device__ __forceinline__ int xcd_tile_m(int b, int n_tiles)
     return x * q + min(x, r) + slot;
 }
 
-// 1D parameters of a Gaussian on this ray and whether it can deposit mass
-// (math.h:436-454)
+// A Gaussian on this pixel's ray: centre, 1 / sd, mass on the ray, and the
+// distance from the centre beyond which every bin holds less than 1e-5 (the
+// reference's per-bin threshold, so bins out there take nothing).
 template <class S>
-__device__ __forceinline__ bool ray_gaussian(const Staged<S>& g, const S* o, const S* d, S b_first, S b_last, Ray1d<S>* r, S* sd, S* inv_sd,
-    S* mor)
+struct RayGauss {
+    S centre, inv_sd, mor, far;
+};
+
+// The far distance: the tail beyond z sd holds at most exp(-z^2 / 2) / 2 of the
+// mass, so z^2 = 2 ln(mor / 1.8e-5) leaves every bin there at most 0.9e-5; the
+// rest of the 1e-5 covers the float cdf's 1.5e-7 (twice, for mor <= 2).  Above
+// that 5.5 sd, and no cut for more than 10 (which could reach 1e-5 by the
+// cdf's error alone).
+__device__ __forceinline__ float far_radius(float mor, float var)
 {
-    *r = intersect_ray(g.mu, g.A, o, d);
-    *sd = sqrt_rn(r->var);
-    *inv_sd = S(1) / *sd;
-    *mor = r->weight * g.mass;
-    if (r->centre != r->centre)
+    const float z2 = 1.3862943611f * (__builtin_amdgcn_logf(mor) + 15.7616f); // 2 ln2 (log2 mor + log2 55556)
+    const float r = __builtin_amdgcn_sqrtf((mor > 1.99f ? 30.25f : z2) * var);
+    return mor > 9.99f ? __builtin_inff() : r;
+}
+
+// A restricted to the ray and whether it can deposit mass (math.h:436-454).
+// Double: the reference's expressions.
+template <class S>
+__device__ __forceinline__ bool ray_gaussian(const Staged<S>& g, const S* o, const S* d, RayGauss<S>* out)
+{
+    const Ray1d<S> r = intersect_staged(g, o, d);
+    const S sd = sqrt_rn(r.var);
+    out->centre = r.centre;
+    out->inv_sd = S(1) / sd;
+    out->mor = r.weight * g.mass;
+    out->far = S(far_radius(float(out->mor), float(r.var)) * 1.00001f);
+    if (r.centre != r.centre)
         return false;
-    if (*mor < S(1.0f / 255.f) || *mor > S(1000))
+    if (out->mor < S(1.0f / 255.f) || out->mor > S(1000))
         return false;
-    if (*sd <= S(0.0001) || *sd != *sd || *mor != *mor || *mor > S(100000))
+    if (sd <= S(0.0001) || sd != sd || out->mor != out->mor)
         return false;
     return true;
 }
 
-// Conservative skip of a chunk whose borders lie > 5.5 sd from the centre:
-// every bin there holds less than 1e-5 (the reference's per-bin threshold)
-// as long as the mass on the ray is at most 10.
-template <class S>
-__device__ __forceinline__ bool chunk_far(S centre, S inv_sd, S mor, S lo, S hi)
+// Float: the centre and the residual o + centre d - mu keep the operations of
+// the exact restriction (the residual's rounding, ~1e-7 of the distance, is
+// what the mass is sensitive to, and it moves with the centre), the rest uses
+// fused multiply-adds, the hardware reciprocal square root and exp2: 60
+// instructions instead of 170.  The result is a few ulp from the exact
+// restriction's, which decides where the mass on the ray is within 1e-3 of a
+// threshold, so no Gaussian changes sides.
+template <>
+__device__ __forceinline__ bool ray_gaussian<float>(const Staged<float>& g, const float* o, const float* d, RayGauss<float>* out)
 {
-    return mor <= S(10) && ((lo - centre) * inv_sd > S(5.5) || (centre - hi) * inv_sd > S(5.5));
+    const float Ad0 = (g.A[0] * d[0] + g.A[1] * d[1]) + g.A[2] * d[2];
+    const float Ad1 = (g.A[1] * d[0] + g.A[3] * d[1]) + g.A[4] * d[2];
+    const float Ad2 = (g.A[2] * d[0] + g.A[4] * d[1]) + g.A[5] * d[2];
+    const float q = (d[0] * Ad0 + d[1] * Ad1) + d[2] * Ad2;
+    const float C = 1.f / q;
+    const float centre = ((Ad0 * g.m[0] + Ad1 * g.m[1]) + Ad2 * g.m[2]) * C;
+    const float r0 = (o[0] + centre * d[0]) - g.mu[0];
+    const float r1 = (o[1] + centre * d[1]) - g.mu[1];
+    const float r2 = (o[2] + centre * d[2]) - g.mu[2];
+    const float Ar0 = fmaf(g.A[2], r2, fmaf(g.A[1], r1, g.A[0] * r0));
+    const float Ar1 = fmaf(g.A[4], r2, fmaf(g.A[3], r1, g.A[1] * r0));
+    const float Ar2 = fmaf(g.A[5], r2, fmaf(g.A[4], r1, g.A[2] * r0));
+    const float E = fmaf(r2, Ar2, fmaf(r1, Ar1, r0 * Ar0));
+    const float sd = __builtin_amdgcn_rsqf(q);
+    // mass norm3 sqrt(2 pi) exp(-E / 2) sd
+    float mor = (g.mass * g.norm3) * (2.5066282746310002f * sd) * __builtin_amdgcn_exp2f(E * -0.7213475204444817f);
+    const bool near_cut = fabsf(fmaf(mor, 255.f, -1.f)) < 1e-3f || mor > 900.f;
+    if (__builtin_amdgcn_ballot_w64(near_cut) != 0) {
+        const Ray1d<float> r = intersect_staged(g, o, d);
+        mor = near_cut ? r.weight * g.mass : mor;
+    }
+    out->centre = centre;
+    out->inv_sd = q * sd;
+    out->mor = mor;
+    out->far = far_radius(mor, C);
+    return centre == centre && mor >= 1.0f / 255.f && mor <= 1000.f && sd > 0.0001f; // false for NaN
 }
 
 // Per-wave candidate masks over the tile's list: bit p of a wave's mask is
@@ -307,10 +446,10 @@ __device__ __forceinline__ bool chunk_far(S centre, S inv_sd, S mor, S lo, S hi)
 // (1/255 <= mass <= 1000, or NaN) on some pixel of the wave.  A Gaussian that
 // fails it on every pixel deposits nothing (math.h:440-443) and has no
 // adjoint, so the deposit and adjoint passes of every large step skip it for
-// the whole wave; the section pass (whose depth break looks at every
-// Gaussian) does not use the masks.  The test does not depend on the large
-// step, so one walk per frame builds the masks.  Positions from kCandEntries
-// on are not tracked and always taken.
+// the whole wave.  The test does not depend on the large step: a 64-entry word
+// is built when a pass first needs one of its entries and kept in LDS (the
+// entries past the depth where the wave's rays saturate are never tested).
+// Positions from kCandEntries on are not tracked and always taken.
 constexpr int kCandWords = 64;
 constexpr uint32_t kCandEntries = 64u * kCandWords;
 
@@ -321,48 +460,113 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t v)
     return (uint64_t(hi) << 32) | lo;
 }
 
-// the candidates among staged entries [j0, j0 + 64) of the batch at list
-// offset `pos` (relative to the tile's first entry), limited to cnt entries
-__device__ __forceinline__ uint64_t candidate_word(const uint64_t* cand, uint32_t pos, int j0, int cnt)
-{
-    const int n = min(64, cnt - j0);
-    const uint64_t valid = n >= 64 ? ~uint64_t(0) : ((uint64_t(1) << n) - 1);
-    const uint32_t p = pos + uint32_t(j0);
-    if (!cand || p >= kCandEntries)
-        return valid;
-    return uniform_u64(cand[p / 64]) & valid;
-}
+// a wave's candidate words and which of them are built
+struct Candidates {
+    uint64_t* words; // LDS, this wave's
+    uint64_t built;
+};
 
-template <class S, int NT>
-__device__ __forceinline__ void build_candidates(uint64_t* cand, const MarchData<S>& md, Staged<S>* s_g, uint32_t first, uint32_t last,
+// the candidates among staged entries [j0, j0 + 64) of the batch at list
+// offset `pos` (relative to the tile's first entry), limited to `mask` (not 0)
+template <class S>
+__device__ __forceinline__ uint64_t candidate_word(Candidates& cand, uint64_t mask, uint64_t valid, uint32_t pos, int j0, const Staged<S>* s_g,
     bool inside, const S* o, const S* d)
 {
-    for (uint32_t base = first; base < last && base - first < kCandEntries; base += NT) {
+    const uint32_t p = pos + uint32_t(j0);
+    if (p >= kCandEntries)
+        return mask;
+    const uint32_t w = p / 64;
+    if (!((cand.built >> w) & 1)) {
+        uint64_t word = 0;
+        for (uint64_t todo = valid; todo != 0; todo &= todo - 1) {
+            const int jj = __builtin_ctzll(todo);
+            const Staged<S>& g = s_g[j0 + jj];
+            const Ray1d<S> r = intersect_staged(g, o, d);
+            const S mor = r.weight * g.mass;
+            if (__builtin_amdgcn_ballot_w64(inside && !(mor < S(1.0f / 255.f)) && !(mor > S(1000))) != 0)
+                word |= uint64_t(1) << jj;
+        }
+        if (lane_id() == 0)
+            cand.words[w] = word;
+        __builtin_amdgcn_wave_barrier(); // LDS operations of a wave execute in order: later reads see the word
+        cand.built |= uint64_t(1) << w;
+        return word & mask;
+    }
+    return uniform_u64(cand.words[w]) & mask;
+}
+
+// the valid entries of a 64-entry word of a batch of cnt
+__device__ __forceinline__ uint64_t valid_entries(int j0, int cnt)
+{
+    const int n = cnt - j0;
+    return n >= 64 ? ~uint64_t(0) : ((uint64_t(1) << n) - 1);
+}
+
+// entries of a word whose window meets (wlo, whi): one entry per lane
+__device__ __forceinline__ uint64_t entries_in(const Reach1d* s_win, int j0, int cnt, float wlo, float whi)
+{
+    const Reach1d w = s_win[min(j0 + int(lane_id()), cnt - 1)];
+    return __builtin_amdgcn_ballot_w64(!(w.lo > whi) && !(w.hi < wlo)) & valid_entries(j0, cnt);
+}
+
+__device__ __forceinline__ float wave_min(float v)
+{
+#pragma unroll
+    for (int k = 32; k > 0; k >>= 1)
+        v = fminf(v, __shfl_xor(v, k));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+__device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
+
+// The tile's list in LDS, NT entries at a time, for the block's passes over it
+template <class S, int NT>
+struct TileList {
+    Staged<S>* s_g;
+    Reach1d* s_win;
+    const MarchData<S>& md;
+    uint32_t first, last;
+    TileAxis axis;
+    uint32_t staged; // first entry of the staged batch; last: none
+
+    // stages the batch at `base` unless it is there already (the lists of most
+    // tiles fit one batch); every thread of the block calls it
+    __device__ __forceinline__ void stage(uint32_t base, const S* o)
+    {
+        if (staged == base)
+            return;
+        __syncthreads(); // the previous batch has been read
         const uint32_t k = base + threadIdx.x;
         if (k < last)
-            stage_gaussian(&s_g[threadIdx.x], md.point_list[k], md.means, md.inv_cov, md.rgb, md.mass, md.depths);
+            stage_gaussian(&s_g[threadIdx.x], &s_win[threadIdx.x], md.point_list[k], md, o, axis);
         __syncthreads();
-        const int cnt = int(min<uint32_t>(NT, last - base));
-        for (int j0 = 0; j0 < cnt; j0 += 64) {
-            uint64_t word = 0;
-            const int n = min(64, cnt - j0);
-            for (int jj = 0; jj < n; ++jj) {
-                const Staged<S>& g = s_g[j0 + jj];
-                bool c = false;
-                if (inside) {
-                    const Ray1d<S> r = intersect_ray(g.mu, g.A, o, d);
-                    const S mor = r.weight * g.mass;
-                    c = !(mor < S(1.0f / 255.f)) && !(mor > S(1000));
-                }
-                if (__builtin_amdgcn_ballot_w64(c) != 0)
-                    word |= uint64_t(1) << jj;
-            }
-            const uint32_t p = base - first + uint32_t(j0);
-            if (p < kCandEntries && lane_id() == 0)
-                cand[p / 64] = word;
-        }
-        __syncthreads();
+        staged = base;
     }
+};
+
+// the block's common ray direction (its first pixel's) and the largest
+// deviation of its pixels' rays from it
+template <class S, int NT>
+__device__ __forceinline__ TileAxis tile_axis(const S* d, bool inside, float* s_axis)
+{
+    if (threadIdx.x == 0) {
+        // thread 0's pixel is inside in every tile
+        s_axis[0] = float(d[0]);
+        s_axis[1] = float(d[1]);
+        s_axis[2] = float(d[2]);
+        s_axis[3] = 0.f;
+    }
+    __syncthreads();
+    TileAxis ax;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        ax.dc[k] = s_axis[k];
+    const float e0 = float(d[0]) - ax.dc[0], e1 = float(d[1]) - ax.dc[1], e2 = float(d[2]) - ax.dc[2];
+    const float dev = inside ? sqrtf(e0 * e0 + e1 * e1 + e2 * e2) : 0.f;
+    atomicMax(reinterpret_cast<uint32_t*>(s_axis + 3), __float_as_uint(dev)); // dev >= 0: ordered as its bits
+    __syncthreads();
+    ax.dev = s_axis[3];
+    return ax;
 }
 
 // A pixel's section list: in LDS for float (48 KB for a 256-pixel tile, which
@@ -397,19 +601,21 @@ __device__ __forceinline__ void attach_sections(L& sec, float* s_sec)
 // double path keeps the full walk (its depths are ordered by their float32
 // rounding only).
 template <class S>
-__device__ __forceinline__ const uint64_t* section_candidates(const MarchData<S>& md, uint32_t first, uint32_t last, const uint64_t* cand)
+__device__ __forceinline__ bool sections_by_candidates(const MarchData<S>& md, uint32_t first, uint32_t last)
 {
     if (sizeof(S) != 4 || first >= last)
-        return nullptr;
+        return false;
     const float dl = float(md.depths[md.point_list[last - 1]]);
-    return (__float_as_uint(dl) >> 31) || dl != dl ? nullptr : cand;
+    return !((__float_as_uint(dl) >> 31) || dl != dl);
 }
 
-// pass 1: sample sections from the tile's Gaussians (vol_marcher_forward.cu:350-403);
-// cand (may be null) as section_candidates allows
+// pass 1: sample sections from the tile's Gaussians (vol_marcher_forward.cu:350-403).
+// by_cand: visit only the candidates whose window meets the part of the ray
+// between the step's start and the list's end (a section outside it is not
+// put; the depth break moves as for the candidates)
 template <class S, int NT, class L>
-__device__ __forceinline__ void build_sections(L& sec, const MarchData<S>& md, Staged<S>* s_g, uint32_t first, uint32_t last, bool skip,
-    const S* o, const S* d, const MarchControl& ctl, const uint64_t* cand)
+__device__ __forceinline__ void build_sections(L& sec, TileList<S, NT>& tl, bool skip, bool inside, const S* o, const S* d, const MarchControl& ctl,
+    bool by_cand, Candidates& cand)
 {
     if (ctl.n_frozen > 0) {
         for (int k = 0; k < ctl.n_frozen; ++k)
@@ -417,106 +623,163 @@ __device__ __forceinline__ void build_sections(L& sec, const MarchData<S>& md, S
         return;
     }
     bool done1 = skip;
-    for (uint32_t base = first; base < last; base += NT) {
+    const float wlo = by_cand ? wave_min(skip ? __builtin_inff() : float(sec.start_)) : 0.f;
+    for (uint32_t base = tl.first; base < tl.last; base += NT) {
         if (__syncthreads_count(!done1) == 0)
             break;
-        const uint32_t k = base + threadIdx.x;
-        if (k < last)
-            stage_gaussian(&s_g[threadIdx.x], md.point_list[k], md.means, md.inv_cov, md.rgb, md.mass, md.depths);
-        __syncthreads();
+        tl.stage(base, o);
         // the batch's first Gaussian is its shallowest: past it, every later
         // one is beyond the list's end too (the break the full walk takes)
-        if (!done1 && sec.end_ < s_g[0].depth)
+        if (!done1 && sec.end_ < tl.s_g[0].depth)
             done1 = true;
-        if (done1)
-            continue;
-        const int cnt = int(min<uint32_t>(NT, last - base));
-        for (int j0 = 0; j0 < cnt && !done1; j0 += 64)
-        for (uint64_t word = candidate_word(cand, base - first, j0, cnt); word != 0; word &= word - 1) {
-            const Staged<S>& g = s_g[j0 + __builtin_ctzll(word)];
-            const Ray1d<S> r = intersect_ray(g.mu, g.A, o, d);
-            const S sd = sqrt_rn(r.var);
-            if (sec.end_ < g.depth) {
-                done1 = true;
+        const int cnt = int(min<uint32_t>(NT, tl.last - base));
+        for (int j0 = 0; j0 < cnt; j0 += 64) {
+            if (__builtin_amdgcn_ballot_w64(!done1) == 0)
                 break;
+            uint64_t word = valid_entries(j0, cnt);
+            if (by_cand) {
+                const uint64_t valid = word;
+                word = entries_in(tl.s_win, j0, cnt, wlo, wave_max(done1 ? -__builtin_inff() : float(sec.end_)));
+                if (word != 0)
+                    word = candidate_word(cand, word, valid, base - tl.first, j0, tl.s_g, inside, o, d);
             }
-            const S mor = r.weight * g.mass;
-            if (mor <= S(1.0f / 255.f) || mor > S(1000))
-                continue;
-            if (r.var <= 0)
-                continue;
-            if (r.centre != r.centre)
-                continue;
-            const S half = sd * S(kRelevanceSigma);
-            sec.put({ r.centre - half, r.centre + half, (sd * S(kRelevanceSigma) * S(2)) / S(kStepsPerGaussian - 1) });
+            for (; word != 0; word &= word - 1) {
+                if (__builtin_amdgcn_ballot_w64(!done1) == 0)
+                    break;
+                const Staged<S>& g = tl.s_g[j0 + __builtin_ctzll(word)];
+                const Ray1d<S> r = intersect_staged(g, o, d);
+                if (sec.end_ < g.depth)
+                    done1 = true;
+                if (done1)
+                    continue;
+                const S mor = r.weight * g.mass;
+                if (mor <= S(1.0f / 255.f) || mor > S(1000))
+                    continue;
+                if (r.var <= 0)
+                    continue;
+                if (r.centre != r.centre)
+                    continue;
+                const S sd = sqrt_rn(r.var);
+                const S half = sd * S(kRelevanceSigma);
+                sec.put({ r.centre - half, r.centre + half, (sd * S(kRelevanceSigma) * S(2)) / S(kStepsPerGaussian - 1) });
+            }
         }
     }
-    __syncthreads(); // LDS reuse by the next pass
 }
 
-// pass 2 for one chunk of bins [bb[0], bb[kk]] (bb[k] = bb[kk] for k > kk, so
-// bb[CB] is the chunk's end): every Gaussian of the tile
+// A lane's share of one Gaussian in the chunk [bb[0], bb[CB]]: whether it can
+// deposit there at all.  The mass within the step's bins must reach 1e-4
+// (math.h:455-460): with at least 1/255 on the ray that is certain when the
+// centre lies in the bins, 0.1 sd from one of their ends (0.04 of the mass);
+// otherwise the cdf at both ends decides.
+template <class S>
+__device__ __forceinline__ bool deposits_in(const RayGauss<S>& r, bool pass, S b_first, S b_last, S lo, S hi)
+{
+    bool need = pass && r.centre + r.far > lo && r.centre - r.far < hi;
+    const S zl = (b_last - r.centre) * r.inv_sd, zf = (b_first - r.centre) * r.inv_sd;
+    const bool sure = (zl > S(0.1) && zf <= S(0)) || (zl >= S(0) && zf < S(-0.1));
+    if (__builtin_amdgcn_ballot_w64(need && !sure) != 0) {
+        const S in_bins = r.mor * (cdf_inv_sd(r.centre, r.inv_sd, b_last) - cdf_inv_sd(r.centre, r.inv_sd, b_first));
+        need = need && (sure || !(in_bins < S(0.0001f)));
+    }
+    return need;
+}
+
+// f(0), f(1), ... f(N - 1) with compile-time arguments: the per-bin arrays a
+// chunk keeps in registers are only ever indexed by constants (a loop that the
+// compiler unrolls late leaves them one register tuple, copied at every branch)
+template <class F, int... I>
+__device__ __forceinline__ void static_for_each(F&& f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I> {}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    static_for_each(f, std::make_integer_sequence<int, N> {});
+}
+
+// Bins per group: a wave evaluates the groups of a chunk that some lane's
+// Gaussian reaches (far_radius), the others hold less than 1e-5 per bin
+constexpr int kBinGroup = 8;
+
+// pass 2 for one chunk of bins [bb[0], bb[CB]] (borders past the chunk's last
+// bin repeat its end, so the bins there are empty): every Gaussian of the tile
 // deposits its ray mass (math.h:430-468), in tile order; pixels with `stopped`
-// take part in the block's staging only; cand (may be null) skips the
-// Gaussians no pixel of the wave can take
+// take part in the block's staging only.  Only the entries whose window meets
+// the wave's part of the chunk are visited, and only the wave's candidates of
+// them.  Bound by VALU issue.  Visiting every candidate in every chunk, with
+// the exact restriction each time and all of a chunk's bins once one pixel's
+// Gaussian reached it, the forward took 52.0 ms on 200k Gaussians at 1024^2 and
+// forward + backward 56.3 ms on 60k at 491x373; with windows, groups and the
+// short restriction 17.4 and 22.3 ms.
 template <class S, int NT, int CB>
-__device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 1], int kk, bool stopped, const MarchData<S>& md,
-    Staged<S>* s_g, uint32_t first, uint32_t last, const S* o, const S* d, S b_first, S b_last, const uint64_t* cand)
+__device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 1], bool stopped, TileList<S, NT>& tl, bool inside,
+    const S* o, const S* d, S b_first, S b_last, Candidates& cand)
 {
 #pragma unroll
     for (int k = 0; k < CB; ++k)
         bins[k][0] = bins[k][1] = bins[k][2] = bins[k][3] = 0;
-    for (uint32_t base = first; base < last; base += NT) {
-        if (__syncthreads_count(!stopped) == 0)
-            break;
-        const uint32_t k = base + threadIdx.x;
-        if (k < last)
-            stage_gaussian(&s_g[threadIdx.x], md.point_list[k], md.means, md.inv_cov, md.rgb, md.mass, md.depths);
-        __syncthreads();
-        if (!stopped) {
-            const int cnt = int(min<uint32_t>(NT, last - base));
-            for (int j0 = 0; j0 < cnt; j0 += 64)
-            for (uint64_t word = candidate_word(cand, base - first, j0, cnt); word != 0; word &= word - 1) {
-                const int j = j0 + __builtin_ctzll(word);
-                const Staged<S>& g = s_g[j];
-                Ray1d<S> r;
-                S sd, inv_sd, mor;
-                if (!ray_gaussian(g, o, d, b_first, b_last, &r, &sd, &inv_sd, &mor))
+    const uint32_t end = __syncthreads_count(!stopped) == 0 ? tl.first : tl.last;
+    const float inf = __builtin_inff();
+    // no entry meets the empty window of a wave whose pixels have all stopped
+    const float wlo = wave_min(stopped ? inf : float(bb[0])), whi = wave_max(stopped ? -inf : float(bb[CB]));
+    for (uint32_t base = tl.first; base < end; base += NT) {
+        tl.stage(base, o);
+        const int cnt = int(min<uint32_t>(NT, tl.last - base));
+        for (int j0 = 0; j0 < cnt; j0 += 64) {
+            uint64_t word = entries_in(tl.s_win, j0, cnt, wlo, whi);
+            if (word != 0)
+                word = candidate_word(cand, word, valid_entries(j0, cnt), base - tl.first, j0, tl.s_g, inside, o, d);
+            for (; word != 0; word &= word - 1) {
+                const Staged<S>& g = tl.s_g[j0 + __builtin_ctzll(word)];
+                RayGauss<S> r;
+                const bool pass = ray_gaussian(g, o, d, &r) && !stopped;
+                if (__builtin_amdgcn_ballot_w64(pass && r.centre + r.far > bb[0] && r.centre - r.far < bb[CB]) == 0)
                     continue;
-                if (chunk_far(r.centre, inv_sd, mor, bb[0], bb[CB]))
-                    continue;
-                const S in_bins = mor * (cdf_inv_sd(r.centre, inv_sd, b_last) - cdf_inv_sd(r.centre, inv_sd, b_first));
-                if (in_bins < S(0.0001f))
-                    continue;
-                S c0 = cdf_inv_sd(r.centre, inv_sd, bb[0]);
-#pragma unroll
-                for (int k = 0; k < CB; ++k) {
-                    if (k < kk) {
-                        const S c1 = cdf_inv_sd(r.centre, inv_sd, bb[k + 1]);
-                        const S m = dmax(S(0), (c1 - c0) * mor);
-                        c0 = c1;
-                        if (!(m < S(0.00001f))) {
-                            bins[k][0] = dfma(g.rgb[0], m, bins[k][0]);
-                            bins[k][1] = dfma(g.rgb[1], m, bins[k][1]);
-                            bins[k][2] = dfma(g.rgb[2], m, bins[k][2]);
-                            bins[k][3] += m;
-                        }
+                const bool need = deposits_in(r, pass, b_first, b_last, bb[0], bb[CB]);
+                const S lo = need ? r.centre - r.far : S(inf), hi = need ? r.centre + r.far : S(-inf);
+                const S mor = need ? r.mor : S(0);
+                const CdfScale<S> cs = cdf_scale(r.inv_sd);
+                S c0 = 0;
+                bool have = false;
+                static_for<CB / kBinGroup>([&](auto group) {
+                    constexpr int k0 = group * kBinGroup;
+                    // bins past the chunk's end are empty (bb repeats), so a group needs no bound
+                    if (__builtin_amdgcn_ballot_w64(hi > bb[k0] && lo < bb[k0 + kBinGroup]) == 0) {
+                        have = false;
+                        return;
                     }
-                }
+                    if (!have)
+                        c0 = cdf_step(r.centre, cs, bb[k0]);
+                    have = true;
+                    static_for<kBinGroup>([&](auto q) {
+                        constexpr int k = k0 + q;
+                        const S c1 = cdf_step(r.centre, cs, bb[k + 1]);
+                        const S mass = (c1 - c0) * mor;
+                        c0 = c1;
+                        const S m = mass >= S(0.00001f) ? mass : S(0); // NaN is not kept
+                        bins[k][0] = dfma(g.rgb[0], m, bins[k][0]);
+                        bins[k][1] = dfma(g.rgb[1], m, bins[k][1]);
+                        bins[k][2] = dfma(g.rgb[2], m, bins[k][2]);
+                        bins[k][3] += m;
+                    });
+                });
             }
         }
     }
-    __syncthreads();
 }
 
 template <class S, int TW, int TH, int CB>
-__global__ __launch_bounds__(TW* TH) void k_march_forward(MarchData<S> md, DevCamera<S> cam, MarchControl ctl, S* __restrict__ framebuffer,
+__global__ __launch_bounds__(TW* TH, sizeof(S) == 4 ? 2 : 1) void k_march_forward(MarchData<S> md, DevCamera<S> cam, MarchControl ctl, S* __restrict__ framebuffer,
     S* __restrict__ remaining, Replay<S> rp)
 {
     constexpr int NT = TW * TH;
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
+    __shared__ Reach1d s_win[NT];
     __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ float s_axis[4];
     __shared__ float s_sec[kSectionLdsFloats<S, NT>];
     if (md.n_pairs && *md.n_pairs == 0)
         return; // no visible Gaussian: the framebuffer stays as the caller cleared it
@@ -528,9 +791,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward(MarchData<S> md, DevCa
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    uint64_t* cand = s_cand[threadIdx.x / 64];
-    build_candidates<S, NT>(cand, md, s_g, first, last, inside, o, d);
-    const uint64_t* sec_cand = section_candidates(md, first, last, cand);
+    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    const bool by_cand = sections_by_candidates(md, first, last);
     S C0 = 0, C1 = 0, C2 = 0, T = 1, start = 0;
     bool done = !inside;
     int steps = 0;
@@ -538,7 +801,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward(MarchData<S> md, DevCa
     attach_sections<S>(sec, s_sec);
     while (true) {
         sec.reset(start);
-        build_sections<S, NT>(sec, md, s_g, first, last, done, o, d, ctl, sec_cand);
+        build_sections<S, NT>(sec, tl, done, inside, o, d, ctl, by_cand, cand);
         // border range of this large step
         BorderWalk<S, kSections> walk;
         walk.begin(sec);
@@ -562,79 +825,29 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward(MarchData<S> md, DevCa
             for (int k = 1; k <= CB; ++k)
                 bb[k] = (k <= kk) ? walk.next(sec) : bb[k - 1];
             S bins[CB][4];
-#pragma unroll
-            for (int k = 0; k < CB; ++k)
-                bins[k][0] = bins[k][1] = bins[k][2] = bins[k][3] = 0;
-            // pass 2, as fill_chunk (kept inline here: as a call, the compiler
-            // allocated this kernel 256 VGPRs and 79 AGPRs instead of 215)
-            for (uint32_t base = first; base < last; base += NT) {
-                if (__syncthreads_count(!stopped) == 0)
-                    break;
-                const uint32_t k = base + threadIdx.x;
-                if (k < last)
-                    stage_gaussian(&s_g[threadIdx.x], md.point_list[k], md.means, md.inv_cov, md.rgb, md.mass, md.depths);
-                __syncthreads();
-                if (!stopped) {
-                    const int cnt = int(min<uint32_t>(NT, last - base));
-                    for (int j0 = 0; j0 < cnt; j0 += 64)
-                    for (uint64_t word = candidate_word(cand, base - first, j0, cnt); word != 0; word &= word - 1) {
-                        const int j = j0 + __builtin_ctzll(word);
-                        const Staged<S>& g = s_g[j];
-                        Ray1d<S> r;
-                        S sd, inv_sd, mor;
-                        if (!ray_gaussian(g, o, d, b_first, b_last, &r, &sd, &inv_sd, &mor))
-                            continue;
-                        if (chunk_far(r.centre, inv_sd, mor, bb[0], bb[CB]))
-                            continue;
-                        const S in_bins = mor * (cdf_inv_sd(r.centre, inv_sd, b_last) - cdf_inv_sd(r.centre, inv_sd, b_first));
-                        if (in_bins < S(0.0001f))
-                            continue;
-                        S c0 = cdf_inv_sd(r.centre, inv_sd, bb[0]);
-#pragma unroll
-                        for (int k = 0; k < CB; ++k) {
-                            if (k < kk) {
-                                const S c1 = cdf_inv_sd(r.centre, inv_sd, bb[k + 1]);
-                                const S m = dmax(S(0), (c1 - c0) * mor);
-                                c0 = c1;
-                                if (!(m < S(0.00001f))) {
-                                    bins[k][0] = dfma(g.rgb[0], m, bins[k][0]);
-                                    bins[k][1] = dfma(g.rgb[1], m, bins[k][1]);
-                                    bins[k][2] = dfma(g.rgb[2], m, bins[k][2]);
-                                    bins[k][3] += m;
-                                }
-                            }
-                        }
-                    }
-                }
-            }
-            __syncthreads();
+            fill_chunk<S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
             if (rec) {
                 S* rb = rec + (int64_t(ch * CB) * NT + threadIdx.x) * 4;
                 S* rd = rec + int64_t(NT) * 4 * kBins + int64_t(ch * CB) * NT + threadIdx.x;
-#pragma unroll
-                for (int k = 0; k < CB; ++k) {
+                static_for<CB>([&](auto k) {
                     if (k < kk) {
-                        store4(rb + int64_t(k) * NT * 4, bins[k][0], bins[k][1], bins[k][2], bins[k][3]);
+                        store4(rb + int64_t(k) * NT * 4, detached(bins[k][0]), detached(bins[k][1]), detached(bins[k][2]), detached(bins[k][3]));
                         rd[int64_t(k) * NT] = bb[k];
                     }
-                }
+                });
                 if (ch == NCH - 1)
                     rd[int64_t(kk) * NT] = bb[CB];
             }
-            if (!stopped) {
-#pragma unroll
-                for (int k = 0; k < CB; ++k) {
-                    if (k < kk && !stopped) {
-                        const S tk = dexp(-bins[k][3]);
-                        C0 += bins[k][0] * T;
-                        C1 += bins[k][1] * T;
-                        C2 += bins[k][2] * T;
-                        T *= tk;
-                        if (T < S(1. / 255.))
-                            stopped = true;
-                    }
-                }
-            }
+            // blend, branch-free (branches around the bins cost copies of them):
+            // a stopped pixel's weight is 0, bins past the chunk's end are empty
+            static_for<CB>([&](auto k) {
+                const S w = stopped ? S(0) : T;
+                C0 += bins[k][0] * w;
+                C1 += bins[k][1] * w;
+                C2 += bins[k][2] * w;
+                T = stopped ? T : T * dexp(-bins[k][3]);
+                stopped = stopped || T < S(1. / 255.);
+            });
         }
         ++steps;
         done = done || sec.size == 0 || T < S(1.f / 255.f) || (ctl.max_large_steps > 0 && steps >= ctl.max_large_steps);
@@ -671,7 +884,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     constexpr int NT = TW * TH;
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
+    __shared__ Reach1d s_win[NT];
     __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ float s_axis[4];
     __shared__ float s_sec[kSectionLdsFloats<S, NT>];
     if (md.n_pairs && *md.n_pairs == 0)
         return; // no visible Gaussian: the framebuffer stays as the caller cleared it
@@ -683,9 +898,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    uint64_t* cand = s_cand[threadIdx.x / 64];
-    build_candidates<S, NT>(cand, md, s_g, first, last, inside, o, d);
-    const uint64_t* sec_cand = section_candidates(md, first, last, cand);
+    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    const bool by_cand = sections_by_candidates(md, first, last);
     const bool bins_mode = ctl.render_mode == 1;
     const int target = int(min(unsigned(ctl.debug_bin), unsigned(kBins - 1)));
     const S max_depth = S(ctl.max_depth);
@@ -696,7 +911,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     attach_sections<S>(sec, s_sec);
     while (true) {
         sec.reset(start);
-        build_sections<S, NT>(sec, md, s_g, first, last, done, o, d, ctl, sec_cand);
+        build_sections<S, NT>(sec, tl, done, inside, o, d, ctl, by_cand, cand);
         BorderWalk<S, kSections> walk;
         walk.begin(sec);
         const S b_first = walk.prev;
@@ -717,7 +932,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
             if (bins_mode && (target < ch * CB || target >= ch * CB + kk))
                 continue; // only the chunk holding the shown bin
             S bins[CB][4];
-            fill_chunk<S, NT, CB>(bins, bb, kk, done, md, s_g, first, last, o, d, b_first, b_last, cand);
+            fill_chunk<S, NT, CB>(bins, bb, done, tl, inside, o, d, b_first, b_last, cand);
 #pragma unroll
             for (int k = 0; k < CB; ++k) {
                 if (k < kk) {
@@ -781,12 +996,11 @@ __device__ __forceinline__ S wave_total(S v)
 // Blend adjoint of one chunk (grad/math.h:529-557), front to back from the
 // running transmittance T and remaining colour Cr: bin k's gradient is
 // dL/d(rgb mass) = Tk[k] dL/dC and dL/d(mass) = Gk[k].  Bins past the chunk
-// end or after the pixel stopped get zero; na = the bins before the stop.
+// end or after the pixel stopped get zero.
 template <class S, int CB>
 __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bool& stopped, S& T, S* Cr, S Tf, S gT, const S* gC, S (&Tk)[CB],
-    S (&Gk)[CB], int& na)
+    S (&Gk)[CB])
 {
-    na = 0;
 #pragma unroll
     for (int k = 0; k < CB; ++k) {
         Tk[k] = 0;
@@ -801,7 +1015,6 @@ __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bo
             Tk[k] = T;
             Gk[k] = -g_tk * tk;
             T *= tk;
-            na = k + 1;
             if (T < S(1. / 255.))
                 stopped = true;
         }
@@ -813,103 +1026,108 @@ __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bo
 // Gaussian (mass 1, rgb 3, means 3, inverse covariance 6).  Per bin the
 // gradient of the bin's mass is Tk (dL/dC . rgb) + Gk; the rgb gradient is
 // dL/dC times the sum of Tk mass, and the centre and inverse-sd gradients
-// collect the cdf derivatives at both borders of every bin.
+// collect the cdf derivatives at both borders of every bin.  Entries, groups of
+// bins and kept bins are fill_chunk's; Tk = Gk = 0 past the pixel's stop.
 template <class S, int NT, int CB>
-__device__ __forceinline__ void adjoint_chunk(const MarchData<S>& md, Staged<S>* s_g, const uint64_t* cand, uint32_t first, uint32_t last,
-    bool active, const S* o, const S* d, const S (&bb)[CB + 1], int kk, int na, S b_first, S b_last, const S (&Tk)[CB], const S (&Gk)[CB],
-    const S* gC, S* __restrict__ render_grads)
+__device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& cand, bool active, bool inside, const S* o, const S* d,
+    const S (&bb)[CB + 1], S b_first, S b_last, const S (&Tk)[CB], const S (&Gk)[CB], const S* gC, S* __restrict__ render_grads)
 {
-    for (uint32_t base = first; base < last; base += NT) {
-        if (__syncthreads_count(active) == 0)
-            break;
-        const uint32_t k = base + threadIdx.x;
-        if (k < last)
-            stage_gaussian(&s_g[threadIdx.x], md.point_list[k], md.means, md.inv_cov, md.rgb, md.mass, md.depths);
-        __syncthreads();
-        const int cnt = int(min<uint32_t>(NT, last - base));
-        for (int j0 = 0; j0 < cnt; j0 += 64)
-        for (uint64_t word = candidate_word(cand, base - first, j0, cnt); word != 0; word &= word - 1) {
-            const int j = j0 + __builtin_ctzll(word);
-            const Staged<S>& g = s_g[j];
-            bool contrib = false;
-            S g_mor = 0, s_tm = 0, s_c = 0, s_i = 0;
-            Ray1d<S> r;
-            S sd = 1, inv_sd = 1, mor = 0;
-            if (active && ray_gaussian(g, o, d, b_first, b_last, &r, &sd, &inv_sd, &mor) && !chunk_far(r.centre, inv_sd, mor, bb[0], bb[CB])) {
-                const S in_bins = mor * (cdf_inv_sd(r.centre, inv_sd, b_last) - cdf_inv_sd(r.centre, inv_sd, b_first));
-                if (!(in_bins < S(0.0001f))) {
-                    const S gcr = (gC[0] * g.rgb[0] + gC[1] * g.rgb[1]) + gC[2] * g.rgb[2];
-                    S c0, p0;
-                    cdf_pdf_inv_sd(r.centre, inv_sd, bb[0], &c0, &p0);
-                    S q0 = (bb[0] - r.centre) * p0;
-#pragma unroll
-                    for (int kq = 0; kq < CB; ++kq) {
-                        if (kq < na) {
-                            S c1, p1;
-                            cdf_pdf_inv_sd(r.centre, inv_sd, bb[kq + 1], &c1, &p1);
-                            const S q1 = (bb[kq + 1] - r.centre) * p1;
-                            const S delta = c1 - c0;
-                            const S m = delta * mor;
-                            // the bin's mass max(0, m) is kept from 1e-5 on (NaN is not)
-                            if (m >= S(0.00001f)) {
-                                contrib = true;
-                                s_tm = dfma(Tk[kq], m, s_tm);
-                                const S g_m = dfma(Tk[kq], gcr, Gk[kq]);
-                                g_mor = dfma(g_m, delta, g_mor);
-                                const S g_delta = g_m * mor;
-                                s_c = dfma(g_delta, p1 - p0, s_c);
-                                s_i = dfma(g_delta, q1 - q0, s_i);
-                            }
-                            c0 = c1;
-                            p0 = p1;
-                            q0 = q1;
-                        }
+    const uint32_t end = __syncthreads_count(active) == 0 ? tl.first : tl.last;
+    const float inf = __builtin_inff();
+    const float wlo = wave_min(active ? float(bb[0]) : inf), whi = wave_max(active ? float(bb[CB]) : -inf);
+    for (uint32_t base = tl.first; base < end; base += NT) {
+        tl.stage(base, o);
+        const int cnt = int(min<uint32_t>(NT, tl.last - base));
+        for (int j0 = 0; j0 < cnt; j0 += 64) {
+            uint64_t word = entries_in(tl.s_win, j0, cnt, wlo, whi);
+            if (word != 0)
+                word = candidate_word(cand, word, valid_entries(j0, cnt), base - tl.first, j0, tl.s_g, inside, o, d);
+            for (; word != 0; word &= word - 1) {
+                const Staged<S>& g = tl.s_g[j0 + __builtin_ctzll(word)];
+                RayGauss<S> r;
+                const bool pass = ray_gaussian(g, o, d, &r) && active;
+                if (__builtin_amdgcn_ballot_w64(pass && r.centre + r.far > bb[0] && r.centre - r.far < bb[CB]) == 0)
+                    continue;
+                const bool need = deposits_in(r, pass, b_first, b_last, bb[0], bb[CB]);
+                const S lo = need ? r.centre - r.far : S(inf), hi = need ? r.centre + r.far : S(-inf);
+                const S mor = need ? r.mor : S(0);
+                const CdfScale<S> cs = cdf_scale(r.inv_sd);
+                const S gcr = dfma(gC[2], g.rgb[2], dfma(gC[1], g.rgb[1], gC[0] * g.rgb[0]));
+                S c0 = 0, p0 = 0, q0 = 0;
+                S s_d = 0, s_tm = 0, s_c = 0, s_i = 0;
+                bool have = false, any = false;
+                static_for<CB / kBinGroup>([&](auto group) {
+                    constexpr int k0 = group * kBinGroup;
+                    if (__builtin_amdgcn_ballot_w64(hi > bb[k0] && lo < bb[k0 + kBinGroup]) == 0) {
+                        have = false;
+                        return;
                     }
-                }
-            }
-            if (__ballot(contrib) == 0)
-                continue;
-            S gr[13];
-#pragma unroll
-            for (int q = 0; q < 13; ++q)
-                gr[q] = 0;
-            if (contrib) {
-                const S g_w = g_mor * g.mass;
-                gr[0] = g_mor * r.weight;
-                gr[1] = gC[0] * s_tm;
-                gr[2] = gC[1] * s_tm;
-                gr[3] = gC[2] * s_tm;
-                // d cdf / d centre = -inv_sd pdf, d cdf / d inv_sd = (x - centre) pdf
-                const S g_centre = -inv_sd * s_c;
-                const S g_sd = -s_i / (sd * sd);
-                const S g_var = g_sd / (S(2) * sd);
-                intersect_ray_grad(g.mu, g.A, o, d, g_w, g_centre, g_var, gr + 4, gr + 7);
-            }
-            S* dst = render_grads + int64_t(g.id) * 13;
-            if constexpr (sizeof(S) == 4) {
-                // two transposing reductions: lane 8m holds values kSum8Order[m] and 8 + kSum8Order[m]
-                const float ta = wave_sum8(gr[0], gr[1], gr[2], gr[3], gr[4], gr[5], gr[6], gr[7]);
-                const float tb = wave_sum8(gr[8], gr[9], gr[10], gr[11], gr[12], 0.f, 0.f, 0.f);
-                const unsigned ln = lane_id();
-                if ((ln & 7u) == 0) {
-                    const int q = kSum8Order[ln >> 3];
-                    unsafeAtomicAdd(dst + q, ta);
-                    if (q < 5)
-                        unsafeAtomicAdd(dst + 8 + q, tb);
-                }
-            } else {
+                    if (!have)
+                        cdf_grad_step(r.centre, cs, bb[k0], &c0, &p0, &q0);
+                    have = any = true;
+                    static_for<kBinGroup>([&](auto bin) {
+                        constexpr int k = k0 + bin;
+                        S c1, p1, q1;
+                        cdf_grad_step(r.centre, cs, bb[k + 1], &c1, &p1, &q1);
+                        const S delta = c1 - c0;
+                        // the bin's mass max(0, m) is kept from 1e-5 on (NaN is not)
+                        const bool kept = delta * mor >= S(0.00001f);
+                        const S tk = kept ? Tk[k] : S(0);
+                        const S g_m = dfma(tk, gcr, kept ? Gk[k] : S(0));
+                        s_tm = dfma(tk, delta, s_tm);
+                        s_d = dfma(g_m, delta, s_d);
+                        s_c = dfma(g_m, p1 - p0, s_c);
+                        s_i = dfma(g_m, q1 - q0, s_i);
+                        c0 = c1;
+                        p0 = p1;
+                        q0 = q1;
+                    });
+                });
+                if (!any)
+                    continue;
+                S gr[13];
 #pragma unroll
                 for (int q = 0; q < 13; ++q)
-                    gr[q] = wave_total(gr[q]);
-                if (lane_id() == 63) {
+                    gr[q] = 0;
+                if (need) {
+                    S fp, fq;
+                    cdf_grad_scale(cs, r.inv_sd, &fp, &fq);
+                    // d L / d mass on the ray = s_d; weight = mor / mass
+                    gr[0] = fast_div(s_d * mor, g.mass);
+                    s_tm *= mor;
+                    gr[1] = gC[0] * s_tm;
+                    gr[2] = gC[1] * s_tm;
+                    gr[3] = gC[2] * s_tm;
+                    // d cdf / d centre = -inv_sd pdf; d cdf / d var = -z pdf / (2 var)
+                    const S g_centre = -(s_c * mor) * fp;
+                    const S g_var = -(s_i * mor) * fq * (S(0.5) * r.inv_sd * r.inv_sd);
+                    intersect_ray_grad(g.mu, g.A, g.m, o, d, r.centre, s_d * mor, g_centre, g_var, gr + 4, gr + 7);
+                }
+                S* dst = render_grads + int64_t(g.id) * 13;
+                if constexpr (sizeof(S) == 4) {
+                    // two transposing reductions: lane 8m holds values kSum8Order[m] and 8 + kSum8Order[m]
+                    const float ta = wave_sum8(gr[0], gr[1], gr[2], gr[3], gr[4], gr[5], gr[6], gr[7]);
+                    const float tb = wave_sum8(gr[8], gr[9], gr[10], gr[11], gr[12], 0.f, 0.f, 0.f);
+                    const unsigned ln = lane_id();
+                    if ((ln & 7u) == 0) {
+                        const int q = kSum8Order[ln >> 3];
+                        unsafeAtomicAdd(dst + q, ta);
+                        if (q < 5)
+                            unsafeAtomicAdd(dst + 8 + q, tb);
+                    }
+                } else {
 #pragma unroll
                     for (int q = 0; q < 13; ++q)
-                        unsafeAtomicAdd(dst + q, gr[q]);
+                        gr[q] = wave_total(gr[q]);
+                    if (lane_id() == 63) {
+#pragma unroll
+                        for (int q = 0; q < 13; ++q)
+                            unsafeAtomicAdd(dst + q, gr[q]);
+                    }
                 }
             }
         }
     }
-    __syncthreads();
 }
 
 // per-pixel state of the backward: dL/dC, the remaining colour C - T_final bg,
@@ -948,7 +1166,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
     constexpr int NT = TW * TH;
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
+    __shared__ Reach1d s_win[NT];
     __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ float s_axis[4];
     __shared__ float s_sec[kSectionLdsFloats<S, NT>];
     const int tile = xcd_tile_m(blockIdx.x, md.n_tiles);
     if (rp.tile_steps && rp.tile_steps[tile] <= uint32_t(rp.steps))
@@ -960,9 +1180,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    uint64_t* cand = s_cand[threadIdx.x / 64];
-    build_candidates<S, NT>(cand, md, s_g, first, last, inside, o, d);
-    const uint64_t* sec_cand = section_candidates(md, first, last, cand);
+    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    const bool by_cand = sections_by_candidates(md, first, last);
     PixelAdjoint<S> pa = load_pixel_adjoint(cam, inside, px, py, framebuffer, remaining, grad_fb);
     S T = 1, start = 0;
     bool done = !inside;
@@ -971,7 +1191,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
     attach_sections<S>(sec, s_sec);
     while (true) {
         sec.reset(start);
-        build_sections<S, NT>(sec, md, s_g, first, last, done, o, d, ctl, sec_cand);
+        build_sections<S, NT>(sec, tl, done, inside, o, d, ctl, by_cand, cand);
         BorderWalk<S, kSections> walk;
         walk.begin(sec);
         const S b_first = walk.prev;
@@ -990,15 +1210,14 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
             for (int k = 1; k <= CB; ++k)
                 bb[k] = (k <= kk) ? walk.next(sec) : bb[k - 1];
             S Tk[CB], Gk[CB];
-            int na;
             const bool active = !stopped;
             {
                 S bins[CB][4];
                 // pass 2 (identical to the forward)
-                fill_chunk<S, NT, CB>(bins, bb, kk, stopped, md, s_g, first, last, o, d, b_first, b_last, cand);
-                blend_adjoint<S, CB>(bins, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk, na);
+                fill_chunk<S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
+                blend_adjoint<S, CB>(bins, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
             }
-            adjoint_chunk<S, NT, CB>(md, s_g, cand, first, last, active, o, d, bb, kk, na, b_first, b_last, Tk, Gk, pa.gC, render_grads);
+            adjoint_chunk<S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
         }
         ++steps;
         done = done || sec.size == 0 || T < S(1.f / 255.f) || (ctl.max_large_steps > 0 && steps >= ctl.max_large_steps);
@@ -1020,7 +1239,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
     constexpr int NT = TW * TH;
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
+    __shared__ Reach1d s_win[NT];
     __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ float s_axis[4];
     const int tile = xcd_tile_m(blockIdx.x, md.n_tiles);
     const uint32_t n_steps = rp.tile_steps[tile];
     if (n_steps > uint32_t(rp.steps))
@@ -1032,8 +1253,8 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    uint64_t* cand = s_cand[threadIdx.x / 64];
-    build_candidates<S, NT>(cand, md, s_g, first, last, inside, o, d);
+    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
     PixelAdjoint<S> pa = load_pixel_adjoint(cam, inside, px, py, framebuffer, remaining, grad_fb);
     S T = 1;
     for (uint32_t step = 0; step < n_steps; ++step) {
@@ -1049,7 +1270,6 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
             for (int k = 0; k <= CB; ++k)
                 bb[k] = rd[int64_t(ch * CB + min(k, kk)) * NT];
             S Tk[CB], Gk[CB];
-            int na = 0;
             const bool active = !stopped;
             if (active) {
                 S bins[CB][4];
@@ -1061,13 +1281,13 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
                     else
                         bins[k][0] = bins[k][1] = bins[k][2] = bins[k][3] = 0;
                 }
-                blend_adjoint<S, CB>(bins, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk, na);
+                blend_adjoint<S, CB>(bins, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
             } else {
 #pragma unroll
                 for (int k = 0; k < CB; ++k)
                     Tk[k] = Gk[k] = 0;
             }
-            adjoint_chunk<S, NT, CB>(md, s_g, cand, first, last, active, o, d, bb, kk, na, b_first, b_last, Tk, Gk, pa.gC, render_grads);
+            adjoint_chunk<S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
         }
     }
 }

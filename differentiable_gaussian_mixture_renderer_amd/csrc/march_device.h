@@ -206,19 +206,29 @@ __device__ __forceinline__ float derf<float>(float v) { return erff(v); }
 template <>
 __device__ __forceinline__ double derf<double>(double v) { return erf(v); }
 
+template <class S>
+__device__ __forceinline__ S sym3_det(const S* A)
+{
+    return A[0] * (A[3] * A[5] - A[4] * A[4]) - A[1] * (A[1] * A[5] - A[4] * A[2]) + A[2] * (A[1] * A[4] - A[3] * A[2]);
+}
+
+// normalisation of the 3D Gaussian with inverse covariance A
+template <class S>
+__device__ __forceinline__ S ray_norm3(S detA) { return sqrt_rn(detA) / S(15.749609945722419); } // sqrt((2 pi)^3)
+
 // restriction of N(mu, A^-1) to o + t d (stroke::gaussian::intersect_with_ray_inv_C
 // as used at math.h:436): variance 1/(d^T A d), centre d^T A (mu - o) / (d^T A d),
-// weight = integral of the normalised density along the ray
+// weight = integral of the normalised density along the ray.  m = mu - o and
+// norm3 = ray_norm3(det A) do not depend on the ray.
 template <class S>
-__device__ __forceinline__ Ray1d<S> intersect_ray(const S* mu, const S* A, const S* o, const S* d)
+__device__ __forceinline__ Ray1d<S> intersect_ray_pre(const S* mu, const S* A, const S* m, S norm3, const S* o, const S* d)
 {
     const S Ad0 = (A[0] * d[0] + A[1] * d[1]) + A[2] * d[2];
     const S Ad1 = (A[1] * d[0] + A[3] * d[1]) + A[4] * d[2];
     const S Ad2 = (A[2] * d[0] + A[4] * d[1]) + A[5] * d[2];
-    const S m0 = mu[0] - o[0], m1 = mu[1] - o[1], m2 = mu[2] - o[2];
     const S q = (d[0] * Ad0 + d[1] * Ad1) + d[2] * Ad2;
     const S C = S(1) / q;
-    const S centre = ((Ad0 * m0 + Ad1 * m1) + Ad2 * m2) * C;
+    const S centre = ((Ad0 * m[0] + Ad1 * m[1]) + Ad2 * m[2]) * C;
     const S r0 = (o[0] + centre * d[0]) - mu[0];
     const S r1 = (o[1] + centre * d[1]) - mu[1];
     const S r2 = (o[2] + centre * d[2]) - mu[2];
@@ -226,47 +236,51 @@ __device__ __forceinline__ Ray1d<S> intersect_ray(const S* mu, const S* A, const
     const S Ar1 = (A[1] * r0 + A[3] * r1) + A[4] * r2;
     const S Ar2 = (A[2] * r0 + A[4] * r1) + A[5] * r2;
     const S E = (r0 * Ar0 + r1 * Ar1) + r2 * Ar2;
-    const S detA = A[0] * (A[3] * A[5] - A[4] * A[4]) - A[1] * (A[1] * A[5] - A[4] * A[2]) + A[2] * (A[1] * A[4] - A[3] * A[2]);
-    const S norm3 = sqrt_rn(detA) / S(15.749609945722419); // sqrt((2 pi)^3)
     const S norm1 = S(1) / sqrt_rn(S(2 * kPi) * C);
     return { norm3 / norm1 * dexp(S(-0.5) * E), centre, C };
 }
 
-// adjoint w.r.t. mu and the stored inverse covariance
 template <class S>
-__device__ __forceinline__ void intersect_ray_grad(const S* mu, const S* A, const S* o, const S* d, S g_w, S g_centre, S g_var, S* g_mu,
-    S* g_A)
+__device__ __forceinline__ Ray1d<S> intersect_ray(const S* mu, const S* A, const S* o, const S* d)
 {
+    const S m[3] = { mu[0] - o[0], mu[1] - o[1], mu[2] - o[2] };
+    return intersect_ray_pre(mu, A, m, ray_norm3(sym3_det(A)), o, d);
+}
+
+// adjoint w.r.t. mu and the stored inverse covariance; g_wW is the gradient
+// of the weight times the weight.  Gradient values only: contraction and (in
+// float) hardware reciprocals.
+template <class S>
+__device__ __forceinline__ void intersect_ray_grad(const S* mu, const S* A, const S* m, const S* o, const S* d, S centre, S g_wW, S g_centre,
+    S g_var, S* g_mu, S* g_A)
+{
+#pragma clang fp contract(fast)
     const S Ad[3] = { (A[0] * d[0] + A[1] * d[1]) + A[2] * d[2], (A[1] * d[0] + A[3] * d[1]) + A[4] * d[2],
         (A[2] * d[0] + A[4] * d[1]) + A[5] * d[2] };
-    const S m[3] = { mu[0] - o[0], mu[1] - o[1], mu[2] - o[2] };
-    const S q = dot3(d, Ad);
-    const S C = S(1) / q;
-    const S k = dot3(Ad, m);
-    const S centre = k * C;
-    const S r[3] = { (o[0] + centre * d[0]) - mu[0], (o[1] + centre * d[1]) - mu[1], (o[2] + centre * d[2]) - mu[2] };
+    const S C = fast_div(S(1), dot3(d, Ad));
+    const S r[3] = { centre * d[0] - m[0], centre * d[1] - m[1], centre * d[2] - m[2] };
     const S Ar[3] = { (A[0] * r[0] + A[1] * r[1]) + A[2] * r[2], (A[1] * r[0] + A[3] * r[1]) + A[4] * r[2],
         (A[2] * r[0] + A[4] * r[1]) + A[5] * r[2] };
-    const S E = dot3(r, Ar);
-    const S detA = A[0] * (A[3] * A[5] - A[4] * A[4]) - A[1] * (A[1] * A[5] - A[4] * A[2]) + A[2] * (A[1] * A[4] - A[3] * A[2]);
-    const S W = sqrt_rn(detA) / S(15.749609945722419) * sqrt_rn(S(2 * kPi) * C) * dexp(S(-0.5) * E);
-    const S gwW = g_w * W;
+    const S gc = g_centre * C;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-        g_mu[i] = gwW * Ar[i] + g_centre * Ad[i] * C;
+        g_mu[i] = g_wW * Ar[i] + gc * Ad[i];
     // A^-1 via the adjugate
-    const S inv_det = S(1) / detA;
-    const S Ai[6] = { (A[3] * A[5] - A[4] * A[4]) * inv_det, (A[2] * A[4] - A[1] * A[5]) * inv_det, (A[1] * A[4] - A[2] * A[3]) * inv_det,
-        (A[0] * A[5] - A[2] * A[2]) * inv_det, (A[2] * A[1] - A[0] * A[4]) * inv_det, (A[0] * A[3] - A[1] * A[1]) * inv_det };
+    const S c00 = A[3] * A[5] - A[4] * A[4], c01 = A[2] * A[4] - A[1] * A[5], c02 = A[1] * A[4] - A[2] * A[3];
+    const S inv_det = fast_div(S(1), (A[0] * c00 + A[1] * c01) + A[2] * c02);
+    const S Ai[6] = { c00 * inv_det, c01 * inv_det, c02 * inv_det, (A[0] * A[5] - A[2] * A[2]) * inv_det, (A[2] * A[1] - A[0] * A[4]) * inv_det,
+        (A[0] * A[3] - A[1] * A[1]) * inv_det };
+    // g_A = g_wW / 2 (A^-1 - C d d^T - r r^T) - g_centre C / 2 (d r^T + r d^T) - g_var C^2 d d^T
+    const S h = S(0.5) * g_wW, f = h * C + g_var * (C * C), e = S(0.5) * gc;
     const int idx[6][2] = { { 0, 0 }, { 0, 1 }, { 0, 2 }, { 1, 1 }, { 1, 2 }, { 2, 2 } };
 #pragma unroll
-    for (int e = 0; e < 6; ++e) {
-        const int i = idx[e][0], j = idx[e][1];
-        const S ddT = d[i] * d[j];
-        S G = gwW * S(0.5) * (Ai[e] - C * ddT - r[i] * r[j]) + g_centre * (C * S(0.5) * (d[i] * m[j] + m[i] * d[j]) - k * C * C * ddT)
-            - g_var * C * C * ddT;
-        g_A[e] = (i == j) ? G : S(2) * G;
+    for (int k = 0; k < 6; ++k) {
+        const int i = idx[k][0], j = idx[k][1];
+        const S G = h * (Ai[k] - r[i] * r[j]) - f * (d[i] * d[j]) - e * (d[i] * r[j] + r[i] * d[j]);
+        g_A[k] = (i == j) ? G : S(2) * G;
     }
+    (void)mu;
+    (void)o;
 }
 
 // stroke::gaussian::cdf_inv_SD: standard normal cdf of (x - centre) / sd
@@ -293,30 +307,61 @@ __device__ __forceinline__ float cdf_inv_sd<float>(float centre, float inv_sd, f
     return 0.5f + 0.5f * copysignf(erf_abs, v);
 }
 
-// The cdf and the density at x of the normal (centre, 1 / inv_sd), for the
-// adjoint of a bin's mass (d cdf / d centre = -inv_sd pdf, d cdf / d inv_sd =
-// (x - centre) pdf).  Double: erf and exp.  Float: the cdf above, whose
-// e^{-v^2} with v = z / sqrt 2 is the density's e^{-z^2 / 2}, so one
-// exponential serves both.
+// The cdf less a constant, for differences between bin borders.  Double: the
+// cdf.  Float: formula 7.1.26 as above with the factors that do not depend on
+// the border folded into the scale (u = v sqrt(log2 e), so e^{-v^2} = 2^{-u^2})
+// and the final 1/2 into the coefficients; without adding 1/2 a difference
+// loses nothing to rounding.
 template <class S>
-__device__ __forceinline__ void cdf_pdf_inv_sd(S centre, S inv_sd, S x, S* cdf, S* pdf)
+struct CdfScale {
+    S k;
+};
+__device__ __forceinline__ CdfScale<double> cdf_scale(double inv_sd) { return { inv_sd }; }
+__device__ __forceinline__ CdfScale<float> cdf_scale(float inv_sd) { return { inv_sd * 0.849321800288019f }; } // sqrt(log2(e) / 2)
+
+__device__ __forceinline__ double cdf_step(double centre, const CdfScale<double>& s, double x) { return cdf_inv_sd(centre, s.k, x); }
+
+// e: 2^{-u^2} = e^{-z^2 / 2}
+__device__ __forceinline__ float cdf_step_exp(float u, float* e)
 {
-    const S z = (x - centre) * inv_sd;
-    *cdf = S(0.5) * (S(1) + derf(z * S(0.70710678118654752440)));
-    *pdf = dexp(S(-0.5) * z * z) * S(0.39894228040143267794);
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.272737440f, fabsf(u), 1.f)); // 0.3275911 / sqrt(log2 e)
+    const float poly = fmaf(t, fmaf(t, fmaf(t, fmaf(t, 0.5307027145f, -0.7265760135f), 0.7107068705f), -0.142248368f), 0.127414796f);
+    *e = __builtin_amdgcn_exp2f(-u * u);
+    return copysignf(fmaf(-(t * poly), *e, 0.5f), u);
+}
+__device__ __forceinline__ float cdf_step(float centre, const CdfScale<float>& s, float x)
+{
+    float e;
+    return cdf_step_exp((x - centre) * s.k, &e);
 }
 
-template <>
-__device__ __forceinline__ void cdf_pdf_inv_sd<float>(float centre, float inv_sd, float x, float* cdf, float* pdf)
+// The cdf (less a constant) at x and what its derivatives need, for the adjoint
+// of a bin's mass: p ~ pdf and q ~ z pdf up to the constant factors of
+// cdf_grad_scale (d cdf / d centre = -inv_sd pdf, d cdf / d inv_sd =
+// (x - centre) pdf).  Float: e^{-z^2 / 2} is the one of the cdf.
+__device__ __forceinline__ void cdf_grad_step(double centre, const CdfScale<double>& s, double x, double* cdf, double* p, double* q)
 {
-    const float v = (x - centre) * inv_sd * 0.70710678118654752440f;
-    const float a = fabsf(v);
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, a, 1.f));
-    const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
-    const float e = __builtin_amdgcn_exp2f(-a * a * 1.4426950408889634f);
-    const float erf_abs = fmaf(-poly, e, 1.f);
-    *cdf = 0.5f + 0.5f * copysignf(erf_abs, v);
-    *pdf = e * 0.39894228040143267794f;
+    const double z = (x - centre) * s.k;
+    *cdf = 0.5 * (1.0 + derf(z * 0.70710678118654752440));
+    *p = dexp(-0.5 * z * z);
+    *q = z * *p;
+}
+__device__ __forceinline__ void cdf_grad_step(float centre, const CdfScale<float>& s, float x, float* cdf, float* p, float* q)
+{
+    const float u = (x - centre) * s.k;
+    *cdf = cdf_step_exp(u, p);
+    *q = u * *p;
+}
+// factors that turn sums over p into sums over inv_sd pdf, and over q into sums over z pdf
+__device__ __forceinline__ void cdf_grad_scale(const CdfScale<double>&, double inv_sd, double* fp, double* fq)
+{
+    *fp = inv_sd * 0.39894228040143267794;
+    *fq = 0.39894228040143267794;
+}
+__device__ __forceinline__ void cdf_grad_scale(const CdfScale<float>&, float inv_sd, float* fp, float* fq)
+{
+    *fp = inv_sd * 0.39894228040143267794f;
+    *fq = 0.39894228040143267794f * 1.17741002251547469f; // u = z / sqrt(2 ln 2)
 }
 
 // pixel ray, vol_marcher_forward.cu:308-315
