@@ -383,8 +383,7 @@ __device__ __forceinline__ float far_radius(float mor, float var)
     return mor > 9.99f ? __builtin_inff() : r;
 }
 
-// A restricted to the ray and whether it can deposit mass (math.h:436-454).
-// Double: the reference's expressions.
+// A restricted to the ray and whether it can deposit mass (math.h:436-454)
 template <class S>
 __device__ __forceinline__ bool ray_gaussian(const Staged<S>& g, const S* o, const S* d, RayGauss<S>* out)
 {
@@ -403,53 +402,14 @@ __device__ __forceinline__ bool ray_gaussian(const Staged<S>& g, const S* o, con
     return true;
 }
 
-// Float: the centre and the residual o + centre d - mu keep the operations of
-// the exact restriction (the residual's rounding, ~1e-7 of the distance, is
-// what the mass is sensitive to, and it moves with the centre), the rest uses
-// fused multiply-adds, the hardware reciprocal square root and exp2: 60
-// instructions instead of 170.  The result is a few ulp from the exact
-// restriction's, which decides where the mass on the ray is within 1e-3 of a
-// threshold, so no Gaussian changes sides.
-template <>
-__device__ __forceinline__ bool ray_gaussian<float>(const Staged<float>& g, const float* o, const float* d, RayGauss<float>* out)
-{
-    const float Ad0 = (g.A[0] * d[0] + g.A[1] * d[1]) + g.A[2] * d[2];
-    const float Ad1 = (g.A[1] * d[0] + g.A[3] * d[1]) + g.A[4] * d[2];
-    const float Ad2 = (g.A[2] * d[0] + g.A[4] * d[1]) + g.A[5] * d[2];
-    const float q = (d[0] * Ad0 + d[1] * Ad1) + d[2] * Ad2;
-    const float C = 1.f / q;
-    const float centre = ((Ad0 * g.m[0] + Ad1 * g.m[1]) + Ad2 * g.m[2]) * C;
-    const float r0 = (o[0] + centre * d[0]) - g.mu[0];
-    const float r1 = (o[1] + centre * d[1]) - g.mu[1];
-    const float r2 = (o[2] + centre * d[2]) - g.mu[2];
-    const float Ar0 = fmaf(g.A[2], r2, fmaf(g.A[1], r1, g.A[0] * r0));
-    const float Ar1 = fmaf(g.A[4], r2, fmaf(g.A[3], r1, g.A[1] * r0));
-    const float Ar2 = fmaf(g.A[5], r2, fmaf(g.A[4], r1, g.A[2] * r0));
-    const float E = fmaf(r2, Ar2, fmaf(r1, Ar1, r0 * Ar0));
-    const float sd = __builtin_amdgcn_rsqf(q);
-    // mass norm3 sqrt(2 pi) exp(-E / 2) sd
-    float mor = (g.mass * g.norm3) * (2.5066282746310002f * sd) * __builtin_amdgcn_exp2f(E * -0.7213475204444817f);
-    const bool near_cut = fabsf(fmaf(mor, 255.f, -1.f)) < 1e-3f || mor > 900.f;
-    if (__builtin_amdgcn_ballot_w64(near_cut) != 0) {
-        const Ray1d<float> r = intersect_staged(g, o, d);
-        mor = near_cut ? r.weight * g.mass : mor;
-    }
-    out->centre = centre;
-    out->inv_sd = q * sd;
-    out->mor = mor;
-    out->far = far_radius(mor, C);
-    return centre == centre && mor >= 1.0f / 255.f && mor <= 1000.f && sd > 0.0001f; // false for NaN
-}
-
-// Per-wave candidate masks over the tile's list: bit p of a wave's mask is
-// set when the Gaussian at list position p passes the mass-on-ray test
-// (1/255 <= mass <= 1000, or NaN) on some pixel of the wave.  A Gaussian that
-// fails it on every pixel deposits nothing (math.h:440-443) and has no
-// adjoint, so the deposit and adjoint passes of every large step skip it for
-// the whole wave.  The test does not depend on the large step: a 64-entry word
-// is built when a pass first needs one of its entries and kept in LDS (the
-// entries past the depth where the wave's rays saturate are never tested).
-// Positions from kCandEntries on are not tracked and always taken.
+// Per-wave candidate masks over the tile's list: the Gaussian at list
+// position p is a candidate when it passes the mass-on-ray test (1/255 <=
+// mass <= 1000, or NaN) on some pixel of the wave.  One that fails it on every
+// pixel deposits nothing (math.h:440-443) and has no adjoint, so the passes of
+// every large step skip it for the whole wave.  The test does not depend on the
+// large step: the first pass that visits an entry evaluates its restriction
+// anyway, and records the answer in LDS.  Positions from kCandEntries on are
+// not recorded and always taken.
 constexpr int kCandWords = 64;
 constexpr uint32_t kCandEntries = 64u * kCandWords;
 
@@ -460,40 +420,56 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t v)
     return (uint64_t(hi) << 32) | lo;
 }
 
-// a wave's candidate words and which of them are built
+// a wave's words, in LDS: bit p of `rejected` is set once position p is known
+// not to be a candidate, bit p of `known` once it was tested
 struct Candidates {
-    uint64_t* words; // LDS, this wave's
-    uint64_t built;
+    uint64_t* rejected;
+    uint64_t* known;
 };
 
-// the candidates among staged entries [j0, j0 + 64) of the batch at list
-// offset `pos` (relative to the tile's first entry), limited to `mask` (not 0)
-template <class S>
-__device__ __forceinline__ uint64_t candidate_word(Candidates& cand, uint64_t mask, uint64_t valid, uint32_t pos, int j0, const Staged<S>* s_g,
-    bool inside, const S* o, const S* d)
-{
-    const uint32_t p = pos + uint32_t(j0);
-    if (p >= kCandEntries)
-        return mask;
-    const uint32_t w = p / 64;
-    if (!((cand.built >> w) & 1)) {
-        uint64_t word = 0;
-        for (uint64_t todo = valid; todo != 0; todo &= todo - 1) {
-            const int jj = __builtin_ctzll(todo);
-            const Staged<S>& g = s_g[j0 + jj];
-            const Ray1d<S> r = intersect_staged(g, o, d);
-            const S mor = r.weight * g.mass;
-            if (__builtin_amdgcn_ballot_w64(inside && !(mor < S(1.0f / 255.f)) && !(mor > S(1000))) != 0)
-                word |= uint64_t(1) << jj;
+// the 64-entry word at a list position, while a pass visits its entries
+struct CandidateWord {
+    uint64_t rejected, known;
+    int at; // -1: not recorded
+
+    __device__ __forceinline__ CandidateWord(const Candidates& c, uint32_t pos) : rejected(0), known(0), at(-1)
+    {
+        if (pos < kCandEntries) {
+            at = int(pos / 64);
+            rejected = uniform_u64(c.rejected[at]);
+            known = uniform_u64(c.known[at]);
         }
-        if (lane_id() == 0)
-            cand.words[w] = word;
-        __builtin_amdgcn_wave_barrier(); // LDS operations of a wave execute in order: later reads see the word
-        cand.built |= uint64_t(1) << w;
-        return word & mask;
     }
-    return uniform_u64(cand.words[w]) & mask;
+    // entry j was visited; mor: its mass on the lane's ray
+    template <class S>
+    __device__ __forceinline__ void visited(int j, bool inside, S mor)
+    {
+        const uint64_t bit = uint64_t(1) << j;
+        if ((known & bit) == 0) {
+            known |= bit;
+            if (__builtin_amdgcn_ballot_w64(inside && !(mor < S(1.0f / 255.f)) && !(mor > S(1000))) == 0)
+                rejected |= bit;
+        }
+    }
+    __device__ __forceinline__ void store(const Candidates& c) const
+    {
+        if (at >= 0 && lane_id() == 0) {
+            c.rejected[at] = rejected;
+            c.known[at] = known;
+        }
+        __builtin_amdgcn_wave_barrier(); // LDS operations of a wave execute in order: later reads see the word
+    }
+};
+
+// clears a wave's words; every lane of the wave calls it
+__device__ __forceinline__ Candidates clear_candidates(uint64_t (*words)[kCandWords])
+{
+    words[0][lane_id()] = 0;
+    words[1][lane_id()] = 0;
+    __builtin_amdgcn_wave_barrier();
+    return { words[0], words[1] };
 }
+static_assert(kCandWords == 64, "one word per lane");
 
 // the valid entries of a 64-entry word of a batch of cnt
 __device__ __forceinline__ uint64_t valid_entries(int j0, int cnt)
@@ -569,26 +545,22 @@ __device__ __forceinline__ TileAxis tile_axis(const S* d, bool inside, float* s_
     return ax;
 }
 
-// A pixel's section list: in LDS for float (48 KB for a 256-pixel tile, which
-// two workgroups per CU can hold beside their staging; indexed at run time,
-// the list would live in private memory), in the thread's own array for
-// double (twice the bytes)
+// The tile's section lists, in LDS: indexed at run time by the border walk,
+// and (in the in-order insertion) by the list itself, they would live in private
+// memory as a thread's own array.  52 KB for a 256-pixel tile in float, which
+// two workgroups per CU hold beside their staging; 104 KB in double, one
+// workgroup per CU, which is what the double kernels' registers allow.
 template <class S, int NT>
-struct SectionListFor {
-    using type = SectionList<S, kSections>;
+struct SectionSmem {
+    S words[3 * SectionStore<S, kSections, NT>::kSlots * NT];
 };
-template <int NT>
-struct SectionListFor<float, NT> {
-    using type = SectionList<float, kSections, SectionLds<NT>>;
-};
-template <class S, int NT>
-constexpr int kSectionLdsFloats = sizeof(S) == 4 ? kSections * 3 * NT : 1;
 
-template <class S, class L>
-__device__ __forceinline__ void attach_sections(L& sec, float* s_sec)
+template <class S, int NT>
+__device__ __forceinline__ SectionList<S, kSections, NT> section_list(SectionSmem<S, NT>& sm)
 {
-    if constexpr (sizeof(S) == 4)
-        sec.data.base = s_sec + threadIdx.x;
+    SectionList<S, kSections, NT> sec;
+    sec.data.base = sm.words + threadIdx.x;
+    return sec;
 }
 
 // Whether the section pass may visit only the wave's candidates: a Gaussian
@@ -615,7 +587,7 @@ __device__ __forceinline__ bool sections_by_candidates(const MarchData<S>& md, u
 // put; the depth break moves as for the candidates)
 template <class S, int NT, class L>
 __device__ __forceinline__ void build_sections(L& sec, TileList<S, NT>& tl, bool skip, bool inside, const S* o, const S* d, const MarchControl& ctl,
-    bool by_cand, Candidates& cand)
+    bool by_cand, const Candidates& cand)
 {
     if (ctl.n_frozen > 0) {
         for (int k = 0; k < ctl.n_frozen; ++k)
@@ -624,46 +596,81 @@ __device__ __forceinline__ void build_sections(L& sec, TileList<S, NT>& tl, bool
     }
     bool done1 = skip;
     const float wlo = by_cand ? wave_min(skip ? __builtin_inff() : float(sec.start_)) : 0.f;
+    // A pixel's accepted Gaussians wait here, so that one insertion serves
+    // pixels that took different Gaussians (a wave visits about 50 Gaussians
+    // per large step, a pixel takes a third of them).  Each is inserted, or
+    // stops the pass, exactly as if it had been at once: its depth is held
+    // against the list's end when its turn comes.
+    constexpr int Q = 4;
+    S q_centre[Q], q_sd[Q], q_depth[Q];
+    int waiting = 0;
+    static_for<Q>([&](auto k) { q_centre[k] = q_sd[k] = q_depth[k] = 0; });
     for (uint32_t base = tl.first; base < tl.last; base += NT) {
         if (__syncthreads_count(!done1) == 0)
             break;
         tl.stage(base, o);
         // the batch's first Gaussian is its shallowest: past it, every later
         // one is beyond the list's end too (the break the full walk takes)
-        if (!done1 && sec.end_ < tl.s_g[0].depth)
+        if (sec.end_ < tl.s_g[0].depth)
             done1 = true;
         const int cnt = int(min<uint32_t>(NT, tl.last - base));
-        for (int j0 = 0; j0 < cnt; j0 += 64) {
-            if (__builtin_amdgcn_ballot_w64(!done1) == 0)
-                break;
-            uint64_t word = valid_entries(j0, cnt);
-            if (by_cand) {
-                const uint64_t valid = word;
-                word = entries_in(tl.s_win, j0, cnt, wlo, wave_max(done1 ? -__builtin_inff() : float(sec.end_)));
-                if (word != 0)
-                    word = candidate_word(cand, word, valid, base - tl.first, j0, tl.s_g, inside, o, d);
+        int j0 = -64;
+        uint64_t word = 0;
+        CandidateWord cw(cand, kCandEntries);
+        while (true) {
+            while (word == 0 && j0 + 64 < cnt) {
+                j0 += 64;
+                cw.store(cand);
+                cw = CandidateWord(cand, base - tl.first + uint32_t(j0));
+                word = valid_entries(j0, cnt);
+                if (by_cand)
+                    word = entries_in(tl.s_win, j0, cnt, wlo, wave_max(done1 ? -__builtin_inff() : float(sec.end_))) & ~cw.rejected;
             }
-            for (; word != 0; word &= word - 1) {
-                if (__builtin_amdgcn_ballot_w64(!done1) == 0)
-                    break;
-                const Staged<S>& g = tl.s_g[j0 + __builtin_ctzll(word)];
-                const Ray1d<S> r = intersect_staged(g, o, d);
+            const bool visit = word != 0 && __builtin_amdgcn_ballot_w64(!done1) != 0;
+            if (visit) {
+                const int j = __builtin_ctzll(word);
+                const Staged<S>& g = tl.s_g[j0 + j];
+                word &= word - 1;
                 if (sec.end_ < g.depth)
                     done1 = true;
-                if (done1)
-                    continue;
+                const Ray1d<S> r = intersect_staged(g, o, d);
                 const S mor = r.weight * g.mass;
-                if (mor <= S(1.0f / 255.f) || mor > S(1000))
-                    continue;
-                if (r.var <= 0)
-                    continue;
-                if (r.centre != r.centre)
-                    continue;
-                const S sd = sqrt_rn(r.var);
-                const S half = sd * S(kRelevanceSigma);
-                sec.put({ r.centre - half, r.centre + half, (sd * S(kRelevanceSigma) * S(2)) / S(kStepsPerGaussian - 1) });
+                cw.visited(j, inside, mor);
+                const S sd = sqrt_rn(r.var), half = sd * S(kRelevanceSigma);
+                const bool out = r.centre + half <= sec.start_ || r.centre - half >= sec.end_; // put would return
+                const bool take = !done1 && !(mor <= S(1.0f / 255.f) || mor > S(1000)) && !(r.var <= 0) && r.centre == r.centre && !out;
+                static_for<Q>([&](auto k) {
+                    const bool here = take && waiting == k;
+                    q_centre[k] = here ? r.centre : q_centre[k];
+                    q_sd[k] = here ? sd : q_sd[k];
+                    q_depth[k] = here ? g.depth : q_depth[k];
+                });
+                waiting += take ? 1 : 0;
             }
+            // a full walk (depths not ascending) inserts at once; so does the
+            // end of a batch
+            const int limit = visit && by_cand ? Q : 1;
+            while (__builtin_amdgcn_ballot_w64(waiting >= limit) != 0) {
+                if (waiting > 0) {
+                    if (sec.end_ < q_depth[0]) {
+                        done1 = true;
+                        waiting = 1; // the later ones are deeper
+                    } else {
+                        const S half = q_sd[0] * S(kRelevanceSigma);
+                        sec.put({ q_centre[0] - half, q_centre[0] + half, (q_sd[0] * S(kRelevanceSigma) * S(2)) / S(kStepsPerGaussian - 1) });
+                    }
+                    --waiting;
+                }
+                static_for<Q - 1>([&](auto k) {
+                    q_centre[k] = q_centre[k + 1];
+                    q_sd[k] = q_sd[k + 1];
+                    q_depth[k] = q_depth[k + 1];
+                });
+            }
+            if (!visit)
+                break;
         }
+        cw.store(cand);
     }
 }
 
@@ -685,20 +692,6 @@ __device__ __forceinline__ bool deposits_in(const RayGauss<S>& r, bool pass, S b
     return need;
 }
 
-// f(0), f(1), ... f(N - 1) with compile-time arguments: the per-bin arrays a
-// chunk keeps in registers are only ever indexed by constants (a loop that the
-// compiler unrolls late leaves them one register tuple, copied at every branch)
-template <class F, int... I>
-__device__ __forceinline__ void static_for_each(F&& f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I> {}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    static_for_each(f, std::make_integer_sequence<int, N> {});
-}
-
 // Bins per group: a wave evaluates the groups of a chunk that some lane's
 // Gaussian reaches (far_radius), the others hold less than 1e-5 per bin
 constexpr int kBinGroup = 8;
@@ -715,7 +708,7 @@ constexpr int kBinGroup = 8;
 // short restriction 17.4 and 22.3 ms.
 template <class S, int NT, int CB>
 __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 1], bool stopped, TileList<S, NT>& tl, bool inside,
-    const S* o, const S* d, S b_first, S b_last, Candidates& cand)
+    const S* o, const S* d, S b_first, S b_last, const Candidates& cand)
 {
 #pragma unroll
     for (int k = 0; k < CB; ++k)
@@ -729,18 +722,20 @@ __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 
         const int cnt = int(min<uint32_t>(NT, tl.last - base));
         for (int j0 = 0; j0 < cnt; j0 += 64) {
             uint64_t word = entries_in(tl.s_win, j0, cnt, wlo, whi);
-            if (word != 0)
-                word = candidate_word(cand, word, valid_entries(j0, cnt), base - tl.first, j0, tl.s_g, inside, o, d);
-            for (; word != 0; word &= word - 1) {
-                const Staged<S>& g = tl.s_g[j0 + __builtin_ctzll(word)];
+            if (word == 0)
+                continue;
+            CandidateWord cw(cand, base - tl.first + uint32_t(j0));
+            for (word &= ~cw.rejected; word != 0; word &= word - 1) {
+                const int j = __builtin_ctzll(word);
+                const Staged<S>& g = tl.s_g[j0 + j];
                 RayGauss<S> r;
                 const bool pass = ray_gaussian(g, o, d, &r) && !stopped;
+                cw.visited(j, inside, r.mor);
                 if (__builtin_amdgcn_ballot_w64(pass && r.centre + r.far > bb[0] && r.centre - r.far < bb[CB]) == 0)
                     continue;
                 const bool need = deposits_in(r, pass, b_first, b_last, bb[0], bb[CB]);
                 const S lo = need ? r.centre - r.far : S(inf), hi = need ? r.centre + r.far : S(-inf);
                 const S mor = need ? r.mor : S(0);
-                const CdfScale<S> cs = cdf_scale(r.inv_sd);
                 S c0 = 0;
                 bool have = false;
                 static_for<CB / kBinGroup>([&](auto group) {
@@ -751,11 +746,11 @@ __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 
                         return;
                     }
                     if (!have)
-                        c0 = cdf_step(r.centre, cs, bb[k0]);
+                        c0 = cdf_inv_sd(r.centre, r.inv_sd, bb[k0]);
                     have = true;
                     static_for<kBinGroup>([&](auto q) {
                         constexpr int k = k0 + q;
-                        const S c1 = cdf_step(r.centre, cs, bb[k + 1]);
+                        const S c1 = cdf_inv_sd(r.centre, r.inv_sd, bb[k + 1]);
                         const S mass = (c1 - c0) * mor;
                         c0 = c1;
                         const S m = mass >= S(0.00001f) ? mass : S(0); // NaN is not kept
@@ -766,6 +761,7 @@ __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 
                     });
                 });
             }
+            cw.store(cand);
         }
     }
 }
@@ -778,9 +774,9 @@ __global__ __launch_bounds__(TW* TH, sizeof(S) == 4 ? 2 : 1) void k_march_forwar
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
     __shared__ Reach1d s_win[NT];
-    __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ uint64_t s_cand[NT / 64][2][kCandWords];
     __shared__ float s_axis[4];
-    __shared__ float s_sec[kSectionLdsFloats<S, NT>];
+    __shared__ SectionSmem<S, NT> s_sec;
     if (md.n_pairs && *md.n_pairs == 0)
         return; // no visible Gaussian: the framebuffer stays as the caller cleared it
     const int tile = xcd_tile_m(blockIdx.x, md.n_tiles);
@@ -791,14 +787,13 @@ __global__ __launch_bounds__(TW* TH, sizeof(S) == 4 ? 2 : 1) void k_march_forwar
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
     TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
     const bool by_cand = sections_by_candidates(md, first, last);
     S C0 = 0, C1 = 0, C2 = 0, T = 1, start = 0;
     bool done = !inside;
     int steps = 0;
-    typename SectionListFor<S, NT>::type sec;
-    attach_sections<S>(sec, s_sec);
+    SectionList<S, kSections, NT> sec = section_list<S, NT>(s_sec);
     while (true) {
         sec.reset(start);
         build_sections<S, NT>(sec, tl, done, inside, o, d, ctl, by_cand, cand);
@@ -885,9 +880,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
     __shared__ Reach1d s_win[NT];
-    __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ uint64_t s_cand[NT / 64][2][kCandWords];
     __shared__ float s_axis[4];
-    __shared__ float s_sec[kSectionLdsFloats<S, NT>];
+    __shared__ SectionSmem<S, NT> s_sec;
     if (md.n_pairs && *md.n_pairs == 0)
         return; // no visible Gaussian: the framebuffer stays as the caller cleared it
     const int tile = xcd_tile_m(blockIdx.x, md.n_tiles);
@@ -898,7 +893,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
     TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
     const bool by_cand = sections_by_candidates(md, first, last);
     const bool bins_mode = ctl.render_mode == 1;
@@ -907,8 +902,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     S C0 = 0, C1 = 0, C2 = 0, T = 1, start = 0, distance = 0;
     bool done = !inside;
     int steps = 0;
-    typename SectionListFor<S, NT>::type sec;
-    attach_sections<S>(sec, s_sec);
+    SectionList<S, kSections, NT> sec = section_list<S, NT>(s_sec);
     while (true) {
         sec.reset(start);
         build_sections<S, NT>(sec, tl, done, inside, o, d, ctl, by_cand, cand);
@@ -1029,7 +1023,7 @@ __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bo
 // collect the cdf derivatives at both borders of every bin.  Entries, groups of
 // bins and kept bins are fill_chunk's; Tk = Gk = 0 past the pixel's stop.
 template <class S, int NT, int CB>
-__device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& cand, bool active, bool inside, const S* o, const S* d,
+__device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candidates& cand, bool active, bool inside, const S* o, const S* d,
     const S (&bb)[CB + 1], S b_first, S b_last, const S (&Tk)[CB], const S (&Gk)[CB], const S* gC, S* __restrict__ render_grads)
 {
     const uint32_t end = __syncthreads_count(active) == 0 ? tl.first : tl.last;
@@ -1040,10 +1034,13 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& c
         const int cnt = int(min<uint32_t>(NT, tl.last - base));
         for (int j0 = 0; j0 < cnt; j0 += 64) {
             uint64_t word = entries_in(tl.s_win, j0, cnt, wlo, whi);
-            if (word != 0)
-                word = candidate_word(cand, word, valid_entries(j0, cnt), base - tl.first, j0, tl.s_g, inside, o, d);
+            if (word == 0)
+                continue;
+            // the chunk's deposit pass has visited these entries
+            word &= ~CandidateWord(cand, base - tl.first + uint32_t(j0)).rejected;
             for (; word != 0; word &= word - 1) {
-                const Staged<S>& g = tl.s_g[j0 + __builtin_ctzll(word)];
+                const int j = __builtin_ctzll(word);
+                const Staged<S>& g = tl.s_g[j0 + j];
                 RayGauss<S> r;
                 const bool pass = ray_gaussian(g, o, d, &r) && active;
                 if (__builtin_amdgcn_ballot_w64(pass && r.centre + r.far > bb[0] && r.centre - r.far < bb[CB]) == 0)
@@ -1051,7 +1048,6 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& c
                 const bool need = deposits_in(r, pass, b_first, b_last, bb[0], bb[CB]);
                 const S lo = need ? r.centre - r.far : S(inf), hi = need ? r.centre + r.far : S(-inf);
                 const S mor = need ? r.mor : S(0);
-                const CdfScale<S> cs = cdf_scale(r.inv_sd);
                 const S gcr = dfma(gC[2], g.rgb[2], dfma(gC[1], g.rgb[1], gC[0] * g.rgb[0]));
                 S c0 = 0, p0 = 0, q0 = 0;
                 S s_d = 0, s_tm = 0, s_c = 0, s_i = 0;
@@ -1063,12 +1059,12 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& c
                         return;
                     }
                     if (!have)
-                        cdf_grad_step(r.centre, cs, bb[k0], &c0, &p0, &q0);
+                        cdf_grad_step(r.centre, r.inv_sd, bb[k0], &c0, &p0, &q0);
                     have = any = true;
                     static_for<kBinGroup>([&](auto bin) {
                         constexpr int k = k0 + bin;
                         S c1, p1, q1;
-                        cdf_grad_step(r.centre, cs, bb[k + 1], &c1, &p1, &q1);
+                        cdf_grad_step(r.centre, r.inv_sd, bb[k + 1], &c1, &p1, &q1);
                         const S delta = c1 - c0;
                         // the bin's mass max(0, m) is kept from 1e-5 on (NaN is not)
                         const bool kept = delta * mor >= S(0.00001f);
@@ -1091,7 +1087,7 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& c
                     gr[q] = 0;
                 if (need) {
                     S fp, fq;
-                    cdf_grad_scale(cs, r.inv_sd, &fp, &fq);
+                    cdf_grad_scale(r.inv_sd, &fp, &fq);
                     // d L / d mass on the ray = s_d; weight = mor / mass
                     gr[0] = fast_div(s_d * mor, g.mass);
                     s_tm *= mor;
@@ -1101,7 +1097,7 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, Candidates& c
                     // d cdf / d centre = -inv_sd pdf; d cdf / d var = -z pdf / (2 var)
                     const S g_centre = -(s_c * mor) * fp;
                     const S g_var = -(s_i * mor) * fq * (S(0.5) * r.inv_sd * r.inv_sd);
-                    intersect_ray_grad(g.mu, g.A, g.m, o, d, r.centre, s_d * mor, g_centre, g_var, gr + 4, gr + 7);
+                    intersect_ray_grad(g.mu, g.A, o, d, r.centre, s_d * mor, g_centre, g_var, gr + 4, gr + 7);
                 }
                 S* dst = render_grads + int64_t(g.id) * 13;
                 if constexpr (sizeof(S) == 4) {
@@ -1167,9 +1163,9 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
     __shared__ Reach1d s_win[NT];
-    __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ uint64_t s_cand[NT / 64][2][kCandWords];
     __shared__ float s_axis[4];
-    __shared__ float s_sec[kSectionLdsFloats<S, NT>];
+    __shared__ SectionSmem<S, NT> s_sec;
     const int tile = xcd_tile_m(blockIdx.x, md.n_tiles);
     if (rp.tile_steps && rp.tile_steps[tile] <= uint32_t(rp.steps))
         return;
@@ -1180,15 +1176,14 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
     TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
     const bool by_cand = sections_by_candidates(md, first, last);
     PixelAdjoint<S> pa = load_pixel_adjoint(cam, inside, px, py, framebuffer, remaining, grad_fb);
     S T = 1, start = 0;
     bool done = !inside;
     int steps = 0;
-    typename SectionListFor<S, NT>::type sec;
-    attach_sections<S>(sec, s_sec);
+    SectionList<S, kSections, NT> sec = section_list<S, NT>(s_sec);
     while (true) {
         sec.reset(start);
         build_sections<S, NT>(sec, tl, done, inside, o, d, ctl, by_cand, cand);
@@ -1240,7 +1235,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
     constexpr int NCH = (kBins + CB - 1) / CB;
     __shared__ Staged<S> s_g[NT];
     __shared__ Reach1d s_win[NT];
-    __shared__ uint64_t s_cand[NT / 64][kCandWords];
+    __shared__ uint64_t s_cand[NT / 64][2][kCandWords];
     __shared__ float s_axis[4];
     const int tile = xcd_tile_m(blockIdx.x, md.n_tiles);
     const uint32_t n_steps = rp.tile_steps[tile];
@@ -1253,7 +1248,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
     S d[3];
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
-    Candidates cand { s_cand[threadIdx.x / 64], 0 };
+    const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
     TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
     PixelAdjoint<S> pa = load_pixel_adjoint(cam, inside, px, py, framebuffer, remaining, grad_fb);
     S T = 1;

@@ -1,12 +1,13 @@
 // SPDX-License-Identifier: GPL-3.0-or-later
-// Device pieces of the volumetric ray marcher: the sample-section list, the
-// border walk, the 1D restriction of a 3D Gaussian to a ray, the normal cdf and
+// Device pieces of the volumetric ray marcher: the border walk over the sample
+// sections (sections.h), the 1D restriction of a 3D Gaussian to a ray, the normal cdf and
 // their adjoints.  References: src/dgmr/marching_steps.h:28-220,
 // src/dgmr/math.h:412-468, src/dgmr/grad/math.h:529-620.
 #pragma once
 
 #include "device_grad.h"
 #include "device_math.h"
+#include "sections.h"
 
 namespace dgmr {
 
@@ -17,150 +18,6 @@ constexpr int kBins = kBorders - 1;
 constexpr int kStepsPerGaussian = 32;
 constexpr float kRelevanceSigma = 3.f;
 constexpr float kFilterSD = 0.55f;
-
-template <class S>
-struct Section {
-    S start, end, dt;
-};
-
-// Storage of a pixel's sections: in the thread's own array (private memory
-// once indexed at run time), or in LDS, where thread t keeps field f of its
-// section i at base[(3 i + f) NT] (base = the kernel's array + t, so the
-// lanes of a wave touch consecutive words).
-template <class S, int CAP>
-struct SectionRegs {
-    Section<S> d[CAP];
-    __device__ __forceinline__ Section<S> get(int i) const { return d[i]; }
-    __device__ __forceinline__ S start(int i) const { return d[i].start; }
-    __device__ __forceinline__ S end(int i) const { return d[i].end; }
-    __device__ __forceinline__ S dt(int i) const { return d[i].dt; }
-    __device__ __forceinline__ void set(int i, const Section<S>& v) { d[i] = v; }
-};
-
-template <int NT>
-struct SectionLds {
-    float* base;
-    __device__ __forceinline__ Section<float> get(int i) const { return { base[(3 * i) * NT], base[(3 * i + 1) * NT], base[(3 * i + 2) * NT] }; }
-    __device__ __forceinline__ float start(int i) const { return base[(3 * i) * NT]; }
-    __device__ __forceinline__ float end(int i) const { return base[(3 * i + 1) * NT]; }
-    __device__ __forceinline__ float dt(int i) const { return base[(3 * i + 2) * NT]; }
-    __device__ __forceinline__ void set(int i, const Section<float>& v)
-    {
-        base[(3 * i) * NT] = v.start;
-        base[(3 * i + 1) * NT] = v.end;
-        base[(3 * i + 2) * NT] = v.dt;
-    }
-};
-
-// marching_steps::DensityArray (marching_steps.h:35-200): a sorted list of
-// disjoint sections over [start, end) holding the minimum step; when full,
-// end() shrinks to the last section's end.  put() follows the reference's
-// insertion step for step (in-place merge through a small ring buffer),
-// because the boundaries it leaves decide where the bin borders fall.
-template <class S, int CAP, class Store = SectionRegs<S, CAP>>
-struct SectionList {
-    Store data;
-    int size;
-    S start_, end_;
-
-    __device__ __forceinline__ void reset(S start)
-    {
-        size = 0;
-        start_ = start;
-        end_ = S(__builtin_huge_val());
-    }
-
-    __device__ __forceinline__ int first_ending_after(S v, int from) const
-    {
-        for (int i = from; i < size; ++i)
-            if (data.end(i) > v)
-                return i;
-        return size;
-    }
-
-    __device__ __forceinline__ static void combine(const Section<S>& a, const Section<S>& b, Section<S>* out)
-    {
-        if (a.start < b.start)
-            out[0] = { a.start, dmin(a.end, b.start), a.dt };
-        else
-            out[0] = { b.start, dmin(b.end, a.start), b.dt };
-        if (b.end < a.end)
-            out[2] = { b.end, a.end, a.dt };
-        else
-            out[2] = { a.end, b.end, b.dt };
-        out[1] = { out[0].end, out[2].start, dmin(a.dt, b.dt) };
-    }
-
-    __device__ void put(Section<S> e)
-    {
-        if (e.end <= start_ || e.start >= end_)
-            return;
-        e.start = dmax(start_, e.start);
-        e.end = dmin(end_, e.end);
-        const int first = first_ending_after(e.start, 0);
-        if (first >= size) {
-            if (first < CAP)
-                data.set(size++, e);
-            else
-                end_ = e.start;
-            return;
-        }
-        int stop = first_ending_after(e.end, first);
-        if (stop < size && data.start(stop) < e.end)
-            ++stop;
-        Section<S> ring[CAP];
-        unsigned ring_r = 0, ring_w = 0;
-        int rd = first, wr = first, inserted = 0;
-        while (rd < stop + inserted && wr < CAP) {
-            if (rd < size)
-                ring[(ring_w++) % CAP] = data.get(rd++);
-            if (ring_r >= ring_w)
-                break;
-            const Section<S> head = ring[ring_r % CAP];
-            if (head.end <= e.start) {
-                data.set(wr++, ring[(ring_r++) % CAP]);
-                continue;
-            }
-            if (head.start >= e.end)
-                break;
-            Section<S> parts[3];
-            combine(ring[(ring_r++) % CAP], e, parts);
-            if (parts[0].dt == parts[1].dt) {
-                parts[1].start = parts[0].start;
-                parts[0].end = parts[0].start;
-            }
-            e = parts[2];
-            if (parts[0].end - parts[0].start <= 0) {
-                if (parts[1].dt == parts[2].dt) {
-                    e.start = parts[1].start;
-                    continue;
-                }
-                data.set(wr++, parts[1]);
-            } else {
-                data.set(wr++, parts[0]);
-                if (parts[1].dt == parts[2].dt) {
-                    e.start = parts[1].start;
-                    continue;
-                }
-                ++inserted;
-                ring[(--ring_r) % CAP] = parts[1];
-            }
-        }
-        if (e.end - e.start > 0 && wr < CAP) {
-            if (rd < size)
-                ring[(ring_w++) % CAP] = data.get(rd++);
-            data.set(wr++, e);
-        }
-        while (ring_w - ring_r && wr < CAP) {
-            if (rd < size)
-                ring[(ring_w++) % CAP] = data.get(rd++);
-            data.set(wr++, ring[(ring_r++) % CAP]);
-        }
-        size = wr + size - rd;
-        if (size == CAP)
-            end_ = dmin(end_, data.end(size - 1));
-    }
-};
 
 // sample<n> (marching_steps.h:202-220) as a generator: border i+1 from border i
 template <class S, int CAP>
@@ -247,18 +104,29 @@ __device__ __forceinline__ Ray1d<S> intersect_ray(const S* mu, const S* A, const
     return intersect_ray_pre(mu, A, m, ray_norm3(sym3_det(A)), o, d);
 }
 
+// the ray's nearest point (in the A-norm) to mu, minus mu, rounded as the
+// restriction rounds it
+template <class S>
+__device__ __forceinline__ void ray_residual(const S* mu, const S* o, const S* d, S centre, S* r)
+{
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        r[i] = (o[i] + centre * d[i]) - mu[i];
+}
+
 // adjoint w.r.t. mu and the stored inverse covariance; g_wW is the gradient
 // of the weight times the weight.  Gradient values only: contraction and (in
 // float) hardware reciprocals.
 template <class S>
-__device__ __forceinline__ void intersect_ray_grad(const S* mu, const S* A, const S* m, const S* o, const S* d, S centre, S g_wW, S g_centre,
-    S g_var, S* g_mu, S* g_A)
+__device__ __forceinline__ void intersect_ray_grad(const S* mu, const S* A, const S* o, const S* d, S centre, S g_wW, S g_centre, S g_var,
+    S* g_mu, S* g_A)
 {
 #pragma clang fp contract(fast)
+    S r[3];
+    ray_residual(mu, o, d, centre, r);
     const S Ad[3] = { (A[0] * d[0] + A[1] * d[1]) + A[2] * d[2], (A[1] * d[0] + A[3] * d[1]) + A[4] * d[2],
         (A[2] * d[0] + A[4] * d[1]) + A[5] * d[2] };
     const S C = fast_div(S(1), dot3(d, Ad));
-    const S r[3] = { centre * d[0] - m[0], centre * d[1] - m[1], centre * d[2] - m[2] };
     const S Ar[3] = { (A[0] * r[0] + A[1] * r[1]) + A[2] * r[2], (A[1] * r[0] + A[3] * r[1]) + A[4] * r[2],
         (A[2] * r[0] + A[4] * r[1]) + A[5] * r[2] };
     const S gc = g_centre * C;
@@ -271,16 +139,16 @@ __device__ __forceinline__ void intersect_ray_grad(const S* mu, const S* A, cons
     const S Ai[6] = { c00 * inv_det, c01 * inv_det, c02 * inv_det, (A[0] * A[5] - A[2] * A[2]) * inv_det, (A[2] * A[1] - A[0] * A[4]) * inv_det,
         (A[0] * A[3] - A[1] * A[1]) * inv_det };
     // g_A = g_wW / 2 (A^-1 - C d d^T - r r^T) - g_centre C / 2 (d r^T + r d^T) - g_var C^2 d d^T
-    const S h = S(0.5) * g_wW, f = h * C + g_var * (C * C), e = S(0.5) * gc;
+    // (A^-1 - C d d^T is formed first: the two nearly cancel along the ray)
+    const S h = S(0.5) * g_wW, f = g_var * (C * C), e = S(0.5) * gc;
     const int idx[6][2] = { { 0, 0 }, { 0, 1 }, { 0, 2 }, { 1, 1 }, { 1, 2 }, { 2, 2 } };
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         const int i = idx[k][0], j = idx[k][1];
-        const S G = h * (Ai[k] - r[i] * r[j]) - f * (d[i] * d[j]) - e * (d[i] * r[j] + r[i] * d[j]);
+        const S dd = d[i] * d[j];
+        const S G = h * ((Ai[k] - C * dd) - r[i] * r[j]) - f * dd - e * (d[i] * r[j] + r[i] * d[j]);
         g_A[k] = (i == j) ? G : S(2) * G;
     }
-    (void)mu;
-    (void)o;
 }
 
 // stroke::gaussian::cdf_inv_SD: standard normal cdf of (x - centre) / sd
@@ -295,73 +163,50 @@ __device__ __forceinline__ S cdf_inv_sd(S centre, S inv_sd, S x)
 // formula 7.1.26, erf(x) = 1 - t (a1 + t (a2 + t (a3 + t (a4 + t a5)))) e^{-x^2}
 // with t = 1 / (1 + p x), x >= 0, |error| <= 1.5e-7: one reciprocal and one
 // exponential instead of a library erf.  The double path keeps erf.
-template <>
-__device__ __forceinline__ float cdf_inv_sd<float>(float centre, float inv_sd, float x)
+// v: z / sqrt 2, e: e^{-v^2}
+__device__ __forceinline__ float cdf_exp(float v, float* e)
 {
-    const float v = (x - centre) * inv_sd * 0.70710678118654752440f;
     const float a = fabsf(v);
     const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, a, 1.f));
     const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
-    const float e = __builtin_amdgcn_exp2f(-a * a * 1.4426950408889634f);
-    const float erf_abs = fmaf(-poly, e, 1.f);
-    return 0.5f + 0.5f * copysignf(erf_abs, v);
+    *e = __builtin_amdgcn_exp2f(-a * a * 1.4426950408889634f);
+    return fmaf(0.5f, copysignf(fmaf(-poly, *e, 1.f), v), 0.5f);
 }
-
-// The cdf less a constant, for differences between bin borders.  Double: the
-// cdf.  Float: formula 7.1.26 as above with the factors that do not depend on
-// the border folded into the scale (u = v sqrt(log2 e), so e^{-v^2} = 2^{-u^2})
-// and the final 1/2 into the coefficients; without adding 1/2 a difference
-// loses nothing to rounding.
-template <class S>
-struct CdfScale {
-    S k;
-};
-__device__ __forceinline__ CdfScale<double> cdf_scale(double inv_sd) { return { inv_sd }; }
-__device__ __forceinline__ CdfScale<float> cdf_scale(float inv_sd) { return { inv_sd * 0.849321800288019f }; } // sqrt(log2(e) / 2)
-
-__device__ __forceinline__ double cdf_step(double centre, const CdfScale<double>& s, double x) { return cdf_inv_sd(centre, s.k, x); }
-
-// e: 2^{-u^2} = e^{-z^2 / 2}
-__device__ __forceinline__ float cdf_step_exp(float u, float* e)
-{
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.272737440f, fabsf(u), 1.f)); // 0.3275911 / sqrt(log2 e)
-    const float poly = fmaf(t, fmaf(t, fmaf(t, fmaf(t, 0.5307027145f, -0.7265760135f), 0.7107068705f), -0.142248368f), 0.127414796f);
-    *e = __builtin_amdgcn_exp2f(-u * u);
-    return copysignf(fmaf(-(t * poly), *e, 0.5f), u);
-}
-__device__ __forceinline__ float cdf_step(float centre, const CdfScale<float>& s, float x)
+template <>
+__device__ __forceinline__ float cdf_inv_sd<float>(float centre, float inv_sd, float x)
 {
     float e;
-    return cdf_step_exp((x - centre) * s.k, &e);
+    return cdf_exp((x - centre) * inv_sd * 0.70710678118654752440f, &e);
 }
 
-// The cdf (less a constant) at x and what its derivatives need, for the adjoint
-// of a bin's mass: p ~ pdf and q ~ z pdf up to the constant factors of
-// cdf_grad_scale (d cdf / d centre = -inv_sd pdf, d cdf / d inv_sd =
-// (x - centre) pdf).  Float: e^{-z^2 / 2} is the one of the cdf.
-__device__ __forceinline__ void cdf_grad_step(double centre, const CdfScale<double>& s, double x, double* cdf, double* p, double* q)
+// The cdf at x and what its derivatives need, for the adjoint of a bin's mass:
+// p ~ pdf and q ~ z pdf up to the constant factors of cdf_grad_scale (d cdf /
+// d centre = -inv_sd pdf, d cdf / d inv_sd = (x - centre) pdf).  Double: erf
+// and exp.  Float: the cdf above, whose e^{-v^2} with v = z / sqrt 2 is the
+// density's e^{-z^2 / 2}, so one exponential serves both.
+__device__ __forceinline__ void cdf_grad_step(double centre, double inv_sd, double x, double* cdf, double* p, double* q)
 {
-    const double z = (x - centre) * s.k;
+    const double z = (x - centre) * inv_sd;
     *cdf = 0.5 * (1.0 + derf(z * 0.70710678118654752440));
     *p = dexp(-0.5 * z * z);
     *q = z * *p;
 }
-__device__ __forceinline__ void cdf_grad_step(float centre, const CdfScale<float>& s, float x, float* cdf, float* p, float* q)
+__device__ __forceinline__ void cdf_grad_step(float centre, float inv_sd, float x, float* cdf, float* p, float* q)
 {
-    const float u = (x - centre) * s.k;
-    *cdf = cdf_step_exp(u, p);
-    *q = u * *p;
+    const float v = (x - centre) * inv_sd * 0.70710678118654752440f;
+    *cdf = cdf_exp(v, p);
+    *q = v * *p;
 }
 // factors that turn sums over p into sums over inv_sd pdf, and over q into sums over z pdf
-__device__ __forceinline__ void cdf_grad_scale(const CdfScale<double>&, double inv_sd, double* fp, double* fq)
+__device__ __forceinline__ void cdf_grad_scale(double inv_sd, double* fp, double* fq)
 {
     *fp = inv_sd * 0.39894228040143267794;
     *fq = 0.39894228040143267794;
 }
-__device__ __forceinline__ void cdf_grad_scale(const CdfScale<float>&, float inv_sd, float* fp, float* fq)
+__device__ __forceinline__ void cdf_grad_scale(float inv_sd, float* fp, float* fq)
 {
     *fp = inv_sd * 0.39894228040143267794f;
-    *fq = 0.39894228040143267794f * 1.17741002251547469f; // u = z / sqrt(2 ln 2)
+    *fq = 0.39894228040143267794f * 1.41421356237309504880f;
 }
 
 // pixel ray, vol_marcher_forward.cu:308-315

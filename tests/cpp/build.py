@@ -1,7 +1,8 @@
 """Builds tests/cpp/_build/libfacade_check.so: the C++ façade check
 (facade_check.cpp over include/dgmr.hpp) that tests/test_gpu_facade.py loads,
-and libreach_check.so, the host build of the blends' tile-reach test that
-tests/test_tile_reach.py checks.  Run by __graft_entry__.build() after the
+libreach_check.so, the host build of the blends' tile-reach test that
+tests/test_tile_reach.py checks, and libsection_check.so, the host build of the
+marcher's section list that tests/test_section_list.py checks.  Run by __graft_entry__.build() after the
 library itself."""
 import os
 import subprocess
@@ -15,17 +16,29 @@ OUT = os.path.join(HERE, "_build", "libfacade_check.so")
 REACH_OUT = os.path.join(HERE, "_build", "libreach_check.so")
 
 
-def build_reach() -> str:
-    """The tile-reach test of the blends, built for the host (g++, no
-    contraction, as the kernels compile) for a CPU brute-force check."""
-    os.makedirs(os.path.dirname(REACH_OUT), exist_ok=True)
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", os.path.join(HERE, "reach_check.cpp"), "-o",
-           REACH_OUT + ".tmp"]
+SECTION_OUT = os.path.join(HERE, "_build", "libsection_check.so")
+
+
+def _build_host(source: str, out: str) -> str:
+    """A device header built for the host (g++, no contraction, as the
+    kernels compile)."""
+    os.makedirs(os.path.dirname(out), exist_ok=True)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", os.path.join(HERE, source), "-o", out + ".tmp"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed:\n{res.stdout}{res.stderr}")
-    os.replace(REACH_OUT + ".tmp", REACH_OUT)
-    return REACH_OUT
+    os.replace(out + ".tmp", out)
+    return out
+
+
+def build_reach() -> str:
+    """The tile-reach test of the blends, for a CPU brute-force check."""
+    return _build_host("reach_check.cpp", REACH_OUT)
+
+
+def build_sections() -> str:
+    """The marcher's section list, for a CPU check against the restatement."""
+    return _build_host("section_check.cpp", SECTION_OUT)
 
 
 def build() -> str:
@@ -41,4 +54,5 @@ def build() -> str:
 
 if __name__ == "__main__":
     print(build_reach())
+    print(build_sections())
     print(build())
