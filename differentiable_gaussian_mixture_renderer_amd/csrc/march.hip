@@ -178,65 +178,32 @@ struct alignas(16) Staged {
     uint32_t id;
 };
 
-// Where along any ray of the tile a staged Gaussian can matter: outside
-// [lo, hi] it holds neither a sample section nor a bin mass of 1e-5.  One
-// float pair per list entry, read by one lane each.
-struct Reach1d {
-    float lo, hi;
-};
-
 template <class S>
 __device__ __forceinline__ Ray1d<S> intersect_staged(const Staged<S>& g, const S* o, const S* d)
 {
     return intersect_ray_pre(g.mu, g.A, g.m, g.norm3, o, d);
 }
 
-// The window of a Gaussian over the tile's rays.  A point x d of the ray lies
-// at A-distance^2 E + z^2 from the centre mu (E: of the ray's nearest point, z:
-// standard deviations along the ray), so |x d - m| <= K sqrt(lambda) for every
-// point with E + z^2 <= K^2, lambda the largest eigenvalue of A^-1 (bounded by
-// the Frobenius norm), m = mu - o; as long as x >= 0 that bounds x by
-// |m| +- K sqrt(lambda).  The mass on the ray is at most M exp(-E / 2) with
-// M = mass norm3 sqrt(2 pi lambda), and a section or a bin of the Gaussian
-// needs
+// The window of a Gaussian over the tile's rays (gaussian_window): a section or
+// a bin of it needs
 //   mass on the ray >= 1/255 and z <= 3:   E + z^2 <= 2 ln M + 2 ln 255 + 9
 //   z within far_radius' cut:              E + z^2 <= 2 ln M + 2 ln 55556, or
 //                                          + 5.5^2 - 2 ln 2 when M can exceed 2
-// Rounding is covered by the widened K and an absolute term; where it could
-// not be (ill-conditioned A), for M >= 10 (never cut) and for rays that may
-// point away from the Gaussian, the window is the whole axis.
+// and with M >= 10 (never cut) it is the whole axis.
 template <class S>
-__device__ __forceinline__ Reach1d ray_window(const Staged<S>& g, S detA, const float* dc, float dev)
+__device__ __forceinline__ Reach1d ray_window(const Staged<S>& g, S detA, const TileAxis& ax)
 {
     const float inf = __builtin_inff();
-    const Reach1d all { -inf, inf };
-    const float a0 = float(g.A[0]), a1 = float(g.A[1]), a2 = float(g.A[2]), a3 = float(g.A[3]), a4 = float(g.A[4]), a5 = float(g.A[5]);
-    const float det = float(detA);
-    if (!(a0 > 0.f && a0 * a3 - a1 * a1 > 0.f && det > 0.f))
-        return all;
-    const float id = 1.f / det;
-    const float c0 = (a3 * a5 - a4 * a4) * id, c1 = (a2 * a4 - a1 * a5) * id, c2 = (a1 * a4 - a2 * a3) * id, c3 = (a0 * a5 - a2 * a2) * id,
-                c4 = (a2 * a1 - a0 * a4) * id, c5 = (a0 * a3 - a1 * a1) * id;
-    const float lam = sqrtf(c0 * c0 + c3 * c3 + c5 * c5 + 2.f * (c1 * c1 + c2 * c2 + c4 * c4));
-    const float tr = a0 + a3 + a5;
-    const float cond = tr * lam;
-    const float m0 = float(g.m[0]), m1 = float(g.m[1]), m2 = float(g.m[2]);
-    const float len = sqrtf(m0 * m0 + m1 * m1 + m2 * m2);
-    const float M = float(g.mass) * float(g.norm3) * sqrtf(float(2 * kPi) * lam);
-    if (!(cond < 1e4f) || !(1e-6f * len * sqrtf(tr) < 0.02f) || !(M < 9.9f) || !(m0 * dc[0] + m1 * dc[1] + m2 * dc[2] > 1.01f * dev * len + 1e-6f * len))
-        return all;
-    if (M < 0.0039f)
+    const float A[6] = { float(g.A[0]), float(g.A[1]), float(g.A[2]), float(g.A[3]), float(g.A[4]), float(g.A[5]) };
+    const float m[3] = { float(g.m[0]), float(g.m[1]), float(g.m[2]) };
+    const GaussianExtent e = gaussian_extent(A, float(detA), m, float(g.mass) * float(g.norm3), ax);
+    if (!e.bounded || !(e.mass < 9.9f))
+        return Reach1d { -inf, inf };
+    if (e.mass < 0.0039f)
         return Reach1d { inf, -inf }; // under 1/255 on every ray
-    const float K2 = 2.f * logf(M) + (M > 1.9f ? 29.f : 22.f);
-    const float half = (1.02f * sqrtf(fmaxf(K2, 0.f)) + 0.1f) * sqrtf(lam) + 1e-6f * cond * len;
-    return Reach1d { len - half, len + half };
+    const float half = extent_half(e, e.mass > 1.9f ? 29.f : 22.f);
+    return Reach1d { e.len - half, e.len + half };
 }
-
-// the direction the tile's rays deviate from by at most dev
-struct TileAxis {
-    float dc[3];
-    float dev;
-};
 
 template <class S>
 struct MarchData;
@@ -302,7 +269,7 @@ __device__ __forceinline__ void stage_gaussian(Staged<S>* dst, Reach1d* win, uin
         g.m[k] = g.mu[k] - o[k];
     const S detA = sym3_det(g.A);
     g.norm3 = ray_norm3(detA);
-    *win = ray_window(g, detA, ax.dc, ax.dev);
+    *win = ray_window(g, detA, ax);
     *dst = g;
 }
 
@@ -413,13 +380,6 @@ __device__ __forceinline__ bool ray_gaussian(const Staged<S>& g, const S* o, con
 constexpr int kCandWords = 64;
 constexpr uint32_t kCandEntries = 64u * kCandWords;
 
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v)
-{
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(v));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(v >> 32));
-    return (uint64_t(hi) << 32) | lo;
-}
-
 // a wave's words, in LDS: bit p of `rejected` is set once position p is known
 // not to be a candidate, bit p of `known` once it was tested
 struct Candidates {
@@ -471,30 +431,6 @@ __device__ __forceinline__ Candidates clear_candidates(uint64_t (*words)[kCandWo
 }
 static_assert(kCandWords == 64, "one word per lane");
 
-// the valid entries of a 64-entry word of a batch of cnt
-__device__ __forceinline__ uint64_t valid_entries(int j0, int cnt)
-{
-    const int n = cnt - j0;
-    return n >= 64 ? ~uint64_t(0) : ((uint64_t(1) << n) - 1);
-}
-
-// entries of a word whose window meets (wlo, whi): one entry per lane
-__device__ __forceinline__ uint64_t entries_in(const Reach1d* s_win, int j0, int cnt, float wlo, float whi)
-{
-    const Reach1d w = s_win[min(j0 + int(lane_id()), cnt - 1)];
-    return __builtin_amdgcn_ballot_w64(!(w.lo > whi) && !(w.hi < wlo)) & valid_entries(j0, cnt);
-}
-
-__device__ __forceinline__ float wave_min(float v)
-{
-#pragma unroll
-    for (int k = 32; k > 0; k >>= 1)
-        v = fminf(v, __shfl_xor(v, k));
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-
-__device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
-
 // The tile's list in LDS, NT entries at a time, for the block's passes over it
 template <class S, int NT>
 struct TileList {
@@ -519,31 +455,6 @@ struct TileList {
         staged = base;
     }
 };
-
-// the block's common ray direction (its first pixel's) and the largest
-// deviation of its pixels' rays from it
-template <class S, int NT>
-__device__ __forceinline__ TileAxis tile_axis(const S* d, bool inside, float* s_axis)
-{
-    if (threadIdx.x == 0) {
-        // thread 0's pixel is inside in every tile
-        s_axis[0] = float(d[0]);
-        s_axis[1] = float(d[1]);
-        s_axis[2] = float(d[2]);
-        s_axis[3] = 0.f;
-    }
-    __syncthreads();
-    TileAxis ax;
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        ax.dc[k] = s_axis[k];
-    const float e0 = float(d[0]) - ax.dc[0], e1 = float(d[1]) - ax.dc[1], e2 = float(d[2]) - ax.dc[2];
-    const float dev = inside ? sqrtf(e0 * e0 + e1 * e1 + e2 * e2) : 0.f;
-    atomicMax(reinterpret_cast<uint32_t*>(s_axis + 3), __float_as_uint(dev)); // dev >= 0: ordered as its bits
-    __syncthreads();
-    ax.dev = s_axis[3];
-    return ax;
-}
 
 // The tile's section lists, in LDS: indexed at run time by the border walk,
 // and (in the in-order insertion) by the list itself, they would live in private
@@ -788,7 +699,7 @@ __global__ __launch_bounds__(TW* TH, sizeof(S) == 4 ? 2 : 1) void k_march_forwar
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
     const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
-    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S>(d, inside, s_axis), last };
     const bool by_cand = sections_by_candidates(md, first, last);
     S C0 = 0, C1 = 0, C2 = 0, T = 1, start = 0;
     bool done = !inside;
@@ -894,7 +805,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
     const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
-    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S>(d, inside, s_axis), last };
     const bool by_cand = sections_by_candidates(md, first, last);
     const bool bins_mode = ctl.render_mode == 1;
     const int target = int(min(unsigned(ctl.debug_bin), unsigned(kBins - 1)));
@@ -1177,7 +1088,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
     const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
-    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S>(d, inside, s_axis), last };
     const bool by_cand = sections_by_candidates(md, first, last);
     PixelAdjoint<S> pa = load_pixel_adjoint(cam, inside, px, py, framebuffer, remaining, grad_fb);
     S T = 1, start = 0;
@@ -1249,7 +1160,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
     pixel_ray(cam, inside ? px : 0, inside ? py : 0, d);
     const uint32_t first = md.ranges[2 * tile], last = md.ranges[2 * tile + 1];
     const Candidates cand = clear_candidates(s_cand[threadIdx.x / 64]);
-    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S, NT>(d, inside, s_axis), last };
+    TileList<S, NT> tl { s_g, s_win, md, first, last, tile_axis<S>(d, inside, s_axis), last };
     PixelAdjoint<S> pa = load_pixel_adjoint(cam, inside, px, py, framebuffer, remaining, grad_fb);
     S T = 1;
     for (uint32_t step = 0; step < n_steps; ++step) {

@@ -227,6 +227,116 @@ __device__ __forceinline__ void pixel_ray(const DevCamera<S>& cam, int px, int p
         dir[i] = p[i] * inv_len;
 }
 
+// ------------------------------------------------ windows along a tile's rays
+// Where along any ray of the tile a staged Gaussian can matter: outside
+// [lo, hi] it holds neither a sample section nor a bin mass of 1e-5.  One
+// float pair per list entry, read by one lane each.
+struct Reach1d {
+    float lo, hi;
+};
+
+// the direction the tile's rays deviate from by at most dev
+struct TileAxis {
+    float dc[3];
+    float dev;
+};
+
+// The part of a tile's rays near a Gaussian.  A point x d of a ray lies at
+// A-distance^2 E + z^2 from the centre mu (E: of the ray's nearest point, z:
+// standard deviations along the ray), so |x d - m| <= K sqrt(lambda) for every
+// point with E + z^2 <= K^2, lambda the largest eigenvalue of A^-1 (bounded by
+// the Frobenius norm), m = mu - o; as long as the rays point towards m that
+// bounds x >= 0 by |m| +- K sqrt(lambda).  The mass on a ray is at most
+// M exp(-E / 2) with M = mass norm3 sqrt(2 pi lambda).  Rounding is covered by
+// a widened K and an absolute term; where it could not be (ill-conditioned A)
+// and for rays that may point away from the Gaussian, bounded is false.
+struct GaussianExtent {
+    float len, sqrt_lam, err, mass; // |m|, sqrt(lambda), rounding, M
+    bool bounded;
+};
+
+__device__ __forceinline__ GaussianExtent gaussian_extent(const float* A, float det, const float* m, float mass_norm3, const TileAxis& ax)
+{
+    GaussianExtent e { 0.f, 0.f, 0.f, 0.f, false };
+    if (!(A[0] > 0.f && A[0] * A[3] - A[1] * A[1] > 0.f && det > 0.f))
+        return e;
+    const float id = 1.f / det;
+    const float c0 = (A[3] * A[5] - A[4] * A[4]) * id, c1 = (A[2] * A[4] - A[1] * A[5]) * id, c2 = (A[1] * A[4] - A[2] * A[3]) * id,
+                c3 = (A[0] * A[5] - A[2] * A[2]) * id, c4 = (A[2] * A[1] - A[0] * A[4]) * id, c5 = (A[0] * A[3] - A[1] * A[1]) * id;
+    const float lam = sqrtf(c0 * c0 + c3 * c3 + c5 * c5 + 2.f * (c1 * c1 + c2 * c2 + c4 * c4));
+    const float tr = A[0] + A[3] + A[5];
+    const float cond = tr * lam;
+    e.len = sqrtf(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]);
+    e.sqrt_lam = sqrtf(lam);
+    e.err = 1e-6f * cond * e.len;
+    e.mass = mass_norm3 * (2.5066282746310002f * e.sqrt_lam);
+    e.bounded = cond < 1e4f && 1e-6f * e.len * sqrtf(tr) < 0.02f && e.mass == e.mass
+        && m[0] * ax.dc[0] + m[1] * ax.dc[1] + m[2] * ax.dc[2] > 1.01f * ax.dev * e.len + 1e-6f * e.len;
+    return e;
+}
+
+// half the window of the points with E + z^2 <= 2 ln M + above
+__device__ __forceinline__ float extent_half(const GaussianExtent& e, float above)
+{
+    return (1.02f * sqrtf(fmaxf(2.f * logf(e.mass) + above, 0.f)) + 0.1f) * e.sqrt_lam + e.err;
+}
+
+// the block's common ray direction (its first pixel's) and the largest
+// deviation of its pixels' rays from it
+template <class S>
+__device__ __forceinline__ TileAxis tile_axis(const S* d, bool inside, float* s_axis)
+{
+    if (threadIdx.x == 0) {
+        // thread 0's pixel is inside in every tile
+        s_axis[0] = float(d[0]);
+        s_axis[1] = float(d[1]);
+        s_axis[2] = float(d[2]);
+        s_axis[3] = 0.f;
+    }
+    __syncthreads();
+    TileAxis ax;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        ax.dc[k] = s_axis[k];
+    const float e0 = float(d[0]) - ax.dc[0], e1 = float(d[1]) - ax.dc[1], e2 = float(d[2]) - ax.dc[2];
+    const float dev = inside ? sqrtf(e0 * e0 + e1 * e1 + e2 * e2) : 0.f;
+    atomicMax(reinterpret_cast<uint32_t*>(s_axis + 3), __float_as_uint(dev)); // dev >= 0: ordered as its bits
+    __syncthreads();
+    ax.dev = s_axis[3];
+    return ax;
+}
+
+__device__ __forceinline__ uint64_t uniform_u64(uint64_t v)
+{
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(v >> 32));
+    return (uint64_t(hi) << 32) | lo;
+}
+
+// the valid entries of a 64-entry word of a batch of cnt
+__device__ __forceinline__ uint64_t valid_entries(int j0, int cnt)
+{
+    const int n = cnt - j0;
+    return n >= 64 ? ~uint64_t(0) : ((uint64_t(1) << n) - 1);
+}
+
+// entries of a word whose window meets (wlo, whi): one entry per lane
+__device__ __forceinline__ uint64_t entries_in(const Reach1d* s_win, int j0, int cnt, float wlo, float whi)
+{
+    const Reach1d w = s_win[min(j0 + int(lane_id()), cnt - 1)];
+    return __builtin_amdgcn_ballot_w64(!(w.lo > whi) && !(w.hi < wlo)) & valid_entries(j0, cnt);
+}
+
+__device__ __forceinline__ float wave_min(float v)
+{
+#pragma unroll
+    for (int k = 32; k > 0; k >>= 1)
+        v = fminf(v, __shfl_xor(v, k));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+__device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
+
 template <int CTRL, int ROW_MASK = 0xf, int BANK_MASK = 0xf>
 __device__ __forceinline__ double dpp_f64(double v)
 {

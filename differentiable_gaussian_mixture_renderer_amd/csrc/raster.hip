@@ -9,11 +9,10 @@
 //   2. bin_gaussians: the splatter's binning (same keys, same order).
 //   3. k_raster_render: one 16x16 tile per 256-thread workgroup, one pixel per
 //      thread.  Pass 1 sizes 32 bins per pixel (math::RasterBinSizer, kept in
-//      registers with fully unrolled, select-based updates so no runtime index
-//      sends the arrays to scratch); pass 2 rasterises the tile's Gaussians
-//      into the bins kChunk bins at a time and integrates each chunk's bins
-//      piecewise-linearly before the next chunk, so only kChunk bins of
-//      (rgb*mass, mass) and kChunk + 1 border evaluations are live.
+//      registers, every slot indexed by a constant); pass 2 rasterises the
+//      tile's Gaussians into the bins kChunk bins at a time and integrates each
+//      chunk's bins piecewise-linearly before the next chunk, so only kChunk
+//      bins of (rgb*mass, mass) and kChunk + 1 border evaluations are live.
 #include <cmath>
 
 #include "device_grad.h"
@@ -31,7 +30,8 @@ constexpr float kRasterFilterSD = 0.55f; // vol_raster::config::filter_kernel_SD
 constexpr float kRelevanceSigma = 3.f;  // vol_raster::config::gaussian_relevance_sigma
 constexpr int kTile = 16;               // render_block_width/height (constants.h:45-46)
 constexpr int kThreads = kTile * kTile;
-constexpr int kChunk = 8;               // bins rasterised per walk of the tile's list
+constexpr int kChunk = 16;              // bins rasterised per walk of the tile's list
+constexpr int kGroup = 4;               // bins evaluated together when some pixel of the wave needs one
 constexpr int kBorderStride = kRasterBins + 1; // odd: one LDS row per pixel, conflict-free
 
 // vol_raster_forward.cu:100-136 for the Gaussians the splatter preprocess kept:
@@ -79,12 +79,6 @@ __device__ __forceinline__ float cdf_sd(float centre, float inv_sd, float x)
     return 0.5f * (1.f + erff((x - centre) * inv_sd * 0.70710678118654752440f));
 }
 
-__device__ __forceinline__ float eval_exponential(float centre, float var, float x)
-{
-    const float d = x - centre;
-    return expf(-0.5f * d * d / var);
-}
-
 // math::RasterBinSizer<vol_raster::config> (raster_bin_sizers.h:271-485)
 struct BinSizer {
     float m[kRasterBins], b[kRasterBins], s[kRasterBins];
@@ -116,8 +110,8 @@ struct BinSizer {
         s[L] = sd;
         // insertion from the back: swap while the left neighbour lies further
         bool moving = true;
-#pragma unroll
-        for (int i = L; i > 0; --i) {
+        static_for<L>([&](auto q) {
+            constexpr int i = L - q;
             const bool sw = moving && b[i - 1] > b[i];
             const float bl = b[i - 1], br = b[i], sl = s[i - 1], sr = s[i], ml = m[i - 1], mr = m[i];
             b[i - 1] = sw ? br : bl;
@@ -127,37 +121,35 @@ struct BinSizer {
             m[i - 1] = sw ? mr : ml;
             m[i] = sw ? ml : mr;
             moving = sw;
-        }
+        });
         if (!(m[L] > 0.f))
             return;
         // every slot is taken: merge the cheapest adjacent pair
         float tr[L];
         float t = 1.f;
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-            t *= expf(-m[i]);
+        static_for<L>([&](auto i) {
+            t *= __builtin_amdgcn_exp2f(m[i] * -1.4426950408889634f);
             tr[i] = t;
-        }
+        });
         int best = -1;
         float best_val = __builtin_inff();
-#pragma unroll
-        for (int j = 0; j < L; ++j) {
-            const float ta = j == 0 ? 1.f : tr[j - 1];
-            float nm, nc, nsd;
-            merge(ta, tr[j], j, &nm, &nc, &nsd);
-            const float v = tr[j] * (kl(b[j], s[j], nc, nsd) + kl(b[j + 1], s[j + 1], nc, nsd));
+        static_for<L>([&](auto j) {
+            float ta = 1.f;
+            if constexpr (j > 0)
+                ta = tr[j - 1];
+            const float v = tr[j] * merge_cost(ta, tr[j], m[j], m[j + 1], b[j], b[j + 1], s[j], s[j + 1]);
             if (v < best_val) {
                 best_val = v;
                 best = j;
             }
-        }
+        });
         // the reference asserts a candidate exists; with none its merge would
         // index slot -1, here slot 0 merges
         best = best < 0 ? 0 : best;
         // gather the pair (best, best + 1) without a runtime index
         float ba = b[0], bb = b[1], sa = s[0], sb = s[1], ma = m[0], mb = m[1], tb_a = 1.f, tb_b = tr[0];
-#pragma unroll
-        for (int j = 1; j < L; ++j) {
+        static_for<L - 1>([&](auto q) {
+            constexpr int j = q + 1;
             const bool h = best == j;
             ba = h ? b[j] : ba;
             bb = h ? b[j + 1] : bb;
@@ -167,24 +159,37 @@ struct BinSizer {
             mb = h ? m[j + 1] : mb;
             tb_a = h ? tr[j - 1] : tb_a;
             tb_b = h ? tr[j] : tb_b;
-        }
+        });
         float nm, nc, nsd;
         merge_values(tb_a, tb_b, ma, mb, ba, bb, sa, sb, &nm, &nc, &nsd);
-#pragma unroll
-        for (int j = 0; j < L; ++j) {
+        static_for<L>([&](auto j) {
             const bool here = j == best, after = j > best;
-            const float bn = j + 1 < kRasterBins ? b[j + 1] : b[j];
-            const float sn = j + 1 < kRasterBins ? s[j + 1] : s[j];
-            const float mn = j + 1 < kRasterBins ? m[j + 1] : m[j];
-            b[j] = here ? nc : (after ? bn : b[j]);
-            s[j] = here ? nsd : (after ? sn : s[j]);
-            m[j] = here ? nm : (after ? mn : m[j]);
-        }
+            b[j] = here ? nc : (after ? b[j + 1] : b[j]);
+            s[j] = here ? nsd : (after ? s[j + 1] : s[j]);
+            m[j] = here ? nm : (after ? m[j + 1] : m[j]);
+        });
     }
 
-    static __device__ __forceinline__ float kl(float c1, float sd1, float c2, float sd2)
+    // kl(a, merged) + kl(b, merged) of two adjacent slots and their merge, kl of
+    // normals (c1, s1), (c2, s2) being ((c1 - c2)^2 + s1^2 - s2^2) / (2 s2^2) +
+    // log(s2 / s1): both logarithms as one, no square root (only variances are
+    // needed), and the hardware reciprocal.  A merge computes 31 of these, which
+    // was two thirds of pass 1's instructions as five divisions, two logarithms
+    // and a square root each.
+    static __device__ __forceinline__ float merge_cost(float tb_a, float tb_b, float ma, float mb, float ba, float bb, float sa, float sb)
     {
-        return ((c1 - c2) * (c1 - c2) + sd1 * sd1 - sd2 * sd2) / (2.f * (sd2 * sd2)) + logf(sd2 / sd1);
+        const float xa = tb_a * ma, xb = tb_b * mb;
+        const float x = xa + xb;
+        const float pa = x >= 0.0000001f ? fminf_ordered(xa * __builtin_amdgcn_rcpf(x), 0.999999f) : 0.5f;
+        const float pb = 1.f - pa;
+        const float nc = fmaf(pa, ba, pb * bb);
+        const float va = sa * sa, vb = sb * sb;
+        const float da = ba - nc, db = bb - nc;
+        const float qa = fmaf(da, da, va), qb = fmaf(db, db, vb);
+        const float nv = fmaf(pa, qa, pb * qb);
+        const float inv = __builtin_amdgcn_rcpf(nv);
+        const float ratio = (nv * __builtin_amdgcn_rcpf(va)) * (nv * __builtin_amdgcn_rcpf(vb));
+        return 0.5f * (fmaf(qa - nv, inv, (qb - nv) * inv) + logf(ratio));
     }
 
     static __device__ __forceinline__ void merge_values(float tb_a, float tb_b, float ma, float mb, float ba, float bb, float sa, float sb,
@@ -204,11 +209,6 @@ struct BinSizer {
 
     // std::min(a, b) = b < a ? b : a
     static __device__ __forceinline__ float fminf_ordered(float a, float b) { return b < a ? b : a; }
-
-    __device__ __forceinline__ void merge(float tb_a, float tb_b, int j, float* nm, float* nc, float* nsd) const
-    {
-        merge_values(tb_a, tb_b, m[j], m[j + 1], b[j], b[j + 1], s[j], s[j + 1], nm, nc, nsd);
-    }
 
     __device__ __forceinline__ bool full(float threshold) const { return acc >= threshold; }
 
@@ -266,11 +266,52 @@ __device__ __forceinline__ Linear fit_channel(float total, float el, float er, f
     return f;
 }
 
-__device__ __forceinline__ float sample_channel(const Linear& f, float t)
+// The channel over the bin's steps, for the integration's inner loop: at step i
+// (midpoint (i + 1/2) dt) the value times dt is
+//   max(med3(l0 + l1 i, r0 + r1 i, pick), 0)
+// of the left and the right segment's lines.  The two segments meet at t1 = t2,
+// where the larger line is the one in force if the channel is convex there and
+// the smaller if it is concave (pick = +inf, -inf: med3 is their max, min); with
+// a gap of zeros between t1 and t2 each line is negative beyond its end, so
+// the larger, and 0, is in force.
+struct StepLines {
+    float l0, l1, r0, r1, pick;
+};
+
+__device__ __forceinline__ StepLines step_lines(const Linear& f, float t_right, float dt)
 {
-    const float left = f.d0 + f.k0 * t;
-    const float right = f.d0 + f.t1 * f.k0 + (t - f.t2) * f.k2;
-    return t <= f.t1 ? left : (t <= f.t2 ? 0.f : right);
+    const float base = f.d0 + f.t1 * f.k0; // the right line at t2
+    float l0 = f.d0, l1 = f.k0, r0 = base - f.t2 * f.k2, r1 = f.k2;
+    const bool apart = f.t2 > f.t1;
+    if (apart && f.d0 == 0.f && f.k0 == 0.f && f.k2 == 0.f) {
+        r0 = 0.f; // an empty channel
+    } else if (apart) {
+        r0 = -(f.t2 * f.k2); // the left line ends at 0
+    } else if (!(f.t1 > 0.f)) {
+        l0 = r0; // no left segment
+        l1 = r1;
+    } else if (f.k2 == 0.f && !(f.t1 < t_right)) {
+        r0 = l0; // no right segment
+        r1 = l1;
+    }
+    const float pick = !apart && f.k0 > f.k2 ? -__builtin_inff() : __builtin_inff();
+    const float h = 0.5f * dt;
+    return { fmaf(l1, h, l0) * dt, l1 * dt * dt, fmaf(r1, h, r0) * dt, r1 * dt * dt, pick };
+}
+
+__device__ __forceinline__ float step_value(const StepLines& c, float i)
+{
+    return fmaxf(__builtin_amdgcn_fmed3f(fmaf(c.l1, i, c.l0), fmaf(c.r1, i, c.r0), c.pick), 0.f);
+}
+
+// The distance from the centre beyond which every bin holds less than the
+// 1e-4 that counts (see far_radius in the marcher): z^2 = 2 ln(w 5 750) leaves
+// at most 0.87e-4, the rest covers the cdf's rounding (1.2e-7 of w) up to w = 100
+__device__ __forceinline__ float raster_far(float w, float var)
+{
+    const float z2 = 1.3862943611f * (__builtin_amdgcn_logf(w) + 12.4893f);
+    const float r = __builtin_amdgcn_sqrtf(fmaxf(z2, 0.f) * var) * 1.0001f;
+    return w > 100.f ? __builtin_inff() : r;
 }
 
 struct RasterArgs {
@@ -291,11 +332,41 @@ struct RasterArgs {
     float* framebuffer;
 };
 
-__global__ __launch_bounds__(kThreads) void k_raster_render(RasterArgs a)
+// What a wave knows of the first 64 kSeenWords entries of its tile's list: the
+// entries it has tested and those whose mass on every pixel's ray is at most the
+// 1e-3 that the rasterisation asks for, which no chunk needs to visit again
+constexpr int kSeenWords = 64;
+
+// Where along the tile's rays a Gaussian matters to the bins (gaussian_window,
+// E + z^2 <= 2 ln M + 2 ln 5 750 for raster_far's cut), and how far its density
+// at a border is not zero in float (z = 13.5: the last border takes it from
+// every Gaussian).  One entry per lane.
+struct RasterWindow {
+    float lo, hi, trail;
+};
+
+__device__ __forceinline__ RasterWindow raster_window(const float* A, float det, const float* m, float mass_norm3, const TileAxis& ax)
+{
+    const float inf = __builtin_inff();
+    const GaussianExtent e = gaussian_extent(A, det, m, mass_norm3, ax);
+    if (!e.bounded || !(e.mass < 99.f))
+        return RasterWindow { -inf, inf, inf };
+    if (e.mass < 0.00099f)
+        return RasterWindow { inf, -inf, -inf }; // at most 1e-3 on every ray
+    const float half = extent_half(e, 18.f);
+    return RasterWindow { e.len - half, e.len + half, e.len + extent_half(e, 185.f) };
+}
+
+__global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
 {
     __shared__ float s_mu[3][kThreads];
     __shared__ float s_inv[6][kThreads];
+    __shared__ float s_off[3][kThreads]; // mu - camera
+    __shared__ float s_norm3[kThreads];
     __shared__ float s_mass[kThreads];
+    __shared__ RasterWindow s_win[kThreads];
+    __shared__ float s_axis[4];
+    __shared__ uint64_t s_seen[kThreads / 64][2][kSeenWords];
     __shared__ float s_rgb[3][kThreads];
     __shared__ float s_border[kThreads * kBorderStride];
     // the reference returns before rendering when no Gaussian is binned
@@ -322,10 +393,15 @@ __global__ __launch_bounds__(kThreads) void k_raster_render(RasterArgs a)
         for (int i = 0; i < 3; ++i)
             dir[i] = pv[i] * inv_len;
     }
+    const TileAxis axis = tile_axis<float>(dir, inside, s_axis);
     const uint32_t first = a.ranges[2 * tile], last = a.ranges[2 * tile + 1];
     const int n_rounds = int((last - first + kThreads - 1) / kThreads);
 
+    int staged = -1; // the batch in LDS (the lists of most tiles fit one)
     const auto stage = [&](int round) {
+        if (staged == round)
+            return;
+        __syncthreads(); // the previous batch has been read
         const uint32_t k = first + uint32_t(round) * kThreads + uint32_t(t_id);
         if (k < last) {
             const uint32_t id = a.point_list[k];
@@ -334,16 +410,27 @@ __global__ __launch_bounds__(kThreads) void k_raster_render(RasterArgs a)
                 s_mu[c][t_id] = a.means[3 * id + c];
                 s_rgb[c][t_id] = a.rgb[3 * id + c];
             }
+            float A[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c)
-                s_inv[c][t_id] = a.inv_cov[6 * id + c];
-            s_mass[t_id] = a.mass[id];
+                s_inv[c][t_id] = A[c] = a.inv_cov[6 * id + c];
+            float m[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                s_off[c][t_id] = m[c] = s_mu[c][t_id] - a.pos[c];
+            const float det = sym3_det(A), norm3 = ray_norm3(det), mass = a.mass[id];
+            s_norm3[t_id] = norm3;
+            s_mass[t_id] = mass;
+            s_win[t_id] = raster_window(A, det, m, mass * norm3, axis);
         }
+        __syncthreads();
+        staged = round;
     };
     const auto ray1d = [&](int j) {
         const float mu[3] = { s_mu[0][j], s_mu[1][j], s_mu[2][j] };
         const float A[6] = { s_inv[0][j], s_inv[1][j], s_inv[2][j], s_inv[3][j], s_inv[4][j], s_inv[5][j] };
-        return intersect_ray(mu, A, a.pos, dir);
+        const float m[3] = { s_off[0][j], s_off[1][j], s_off[2][j] };
+        return intersect_ray_pre(mu, A, m, s_norm3[j], a.pos, dir);
     };
 
     // ---------------------------------------------------------------- pass 1
@@ -351,26 +438,53 @@ __global__ __launch_bounds__(kThreads) void k_raster_render(RasterArgs a)
     z.init();
     if (a.mode != 1) { // Bins mode renders the background only
         bool done = !inside;
+        // A pixel's accepted Gaussians wait here, so that one addition to the
+        // bins serves pixels that took different Gaussians.  Each is added
+        // exactly as if it had been at once; what waits when the bins are full
+        // is dropped.
+        constexpr int Q = 4;
+        float q_mor[Q] = { 0.f, 0.f, 0.f, 0.f }, q_centre[Q] = { 0.f, 0.f, 0.f, 0.f }, q_sd[Q] = { 0.f, 0.f, 0.f, 0.f };
+        int waiting = 0;
         for (int r = 0; r < n_rounds; ++r) {
             if (__syncthreads_and(done))
                 break;
             stage(r);
-            __syncthreads();
-            if (done)
-                continue;
             const int count = int(min(uint32_t(kThreads), last - first - uint32_t(r) * kThreads));
-            for (int j = 0; j < count; ++j) {
-                const Ray1d<float> g = ray1d(j);
-                const float mor = g.weight * s_mass[j];
-                if (mor < 0.001f || mor > 1000.f)
-                    continue;
-                if (g.var <= 0.f)
-                    continue;
-                z.add(mor, g.centre, sqrt_rn(g.var));
-                if (z.full(a.mass_threshold)) {
-                    done = true;
-                    break;
+            int j = 0;
+            while (true) {
+                const bool visit = j < count && __builtin_amdgcn_ballot_w64(!done) != 0;
+                if (visit) {
+                    const Ray1d<float> g = ray1d(j);
+                    const float mor = g.weight * s_mass[j];
+                    const bool take = !done && !(mor < 0.001f || mor > 1000.f) && !(g.var <= 0.f);
+                    const float sd = sqrt_rn(g.var);
+                    static_for<Q>([&](auto k) {
+                        const bool here = take && waiting == k;
+                        q_mor[k] = here ? mor : q_mor[k];
+                        q_centre[k] = here ? g.centre : q_centre[k];
+                        q_sd[k] = here ? sd : q_sd[k];
+                    });
+                    waiting += take ? 1 : 0;
+                    ++j;
                 }
+                const int limit = visit ? Q : 1;
+                while (__builtin_amdgcn_ballot_w64(waiting >= limit) != 0) {
+                    if (waiting > 0) {
+                        z.add(q_mor[0], q_centre[0], q_sd[0]);
+                        if (z.full(a.mass_threshold)) {
+                            done = true;
+                            waiting = 1;
+                        }
+                        --waiting;
+                    }
+                    static_for<Q - 1>([&](auto k) {
+                        q_mor[k] = q_mor[k + 1];
+                        q_centre[k] = q_centre[k + 1];
+                        q_sd[k] = q_sd[k + 1];
+                    });
+                }
+                if (!visit)
+                    break;
             }
         }
         __syncthreads();
@@ -392,100 +506,146 @@ __global__ __launch_bounds__(kThreads) void k_raster_render(RasterArgs a)
         float result[3] = { 0.f, 0.f, 0.f };
         float transparency = 1.f;
         const float max_distance = end_of(kRasterBins - 1);
+        const unsigned lane = lane_id();
+        uint64_t* rejected = s_seen[t_id / 64][0];
+        uint64_t* known = s_seen[t_id / 64][1];
+        rejected[lane] = known[lane] = 0;
+        __builtin_amdgcn_wave_barrier();
         for (int k0 = 0; k0 < kRasterBins; k0 += kChunk) {
             float bm[kChunk][4], be[kChunk + 1][4];
-#pragma unroll
-            for (int q = 0; q < kChunk; ++q)
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    bm[q][c] = 0.f;
-#pragma unroll
-            for (int q = 0; q <= kChunk; ++q)
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    be[q][c] = 0.f;
+            static_for<kChunk>([&](auto q) { bm[q][0] = bm[q][1] = bm[q][2] = bm[q][3] = 0.f; });
+            static_for<kChunk + 1>([&](auto q) { be[q][0] = be[q][1] = be[q][2] = be[q][3] = 0.f; });
             const bool last_chunk = k0 + kChunk == kRasterBins;
+            // the chunk's borders and, for the bin after it, one more
+            const float x_first = begin_of(k0), x_right = end_of(k0 + kChunk - 1);
+            const float x_end = last_chunk ? x_right : end_of(k0 + kChunk);
+            // the wave's part of the rays
+            const float w_first = wave_min(inside ? x_first : __builtin_inff()), w_end = wave_max(inside ? x_end : -__builtin_inff());
+            const float w_right = wave_min(inside ? x_right : __builtin_inff());
             for (int r = 0; r < n_rounds; ++r) {
-                __syncthreads();
                 stage(r);
-                __syncthreads();
-                if (!inside)
-                    continue;
                 const int count = int(min(uint32_t(kThreads), last - first - uint32_t(r) * kThreads));
-                for (int j = 0; j < count; ++j) {
-                    const Ray1d<float> g = ray1d(j);
-                    const float c = g.centre;
-                    const float var = g.var;
-                    const float inv_sd = 1.f / sqrt_rn(var);
-                    const float w = g.weight * s_mass[j];
-                    if (var <= 0.f || __builtin_isnan(var) || __builtin_isnan(w) || w > 100000.f)
-                        continue;
-                    if (w * (cdf_sd(c, inv_sd, max_distance) - cdf_sd(c, inv_sd, 0.f)) <= 0.001f)
-                        continue;
-                    const float rgb[3] = { s_rgb[0][j], s_rgb[1][j], s_rgb[2][j] };
-                    float cdf_start = cdf_sd(c, inv_sd, begin_of(k0));
-#pragma unroll
-                    for (int q = 0; q < kChunk; ++q) {
-                        const float cdf_end = cdf_sd(c, inv_sd, end_of(k0 + q));
-                        const float mq = (cdf_end - cdf_start) * w;
-                        cdf_start = cdf_end;
-                        if (mq < 0.0001f)
+                for (int j0 = 0; j0 < count; j0 += 64) {
+                    const int w_at = (r * kThreads + j0) / 64;
+                    const bool tracked = w_at < kSeenWords;
+                    uint64_t w_rej = tracked ? uniform_u64(rejected[w_at]) : 0, w_known = tracked ? uniform_u64(known[w_at]) : 0;
+                    const RasterWindow win = s_win[min(j0 + int(lane), count - 1)];
+                    // beyond the chunk nothing of it counts; before the last
+                    // chunk only its density at the last border does
+                    const bool met = !(win.lo > w_end) && (!(win.hi < w_first) || (last_chunk && !(win.trail < w_right)));
+                    const uint64_t meets = __builtin_amdgcn_ballot_w64(met) & valid_entries(j0, count);
+                    for (uint64_t word = meets & ~w_rej; word != 0; word &= word - 1) {
+                        const int jj = __builtin_ctzll(word), j = j0 + jj;
+                        const Ray1d<float> g = ray1d(j);
+                        const float c = g.centre;
+                        const float var = g.var;
+                        const float w = g.weight * s_mass[j];
+                        if (((w_known >> jj) & 1) == 0) {
+                            w_known |= uint64_t(1) << jj;
+                            if (__builtin_amdgcn_ballot_w64(inside && w > 0.001f) == 0)
+                                w_rej |= uint64_t(1) << jj; // the mass within the borders is no larger
+                        }
+                        const float inv_sd = 1.f / sqrt_rn(var);
+                        const float far = raster_far(w, var);
+                        bool need = inside && !(var <= 0.f || __builtin_isnan(var) || __builtin_isnan(w) || w > 100000.f);
+                        // the last chunk's right border is evaluated for every Gaussian
+                        need = need && w > 0.001f && (last_chunk || (c + far > x_first && c - far < x_end));
+                        if (__builtin_amdgcn_ballot_w64(need) == 0)
                             continue;
-#pragma unroll
-                        for (int ch = 0; ch < 3; ++ch)
-                            bm[q][ch] += rgb[ch] * mq;
-                        bm[q][3] += mq;
-                        const float e = w * eval_exponential(c, var, begin_of(k0 + q));
-#pragma unroll
-                        for (int ch = 0; ch < 3; ++ch)
-                            be[q][ch] += rgb[ch] * e;
-                        be[q][3] += e;
+                        // with both ends over 3.1 sd away 0.998 of the mass lies within
+                        const bool sure = w > 0.00101f && (max_distance - c) * inv_sd > 3.1f && c * inv_sd > 3.1f;
+                        if (__builtin_amdgcn_ballot_w64(need && !sure) != 0)
+                            need = need && (sure || !(w * (cdf_sd(c, inv_sd, max_distance) - cdf_sd(c, inv_sd, 0.f)) <= 0.001f));
+                        const float lo = need ? c - far : __builtin_inff(), hi = need ? c + far : -__builtin_inff();
+                        const float wk = need ? w : 0.f;
+                        const float rgb[3] = { s_rgb[0][j], s_rgb[1][j], s_rgb[2][j] };
+                        const float e_scale = -0.72134752044448170f * __builtin_amdgcn_rcpf(var); // exp(-d^2 / (2 var)) = 2^(e_scale d^2)
+                        float cdf_start = 0.f;
+                        bool have = false;
+                        static_for<kChunk / kGroup>([&](auto group) {
+                            constexpr int g0 = group * kGroup;
+                            const float x0 = begin_of(k0 + g0);
+                            if (__builtin_amdgcn_ballot_w64(hi > x0 && lo < end_of(k0 + g0 + kGroup - 1)) == 0) {
+                                have = false;
+                                return;
+                            }
+                            if (!have)
+                                cdf_start = cdf_sd(c, inv_sd, x0);
+                            have = true;
+                            float x = x0;
+                            static_for<kGroup>([&](auto i) {
+                                constexpr int q = g0 + i;
+                                const float xe = end_of(k0 + q);
+                                const float cdf_end = cdf_sd(c, inv_sd, xe);
+                                const float mass = (cdf_end - cdf_start) * wk;
+                                cdf_start = cdf_end;
+                                const bool on = !(mass < 0.0001f) && need;
+                                const float mq = on ? mass : 0.f;
+                                const float d = x - c;
+                                const float e = on ? wk * __builtin_amdgcn_exp2f(d * d * e_scale) : 0.f;
+                                x = xe;
+                                bm[q][0] = fmaf(rgb[0], mq, bm[q][0]);
+                                bm[q][1] = fmaf(rgb[1], mq, bm[q][1]);
+                                bm[q][2] = fmaf(rgb[2], mq, bm[q][2]);
+                                bm[q][3] += mq;
+                                be[q][0] = fmaf(rgb[0], e, be[q][0]);
+                                be[q][1] = fmaf(rgb[1], e, be[q][1]);
+                                be[q][2] = fmaf(rgb[2], e, be[q][2]);
+                                be[q][3] += e;
+                            });
+                        });
+                        // the evaluation at the chunk's right border belongs to the
+                        // next bin, added when that bin's mass passes (or, after the
+                        // last bin, always)
+                        const bool next = last_chunk ? need : (hi > x_right && lo < x_end);
+                        if (__builtin_amdgcn_ballot_w64(next) != 0) {
+                            bool add_right = next;
+                            if (!last_chunk)
+                                add_right = next && !((cdf_sd(c, inv_sd, x_end) - cdf_sd(c, inv_sd, x_right)) * wk < 0.0001f);
+                            const float d = x_right - c;
+                            const float e = add_right ? wk * __builtin_amdgcn_exp2f(d * d * e_scale) : 0.f;
+                            be[kChunk][0] = fmaf(rgb[0], e, be[kChunk][0]);
+                            be[kChunk][1] = fmaf(rgb[1], e, be[kChunk][1]);
+                            be[kChunk][2] = fmaf(rgb[2], e, be[kChunk][2]);
+                            be[kChunk][3] += e;
+                        }
                     }
-                    // the evaluation at the chunk's right border belongs to the
-                    // next bin, added when that bin's mass passes (or, after the
-                    // last bin, always)
-                    bool add_right = last_chunk;
-                    float x_right = max_distance;
-                    if (!last_chunk) {
-                        const float cdf_end = cdf_sd(c, inv_sd, end_of(k0 + kChunk));
-                        add_right = !((cdf_end - cdf_start) * w < 0.0001f);
-                        x_right = begin_of(k0 + kChunk);
+                    if (tracked && lane == 0) {
+                        rejected[w_at] = w_rej;
+                        known[w_at] = w_known;
                     }
-                    if (add_right) {
-                        const float e = w * eval_exponential(c, var, x_right);
-#pragma unroll
-                        for (int ch = 0; ch < 3; ++ch)
-                            be[kChunk][ch] += rgb[ch] * e;
-                        be[kChunk][3] += e;
-                    }
+                    __builtin_amdgcn_wave_barrier();
                 }
             }
-            // integrate the chunk's bins (piecewise_linear.h:152-178)
-#pragma unroll
-            for (int q = 0; q < kChunk; ++q) {
+            // integrate the chunk's bins (piecewise_linear.h:152-178): per step
+            // the channels times dt, the colours weighed with the transparency
+            // before the step.  A bin empty on the whole wave changes nothing.
+            static_for<kChunk>([&](auto q) {
                 const float t_right = end_of(k0 + q) - begin_of(k0 + q);
-                if (!(t_right > 0.f))
-                    continue;
-                Linear f[4];
-#pragma unroll
-                for (int ch = 0; ch < 4; ++ch)
-                    f[ch] = fit_channel(bm[q][ch], be[q][ch], be[q + 1][ch], t_right);
+                const bool some = t_right > 0.f && (bm[q][0] > 0.000001f || bm[q][1] > 0.000001f || bm[q][2] > 0.000001f || bm[q][3] > 0.000001f);
+                if (__builtin_amdgcn_ballot_w64(some) == 0)
+                    return;
                 const float dt = t_right / float(kRasterSteps);
-                float t = dt / 2.f;
+                StepLines f[4];
+                static_for<4>([&](auto ch) {
+                    f[ch] = some ? step_lines(fit_channel(bm[q][ch], be[q][ch], be[q + 1][ch], t_right), t_right, dt)
+                                 : StepLines { 0.f, 0.f, 0.f, 0.f, 0.f };
+                });
+                float i = 0.f;
+#pragma unroll 4
                 for (int st = 0; st < kRasterSteps; ++st) {
-                    const float e0 = sample_channel(f[0], t), e1 = sample_channel(f[1], t), e2 = sample_channel(f[2], t);
-                    const float e3 = sample_channel(f[3], t);
-                    result[0] += e0 * transparency * dt;
-                    result[1] += e1 * transparency * dt;
-                    result[2] += e2 * transparency * dt;
-                    transparency *= larger_of(0.f, 1.f - e3 * dt);
-                    t += dt;
+                    const float e0 = step_value(f[0], i), e1 = step_value(f[1], i), e2 = step_value(f[2], i), e3 = step_value(f[3], i);
+                    result[0] = fmaf(e0, transparency, result[0]);
+                    result[1] = fmaf(e1, transparency, result[1]);
+                    result[2] = fmaf(e2, transparency, result[2]);
+                    transparency *= fmaxf(1.f - e3, 0.f);
+                    i += 1.f;
                 }
-#pragma unroll
-                for (int ch = 0; ch < 3; ++ch)
-                    C[ch] = result[ch];
-            }
+            });
         }
+        C[0] = result[0];
+        C[1] = result[1];
+        C[2] = result[2];
     } else if (a.mode == 2) {
         const int bin = int(min(unsigned(a.debug_bin), unsigned(kRasterBins - 1)));
         const float dist = end_of(bin);
