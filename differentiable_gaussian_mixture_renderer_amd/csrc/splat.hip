@@ -493,33 +493,31 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const KeyT* __restrict__ ke
     ranges[2 * g + 1] = lo0 < lo1 ? lo1 : 0u;
 }
 
-// kBlendWaves independent waves per workgroup, one tile each, LDS private per wave
-template <int TW, int TH, int B>
+// kBlendWaves independent waves per workgroup, LDS private per wave, each on one
+// of a tile's SPLIT bands of TH / SPLIT rows (SPLIT waves walk the tile's list)
+template <int TW, int TH, int B, int SPLIT>
 __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_forward(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ point_list,
     const float2* __restrict__ xy, const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, int width, int height, int grid_x,
     int n_tiles, float bg0, float bg1, float bg2, float* __restrict__ framebuffer, float* __restrict__ final_T)
 {
     __shared__ BlendSmem<B> sm_all[kBlendWaves];
     const int wave = int(uniform(threadIdx.x / 64));
-    const int tile = xcd_tile(blockIdx.x, gridDim.x) * kBlendWaves + wave;
+    const int unit = xcd_tile(blockIdx.x, gridDim.x) * kBlendWaves + wave;
+    const int tile = unit / SPLIT, part = unit % SPLIT;
     if (tile >= n_tiles)
         return;
     BlendSmem<B>& sm = sm_all[wave];
     const uint32_t first = uniform(ranges[2 * tile]), last = uniform(ranges[2 * tile + 1]);
-    blend_tile_forward<TW, TH, B>(sm, first, last, (tile % grid_x) * TW, (tile / grid_x) * TH, width, height, bg0, bg1,
-        bg2, point_list, xy, conic_opacity, rgb, framebuffer, final_T);
+    blend_tile_forward<TW, TH / SPLIT, B>(sm, first, last, (tile % grid_x) * TW, (tile / grid_x) * TH + part * (TH / SPLIT), width, height, bg0,
+        bg1, bg2, point_list, xy, conic_opacity, rgb, framebuffer, final_T);
 }
 
-template <int TW, int TH, int B>
+template <int TW, int TH, int B, int SPLIT>
 __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_backward(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ point_list,
     const float2* __restrict__ xy, const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, int width, int height, int grid_x,
     int n_tiles, float bg0, float bg1, float bg2, const float* __restrict__ framebuffer, const float* __restrict__ final_T,
     const float* __restrict__ grad_fb, float* __restrict__ screen_grads, WavePriority prio)
 {
-    // kBwdSplit waves per tile, each on TH / kBwdSplit rows: the tile's list
-    // is walked once per part, and the longest tile's work is spread over
-    // kBwdSplit waves with less per-lane state
-    constexpr int SPLIT = (TW * TH / kBwdSplit >= 64) ? kBwdSplit : 1;
     __shared__ BlendSmemBwd<B> sm_all[kBlendWaves];
     const int wave = int(uniform(threadIdx.x / 64));
     const int unit = xcd_tile(blockIdx.x, gridDim.x) * kBlendWaves + wave;
@@ -671,18 +669,57 @@ size_t splat_workspace_bytes(int64_t n, int64_t cap, bool cull)
     return cv.used;
 }
 
+// Waves per tile: a wave walks its tile's list alone, so with fewer tiles than
+// the chip has wave slots the longest walk is the launch's time, and a wave on
+// a quarter of the tile's pixels takes a step in less than half the time.  With
+// the slots filled, the parts of a step that every wave repeats (fetching and
+// staging the list, the per-Gaussian terms and, in the backward, its reduction)
+// count instead.
+#ifndef DGMR_FWD_SPLIT_TILES
+#define DGMR_FWD_SPLIT_TILES 1024
+#endif
+#ifndef DGMR_BWD_SPLIT_TILES
+#define DGMR_BWD_SPLIT_TILES 1024
+#endif
+
+template <int TW, int TH, int SPLIT>
+static void launch_blend_fwd_as(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
+    const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T)
+{
+    const dim3 grid(unsigned(ceil_div64(int64_t(n_tiles) * SPLIT, kBlendWaves))), block(64 * kBlendWaves);
+    const float b0 = float(bg[0]), b1 = float(bg[1]), b2 = float(bg[2]);
+    if (batch == 64)
+        k_blend_forward<TW, TH, 64, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+    else if (batch == 128)
+        k_blend_forward<TW, TH, 128, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+    else
+        k_blend_forward<TW, TH, 256, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+}
+
 template <int TW, int TH>
 static void launch_blend_fwd(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
     const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T)
 {
-    const dim3 grid(unsigned(ceil_div64(n_tiles, kBlendWaves))), block(64 * kBlendWaves);
+    constexpr int SPLIT = TW * TH / 64;
+    if (SPLIT > 1 && n_tiles <= DGMR_FWD_SPLIT_TILES)
+        launch_blend_fwd_as<TW, TH, SPLIT>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T);
+    else
+        launch_blend_fwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T);
+}
+
+template <int TW, int TH, int SPLIT>
+static void launch_blend_bwd_as(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
+    const float4* co, const float* rgb, int W, int H, int gx, const double* bg, const float* fb, const float* T, const float* gfb, float* sg,
+    WavePriority prio)
+{
+    const dim3 grid(unsigned(ceil_div64(int64_t(n_tiles) * SPLIT, kBlendWaves))), block(64 * kBlendWaves);
     const float b0 = float(bg[0]), b1 = float(bg[1]), b2 = float(bg[2]);
     if (batch == 64)
-        k_blend_forward<TW, TH, 64><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+        k_blend_backward<TW, TH, 64, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, gfb, sg, prio);
     else if (batch == 128)
-        k_blend_forward<TW, TH, 128><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+        k_blend_backward<TW, TH, 128, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, gfb, sg, prio);
     else
-        k_blend_forward<TW, TH, 256><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+        k_blend_backward<TW, TH, 256, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, gfb, sg, prio);
 }
 
 template <int TW, int TH>
@@ -690,15 +727,11 @@ static void launch_blend_bwd(int batch, int n_tiles, hipStream_t st, const uint3
     const float4* co, const float* rgb, int W, int H, int gx, const double* bg, const float* fb, const float* T, const float* gfb, float* sg,
     WavePriority prio)
 {
-    constexpr int SPLIT = (TW * TH / kBwdSplit >= 64) ? kBwdSplit : 1;
-    const dim3 grid(unsigned(ceil_div64(int64_t(n_tiles) * SPLIT, kBlendWaves))), block(64 * kBlendWaves);
-    const float b0 = float(bg[0]), b1 = float(bg[1]), b2 = float(bg[2]);
-    if (batch == 64)
-        k_blend_backward<TW, TH, 64><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, gfb, sg, prio);
-    else if (batch == 128)
-        k_blend_backward<TW, TH, 128><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, gfb, sg, prio);
+    constexpr int SPLIT = TW * TH / 64;
+    if (SPLIT > 1 && n_tiles <= DGMR_BWD_SPLIT_TILES)
+        launch_blend_bwd_as<TW, TH, SPLIT>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, gfb, sg, prio);
     else
-        k_blend_backward<TW, TH, 256><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, gfb, sg, prio);
+        launch_blend_bwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, gfb, sg, prio);
 }
 
 void splat_blend_forward(const dgmr_tiling& t, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float* xy,

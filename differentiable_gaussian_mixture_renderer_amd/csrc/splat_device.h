@@ -631,12 +631,6 @@ __device__ __forceinline__ void blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
     }
 }
 
-// waves per tile in the plain blend backward
-#ifndef DGMR_BWD_SPLIT
-#define DGMR_BWD_SPLIT 1
-#endif
-constexpr int kBwdSplit = DGMR_BWD_SPLIT;
-
 // Issue priority of a backward blend wave from its tile's list length
 // (thresholds t1 < t2 < t3, set from the frame's mean list length): waves on
 // longer lists issue first on their SIMD, so they finish with the rest of the
