@@ -120,6 +120,23 @@ struct BatchBinning {
     int64_t max_view_tiles; // largest grid_x * grid_y over the views
 };
 
+// Prefix binning (single views without tight culling): bins->pair_capacity
+// holds the first pairs of the depth order, and what the extension of the lists
+// needs comes back here, valid until the workspace is used again.
+struct PrefixBinning {
+    const uint32_t* origin; // tile rectangles by position of the depth order
+    const uint32_t* size;
+    const uint32_t* ids;    // Gaussian ids by position of the depth order
+    const uint32_t* n_pairs;
+    uint32_t* used;         // cleared with the tile ranges, as group_noted and groups[0]
+    uint32_t* n_owners;
+    uint32_t* open;         // one word per wave of the blend
+    uint32_t* group_noted;  // one word per group of 8 x 8 tiles
+    uint32_t* groups;       // the number of open groups, then the groups
+    uint32_t* counts;       // counts_room words
+    int64_t counts_room;
+};
+
 // binning shared by both renderers (implemented with the splatter): depth sort,
 // scan, emission, pair sort, tile ranges.  The preprocess must have filled the
 // depth-key and id buffers returned by binning_key_buffers, and its records
@@ -130,7 +147,7 @@ struct BatchBinning {
 // truncated, in-bounds binning that the caller reports as DGMR_ERR_CAPACITY.
 int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const void* xy, bool xy_double, bool bin_rects_written, bool cull,
     int grid_x, int grid_y, int tile_w, int tile_h, dgmr_binning* bins, Carver& cv, PendingCount* pending, hipStream_t st,
-    const BatchBinning* batch);
+    const BatchBinning* batch, PrefixBinning* prefix = nullptr);
 // the preprocess's outputs in the workspace: depth keys, ids and the
 // per-Gaussian records (cull: ReachRec; otherwise uint2 bin rectangles
 // (first tile y0 * grid_x + x0, (y1 - y0) << 16 | (x1 - x0)), zero when culled).

@@ -71,7 +71,7 @@ constexpr int kEmitWindow = 2048; // owners a block stages in LDS (more take the
 // [offsets[k], offsets[k + 1]) and writes the entries whose pair falls in its
 // range, so each entry is written exactly once and no block searches.
 __global__ void k_emit_bounds(int64_t n, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ n_pairs, uint32_t capacity,
-    uint32_t block_pairs, uint32_t* __restrict__ bounds)
+    uint32_t block_pairs, uint32_t* __restrict__ bounds, uint32_t* __restrict__ n_owners)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k >= n)
@@ -79,7 +79,10 @@ __global__ void k_emit_bounds(int64_t n, const uint32_t* __restrict__ offsets, c
     const uint64_t total = *n_pairs;
     const uint64_t R = min(total, uint64_t(capacity)); // pairs past the capacity are not emitted
     const uint64_t lo = offsets[k];
-    const uint64_t hi = min(k + 1 < n ? uint64_t(offsets[k + 1]) : total, R);
+    const uint64_t next = k + 1 < n ? uint64_t(offsets[k + 1]) : total;
+    if (n_owners && lo < total && next == total)
+        *n_owners = uint32_t(k + 1); // the last position that owns pairs
+    const uint64_t hi = min(next, R);
     if (lo >= hi)
         return;
     for (uint64_t b = (lo + block_pairs - 1) / block_pairs; b * block_pairs < hi; ++b)
@@ -113,6 +116,13 @@ __device__ __forceinline__ void owner_rect(uint32_t id, const int32_t* __restric
     *shape = (uint32_t(gx) << 16) | uint32_t(c - a);
 }
 
+// Tile rectangles by position of the depth order for the lists' extension (null: not
+// wanted): (row << 16 | column) of the first tile, (rows << 16 | columns)
+struct PrefixRects {
+    uint32_t* origin;
+    uint32_t* size;
+};
+
 // Per position j of the depth order: the pair count of Gaussian ids[j] (for
 // the scan) and its tile rectangle (for the emission).  The random reads of
 // per-Gaussian data happen here, in a streaming kernel, so the emission reads
@@ -123,7 +133,7 @@ __global__ __launch_bounds__(256) void k_gather_owners(int64_t n, const uint32_t
     const uint2* __restrict__ bin_rects,
     const int32_t* __restrict__ rects, const uint32_t* __restrict__ tiles, const S* __restrict__ xy, int grid_x, int grid_y, int tile_w,
     int tile_h, const int4* __restrict__ views, int64_t n_per_view, uint32_t* __restrict__ counts, uint2* __restrict__ owner_rects,
-    ScanState scan)
+    ScanState scan, PrefixRects prefix)
 {
     scan_clear(scan); // for the scan of counts that follows
     const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -144,6 +154,11 @@ __global__ __launch_bounds__(256) void k_gather_owners(int64_t n, const uint32_t
         start = r.x;
         shape = cols * rows == 0 ? 0u : (gx << 16) | cols;
         count = cols * rows;
+        if (prefix.origin) {
+            const uint32_t y = start / gx;
+            prefix.origin[j] = (y << 16) | (start - y * gx);
+            prefix.size[j] = r.y;
+        }
     } else {
         owner_rect(id, rects, tiles, xy, grid_x, grid_y, tile_w, tile_h, views, n_per_view, &start, &shape);
         count = tiles[id];
@@ -446,11 +461,17 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_pairs(int64_t n, const ui
 template <class KeyT>
 __global__ __launch_bounds__(256) void k_tile_ranges(const KeyT* __restrict__ keys, const uint32_t* __restrict__ vals,
     const uint32_t* __restrict__ n_pairs, uint32_t capacity, const int4* __restrict__ views, int n_views, int64_t n_per_view, int64_t n_tiles,
-    uint32_t* __restrict__ ranges)
+    uint32_t* __restrict__ ranges, uint32_t* __restrict__ used, uint32_t* __restrict__ groups, uint32_t* __restrict__ group_noted)
 {
     const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (g >= n_tiles)
         return;
+    if (used) {
+        // for the blend and the extension of the lists (no more groups than tiles)
+        group_noted[g] = 0;
+        if (g == 0)
+            *used = groups[0] = 0;
+    }
     const uint32_t R = min(*n_pairs, capacity);
     uint32_t t0 = uint32_t(g), t1 = uint32_t(g) + 1;
     uint64_t b0 = 0, b1 = 0;
@@ -493,23 +514,260 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const KeyT* __restrict__ ke
     ranges[2 * g + 1] = lo0 < lo1 ? lo1 : 0u;
 }
 
+// prefix binning (below): open notes the tiles whose list ended with an open
+// pixel; the second pass (again) blends only those, when there are any
+struct PrefixPass {
+    uint32_t* open;        // [tiles * waves per tile], null: whole lists
+    uint32_t* groups;      // [0]: number of groups of 8 x 8 tiles with an open one, then their numbers
+    uint32_t* group_noted; // [groups], 0 before the blend
+    const uint32_t* n_pairs;
+    uint32_t pairs;
+    bool again;
+};
+
 // kBlendWaves independent waves per workgroup, LDS private per wave, each on one
 // of a tile's SPLIT bands of TH / SPLIT rows (SPLIT waves walk the tile's list)
 template <int TW, int TH, int B, int SPLIT>
 __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_forward(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ point_list,
     const float2* __restrict__ xy, const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, int width, int height, int grid_x,
-    int n_tiles, float bg0, float bg1, float bg2, float* __restrict__ framebuffer, float* __restrict__ final_T)
+    int n_tiles, float bg0, float bg1, float bg2, float* __restrict__ framebuffer, float* __restrict__ final_T, PrefixPass prefix)
 {
     __shared__ BlendSmem<B> sm_all[kBlendWaves];
+    if (prefix.again && *prefix.n_pairs <= prefix.pairs)
+        return; // the lists were whole the first time
     const int wave = int(uniform(threadIdx.x / 64));
     const int unit = xcd_tile(blockIdx.x, gridDim.x) * kBlendWaves + wave;
     const int tile = unit / SPLIT, part = unit % SPLIT;
     if (tile >= n_tiles)
         return;
+    if (prefix.again) {
+        uint32_t open = 0;
+        for (int k = 0; k < SPLIT; ++k)
+            open |= prefix.open[tile * SPLIT + k];
+        if (uniform(open) == 0)
+            return; // its list was not extended
+    }
     BlendSmem<B>& sm = sm_all[wave];
     const uint32_t first = uniform(ranges[2 * tile]), last = uniform(ranges[2 * tile + 1]);
-    blend_tile_forward<TW, TH / SPLIT, B>(sm, first, last, (tile % grid_x) * TW, (tile / grid_x) * TH + part * (TH / SPLIT), width, height, bg0,
-        bg1, bg2, point_list, xy, conic_opacity, rgb, framebuffer, final_T);
+    const bool open = blend_tile_forward<TW, TH / SPLIT, B>(sm, first, last, (tile % grid_x) * TW, (tile / grid_x) * TH + part * (TH / SPLIT),
+        width, height, bg0, bg1, bg2, point_list, xy, conic_opacity, rgb, framebuffer, final_T);
+    if (prefix.open && !prefix.again && lane_id() == 0) {
+        prefix.open[unit] = open ? 1u : 0u;
+        const int group = (tile / grid_x) / 8 * ((grid_x + 7) / 8) + (tile % grid_x) / 8;
+        if (open && atomicExch(&prefix.group_noted[group], 1u) == 0)
+            prefix.groups[1 + atomicAdd(&prefix.groups[0], 1u)] = uint32_t(group);
+    }
+}
+
+// ------------------------------------------------------------ prefix binning
+// A deep view's tiles saturate long before their lists end: 1M Gaussians at
+// 1920x1080 make 14.9M pairs, 1 827 per tile, of which a tile walks 76 on
+// average and 166 at most.  Emission and pair sort of all of them are
+// bandwidth bound and were a fifth of the forward.  With prefix binning only
+// the first pairs of the depth order (kPrefixPerTile per tile of the image) are
+// emitted and sorted, so every tile's list is a prefix of its whole list; the
+// blend notes the tiles whose list ends with a pixel still open, and
+// the extension builds those tiles' whole lists behind the sorted pairs from
+// the depth-ordered rectangles, for a second blend of these tiles.  Nothing
+// waits for the host: both launches leave at once when there is nothing to do.
+// (kPrefixMin: whole lists below three times the prefix, where the emission and
+// sort that is saved is small against an extension.)
+constexpr int64_t kPrefixPerTile = 256;
+constexpr int64_t kPrefixMin = 3;
+
+// the first pairs that a view of n_tiles tiles bins with prefix binning, 0 when
+// its whole lists are binned
+static int64_t prefix_pairs(int64_t n_tiles, int64_t pair_capacity)
+{
+    const int64_t pairs = kPrefixPerTile * n_tiles;
+    return pair_capacity >= kPrefixMin * pairs && pair_capacity + pairs <= int64_t(UINT32_MAX) && n_tiles <= (int64_t(1) << 22) ? pairs : 0;
+}
+
+// The extension works on groups of 8 x 8 tiles, a lane per tile, over segments
+// of the depth order, a wave per (open group, segment): the wave reads 64
+// Gaussians' rectangles at a time and hands each that covers the group to all
+// lanes as a 64-bit tile mask, so a lane counts (k_extend_count) or appends
+// (k_extend_write) its tile's Gaussians in depth order.  In between
+// k_extend_place turns the counts into places.  With few open tiles the
+// segments spread them over the chip.
+struct ExtendArgs {
+    const uint32_t* n_pairs;
+    uint32_t prefix;
+    uint64_t capacity;     // entries of point_list
+    const uint32_t* n_owners;
+    const uint32_t* origin;
+    const uint32_t* size;
+    const uint32_t* ids;
+    const uint32_t* open;  // per wave of the blend
+    const uint32_t* groups; // [0]: number of open groups, then their numbers
+    uint32_t* counts;      // [groups * segments * 64]
+    uint32_t* used;
+    int split, grid_x, grid_y, segments;
+};
+
+constexpr int kExtendBlocks = 1024;
+
+// this lane's tile of group g: whether the blend left it open
+__device__ __forceinline__ bool extend_lane_open(const ExtendArgs& a, int g, int* gx0, int* gy0, int* tile)
+{
+    const int groups_x = (a.grid_x + 7) / 8;
+    *gx0 = g % groups_x * 8;
+    *gy0 = g / groups_x * 8;
+    const int lane = int(lane_id());
+    const int tx = *gx0 + lane % 8, ty = *gy0 + lane / 8;
+    *tile = ty * a.grid_x + tx;
+    uint32_t any = 0;
+    if (tx < a.grid_x && ty < a.grid_y)
+        for (int k = 0; k < a.split; ++k)
+            any |= a.open[int64_t(*tile) * a.split + k];
+    return any != 0;
+}
+
+// calls f(id position, this lane's tile is covered) for the positions of segment
+// `seg` that cover an open tile of the group, in order
+template <class F>
+__device__ __forceinline__ void extend_walk(const ExtendArgs& a, int gx0, int gy0, int seg, uint64_t open_tiles, F&& f)
+{
+    const uint32_t n = *a.n_owners;
+    const uint32_t per = (n + uint32_t(a.segments) * 64 - 1) / (uint32_t(a.segments) * 64) * 64;
+    const uint64_t k0 = uint64_t(seg) * per;
+    const uint32_t k1 = uint32_t(min(uint64_t(n), k0 + per));
+    const unsigned lane = lane_id();
+    constexpr int U = 4; // rectangles in flight per lane
+    for (uint64_t kb = k0; kb < k1; kb += 64 * U) {
+        uint32_t o[U], sz[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t k = uint32_t(min(kb + uint64_t(64 * u) + lane, uint64_t(k1 - 1)));
+            o[u] = a.origin[k];
+            sz[u] = a.size[k];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t kbu = kb + uint64_t(64 * u);
+            uint64_t m = 0;
+            if (kbu + lane < k1) {
+                const int x0 = int(o[u] & 0xffffu) - gx0, y0 = int(o[u] >> 16) - gy0;
+                const int x1 = min(x0 + int(sz[u] & 0xffffu), 8), y1 = min(y0 + int(sz[u] >> 16), 8);
+                const int xa = max(x0, 0), ya = max(y0, 0);
+                if (xa < x1 && ya < y1) {
+                    const uint64_t cols = ((0xffu << xa) & (0xffu >> (8 - x1))) * 0x0101010101010101ull;
+                    const uint64_t rows = (~uint64_t(0) << (8 * ya)) & (~uint64_t(0) >> (64 - 8 * y1));
+                    m = cols & rows & open_tiles;
+                }
+            }
+            for (uint64_t hit = __builtin_amdgcn_ballot_w64(m != 0); hit != 0; hit &= hit - 1) {
+                const int j = __builtin_ctzll(hit);
+                const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(m), j), hi = __builtin_amdgcn_readlane(uint32_t(m >> 32), j);
+                f(uint32_t(kbu) + uint32_t(j), (((lane & 32u) ? hi : lo) >> (lane & 31u)) & 1u);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_extend_count(ExtendArgs a)
+{
+    if (*a.n_pairs <= a.prefix)
+        return;
+    const uint32_t items = a.groups[0] * uint32_t(a.segments);
+    for (uint32_t i = uniform(blockIdx.x * 4 + threadIdx.x / 64); i < items; i += kExtendBlocks * 4) {
+        const int at = int(i / uint32_t(a.segments)), seg = int(i % uint32_t(a.segments));
+        int gx0, gy0, tile;
+        const bool open = extend_lane_open(a, int(a.groups[1 + at]), &gx0, &gy0, &tile);
+        uint32_t count = 0;
+        extend_walk(a, gx0, gy0, seg, __builtin_amdgcn_ballot_w64(open), [&](uint32_t, uint32_t covered) { count += covered; });
+        a.counts[int64_t(i) * 64 + lane_id()] = count;
+    }
+}
+
+// per open group: every (segment, tile) run's place in point_list, and the
+// tiles' ranges.  A wave takes a sixteenth of the segments.
+constexpr int kPlaceWaves = 16;
+__global__ __launch_bounds__(64 * kPlaceWaves) void k_extend_place(ExtendArgs a, uint32_t* __restrict__ ranges)
+{
+    __shared__ uint32_t s_run[kPlaceWaves][64];
+    __shared__ uint32_t s_fits;
+    if (*a.n_pairs <= a.prefix)
+        return;
+    const unsigned lane = lane_id();
+    const int wave = int(uniform(threadIdx.x / 64));
+    const int per = (a.segments + kPlaceWaves - 1) / kPlaceWaves;
+    const int s0 = min(a.segments, wave * per), s1 = min(a.segments, s0 + per);
+    for (uint32_t at = blockIdx.x; at < a.groups[0]; at += gridDim.x) {
+        uint32_t* rows = a.counts + int64_t(at) * a.segments * 64 + lane;
+        uint32_t sum = 0;
+#pragma unroll 8
+        for (int s = s0; s < s1; ++s)
+            sum += rows[s * 64];
+        s_run[wave][lane] = sum;
+        __syncthreads();
+        if (wave == 0) {
+            int gx0, gy0, tile;
+            const bool open = extend_lane_open(a, int(a.groups[1 + at]), &gx0, &gy0, &tile);
+            uint32_t total = 0;
+            for (int w = 0; w < kPlaceWaves; ++w)
+                total += s_run[w][lane];
+            uint32_t before = total; // inclusive sum over the lanes
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t v = __shfl_up(before, d);
+                before += lane >= unsigned(d) ? v : 0u;
+            }
+            const uint32_t all = __shfl(before, 63);
+            uint32_t base = 0;
+            if (lane == 0)
+                base = atomicAdd(a.used, all);
+            base = a.prefix + __shfl(base, 0);
+            const bool fits = uint64_t(base) + all <= a.capacity; // always, unless the pairs exceed the caller's capacity
+            uint32_t run = base + (before - total);
+            if (open) {
+                ranges[2 * tile] = fits && total ? run : 0u;
+                ranges[2 * tile + 1] = fits && total ? run + total : 0u;
+            }
+            for (int w = 0; w < kPlaceWaves; ++w) {
+                const uint32_t c = s_run[w][lane];
+                s_run[w][lane] = run;
+                run += c;
+            }
+            if (lane == 0)
+                s_fits = fits;
+        }
+        __syncthreads();
+        uint32_t run = s_run[wave][lane];
+        const bool fits = s_fits != 0;
+        for (int s = s0; s < s1; s += 8) {
+            uint32_t c[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                c[u] = s + u < s1 ? rows[(s + u) * 64] : 0u;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (s + u < s1)
+                    rows[(s + u) * 64] = fits ? run : 0xffffffffu;
+                run += c[u];
+            }
+        }
+        __syncthreads(); // s_run and s_fits are written again
+    }
+}
+
+__global__ __launch_bounds__(256) void k_extend_write(ExtendArgs a, uint32_t* __restrict__ point_list)
+{
+    if (*a.n_pairs <= a.prefix)
+        return;
+    const uint32_t items = a.groups[0] * uint32_t(a.segments);
+    for (uint32_t i = uniform(blockIdx.x * 4 + threadIdx.x / 64); i < items; i += kExtendBlocks * 4) {
+        const int at = int(i / uint32_t(a.segments)), seg = int(i % uint32_t(a.segments));
+        int gx0, gy0, tile;
+        const bool open = extend_lane_open(a, int(a.groups[1 + at]), &gx0, &gy0, &tile);
+        uint32_t place = a.counts[int64_t(i) * 64 + lane_id()];
+        if (uniform(place) == 0xffffffffu)
+            continue; // did not fit (the whole group)
+        extend_walk(a, gx0, gy0, seg, __builtin_amdgcn_ballot_w64(open), [&](uint32_t k, uint32_t covered) {
+            const uint32_t id = a.ids[k];
+            if (covered)
+                point_list[place++] = id;
+        });
+    }
 }
 
 template <int TW, int TH, int B, int SPLIT>
@@ -635,6 +893,7 @@ struct SplatWorkspace {
     uint32_t* counter;
     void* sort_scratch;
     void* scan_scratch;
+    uint32_t* prefix_open; // prefix binning: [4 tiles] open waves, [tiles] groups noted, [1 + tiles] open groups, counts
 };
 
 static SplatWorkspace carve_splat(Carver& cv, int64_t n, int64_t cap, bool cull)
@@ -659,6 +918,9 @@ static SplatWorkspace carve_splat(Carver& cv, int64_t n, int64_t cap, bool cull)
     w.owner_rects = reinterpret_cast<uint2*>(w.owner_reach);
     w.sort_scratch = cv.take<char>(radix_scratch_bytes(std::max(nn, cc)));
     w.scan_scratch = cv.take<char>(scan_scratch_bytes(nn, 2));
+    // the rest of the workspace: a caller of prefix binning has one for at least
+    // kPrefixMin times the pairs that are carved here, 6 words more per pair
+    w.prefix_open = reinterpret_cast<uint32_t*>(cv.base ? cv.base + cv.used : nullptr);
     return w;
 }
 
@@ -673,38 +935,38 @@ size_t splat_workspace_bytes(int64_t n, int64_t cap, bool cull)
 // the chip has wave slots the longest walk is the launch's time, and a wave on
 // a quarter of the tile's pixels takes a step in less than half the time.  With
 // the slots filled, the parts of a step that every wave repeats (fetching and
-// staging the list, the per-Gaussian terms and, in the backward, its reduction)
-// count instead.
-#ifndef DGMR_FWD_SPLIT_TILES
-#define DGMR_FWD_SPLIT_TILES 1024
-#endif
-#ifndef DGMR_BWD_SPLIT_TILES
-#define DGMR_BWD_SPLIT_TILES 1024
-#endif
+// staging the list, the per-Gaussian terms and, in the backward, its reduction
+// and atomics) count instead.  Measured in us with one / four waves per tile:
+// forward 98 / 38 at 192 tiles, 67 / 37 at 920, 66 / 52 and 55 / 49 at 3 600
+// (300k and 1M Gaussians), 108 / 96 and 75 / 82 at 8 160; backward 204 / 80 at
+// 192 tiles, 143 / 85 at 920, 130 / 98 at 1 200, 114 / 120 and 100 / 170 at
+// 1 900 (two waves per tile: 105 and 118).
+constexpr int kFwdSplitTiles = 6144;
+constexpr int kBwdSplitTiles = 1280;
 
 template <int TW, int TH, int SPLIT>
 static void launch_blend_fwd_as(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
-    const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T)
+    const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T, const PrefixPass& prefix)
 {
     const dim3 grid(unsigned(ceil_div64(int64_t(n_tiles) * SPLIT, kBlendWaves))), block(64 * kBlendWaves);
     const float b0 = float(bg[0]), b1 = float(bg[1]), b2 = float(bg[2]);
     if (batch == 64)
-        k_blend_forward<TW, TH, 64, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+        k_blend_forward<TW, TH, 64, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, prefix);
     else if (batch == 128)
-        k_blend_forward<TW, TH, 128, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+        k_blend_forward<TW, TH, 128, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, prefix);
     else
-        k_blend_forward<TW, TH, 256, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T);
+        k_blend_forward<TW, TH, 256, SPLIT><<<grid, block, 0, st>>>(ranges, pl, xy, co, rgb, W, H, gx, n_tiles, b0, b1, b2, fb, T, prefix);
 }
 
 template <int TW, int TH>
 static void launch_blend_fwd(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
-    const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T)
+    const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T, const PrefixPass& prefix)
 {
     constexpr int SPLIT = TW * TH / 64;
-    if (SPLIT > 1 && n_tiles <= DGMR_FWD_SPLIT_TILES)
-        launch_blend_fwd_as<TW, TH, SPLIT>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T);
+    if (SPLIT > 1 && n_tiles <= kFwdSplitTiles)
+        launch_blend_fwd_as<TW, TH, SPLIT>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, prefix);
     else
-        launch_blend_fwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T);
+        launch_blend_fwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, prefix);
 }
 
 template <int TW, int TH, int SPLIT>
@@ -728,23 +990,26 @@ static void launch_blend_bwd(int batch, int n_tiles, hipStream_t st, const uint3
     WavePriority prio)
 {
     constexpr int SPLIT = TW * TH / 64;
-    if (SPLIT > 1 && n_tiles <= DGMR_BWD_SPLIT_TILES)
+    if (SPLIT > 1 && n_tiles <= kBwdSplitTiles)
         launch_blend_bwd_as<TW, TH, SPLIT>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, gfb, sg, prio);
     else
         launch_blend_bwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, gfb, sg, prio);
 }
 
+// waves per tile of the forward blend at a tiling and tile count
+static int blend_forward_split(const dgmr_tiling& t, int64_t n_tiles) { return n_tiles <= kFwdSplitTiles ? t.tile_w * t.tile_h / 64 : 1; }
+
 void splat_blend_forward(const dgmr_tiling& t, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float* xy,
-    const float* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T)
+    const float* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T, const PrefixPass& prefix = PrefixPass {})
 {
     const auto* xy2 = reinterpret_cast<const float2*>(xy);
     const auto* co4 = reinterpret_cast<const float4*>(co);
     if (t.tile_w == 16)
-        launch_blend_fwd<16, 16>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T);
+        launch_blend_fwd<16, 16>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T, prefix);
     else if (t.tile_w == 8)
-        launch_blend_fwd<8, 8>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T);
+        launch_blend_fwd<8, 8>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T, prefix);
     else
-        launch_blend_fwd<32, 8>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T);
+        launch_blend_fwd<32, 8>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T, prefix);
 }
 
 void splat_blend_backward(const dgmr_tiling& t, int n_tiles, int64_t n_pairs, hipStream_t st, const uint32_t* ranges, const uint32_t* pl,
@@ -778,6 +1043,7 @@ struct EmitArgs {
     int n_views;
     int tile_w, tile_h;
     bool cull;
+    const PrefixBinning* prefix; // null: whole lists
 };
 
 // emission, pair sort on the tile bits, tile ranges; pair keys of type KeyT
@@ -799,7 +1065,7 @@ static int emit_sort_ranges(const EmitArgs& a, const SplatWorkspace& w, dgmr_bin
     {
         StageScope sc("bin.emit", st);
         pending->add_stage(sc.slot, 4.0 + sizeof(KeyT), 28.0 * double(a.n));
-        k_emit_bounds<<<a.blocks_n, 256, 0, st>>>(a.n, w.pair_offsets, w.counter, a.cap, block_pairs, w.emit_bounds);
+        k_emit_bounds<<<a.blocks_n, 256, 0, st>>>(a.n, w.pair_offsets, w.counter, a.cap, block_pairs, w.emit_bounds, a.prefix ? a.prefix->n_owners : nullptr);
         DGMR_HIP_CHECK(hipGetLastError());
         if (a.cull && per == kEmitPerLarge)
             k_emit_reach<KeyT, kEmitPerLarge><<<emit_blocks, kEmitThreads, 0, st>>>(w.counter, a.cap, a.sorted_ids, w.emit_bounds,
@@ -826,7 +1092,8 @@ static int emit_sort_ranges(const EmitArgs& a, const SplatWorkspace& w, dgmr_bin
         StageScope sc("bin.ranges", st);
         pending->add_stage(sc.slot, 0.0, 8.0 * double(a.n_tiles));
         k_tile_ranges<KeyT><<<unsigned(ceil_div64(a.n_tiles, 256)), 256, 0, st>>>(sorted_keys, sorted_vals, w.counter, a.cap, a.views,
-            a.n_views, a.n_per_view, a.n_tiles, bins->ranges);
+            a.n_views, a.n_per_view, a.n_tiles, bins->ranges, a.prefix ? a.prefix->used : nullptr,
+            a.prefix ? a.prefix->groups : nullptr, a.prefix ? a.prefix->group_noted : nullptr);
         DGMR_HIP_CHECK(hipGetLastError());
     }
     return DGMR_OK;
@@ -837,7 +1104,7 @@ static int emit_sort_ranges(const EmitArgs& a, const SplatWorkspace& w, dgmr_bin
 // the preprocess.  Returns the pair count through *n_pairs (host).
 int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const void* xy, bool xy_double, bool bin_rects_written, bool cull,
     int grid_x, int grid_y, int tile_w, int tile_h, dgmr_binning* bins, Carver& cv, PendingCount* pending, hipStream_t st,
-    const BatchBinning* batch)
+    const BatchBinning* batch, PrefixBinning* prefix)
 {
     const int4* views = batch ? batch->views : nullptr;
     const int64_t n_per_view = batch ? batch->n_per_view : 0;
@@ -881,6 +1148,15 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
         }
     }
     const uint32_t* sorted_ids = V;
+    // prefix binning: the sorted depth keys are not read again, their buffers
+    // hold the rectangles
+    PrefixRects rects_out { nullptr, nullptr };
+    if (prefix) {
+        rects_out = PrefixRects { K, K2 };
+        const int64_t tiles = int64_t(grid_x) * grid_y;
+        *prefix = PrefixBinning { K, K2, sorted_ids, w.counter, w.counter + 2, w.counter + 3, w.prefix_open, w.prefix_open + 4 * tiles,
+            w.prefix_open + 5 * tiles, w.prefix_open + 6 * tiles + 1, 4 * bins->pair_capacity };
+    }
     const unsigned blocks_n = unsigned(ceil_div64(n, 256));
     {
         StageScope sc("bin.scan", st, 44.0 * double(n));
@@ -895,13 +1171,13 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
                 sorted_ids, w.reach, tile_w, tile_h, w.counts, w.owner_reach, scan);
         else if (bin_rects_written)
             k_gather_owners<float, true><<<blocks_n, 256, 0, st>>>(n, n_sorted, sorted_ids, w.bin_rects, rects, tiles, static_cast<const float*>(xy),
-                grid_x, grid_y, tile_w, tile_h, views, n_per_view, w.counts, w.owner_rects, scan);
+                grid_x, grid_y, tile_w, tile_h, views, n_per_view, w.counts, w.owner_rects, scan, rects_out);
         else if (xy_double)
             k_gather_owners<double, false><<<blocks_n, 256, 0, st>>>(n, n_sorted, sorted_ids, w.bin_rects, rects, tiles,
-                static_cast<const double*>(xy), grid_x, grid_y, tile_w, tile_h, views, n_per_view, w.counts, w.owner_rects, scan);
+                static_cast<const double*>(xy), grid_x, grid_y, tile_w, tile_h, views, n_per_view, w.counts, w.owner_rects, scan, rects_out);
         else
             k_gather_owners<float, false><<<blocks_n, 256, 0, st>>>(n, n_sorted, sorted_ids, w.bin_rects, rects, tiles,
-                static_cast<const float*>(xy), grid_x, grid_y, tile_w, tile_h, views, n_per_view, w.counts, w.owner_rects, scan);
+                static_cast<const float*>(xy), grid_x, grid_y, tile_w, tile_h, views, n_per_view, w.counts, w.owner_rects, scan, rects_out);
         DGMR_HIP_CHECK(hipGetLastError());
         DGMR_HIP_CHECK(scan_u32_arrays(scans, n_scans, n, w.scan_scratch, st, true));
     }
@@ -919,7 +1195,7 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
     // traffic in emission and sort), else 32
     const int tile_bits = int(higher_msb(uint32_t(batch ? batch->max_view_tiles : n_tiles)));
     EmitArgs ea { n, blocks_n, uint32_t(cap), n_tiles, tile_bits, sorted_ids, views, n_per_view, batch ? int(batch->n_views) : 0, tile_w, tile_h,
-        cull };
+        cull, prefix };
     if (tile_bits <= 16)
         return emit_sort_ranges<uint16_t>(ea, w, bins, pending, st);
     return emit_sort_ranges<uint32_t>(ea, w, bins, pending, st);
@@ -943,18 +1219,9 @@ void binning_key_buffers(void* workspace, int64_t n, bool cull, uint32_t** keys,
 
 using namespace dgmr;
 
-extern "C" {
-
-int dgmr_workspace_size(int64_t n, int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, size_t* bytes)
-{
-    DGMR_ARG_CHECK(bytes && n >= 0 && valid_image(width, height) && valid_tiling(tiling) && pair_capacity >= 0, "dgmr_workspace_size: bad argument");
-    *bytes = splat_workspace_bytes(n, pair_capacity, tiling->cull != 0);
-    return DGMR_OK;
-}
-
-int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, dgmr_splat_geometry* geom,
+static int splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, dgmr_splat_geometry* geom,
     dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, dgmr_stats* stats,
-    dgmr_stream stream)
+    dgmr_stream stream, bool allow_prefix)
 {
     DGMR_ARG_CHECK(g && cam && geom && bins && framebuffer && final_transmittance && workspace, "dgmr_splat_forward: null argument");
     DGMR_ARG_CHECK(g->dtype == DGMR_F32, "dgmr_splat_forward: the splatter computes in float32");
@@ -993,17 +1260,40 @@ int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dg
     }
     Carver cv(workspace, workspace_bytes);
     PendingCount pending;
-    const int rc = bin_gaussians(n, geom->rects, geom->tiles_touched, geom->xy, false, true, cull, dc.grid_x, dc.grid_y, dc.tile_w, dc.tile_h, bins, cv,
-        &pending, st, nullptr);
+    const int64_t prefix = allow_prefix && !cull ? prefix_pairs(n_tiles, bins->pair_capacity) : 0;
+    PrefixBinning pb {};
+    dgmr_binning first = *bins;
+    if (prefix)
+        first.pair_capacity = prefix;
+    const int rc = bin_gaussians(n, geom->rects, geom->tiles_touched, geom->xy, false, true, cull, dc.grid_x, dc.grid_y, dc.tile_w, dc.tile_h, &first,
+        cv, &pending, st, nullptr, prefix ? &pb : nullptr);
     if (rc != DGMR_OK)
         return rc;
     int blend_slot = -1;
+    PrefixPass pass { pb.open, pb.groups, pb.group_noted, pb.n_pairs, uint32_t(prefix), false };
     {
         StageScope sc("splat.blend_forward", st);
         blend_slot = sc.slot;
         splat_blend_forward(*tiling, int(n_tiles), st, bins->ranges, bins->point_list, geom->xy, geom->conic_opacity, geom->rgb, cam->width,
-            cam->height, dc.grid_x, cam->background, framebuffer, final_transmittance);
+            cam->height, dc.grid_x, cam->background, framebuffer, final_transmittance, pass);
         DGMR_HIP_CHECK(hipGetLastError());
+        if (prefix) {
+            const int64_t groups = ceil_div64(dc.grid_x, 8) * ceil_div64(dc.grid_y, 8);
+            // as many segments as there is room for counts, at most 512
+            const int segments = int(std::min<int64_t>(512, pb.counts_room / (groups * 64)));
+            const ExtendArgs ea { pb.n_pairs, uint32_t(prefix), uint64_t(prefix + bins->pair_capacity), pb.n_owners, pb.origin, pb.size, pb.ids,
+                pb.open, pb.groups, pb.counts, pb.used, blend_forward_split(*tiling, n_tiles), dc.grid_x, dc.grid_y, segments };
+            k_extend_count<<<kExtendBlocks, 256, 0, st>>>(ea);
+            DGMR_HIP_CHECK(hipGetLastError());
+            k_extend_place<<<unsigned(std::min<int64_t>(groups, 256)), 64 * kPlaceWaves, 0, st>>>(ea, bins->ranges);
+            DGMR_HIP_CHECK(hipGetLastError());
+            k_extend_write<<<kExtendBlocks, 256, 0, st>>>(ea, bins->point_list);
+            DGMR_HIP_CHECK(hipGetLastError());
+            pass.again = true;
+            splat_blend_forward(*tiling, int(n_tiles), st, bins->ranges, bins->point_list, geom->xy, geom->conic_opacity, geom->rgb, cam->width,
+                cam->height, dc.grid_x, cam->background, framebuffer, final_transmittance, pass);
+            DGMR_HIP_CHECK(hipGetLastError());
+        }
     }
     pending.add_stage(blend_slot, 40.0, 16.0 * double(plane) + 8.0 * double(n_tiles));
     // every launch is queued: now wait for the pair count
@@ -1017,6 +1307,37 @@ int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dg
         return DGMR_ERR_CAPACITY;
     }
     return DGMR_OK;
+}
+
+extern "C" {
+
+int dgmr_workspace_size(int64_t n, int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, size_t* bytes)
+{
+    DGMR_ARG_CHECK(bytes && n >= 0 && valid_image(width, height) && valid_tiling(tiling) && pair_capacity >= 0, "dgmr_workspace_size: bad argument");
+    *bytes = splat_workspace_bytes(n, pair_capacity, tiling->cull != 0);
+    return DGMR_OK;
+}
+
+int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, dgmr_splat_geometry* geom,
+    dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, dgmr_stats* stats,
+    dgmr_stream stream)
+{
+    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream, false);
+}
+
+int dgmr_splat_prefix_pairs(int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, int64_t* pairs)
+{
+    DGMR_ARG_CHECK(pairs && valid_image(width, height) && valid_tiling(tiling) && pair_capacity >= 0, "dgmr_splat_prefix_pairs: bad argument");
+    const int64_t n_tiles = ceil_div64(width, tiling->tile_w) * ceil_div64(height, tiling->tile_h);
+    *pairs = tiling->cull ? 0 : prefix_pairs(n_tiles, pair_capacity);
+    return DGMR_OK;
+}
+
+int dgmr_splat_forward_prefix(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, dgmr_splat_geometry* geom,
+    dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, dgmr_stats* stats,
+    dgmr_stream stream)
+{
+    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream, true);
 }
 
 int dgmr_splat_backward(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, const dgmr_splat_geometry* geom,

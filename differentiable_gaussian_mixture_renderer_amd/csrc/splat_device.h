@@ -550,8 +550,10 @@ __device__ __forceinline__ float gauss_at(const LaneTerms& t, float c_scaled, fl
     return __builtin_amdgcn_exp2f(fmaf(fmaf(c_scaled, dy, t.bdx), dy, t.adx2));
 }
 
+// Returns whether some pixel of the tile would take more Gaussians than the
+// list holds.
 template <int TW, int TH, int B>
-__device__ __forceinline__ void blend_tile_forward(BlendSmem<B>& sm, uint32_t first, uint32_t last, int px0, int py0, int width, int height,
+__device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t first, uint32_t last, int px0, int py0, int width, int height,
     float bg0, float bg1, float bg2, const uint32_t* __restrict__ point_list, const float2* __restrict__ xy,
     const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, float* __restrict__ framebuffer, float* __restrict__ final_T)
 {
@@ -629,6 +631,11 @@ __device__ __forceinline__ void blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
             final_T[p] = Tk;
         }
     }
+    bool live = false;
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+        live |= T[k] > 0.f;
+    return wave_any(live);
 }
 
 // Issue priority of a backward blend wave from its tile's list length

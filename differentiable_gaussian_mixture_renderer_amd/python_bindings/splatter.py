@@ -38,11 +38,14 @@ CACHE_FIELDS = ("framebuffer", "rects", "rgb", "rgb_sh_clamped", "depths", "poin
 
 def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, proj_matrix, cam_position, background,
              render_width: int, render_height: int, tan_fovx: float, tan_fovy: float, sh_degree: int,
-             tile=None, batch: int = 0, scale_multiplier: float = 1.0, activation: int = N.DGMR_ACT_NONE, cull=None):
+             tile=None, batch: int = 0, scale_multiplier: float = 1.0, activation: int = N.DGMR_ACT_NONE, cull=None,
+             whole_lists: bool = True):
     """cull=True bins each Gaussian only into the tiles where its alpha can
     reach 1/255 (dgmr_tiling.cull): same image, transmittance and gradients,
     fewer pairs; b_point_list and i_ranges then differ from the reference's.
-    None: DEFAULT_CULL."""
+    None: DEFAULT_CULL.  whole_lists=False bins no more of a deep view than its
+    tiles can take (dgmr_splat_forward_prefix): same image, transmittance and
+    gradients, but b_point_list holds prefixes of the reference's lists."""
     cull = DEFAULT_CULL if cull is None else bool(cull)
     tile = tile or DEFAULT_TILING[0]
     batch = batch or DEFAULT_TILING[1]
@@ -74,12 +77,15 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
         stats = N.Stats()
         stream = C.stream_handle(dev)
         for _attempt in range(3):
-            point_list = torch.empty((max(cap, 1),), dtype=torch.int32, device=dev)
+            prefix = ctypes.c_int64(0)
+            if not whole_lists:
+                N.check(lib.dgmr_splat_prefix_pairs(W, H, ctypes.byref(tiling), cap, ctypes.byref(prefix)), "dgmr_splat_prefix_pairs")
+            point_list = torch.empty((max(cap + prefix.value, 1),), dtype=torch.int32, device=dev)
             bins = N.Binning(offsets.data_ptr(), point_list.data_ptr(), ranges.data_ptr(), cap)
             ws = C.workspace(dev, n, W, H, tiling, cap)
-            rc = lib.dgmr_splat_forward(ctypes.byref(g), ctypes.byref(cam), ctypes.byref(tiling), ctypes.byref(geom),
-                                        ctypes.byref(bins), fb.data_ptr(), T.data_ptr(), ws.data_ptr(), ws.numel(),
-                                        ctypes.byref(stats), stream)
+            forward = lib.dgmr_splat_forward_prefix if prefix.value else lib.dgmr_splat_forward
+            rc = forward(ctypes.byref(g), ctypes.byref(cam), ctypes.byref(tiling), ctypes.byref(geom), ctypes.byref(bins), fb.data_ptr(),
+                         T.data_ptr(), ws.data_ptr(), ws.numel(), ctypes.byref(stats), stream)
             if rc == N.DGMR_ERR_CAPACITY:
                 cap = int(stats.n_pairs * 1.25) + 1024
                 C.remember_capacity(dev, "splat", cap)
@@ -90,8 +96,11 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
             raise N.DgmrError(N.DGMR_ERR_CAPACITY, "dgmr_splat_forward", "pair capacity kept growing")
         R = int(stats.n_pairs)
         C.remember_capacity(dev, "splat", cap)
-    return [fb, rects, rgb, clamped, depths, xy, conic, tiles, offsets, ranges, point_list[:R], T,
-            torch.tensor([R], dtype=torch.int64)]
+    if R > prefix.value > 0:
+        R = prefix.value  # the pairs binned; extended lists lie behind them
+    else:
+        point_list = point_list[:R]
+    return [fb, rects, rgb, clamped, depths, xy, conic, tiles, offsets, ranges, point_list, T, torch.tensor([R], dtype=torch.int64)]
 
 
 def _backward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, proj_matrix, cam_position, background,
@@ -139,7 +148,7 @@ class Splatter(torch.autograd.Function):
     def forward(ctx, shs, opacity, means3D, scales, rotations, world_view_transform, full_proj_transform, camera_center, bg_color,
                 image_width: int, image_height: int, tanfovx: float, tanfovy: float, active_sh_degree: int):
         cache = cpp_binding.forward(shs, opacity, means3D, scales, rotations, world_view_transform, full_proj_transform, camera_center,
-                                    bg_color, image_width, image_height, tanfovx, tanfovy, active_sh_degree)
+                                    bg_color, image_width, image_height, tanfovx, tanfovy, active_sh_degree, whole_lists=False)
         ctx.scalars = (int(image_width), int(image_height), float(tanfovx), float(tanfovy), int(active_sh_degree))
         ctx.save_for_backward(shs, opacity, means3D, scales, rotations, world_view_transform, full_proj_transform, camera_center,
                               bg_color, *cache)
@@ -172,7 +181,7 @@ class SplatterActivated(torch.autograd.Function):
                 bg_color, image_width: int, image_height: int, tanfovx: float, tanfovy: float, active_sh_degree: int):
         cache = cpp_binding.forward(shs, opacity_logits, means3D, log_scales, rotations, world_view_transform, full_proj_transform,
                                     camera_center, bg_color, image_width, image_height, tanfovx, tanfovy, active_sh_degree,
-                                    activation=N.DGMR_ACT_LOG_NORM_SIGMOID)
+                                    activation=N.DGMR_ACT_LOG_NORM_SIGMOID, whole_lists=False)
         ctx.scalars = (int(image_width), int(image_height), float(tanfovx), float(tanfovy), int(active_sh_degree))
         ctx.save_for_backward(shs, opacity_logits, means3D, log_scales, rotations, world_view_transform, full_proj_transform,
                               camera_center, bg_color, *cache)

@@ -333,3 +333,90 @@ def test_backward_against_finite_differences_of_the_fp64_forward():
             print(f"{name}[{i},{j}]: fd {fd:.7g} (half step {fd2:.7g}), gpu {g:.7g}, rel {abs(g - fd) / max(abs(fd), 1e-30):.2g}")
             assert abs(fd - fd2) <= 1e-5 * abs(fd) + e, (name, i, j, "decision moved")
             assert abs(g - fd) <= 1e-3 * abs(fd) + 1e-4 * s + e, (name, i, j, fd, g)
+
+
+@pytest.mark.parametrize("kind", ["saturating", "half_open", "open", "whole"])
+@pytest.mark.parametrize("tile,w,h", [((16, 16), 203, 117), ((8, 8), 131, 77), ((32, 8), 97, 150)])
+def test_prefix_binning_equals_whole_lists(kind, tile, w, h):
+    """whole_lists=False bins a prefix of a deep view's depth order and extends
+    the lists of the tiles it leaves open: none, some (Gaussians near the view's
+    left half only) or all of them, at ragged tile grids.  The image and
+    transmittance equal whole lists' bit for bit, the gradients up to the order
+    of the atomic sums; an extended list equals the whole one.  "whole": a view
+    too shallow for a prefix keeps its lists."""
+    torch = _torch()
+    from differentiable_gaussian_mixture_renderer_amd import _common, scenes
+    from differentiable_gaussian_mixture_renderer_amd.python_bindings import splatter
+    n = 300 if kind == "whole" else 60_000
+    scene = scenes.make_scene(n, seed=6, extent=1.0, sh_degree=1)
+    opacity, scales = scene.opacity.copy(), scene.scales.copy()
+    if kind == "open":
+        opacity *= 0.004
+        scales *= 2.0
+    if kind == "half_open":
+        opacity[scene.means[:, 0] > 0.1] *= 0.01
+    t = math_tan(0.35)
+    cam = scenes.look_at_camera([0.0, 0.0, -4.0], [0.0, 0.0, 0.0], w, h, t * w / h, t)
+    dev = torch.device("cuda:0")
+    T = lambda a: torch.tensor(np.ascontiguousarray(a), device=dev)
+    args = [T(scene.sh), T(opacity), T(scene.means), T(scales), T(scene.rotations), T(cam.world_view_transform), T(cam.full_proj_transform),
+            T(cam.camera_center), T(np.array([0.1, 0.6, 0.3], np.float32)), w, h, cam.tan_fovx, cam.tan_fovy, 1]
+    print(f"[gpu prefix] {kind} {tile} {w}x{h}", flush=True)
+    whole = splatter.cpp_binding.forward(*args, tile=tile)
+    _common.remember_capacity(dev, "splat", int(whole[12][0]))
+    got = splatter.cpp_binding.forward(*args, tile=tile, whole_lists=False)
+    assert torch.equal(got[0], whole[0]) and torch.equal(got[11], whole[11])
+    tiles = whole[9].shape[0]
+    R, prefix = int(whole[12][0]), 256 * tiles
+    rw, rg = whole[9].cpu().numpy(), got[9].cpu().numpy()
+    lw, lg = rw[:, 1] - rw[:, 0], rg[:, 1] - rg[:, 0]
+    pw, pg = whole[10].cpu().numpy(), got[10].cpu().numpy()
+    extended = 0
+    for k in range(tiles):
+        a, b = pw[rw[k, 0]:rw[k, 1]], pg[rg[k, 0]:rg[k, 1]]
+        assert len(b) <= len(a) and np.array_equal(a[:len(b)], b), k
+        if rg[k, 0] >= prefix:
+            extended += 1
+            assert len(a) == len(b), k
+    print(f"R {R}, prefix {prefix}, extended {extended} of {tiles} tiles, listed {int(lg.sum())} of {int(lw.sum())}")
+    if kind == "whole":
+        assert R <= prefix and lg.sum() == R
+    else:
+        assert R >= 3 * prefix
+        assert {"saturating": lg.sum() < R and extended < tiles, "half_open": 0 < extended < tiles, "open": extended == (lw > 0).sum()}[kind]
+    grad = torch.randn(3, h, w, device=dev, generator=torch.Generator(device=dev).manual_seed(1))
+    gw = splatter.cpp_binding.backward(*args, grad, whole, tile=tile)
+    gg = splatter.cpp_binding.backward(*args, grad, got, tile=tile)
+    for name, a, b in zip(("sh", "opacity", "means", "scales", "rotations"), gw, gg):
+        assert float((a - b).norm()) <= 1e-5 * float(a.norm()), name
+
+
+def math_tan(v):
+    import math
+    return math.tan(v)
+
+
+@pytest.mark.parametrize("w,h", [(640, 512), (656, 512), (1536, 1024), (1552, 1024), (17, 3)])
+def test_blends_at_the_waves_per_tile_limits(w, h):
+    """1 280 / 1 312 tiles (the backward's limit of four waves per tile), 6 144 /
+    6 208 (the forward's), and a 17x3 image, at the bars of the other tests."""
+    torch = _torch()
+    from differentiable_gaussian_mixture_renderer_amd import scenes
+    scene = scenes.make_scene(1500, seed=9, extent=1.0, sh_degree=1)
+    t = math_tan(0.3)
+    cam = scenes.look_at_camera([0.1, 0.0, -4.0], [0.0, 0.0, 0.0], w, h, t * w / h, t)
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    ref64 = O.SplatOracle(O.scene_arrays(scene), cam, dbl=True, float_binning=True)
+    fb64, T64, amb, _ = ref64.render(bg)
+    ok = amb == 0
+    assert (~ok).mean() < 0.02
+    grad = np.random.default_rng(2).normal(size=fb64.shape).astype(np.float32)
+    grad[:, ~ok] = 0.0
+    out = _run_gpu(scene, cam, bg, grad_fb=grad)
+    assert np.abs(out["framebuffer"] - fb64).max(axis=0)[ok].max() <= IMG_TOL
+    assert np.abs(out["final_transparency"] - T64)[ok].max() <= IMG_TOL
+    g = out["grads"]
+    want = ref64.backward(bg, fb64, T64, grad)
+    for name in ("means", "scales", "rotations", "opacity"):
+        a, b = np.asarray(g[name]).reshape(1500, -1), np.asarray(want[name]).reshape(1500, -1)
+        assert np.linalg.norm(a - b) <= GRAD_TOL * np.linalg.norm(b), name
