@@ -154,7 +154,7 @@ SIGNATURES = {
     "dgmr_workspace_size": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _P(Tiling), ctypes.c_int64, _P(ctypes.c_size_t)]),
     "dgmr_splat_forward": (ctypes.c_int, [_P(Gaussians), _P(Camera), _P(Tiling), _P(SplatGeometry), _P(Binning), c_void_p, c_void_p,
                                           c_void_p, ctypes.c_size_t, _P(Stats), c_void_p]),
-    "dgmr_splat_prefix_pairs": (ctypes.c_int, [ctypes.c_int32, ctypes.c_int32, _P(Tiling), ctypes.c_int64, _P(ctypes.c_int64)]),
+    "dgmr_splat_prefix_pairs": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _P(Tiling), ctypes.c_int64, _P(ctypes.c_int64)]),
     "dgmr_splat_forward_prefix": (ctypes.c_int, [_P(Gaussians), _P(Camera), _P(Tiling), _P(SplatGeometry), _P(Binning), c_void_p, c_void_p,
                                                  c_void_p, ctypes.c_size_t, _P(Stats), c_void_p]),
     "dgmr_splat_backward": (ctypes.c_int, [_P(Gaussians), _P(Camera), _P(Tiling), _P(SplatGeometry), _P(Binning), ctypes.c_int64,

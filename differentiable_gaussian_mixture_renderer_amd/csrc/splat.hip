@@ -19,6 +19,7 @@
 // wave-reduced atomics) then k_splat_preprocess_backward (per Gaussian).
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "device_grad.h"
 #include "device_math.h"
@@ -62,33 +63,39 @@ constexpr int kEmitThreads = 256;
 // and setup spread over more pairs: 434M pairs 1.13 -> 1.06 ms; at 15M, with
 // half the blocks, 16 was slower, 0.042 against 0.032 ms)
 constexpr int kEmitPerSmall = 8, kEmitPerLarge = 16;
+static_assert((kEmitThreads & (kEmitThreads - 1)) == 0 && (kEmitPerSmall & (kEmitPerSmall - 1)) == 0 && (kEmitPerLarge & (kEmitPerLarge - 1)) == 0,
+    "an emission block's pairs: a power of two");
 constexpr int64_t kEmitLarge = int64_t(48) << 20;
 constexpr int kEmitWindow = 2048; // owners a block stages in LDS (more take the per-pair search)
 
 // First owners of the emission blocks: bounds[b] is the Gaussian (position
-// in depth order) that owns pair b * block_pairs, for every block that emits,
+// in depth order) that owns pair b << block_shift, for every block that emits,
 // and bounds[n_blocks] owns the last emitted pair.  Position k owns pairs
 // [offsets[k], offsets[k + 1]) and writes the entries whose pair falls in its
 // range, so each entry is written exactly once and no block searches.
+__device__ __forceinline__ void emit_bounds_of(uint32_t k, uint64_t lo, uint64_t next, uint64_t total, uint32_t capacity, int block_shift,
+    uint32_t* __restrict__ bounds, uint32_t* __restrict__ n_owners)
+{
+    const uint64_t R = min(total, uint64_t(capacity)); // pairs past the capacity are not emitted
+    if (n_owners && lo < total && next == total)
+        *n_owners = k + 1; // the last position that owns pairs
+    const uint64_t hi = min(next, R);
+    if (lo >= hi)
+        return;
+    const uint64_t up = (uint64_t(1) << block_shift) - 1;
+    for (uint64_t b = (lo + up) >> block_shift; (b << block_shift) < hi; ++b)
+        bounds[b] = k;
+    if (R - 1 < hi)
+        bounds[(R + up) >> block_shift] = k;
+}
 __global__ void k_emit_bounds(int64_t n, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ n_pairs, uint32_t capacity,
-    uint32_t block_pairs, uint32_t* __restrict__ bounds, uint32_t* __restrict__ n_owners)
+    int block_shift, uint32_t* __restrict__ bounds, uint32_t* __restrict__ n_owners)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k >= n)
         return;
     const uint64_t total = *n_pairs;
-    const uint64_t R = min(total, uint64_t(capacity)); // pairs past the capacity are not emitted
-    const uint64_t lo = offsets[k];
-    const uint64_t next = k + 1 < n ? uint64_t(offsets[k + 1]) : total;
-    if (n_owners && lo < total && next == total)
-        *n_owners = uint32_t(k + 1); // the last position that owns pairs
-    const uint64_t hi = min(next, R);
-    if (lo >= hi)
-        return;
-    for (uint64_t b = (lo + block_pairs - 1) / block_pairs; b * block_pairs < hi; ++b)
-        bounds[b] = uint32_t(k);
-    if (R - 1 < hi)
-        bounds[(R + block_pairs - 1) / block_pairs] = uint32_t(k);
+    emit_bounds_of(uint32_t(k), offsets[k], k + 1 < n ? uint64_t(offsets[k + 1]) : total, total, capacity, block_shift, bounds, n_owners);
 }
 
 // tile rectangle of Gaussian id: first tile and (grid_x << 16 | width); 0 shape when it has no tiles
@@ -165,6 +172,263 @@ __global__ __launch_bounds__(256) void k_gather_owners(int64_t n, const uint32_t
     }
     counts[j] = count;
     owner_rects[j] = make_uint2(start, shape);
+}
+
+// ------------------------------------------------------- small views' binning
+// Depth sort, gather, both scans and the emission's bounds of a view of at most
+// kBinOneMax Gaussians in one workgroup.  As separate launches these are 16 to
+// 18 of a few microseconds each with gaps as long between them; one CU has the
+// whole view in its registers and LDS.  The sort is the stable LSD radix sort
+// of the large path (equal digits found by ballot, a running count per wave and
+// digit), on the visible depth keys less the smallest of them: a view's depths
+// span few octaves, so the bits that all keys share are not sorted.  Culled
+// Gaussians (key ~0) take the key after the last and stay in order behind.
+// Bound by the latency of its passes on one CU: 12.6 us at 301 Gaussians and 39
+// us at 10 000, against 66 us and 75 us of the launches it replaces; above
+// kBinOneMax the keys no longer fit its registers and LDS and the launches of
+// the large path fill more CUs (50 000: 12 launches in 60 us).
+constexpr int kBinOneThreads = 1024;
+constexpr int kBinOneItems = 16;
+constexpr int kBinOneWaves = kBinOneThreads / 64;
+constexpr int64_t kBinOneMax = int64_t(kBinOneThreads) * kBinOneItems;
+constexpr int kBinOneRadix = 512;
+
+struct BinOneArgs {
+    int n;
+    const uint32_t* keys;   // depth bits, ~0 culled
+    const uint2* bin_rects;
+    const uint32_t* tiles;
+    uint32_t grid_x;
+    uint32_t capacity;
+    int block_shift;        // log2 of the pairs of an emission block
+    uint32_t* ids;
+    uint2* owner_rects;
+    uint32_t* offsets;
+    uint32_t* point_offsets; // by a second workgroup
+    uint32_t* n_pairs;
+    uint32_t* bounds;
+    uint32_t* n_owners;      // null: not wanted
+    PrefixRects prefix;
+};
+
+// exclusive scan of s[0..n) in place, by the whole workgroup; returns the sum.
+// A thread's share is an odd number of items, so its lanes fall on different banks.
+__device__ __forceinline__ uint32_t bin_one_scan(uint32_t* s, int n, uint32_t* s_wave)
+{
+    const unsigned lane = lane_id(), wave = threadIdx.x / 64;
+    const int per = ((n + kBinOneThreads - 1) / kBinOneThreads) | 1;
+    const int first = min(int(threadIdx.x) * per, n), last = min(first + per, n);
+    uint32_t sum = 0;
+    for (int i = first; i < last; ++i)
+        sum += s[i];
+    uint32_t v = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(v, d, 64);
+        if (lane >= unsigned(d))
+            v += o;
+    }
+    if (lane == 63)
+        s_wave[wave] = v;
+    __syncthreads();
+    uint32_t run = v - sum, total = 0;
+#pragma unroll
+    for (unsigned w = 0; w < kBinOneWaves; ++w) {
+        const uint32_t c = s_wave[w];
+        run += w < wave ? c : 0u;
+        total += c;
+    }
+    for (int i = first; i < last; ++i) {
+        const uint32_t x = s[i];
+        s[i] = run;
+        run += x;
+    }
+    __syncthreads();
+    return total;
+}
+
+__global__ __launch_bounds__(kBinOneThreads) void k_bin_one(BinOneArgs a)
+{
+    __shared__ uint32_t s_key[kBinOneMax];
+    __shared__ uint16_t s_id[kBinOneMax];
+    __shared__ uint16_t s_count[kBinOneWaves][kBinOneRadix]; // counts, then places: below 2^15
+    __shared__ uint32_t s_wave[kBinOneWaves], s_lo[kBinOneWaves], s_hi[kBinOneWaves];
+    const int n = a.n, t = int(threadIdx.x);
+    const unsigned lane = lane_id(), wave = threadIdx.x / 64;
+    const uint64_t lt = (uint64_t(1) << lane) - 1;
+    const int rounds = (n + kBinOneThreads - 1) / kBinOneThreads;
+    const int own = int(wave) * rounds * 64 + int(lane); // this lane's item of round 0
+    if (blockIdx.x == 1) {
+        // the second workgroup: the inclusive scan of the tile counts in id order
+        for (int j = t; j < n; j += kBinOneThreads)
+            s_key[j] = a.tiles[j];
+        __syncthreads();
+        const uint32_t all = bin_one_scan(s_key, n, s_wave);
+        for (int j = t; j < n; j += kBinOneThreads)
+            a.point_offsets[j] = j + 1 < n ? s_key[j + 1] : all;
+        return;
+    }
+    uint32_t key[kBinOneItems], id[kBinOneItems]; // id: the rank in the (wave, digit) in the upper half
+    uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+    for (int r = 0; r < kBinOneItems; ++r) {
+        const int i = own + r * 64;
+        id[r] = uint32_t(i);
+        key[r] = r < rounds && i < n ? a.keys[i] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int r = 0; r < kBinOneItems; ++r) {
+        if (key[r] != 0xffffffffu) {
+            lo = min(lo, key[r]);
+            hi = max(hi, key[r]);
+        }
+        if (r < rounds && own + r * 64 < n)
+            s_id[own + r * 64] = uint16_t(own + r * 64); // stays when nothing is visible
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        lo = min(lo, uint32_t(__shfl_xor(int(lo), d, 64)));
+        hi = max(hi, uint32_t(__shfl_xor(int(hi), d, 64)));
+    }
+    if (lane == 0) {
+        s_lo[wave] = lo;
+        s_hi[wave] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kBinOneWaves; ++w) {
+        lo = min(lo, s_lo[w]);
+        hi = max(hi, s_hi[w]);
+    }
+    lo = uniform(lo);
+    hi = uniform(hi);
+    const uint32_t behind = hi - lo + 1u; // the culled entries' key
+    const int bits = lo <= hi ? 32 - __clz(int(behind)) : 0;
+#pragma unroll
+    for (int r = 0; r < kBinOneItems; ++r)
+        key[r] = key[r] == 0xffffffffu ? behind : key[r] - lo;
+    const auto pass = [&](int shift, auto width) {
+        constexpr int W = decltype(width)::value;
+        constexpr uint32_t mask = (1u << W) - 1u;
+        constexpr int kWords = (1 << W) / 2; // counters, two to a word
+        for (int i = t; i < kBinOneWaves * kBinOneRadix / 2; i += kBinOneThreads)
+            reinterpret_cast<uint32_t*>(&s_count[0][0])[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBinOneItems; ++r) {
+            if (r < rounds) {
+                const bool valid = own + r * 64 < n;
+                const uint32_t digit = (key[r] >> shift) & mask;
+                const uint64_t valid_lanes = __ballot(valid);
+                uint32_t peers_lo = uint32_t(valid_lanes), peers_hi = uint32_t(valid_lanes >> 32);
+#pragma unroll
+                for (int b = 0; b < W; ++b) {
+                    const uint32_t s = uint32_t(int32_t(digit << (31 - b)) >> 31);
+                    const uint64_t m = __ballot(s != 0u);
+                    peers_lo &= ~(uint32_t(m) ^ s);
+                    peers_hi &= ~(uint32_t(m >> 32) ^ s);
+                }
+                const uint64_t peers = (uint64_t(peers_hi) << 32) | peers_lo;
+                // every lane reads the count before the lowest lane of its digit writes it back
+                const uint32_t before = s_count[wave][digit];
+                id[r] |= (before + uint32_t(__popcll(peers & lt))) << 16;
+                if (valid && (peers & lt) == 0)
+                    s_count[wave][digit] = uint16_t(before + uint32_t(__popcll(peers)));
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        __syncthreads();
+        {
+            // thread d < kWords: the starts of digits 2d and 2d + 1 per wave,
+            // exclusive over the digits (both halves of a word at once: no sum reaches 2^16)
+            uint32_t c[kBinOneWaves], tot = 0;
+#pragma unroll
+            for (int w = 0; w < kBinOneWaves; ++w) {
+                c[w] = t < kWords ? reinterpret_cast<const uint32_t*>(s_count[w])[t] : 0u;
+                tot += c[w];
+            }
+            const uint32_t sum = (tot & 0xffffu) + (tot >> 16);
+            uint32_t v = sum;
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const uint32_t o = __shfl_up(v, k, 64);
+                if (lane >= unsigned(k))
+                    v += o;
+            }
+            if (lane == 63)
+                s_wave[wave] = v;
+            __syncthreads();
+            if (t < kWords) {
+                uint32_t start = v - sum;
+#pragma unroll
+                for (unsigned w = 0; w < kWords / 64; ++w)
+                    start += w < wave ? s_wave[w] : 0u;
+                start |= (start + (tot & 0xffffu)) << 16;
+#pragma unroll
+                for (int w = 0; w < kBinOneWaves; ++w) {
+                    reinterpret_cast<uint32_t*>(s_count[w])[t] = start;
+                    start += c[w];
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBinOneItems; ++r) {
+            if (r < rounds && own + r * 64 < n) {
+                const uint32_t pos = s_count[wave][(key[r] >> shift) & mask] + (id[r] >> 16);
+                s_key[pos] = key[r];
+                s_id[pos] = uint16_t(id[r]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBinOneItems; ++r) {
+            if (r < rounds && own + r * 64 < n) {
+                key[r] = s_key[own + r * 64];
+                id[r] = s_id[own + r * 64];
+            }
+        }
+    };
+    // 9-bit digits (one to three passes) up to 27 bits, 16 octaves; else four of 8
+    if (bits <= 27) {
+        for (int shift = 0; shift < bits; shift += 9)
+            pass(shift, std::integral_constant<int, 9> {});
+    } else {
+        for (int shift = 0; shift < 32; shift += 8)
+            pass(shift, std::integral_constant<int, 8> {});
+    }
+    __syncthreads(); // the keys have been read: their LDS holds the pair counts from here
+    uint2 rect[kBinOneItems];
+#pragma unroll
+    for (int r = 0; r < kBinOneItems; ++r) {
+        const int j = r * kBinOneThreads + t;
+        id[r] = r < rounds && j < n ? uint32_t(s_id[j]) : 0u;
+        rect[r] = r < rounds && j < n ? a.bin_rects[id[r]] : make_uint2(0u, 0u);
+    }
+#pragma unroll
+    for (int r = 0; r < kBinOneItems; ++r) {
+        const int j = r * kBinOneThreads + t;
+        if (r < rounds && j < n) {
+            const uint32_t cols = rect[r].y & 0xffffu, rows = rect[r].y >> 16;
+            a.ids[j] = id[r];
+            a.owner_rects[j] = make_uint2(rect[r].x, cols * rows == 0 ? 0u : (a.grid_x << 16) | cols);
+            s_key[j] = cols * rows;
+            if (a.prefix.origin) {
+                const uint32_t y = rect[r].x / a.grid_x;
+                a.prefix.origin[j] = (y << 16) | (rect[r].x - y * a.grid_x);
+                a.prefix.size[j] = rect[r].y;
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t total = bin_one_scan(s_key, n, s_wave);
+    if (t == 0)
+        *a.n_pairs = total;
+    for (int j = t; j < n; j += kBinOneThreads) {
+        const uint32_t first = s_key[j], next = j + 1 < n ? s_key[j + 1] : total;
+        a.offsets[j] = first;
+        emit_bounds_of(uint32_t(j), first, next, total, a.capacity, a.block_shift, a.bounds, a.n_owners);
+    }
 }
 
 // kEmitPer consecutive pairs at a 16-byte aligned position: 32-bit keys and
@@ -570,17 +834,25 @@ __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_forward(const uint32
 // the extension builds those tiles' whole lists behind the sorted pairs from
 // the depth-ordered rectangles, for a second blend of these tiles.  Nothing
 // waits for the host: both launches leave at once when there is nothing to do.
-// (kPrefixMin: whole lists below three times the prefix, where the emission and
-// sort that is saved is small against an extension.)
+// When the lists are whole the four launches of the extension and the second
+// blend find nothing and cost 16 us, as much as the emission and sort of 1.3M
+// pairs: views with fewer pairs to save, by the 16 pairs a Gaussian makes in an
+// ordinary deep view, and those whose pairs are not three times the prefix keep
+// whole lists.
 constexpr int64_t kPrefixPerTile = 256;
 constexpr int64_t kPrefixMin = 3;
+constexpr int64_t kPrefixPairsPerGaussian = 16;
+constexpr int64_t kPrefixMinSaved = 1300000;
 
-// the first pairs that a view of n_tiles tiles bins with prefix binning, 0 when
-// its whole lists are binned
-static int64_t prefix_pairs(int64_t n_tiles, int64_t pair_capacity)
+// the first pairs that a view of n Gaussians and n_tiles tiles bins with prefix
+// binning, 0 when its whole lists are binned
+static int64_t prefix_pairs(int64_t n, int64_t n_tiles, int64_t pair_capacity)
 {
-    const int64_t pairs = kPrefixPerTile * n_tiles;
-    return pair_capacity >= kPrefixMin * pairs && pair_capacity + pairs <= int64_t(UINT32_MAX) && n_tiles <= (int64_t(1) << 22) ? pairs : 0;
+    const int64_t pairs = kPrefixPerTile * n_tiles, expected = kPrefixPairsPerGaussian * n;
+    return pair_capacity >= kPrefixMin * pairs && expected >= kPrefixMin * pairs && expected - pairs >= kPrefixMinSaved
+            && pair_capacity + pairs <= int64_t(UINT32_MAX) && n_tiles <= (int64_t(1) << 22)
+        ? pairs
+        : 0;
 }
 
 // The extension works on groups of 8 x 8 tiles, a lane per tile, over segments
@@ -1044,7 +1316,11 @@ struct EmitArgs {
     int tile_w, tile_h;
     bool cull;
     const PrefixBinning* prefix; // null: whole lists
+    bool bounds_written;         // by the small views' binning
 };
+
+static int emit_per(int64_t cap) { return cap >= kEmitLarge ? kEmitPerLarge : kEmitPerSmall; }
+static int emit_shift(int per) { return __builtin_ctz(unsigned(kEmitThreads * per)); } // log2 of a block's pairs
 
 // emission, pair sort on the tile bits, tile ranges; pair keys of type KeyT
 template <class KeyT>
@@ -1059,13 +1335,15 @@ static int emit_sort_ranges(const EmitArgs& a, const SplatWorkspace& w, dgmr_bin
         pb = SortBuffersT<KeyT> { ka, bins->point_list, kb, w.pvals_a };
     else
         pb = SortBuffersT<KeyT> { ka, w.pvals_a, kb, bins->point_list };
-    const int per = int64_t(a.cap) >= kEmitLarge ? kEmitPerLarge : kEmitPerSmall;
+    const int per = emit_per(a.cap);
     const uint32_t block_pairs = uint32_t(kEmitThreads * per);
     const unsigned emit_blocks = unsigned(ceil_div64(a.cap, block_pairs));
     {
         StageScope sc("bin.emit", st);
         pending->add_stage(sc.slot, 4.0 + sizeof(KeyT), 28.0 * double(a.n));
-        k_emit_bounds<<<a.blocks_n, 256, 0, st>>>(a.n, w.pair_offsets, w.counter, a.cap, block_pairs, w.emit_bounds, a.prefix ? a.prefix->n_owners : nullptr);
+        if (!a.bounds_written)
+            k_emit_bounds<<<a.blocks_n, 256, 0, st>>>(a.n, w.pair_offsets, w.counter, a.cap, emit_shift(per), w.emit_bounds,
+                a.prefix ? a.prefix->n_owners : nullptr);
         DGMR_HIP_CHECK(hipGetLastError());
         if (a.cull && per == kEmitPerLarge)
             k_emit_reach<KeyT, kEmitPerLarge><<<emit_blocks, kEmitThreads, 0, st>>>(w.counter, a.cap, a.sorted_ids, w.emit_bounds,
@@ -1125,9 +1403,10 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
         n_sorted = count;
     }
     const bool multi_view = batch && batch->n_views > 1;
+    const bool one = bin_rects_written && !cull && !batch && n <= kBinOneMax;
     // with tight culling the culled entries sort last in the view pass, under the key n_views
     const uint32_t culled_view = cull && multi_view ? uint32_t(batch->n_views) : 0xffffffffu;
-    {
+    if (!one) {
         StageScope sc("bin.depth_sort", st, 16.0 * double(n) * radix_passes(0, 32));
         // several views: the last depth pass writes each entry's view as its key
         const KeyOut view_keys = multi_view ? KeyOut { uint32_t(n_per_view), culled_view } : KeyOut {};
@@ -1158,7 +1437,14 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
             w.prefix_open + 5 * tiles, w.prefix_open + 6 * tiles + 1, 4 * bins->pair_capacity };
     }
     const unsigned blocks_n = unsigned(ceil_div64(n, 256));
-    {
+    const int64_t cap = std::min<int64_t>(bins->pair_capacity, int64_t(UINT32_MAX));
+    if (one) {
+        StageScope sc("bin.one", st, 60.0 * double(n));
+        k_bin_one<<<bins->point_offsets ? 2 : 1, kBinOneThreads, 0, st>>>(BinOneArgs { int(n), K, w.bin_rects, tiles, uint32_t(grid_x), uint32_t(std::max<int64_t>(cap, 0)),
+            emit_shift(emit_per(cap)), V, w.owner_rects, w.pair_offsets, bins->point_offsets, w.counter, w.emit_bounds,
+            prefix ? prefix->n_owners : nullptr, rects_out });
+        DGMR_HIP_CHECK(hipGetLastError());
+    } else {
         StageScope sc("bin.scan", st, 44.0 * double(n));
         // the pair offsets of the depth order and, when asked for, the
         // reference cache's inclusive scan of tiles in Gaussian order: one
@@ -1186,7 +1472,6 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
     if (rc_count != DGMR_OK)
         return rc_count;
     const int64_t n_tiles = batch ? batch->total_tiles : int64_t(grid_x) * grid_y;
-    const int64_t cap = std::min<int64_t>(bins->pair_capacity, int64_t(UINT32_MAX));
     if (cap <= 0) {
         DGMR_HIP_CHECK(hipMemsetAsync(bins->ranges, 0, size_t(n_tiles) * 2 * sizeof(uint32_t), st));
         return DGMR_OK;
@@ -1195,7 +1480,7 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
     // traffic in emission and sort), else 32
     const int tile_bits = int(higher_msb(uint32_t(batch ? batch->max_view_tiles : n_tiles)));
     EmitArgs ea { n, blocks_n, uint32_t(cap), n_tiles, tile_bits, sorted_ids, views, n_per_view, batch ? int(batch->n_views) : 0, tile_w, tile_h,
-        cull, prefix };
+        cull, prefix, one };
     if (tile_bits <= 16)
         return emit_sort_ranges<uint16_t>(ea, w, bins, pending, st);
     return emit_sort_ranges<uint32_t>(ea, w, bins, pending, st);
@@ -1260,7 +1545,7 @@ static int splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const 
     }
     Carver cv(workspace, workspace_bytes);
     PendingCount pending;
-    const int64_t prefix = allow_prefix && !cull ? prefix_pairs(n_tiles, bins->pair_capacity) : 0;
+    const int64_t prefix = allow_prefix && !cull ? prefix_pairs(n, n_tiles, bins->pair_capacity) : 0;
     PrefixBinning pb {};
     dgmr_binning first = *bins;
     if (prefix)
@@ -1325,11 +1610,12 @@ int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dg
     return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream, false);
 }
 
-int dgmr_splat_prefix_pairs(int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, int64_t* pairs)
+int dgmr_splat_prefix_pairs(int64_t n, int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, int64_t* pairs)
 {
-    DGMR_ARG_CHECK(pairs && valid_image(width, height) && valid_tiling(tiling) && pair_capacity >= 0, "dgmr_splat_prefix_pairs: bad argument");
+    DGMR_ARG_CHECK(pairs && n >= 0 && n < (int64_t(1) << 31) && valid_image(width, height) && valid_tiling(tiling) && pair_capacity >= 0,
+        "dgmr_splat_prefix_pairs: bad argument");
     const int64_t n_tiles = ceil_div64(width, tiling->tile_w) * ceil_div64(height, tiling->tile_h);
-    *pairs = tiling->cull ? 0 : prefix_pairs(n_tiles, pair_capacity);
+    *pairs = tiling->cull ? 0 : prefix_pairs(n, n_tiles, pair_capacity);
     return DGMR_OK;
 }
 

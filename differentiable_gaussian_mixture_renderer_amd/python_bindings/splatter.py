@@ -79,7 +79,7 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
         for _attempt in range(3):
             prefix = ctypes.c_int64(0)
             if not whole_lists:
-                N.check(lib.dgmr_splat_prefix_pairs(W, H, ctypes.byref(tiling), cap, ctypes.byref(prefix)), "dgmr_splat_prefix_pairs")
+                N.check(lib.dgmr_splat_prefix_pairs(n, W, H, ctypes.byref(tiling), cap, ctypes.byref(prefix)), "dgmr_splat_prefix_pairs")
             point_list = torch.empty((max(cap + prefix.value, 1),), dtype=torch.int32, device=dev)
             bins = N.Binning(offsets.data_ptr(), point_list.data_ptr(), ranges.data_ptr(), cap)
             ws = C.workspace(dev, n, W, H, tiling, cap)

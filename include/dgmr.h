@@ -140,7 +140,8 @@ int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dg
  * bins->point_list then holds pair_capacity + *pairs entries, and ranges may
  * point anywhere in it; dgmr_splat_backward walks such lists as any other.  No
  * counterpart in the reference, which bins every pair. */
-int dgmr_splat_prefix_pairs(int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, int64_t* pairs);
+int dgmr_splat_prefix_pairs(int64_t n, int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity,
+    int64_t* pairs);
 int dgmr_splat_forward_prefix(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling,
     dgmr_splat_geometry* geom, dgmr_binning* bins, float* framebuffer, float* final_transmittance,
     void* workspace, size_t workspace_bytes, dgmr_stats* stats, dgmr_stream stream);

@@ -347,11 +347,11 @@ def test_prefix_binning_equals_whole_lists(kind, tile, w, h):
     torch = _torch()
     from differentiable_gaussian_mixture_renderer_amd import _common, scenes
     from differentiable_gaussian_mixture_renderer_amd.python_bindings import splatter
-    n = 300 if kind == "whole" else 60_000
+    n = 300 if kind == "whole" else 120_000
     scene = scenes.make_scene(n, seed=6, extent=1.0, sh_degree=1)
     opacity, scales = scene.opacity.copy(), scene.scales.copy()
     if kind == "open":
-        opacity *= 0.004
+        opacity *= 0.002
         scales *= 2.0
     if kind == "half_open":
         opacity[scene.means[:, 0] > 0.1] *= 0.01
@@ -420,3 +420,32 @@ def test_blends_at_the_waves_per_tile_limits(w, h):
     for name in ("means", "scales", "rotations", "opacity"):
         a, b = np.asarray(g[name]).reshape(1500, -1), np.asarray(want[name]).reshape(1500, -1)
         assert np.linalg.norm(a - b) <= GRAD_TOL * np.linalg.norm(b), name
+
+
+@pytest.mark.parametrize("kind", ["some_culled", "equal_depths", "all_culled", "wide_depths"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1025, 9000, 16383, 16384, 16385])
+def test_binning_of_small_views(n, kind):
+    """A view of up to 16 384 Gaussians is binned by one workgroup: the lists,
+    offsets and ranges equal the float restatement's at the edges of waves,
+    rounds and the limit, with culled Gaussians, equal depths (id order),
+    nothing visible, and depths over many octaves (four digits to sort)."""
+    _torch()
+    from differentiable_gaussian_mixture_renderer_amd import scenes
+    scene = scenes.make_scene(n, seed=n, extent=1.0, sh_degree=0)
+    rng = np.random.default_rng(n)
+    scene.scales[:] = 0.01
+    if kind == "some_culled":
+        scene.means[rng.random(n) < 0.3, 2] -= 20.0
+    elif kind == "equal_depths":
+        scene.means[:, 2] = 0.0
+    elif kind == "all_culled":
+        scene.means[:, 2] = -30.0
+    else:
+        depth = np.exp2(rng.uniform(-1.0, 16.0, n)).astype(np.float32)
+        scene.means[:] = scene.means * depth[:, None] * 0.1
+        scene.means[:, 2] = depth - 4.0
+    cam = scenes.look_at_camera([0.0, 0.0, -4.0], [0.0, 0.0, 0.0], 100, 67, 0.45, 0.3)
+    out = _run_gpu(scene, cam, np.array([0.25, 0.5, 0.75], np.float32))
+    ref = O.SplatOracle(O.scene_arrays(scene), cam, dbl=False)
+    vis = _check_binning(out, ref)
+    assert vis.any() == (kind != "all_culled") or n < 64
