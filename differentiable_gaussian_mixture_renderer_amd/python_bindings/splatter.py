@@ -60,7 +60,7 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
     gx, gy = (W + tiling.tile_w - 1) // tiling.tile_w, (H + tiling.tile_h - 1) // tiling.tile_h
     f32 = dict(dtype=torch.float32, device=dev)
     with torch.cuda.device(dev):
-        fb = torch.zeros((3, H, W), **f32)
+        fb = torch.empty((3, H, W), **f32)  # the blend writes every pixel
         T = torch.empty((H, W), **f32)
         rects = torch.empty((n, 2), dtype=torch.int32, device=dev)
         tiles = torch.empty((n,), dtype=torch.int32, device=dev)
