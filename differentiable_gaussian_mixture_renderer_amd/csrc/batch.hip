@@ -1,15 +1,14 @@
 // SPDX-License-Identifier: GPL-3.0-or-later
 // Batched multi-view splatting: many cameras of one scene with uneven
-// resolutions in one preprocess launch, one binning pass and one persistent
-// blend launch (forward and backward).
+// resolutions in one preprocess launch, one binning pass and one blend launch
+// (forward and backward).
 //
 // Layout: the Gaussians take slots in the Morton order of their centres
 // (slot s holds Gaussian order[s]; in id order when dgmr_tiling.slot_order is
 // 1), and per-view geometry is stored at entry v * n + s, so the entry ids in the pair list index every array directly;
 // view v's tiles occupy a contiguous range of the global tile index space.
-// The blend runs as a persistent grid whose workgroups take the next tile of
-// any view from a device counter, so small and large views share the chip
-// without per-view launches or syncs.
+// The blend is one launch over all views' tiles, so small and large views share
+// the chip without per-view launches or syncs.
 #include <algorithm>
 #include <numeric>
 #include <type_traits>
@@ -231,46 +230,41 @@ __device__ __forceinline__ int find_view(const ViewBlend* views, int n_views, in
     return lo;
 }
 
-// Persistent blend over the global tile queue: kBlendWaves independent waves
-// per workgroup, each popping tiles for itself.  The queue counter starts at
-// 0; a wave exits once the counter has passed the last tile.  Queue position
-// k is tile k, or tile_order[k] when given.
-template <int TW, int TH, int B, bool BACKWARD>
-__global__ __launch_bounds__(64 * kBlendWaves) void k_batch_blend(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ point_list,
+// Blend of every view's tiles, one wave per workgroup and SPLIT waves per tile
+// (each a TH/SPLIT-row part of it).  The dispatcher hands the tiles out: waves
+// of a persistent grid taking theirs from one counter ran at the rate of its
+// atomics, 14 ns each, whatever the tiles held (39k tiles of 12 views: forward
+// 0.57 -> 0.33 ms, backward 0.78 -> 0.72 ms; workgroups of four waves, which
+// wait for their longest list, 0.34 and 0.76 ms).  The forward gives each XCD a
+// contiguous band of tiles, the backward takes tile_order[k] in turn.
+template <int TW, int TH, int B, int SPLIT, bool BACKWARD>
+__global__ __launch_bounds__(64) void k_batch_blend(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ point_list,
     const float2* __restrict__ xy, const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, const ViewBlend* __restrict__ views,
-    int n_views, int total_tiles, uint32_t* __restrict__ queue, float* __restrict__ screen_grads, const uint32_t* __restrict__ tile_order)
+    int n_views, float* __restrict__ screen_grads, const uint32_t* __restrict__ tile_order)
 {
     using Smem = typename std::conditional<BACKWARD, BlendSmemBwd<B>, BlendSmem<B>>::type;
-    __shared__ Smem sm_all[kBlendWaves];
-    Smem& sm = sm_all[threadIdx.x / 64];
-    while (true) {
-        uint32_t t = 0;
-        if (lane_id() == 0)
-            t = atomicAdd(queue, 1u);
-        // lane 0's value, read into a scalar register: the view record and
-        // its pointers then stay in scalar registers too
-        int tile = int(__builtin_amdgcn_readfirstlane(t));
-        if (tile >= total_tiles)
-            break;
-        if (tile_order)
-            tile = int(tile_order[tile]);
-        const ViewBlend& vb = views[find_view(views, n_views, tile)];
-        const int local = tile - vb.tile_base;
-        const int px0 = (local % vb.grid_x) * TW, py0 = (local / vb.grid_x) * TH;
-        if constexpr (BACKWARD) {
-            // a view with neither a gradient image nor an L1 target has a zero
-            // dL/dimage (or no gradient group): its tiles add nothing, so they
-            // are skipped (the view record is the same for the whole wave)
-            if (!vb.grad_fb && !vb.l1_target)
-                continue;
-            blend_tile_backward<TW, TH, B>(sm, uniform(ranges[2 * tile]), uniform(ranges[2 * tile + 1]), px0, py0, vb.width, vb.height, vb.bg[0],
-                vb.bg[1], vb.bg[2], point_list, xy, conic_opacity, rgb, vb.framebuffer, vb.final_T, vb.grad_fb, screen_grads, vb.l1_target,
-                vb.l1_scale);
-        } else {
-            blend_tile_forward<TW, TH, B>(sm, uniform(ranges[2 * tile]), uniform(ranges[2 * tile + 1]), px0, py0, vb.width, vb.height, vb.bg[0], vb.bg[1],
-                vb.bg[2], point_list, xy, conic_opacity, rgb, vb.framebuffer, vb.final_T);
-        }
-        wave_lds_sync();
+    __shared__ Smem sm;
+    constexpr int PH = TH / SPLIT; // rows of a part
+    const int unit = BACKWARD ? int(blockIdx.x) : xcd_tile(int(blockIdx.x), int(gridDim.x));
+    const int part = unit % SPLIT;
+    int tile = unit / SPLIT;
+    if (BACKWARD)
+        tile = int(uniform(tile_order[tile]));
+    const ViewBlend& vb = views[find_view(views, n_views, tile)];
+    const int local = tile - vb.tile_base;
+    const int px0 = (local % vb.grid_x) * TW, py0 = (local / vb.grid_x) * TH + part * PH;
+    if constexpr (BACKWARD) {
+        // a view with neither a gradient image nor an L1 target has a zero
+        // dL/dimage (or no gradient group): its tiles add nothing, so they
+        // are skipped (the view record is the same for the whole wave)
+        if (!vb.grad_fb && !vb.l1_target)
+            return;
+        blend_tile_backward<TW, PH, B>(sm, uniform(ranges[2 * tile]), uniform(ranges[2 * tile + 1]), px0, py0, vb.width, vb.height, vb.bg[0],
+            vb.bg[1], vb.bg[2], point_list, xy, conic_opacity, rgb, vb.framebuffer, vb.final_T, vb.grad_fb, screen_grads, vb.l1_target,
+            vb.l1_scale);
+    } else {
+        blend_tile_forward<TW, PH, B>(sm, uniform(ranges[2 * tile]), uniform(ranges[2 * tile + 1]), px0, py0, vb.width, vb.height, vb.bg[0], vb.bg[1],
+            vb.bg[2], point_list, xy, conic_opacity, rgb, vb.framebuffer, vb.final_T);
     }
 }
 
@@ -278,11 +272,11 @@ __global__ __launch_bounds__(64 * kBlendWaves) void k_batch_blend(const uint32_t
 // the entry's screen gradients with float atomics, and tiles in flight at the
 // same time that touch the same cache lines (a shared Gaussian, or Gaussians
 // in neighbouring slots, which the spatial order makes neighbours on screen)
-// serialise on them.  The queue therefore visits the views round-robin, the
+// serialise on them.  The launch therefore visits the views round-robin, the
 // largest first, and steps through each view's tiles with a stride near
 // 0.618 of its tile count (coprime with it), so tiles in flight together
 // belong to different views or lie far apart.  by_size[j] = (first tile,
-// tiles, stride) of the j-th largest view; segment q = (first queue
+// tiles, stride) of the j-th largest view; segment q = (first
 // position, first round, views) of the rounds in which the first `views`
 // views still have tiles.
 __global__ __launch_bounds__(256) void k_tile_order(int total, const int4* __restrict__ by_size, const int4* __restrict__ segs, int n_segs,
@@ -492,7 +486,6 @@ struct BatchLayout {
     int32_t* groups;
     ViewBlend* views;
     int4* grids;
-    uint32_t* queue;
     uint32_t* tiles;
     float* xy;
     float4* conic_opacity;
@@ -535,7 +528,6 @@ BatchLayout carve_batch(void* ws, int64_t n, const dgmr_batch_view* views, int n
     L.groups = cv.take<int32_t>(n_views);
     L.views = cv.take<ViewBlend>(n_views);
     L.grids = cv.take<int4>(n_views);
-    L.queue = cv.take<uint32_t>(64);
     L.tiles = cv.take<uint32_t>(m);
     L.xy = cv.take<float>(2 * m);
     L.conic_opacity = cv.take<float4>(m);
@@ -574,18 +566,18 @@ SplatParams slot_params(const BatchLayout& L, const dgmr_gaussians* g, const dgm
         g->sh_degree, float(g->scale_multiplier), g->activation };
 }
 
-template <int TW, int TH>
-void launch_batch_blend(bool backward, int batch, int grid, hipStream_t st, const BatchLayout& L, int n_views)
+template <int TW, int TH, int SPLIT>
+void launch_batch_blend(bool backward, int batch, hipStream_t st, const BatchLayout& L, int n_views)
 {
     const auto* xy2 = reinterpret_cast<const float2*>(L.xy);
-    const int tt = int(L.total_tiles);
+    const unsigned grid = unsigned(L.total_tiles * SPLIT);
 #define DGMR_BATCH_BLEND(B)                                                                                                            \
     if (backward)                                                                                                                      \
-        k_batch_blend<TW, TH, B, true><<<grid, 64 * kBlendWaves, 0, st>>>(L.ranges, L.point_list, xy2, L.conic_opacity, L.rgb, L.views, n_views, tt,  \
-            L.queue, L.screen_grads, L.tile_order);                                                                                    \
+        k_batch_blend<TW, TH, B, SPLIT, true><<<grid, 64, 0, st>>>(L.ranges, L.point_list, xy2, L.conic_opacity, L.rgb, L.views, n_views, \
+            L.screen_grads, L.tile_order);                                                                                             \
     else                                                                                                                               \
-        k_batch_blend<TW, TH, B, false><<<grid, 64 * kBlendWaves, 0, st>>>(L.ranges, L.point_list, xy2, L.conic_opacity, L.rgb, L.views, n_views, tt, \
-            L.queue, L.screen_grads, nullptr);
+        k_batch_blend<TW, TH, B, SPLIT, false><<<grid, 64, 0, st>>>(L.ranges, L.point_list, xy2, L.conic_opacity, L.rgb, L.views, n_views, \
+            L.screen_grads, nullptr);
     if (batch == 64) {
         DGMR_BATCH_BLEND(64)
     } else if (batch == 128) {
@@ -596,16 +588,24 @@ void launch_batch_blend(bool backward, int batch, int grid, hipStream_t st, cons
 #undef DGMR_BATCH_BLEND
 }
 
+template <int TW, int TH>
+void launch_batch_blend(bool backward, int batch, hipStream_t st, const BatchLayout& L, int n_views)
+{
+    constexpr int SPLIT = TW * TH / 64;
+    if (SPLIT > 1 && L.total_tiles <= (backward ? kBwdSplitTiles : kFwdSplitTiles))
+        launch_batch_blend<TW, TH, SPLIT>(backward, batch, st, L, n_views);
+    else
+        launch_batch_blend<TW, TH, 1>(backward, batch, st, L, n_views);
+}
+
 void batch_blend(bool backward, const dgmr_tiling& t, hipStream_t st, const BatchLayout& L, int n_views)
 {
-    // persistent grid: 32 waves per CU, never more waves than there are tiles
-    const int grid = int(std::min<int64_t>(ceil_div64(L.total_tiles, kBlendWaves), 256 * 32 / kBlendWaves));
     if (t.tile_w == 16)
-        launch_batch_blend<16, 16>(backward, t.batch, grid, st, L, n_views);
+        launch_batch_blend<16, 16>(backward, t.batch, st, L, n_views);
     else if (t.tile_w == 8)
-        launch_batch_blend<8, 8>(backward, t.batch, grid, st, L, n_views);
+        launch_batch_blend<8, 8>(backward, t.batch, st, L, n_views);
     else
-        launch_batch_blend<32, 8>(backward, t.batch, grid, st, L, n_views);
+        launch_batch_blend<32, 8>(backward, t.batch, st, L, n_views);
 }
 
 int check_batch_args(const dgmr_gaussians* g, const dgmr_batch_view* views, int32_t n_views, const dgmr_tiling* tiling)
@@ -714,7 +714,6 @@ int dgmr_splat_batch_forward(const dgmr_gaussians* g, const dgmr_batch_view* vie
     {
         StageScope sc("batch.blend_forward", st);
         pending.add_stage(sc.slot, 40.0, 0.0);
-        DGMR_HIP_CHECK(hipMemsetAsync(L.queue, 0, sizeof(uint32_t), st));
         batch_blend(false, *tiling, st, L, n_views);
         DGMR_HIP_CHECK(hipGetLastError());
     }
@@ -820,7 +819,6 @@ int dgmr_splat_batch_backward(const dgmr_gaussians* g, const dgmr_batch_view* vi
                 L.tile_order);
             DGMR_HIP_CHECK(hipGetLastError());
         }
-        DGMR_HIP_CHECK(hipMemsetAsync(L.queue, 0, sizeof(uint32_t), st));
         batch_blend(true, *tiling, st, L, n_views);
         DGMR_HIP_CHECK(hipGetLastError());
     }

@@ -1203,19 +1203,6 @@ size_t splat_workspace_bytes(int64_t n, int64_t cap, bool cull)
     return cv.used;
 }
 
-// Waves per tile: a wave walks its tile's list alone, so with fewer tiles than
-// the chip has wave slots the longest walk is the launch's time, and a wave on
-// a quarter of the tile's pixels takes a step in less than half the time.  With
-// the slots filled, the parts of a step that every wave repeats (fetching and
-// staging the list, the per-Gaussian terms and, in the backward, its reduction
-// and atomics) count instead.  Measured in us with one / four waves per tile:
-// forward 98 / 38 at 192 tiles, 67 / 37 at 920, 66 / 52 and 55 / 49 at 3 600
-// (300k and 1M Gaussians), 108 / 96 and 75 / 82 at 8 160; backward 204 / 80 at
-// 192 tiles, 143 / 85 at 920, 130 / 98 at 1 200, 114 / 120 and 100 / 170 at
-// 1 900 (two waves per tile: 105 and 118).
-constexpr int kFwdSplitTiles = 6144;
-constexpr int kBwdSplitTiles = 1280;
-
 template <int TW, int TH, int SPLIT>
 static void launch_blend_fwd_as(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
     const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T, const PrefixPass& prefix)

@@ -428,7 +428,20 @@ __device__ __forceinline__ void preprocess_view(GaussIn& g, int64_t i, int64_t o
 // blended.  The conic is staged pre-scaled by -log2(e)/2 (diagonal) and
 // -log2(e) (off-diagonal), so G = exp2(A dx^2 + B dx dy + C dy^2).
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kBlendWaves = 4; // tile waves per workgroup
+constexpr int kBlendWaves = 4; // tile waves per workgroup of a single view's blends
+
+// Waves per tile: a wave walks its tile's list alone, so with fewer tiles than
+// the chip has wave slots the longest walk is the launch's time, and a wave on
+// a quarter of the tile's pixels takes a step in less than half the time.  With
+// the slots filled, the parts of a step that every wave repeats (fetching and
+// staging the list, the per-Gaussian terms and, in the backward, its reduction
+// and atomics) count instead.  Measured in us with one / four waves per tile:
+// forward 98 / 38 at 192 tiles, 67 / 37 at 920, 66 / 52 and 55 / 49 at 3 600
+// (300k and 1M Gaussians), 108 / 96 and 75 / 82 at 8 160; backward 204 / 80 at
+// 192 tiles, 143 / 85 at 920, 130 / 98 at 1 200, 114 / 120 and 100 / 170 at
+// 1 900 (two waves per tile: 105 and 118).
+constexpr int kFwdSplitTiles = 6144;
+constexpr int kBwdSplitTiles = 1280;
 
 // conic and opacity co = (a, b, c, o) at screen centre xy (tile_reach.h)
 __device__ __forceinline__ bool reaches_box(float2 xy, float4 co, float bx0, float bx1, float by0, float by1)

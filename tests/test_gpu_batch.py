@@ -1,4 +1,4 @@
-"""Batched multi-view splatting (one persistent launch per stage) against the
+"""Batched multi-view splatting (one launch per stage) against the
 one-camera-per-launch path and the oracle: every view's image and the summed
 gradients agree with rendering each camera alone."""
 import numpy as np
@@ -229,3 +229,33 @@ def test_id_slot_order_matches_spatial_order():
     for ga, gb_ in zip(out[True][1], out[False][1]):
         for a, b in zip(ga, gb_):
             assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b) + 1e-12
+
+
+@pytest.mark.parametrize("resolutions", [[(640, 512)], [(641, 512)], [(1536, 1024)], [(1537, 1024), (33, 17)], [(1280, 720), (50, 40), (1920, 1080)]])
+def test_waves_per_tile_of_batches(resolutions):
+    """The batch's total tiles at the limits of four waves per tile (1 280
+    backward, 6 144 forward) and above both, in views of uneven size: images and
+    gradients as the views rendered alone."""
+    torch = _torch()
+    from differentiable_gaussian_mixture_renderer_amd import scenes
+    from differentiable_gaussian_mixture_renderer_amd.batching import BatchSplatter, render_plain
+    scene = scenes.make_scene(4_000, seed=7, extent=5.0, sh_degree=1)
+    cams = [scenes.sphere_cameras(len(resolutions), seed=3, resolutions=[r])[v] for v, r in enumerate(resolutions)]
+    dev = torch.device("cuda:0")
+    t = lambda a: torch.tensor(np.ascontiguousarray(a), device=dev)
+    params = [t(scene.sh), t(scene.opacity), t(scene.means), t(scene.scales), t(scene.rotations)]
+    bg = (0.1, 0.2, 0.3)
+    print(f"[gpu batch] waves per tile, {resolutions}", flush=True)
+    bs = BatchSplatter()
+    fbs, _ = bs.forward(*params, cams, bg=bg, sh_degree=1)
+    rng = np.random.default_rng(1)
+    grads = [torch.tensor(rng.normal(size=(3, c.height, c.width)).astype(np.float32) / (3 * c.height * c.width), device=dev) for c in cams]
+    gb = bs.backward(grads)
+    gi = iter(grads)
+    imgs, gp = render_plain(*params, cams, bg=bg, sh_degree=1, grad_fn=lambda img: next(gi))
+    torch.cuda.synchronize()
+    for v in range(len(cams)):
+        np.testing.assert_allclose(fbs[v].cpu().numpy(), imgs[v].cpu().numpy(), rtol=0, atol=1e-6)
+    for a, b in zip(gb, gp):
+        a, b = a.cpu().numpy(), b.cpu().numpy()
+        assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b) + 1e-12
