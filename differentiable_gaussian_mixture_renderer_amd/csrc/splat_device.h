@@ -534,14 +534,9 @@ struct BlendFetch {
 // order, so a compiler barrier orders its staging writes before its reads
 __device__ __forceinline__ void wave_lds_sync() { __builtin_amdgcn_wave_barrier(); }
 
-// true when the predicate holds on some lane of the wave: the ballot of the
-// condition itself, so the lane mask is used as it is (a ballot of an int
-// re-materialises the mask through a VGPR first)
-__device__ __forceinline__ bool wave_any(bool pred) { return __builtin_amdgcn_ballot_w64(pred) != 0; }
-
 // lane masks of float comparisons (LLVM predicates), combined with scalar
 // instructions where a wave-uniform decision needs them
-enum : int { kCmpOGT = 2, kCmpOGE = 3, kCmpOLT = 4, kCmpUGE = 11 };
+enum : int { kCmpOGE = 3, kCmpOLT = 4 };
 template <int PRED>
 __device__ __forceinline__ uint64_t lanes_where(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, PRED); }
 
@@ -577,13 +572,14 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
     const float pxf = float(px);
     const float pyf0 = float(py0 + lane / TW);
     const float bx0 = float(px0), bx1 = float(px0 + TW - 1), by0 = float(py0), by1 = float(py0 + TH - 1);
-    // a pixel that has stopped carries its transmittance negated (a live
-    // pixel's T is at least 1e-4), so liveness costs no separate register
+    // the lanes whose pixel k takes more Gaussians, as a wave-uniform mask
+    uint64_t live[NP];
     float T[NP], C0[NP], C1[NP], C2[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
         const int py = py0 + lane / TW + RS * k;
-        T[k] = (px < width && py < height) ? 1.f : -1.f;
+        live[k] = __builtin_amdgcn_ballot_w64(px < width && py < height);
+        T[k] = 1.f;
         C0[k] = C1[k] = C2[k] = 0.f;
     }
     if (first < last) {
@@ -592,11 +588,11 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
         f.load_data(xy, conic_opacity, rgb);
         f.load_ids(first + B, last, point_list);
         for (uint32_t base = first; base < last; base += B) {
-            bool any = false;
+            uint64_t any = 0;
 #pragma unroll
             for (int k = 0; k < NP; ++k)
-                any |= T[k] > 0.f;
-            if (!wave_any(any))
+                any |= live[k];
+            if (any == 0)
                 break;
             wave_lds_sync(); // the previous batch has been read
             const int cnt = f.stage_reaching(sm.geo, sm.col, sm.blue, nullptr, base, last, bx0, bx1, by0, by1);
@@ -609,24 +605,25 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
                 const float4 c = sm.col[j];
                 const float blue = sm.blue[j];
                 const LaneTerms lt(pxf, g);
-                // branch-free: every pixel evaluates, selects apply the blend rule
-                bool still = false;
+                uint64_t still = 0;
 #pragma unroll
                 for (int k = 0; k < NP; ++k) {
                     const float alpha = fminf(0.99f, c.y * gauss_at(lt, c.x, pyf0 + float(RS * k) - g.y));
+                    const uint64_t reach = lanes_where<kCmpOGE>(alpha, 1.0f / 255.0f);
                     const float test_T = T[k] * (1.f - alpha);
-                    const bool blend = T[k] > 0.f && alpha >= 1.0f / 255.0f;
-                    const bool stop = blend && test_T < 0.0001f;
-                    const bool use = blend && !stop;
-                    // one select on the weight: fma(c, 0, C) is C exactly (colours are finite, >= 0)
+                    const uint64_t stop = reach & lanes_where<kCmpOLT>(test_T, 0.0001f);
+                    live[k] &= ~stop;
+                    still |= live[k];
+                    const bool use = __builtin_amdgcn_inverse_ballot_w64(live[k] & reach);
+                    // selects apply the blend rule; one on the weight: fma(c, 0, C) is C
+                    // exactly (colours are finite, >= 0)
                     const float wgt = use ? alpha * T[k] : 0.f;
                     C0[k] = fmaf(c.z, wgt, C0[k]);
                     C1[k] = fmaf(c.w, wgt, C1[k]);
                     C2[k] = fmaf(blue, wgt, C2[k]);
-                    T[k] = use ? test_T : (stop ? -T[k] : T[k]);
-                    still |= T[k] > 0.f;
+                    T[k] = use ? test_T : T[k];
                 }
-                if (!wave_any(still))
+                if (still == 0)
                     break;
             }
         }
@@ -637,18 +634,18 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
         const int py = py0 + lane / TW + RS * k;
         if (px < width && py < height) {
             const int64_t p = int64_t(py) * width + px;
-            const float Tk = fabsf(T[k]);
+            const float Tk = T[k];
             framebuffer[p] = fmaf(Tk, bg0, C0[k]);
             framebuffer[plane + p] = fmaf(Tk, bg1, C1[k]);
             framebuffer[2 * plane + p] = fmaf(Tk, bg2, C2[k]);
             final_T[p] = Tk;
         }
     }
-    bool live = false;
+    uint64_t open = 0;
 #pragma unroll
     for (int k = 0; k < NP; ++k)
-        live |= T[k] > 0.f;
-    return wave_any(live);
+        open |= live[k];
+    return open != 0;
 }
 
 // Issue priority of a backward blend wave from its tile's list length
@@ -714,8 +711,9 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
     // far, i.e. the remaining colour plus T_final * background: D carries the
     // remaining-colour term and dL/dT_final * T_final of the alpha adjoint in
     // one scalar per pixel
-    // T[k] = 0 marks a pixel that takes no further part (outside the image,
-    // no gradient, or stopped); a live pixel's T never falls below 1e-4
+    // live[k]: the lanes whose pixel k takes part (inside the image, with a
+    // gradient, not stopped), as a wave-uniform mask
+    uint64_t live[NP];
     float gC0[NP], gC1[NP], gC2[NP], D[NP], T[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
@@ -738,7 +736,8 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
             }
             D[k] = gC0[k] * f0 + gC1[k] * f1 + gC2[k] * f2;
         }
-        T[k] = (inside && !(gC0[k] == 0.f && gC1[k] == 0.f && gC2[k] == 0.f)) ? 1.f : 0.f;
+        T[k] = 1.f;
+        live[k] = __builtin_amdgcn_ballot_w64(inside && !(gC0[k] == 0.f && gC1[k] == 0.f && gC2[k] == 0.f));
     }
     if (first >= last)
         return;
@@ -766,11 +765,11 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
         }
     };
     for (uint32_t base = first; base < last; base += B) {
-        bool any = false;
+        uint64_t any = 0;
 #pragma unroll
         for (int k = 0; k < NP; ++k)
-            any |= T[k] > 0.f;
-        if (!wave_any(any))
+            any |= live[k];
+        if (any == 0)
             break;
         wave_lds_sync(); // the previous batch has been read
         flush();
@@ -794,20 +793,18 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
             const LaneTerms lt(pxf, g);
             // cheap part for every pixel: the blend decisions
             float Gk[NP], alphak[NP];
-            bool use[NP], stop[NP];
-            uint64_t use_lanes[NP]; // use[k] as a lane mask, for the wave-uniform tests
-            uint64_t any_use = 0;
+            uint64_t use_lanes[NP]; // the pixels that blend the Gaussian
+            uint64_t any_use = 0, still = 0;
 #pragma unroll
             for (int k = 0; k < NP; ++k) {
                 Gk[k] = gauss_at(lt, c.x, pyf0 + float(RS * k) - g.y);
                 alphak[k] = fminf(0.99f, c.y * Gk[k]);
-                const float test_T = T[k] * (1.f - alphak[k]);
-                const bool blend = T[k] > 0.f && alphak[k] >= 1.0f / 255.0f;
-                stop[k] = blend && test_T < 0.0001f;
-                use[k] = blend && !stop[k];
-                use_lanes[k] = lanes_where<kCmpOGT>(T[k], 0.f) & lanes_where<kCmpOGE>(alphak[k], 1.0f / 255.0f)
-                    & lanes_where<kCmpUGE>(test_T, 0.0001f);
+                const uint64_t reach = lanes_where<kCmpOGE>(alphak[k], 1.0f / 255.0f);
+                // a pixel stops before the Gaussian that would take T under 1e-4
+                live[k] &= ~(reach & lanes_where<kCmpOLT>(T[k] * (1.f - alphak[k]), 0.0001f));
+                use_lanes[k] = live[k] & reach;
                 any_use |= use_lanes[k];
+                still |= live[k];
             }
             if (any_use != 0) {
                 float m0 = 0.f, m1 = 0.f, m2 = 0.f, so = 0.f, sr = 0.f, sg = 0.f, sbl = 0.f;
@@ -821,8 +818,9 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
                     const float raw = c.y * Gk[k];
                     const float tk = 1.f - alphak[k];
                     const float test_T = T[k] * tk;
+                    const bool use = __builtin_amdgcn_inverse_ballot_w64(use_lanes[k]);
                     // one select on the weight: fma(x, 0, s) is s exactly for finite x
-                    const float wgt = use[k] ? alphak[k] * T[k] : 0.f;
+                    const float wgt = use ? alphak[k] * T[k] : 0.f;
                     // <dL/dC, rgb> and dL/dalpha as fused multiply-adds (gradient
                     // values only: no blend decision reads them)
                     const float grgb = fmaf(gC2[k], blue, fmaf(gC1[k], c.w, gC0[k] * c.z));
@@ -833,13 +831,13 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
                     // 1 - alpha >= 0.01, so the hardware reciprocal (1 ulp) is ample
                     const float inv_tk = __builtin_amdgcn_rcpf(tk);
                     const float g_alpha = fmaf(grgb, T[k], -(D[k] * inv_tk));
-                    const float g_raw = (use[k] && raw < 0.99f) ? g_alpha : 0.f;
+                    const float g_raw = (use && raw < 0.99f) ? g_alpha : 0.f;
                     so = fmaf(Gk[k], g_raw, so);
                     const float gp = raw * g_raw; // dL/dpower
                     m0 += gp;
                     m1 = fmaf(gp, dy, m1);
                     m2 = fmaf(gp * dy, dy, m2);
-                    T[k] = use[k] ? test_T : T[k];
+                    T[k] = use ? test_T : T[k];
                 }
                 // power = -a/2 dx^2 - b dx dy - c/2 dy^2 with dx = px - x, dy = py - y
                 const float a = g.z * kUnscaleDiag, b = g.w * kUnscaleOff, cc = c.x * kUnscaleDiag;
@@ -854,14 +852,7 @@ __device__ __forceinline__ void blend_tile_backward(BlendSmemBwd<B>& sm, uint32_
                 if (slot8 >= 0)
                     sm.acc[9 * j + slot8] = slot8 == 8 ? t9 : t8;
             }
-            // a pixel stops before the Gaussian that would take T under 1e-4
-            bool still = false;
-#pragma unroll
-            for (int k = 0; k < NP; ++k) {
-                T[k] = stop[k] ? 0.f : T[k];
-                still |= T[k] > 0.f;
-            }
-            if (!wave_any(still))
+            if (still == 0)
                 break;
         }
     }
