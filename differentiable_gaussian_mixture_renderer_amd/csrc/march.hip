@@ -184,7 +184,7 @@ __device__ __forceinline__ Ray1d<S> intersect_staged(const Staged<S>& g, const S
     return intersect_ray_pre(g.mu, g.A, g.m, g.norm3, o, d);
 }
 
-// The window of a Gaussian over the tile's rays (gaussian_window): a section or
+// The window of a Gaussian over the tile's rays (gaussian_extent): a section or
 // a bin of it needs
 //   mass on the ray >= 1/255 and z <= 3:   E + z^2 <= 2 ln M + 2 ln 255 + 9
 //   z within far_radius' cut:              E + z^2 <= 2 ln M + 2 ln 55556, or
@@ -616,7 +616,7 @@ constexpr int kBinGroup = 8;
 // the exact restriction each time and all of a chunk's bins once one pixel's
 // Gaussian reached it, the forward took 52.0 ms on 200k Gaussians at 1024^2 and
 // forward + backward 56.3 ms on 60k at 491x373; with windows, groups and the
-// short restriction 17.4 and 22.3 ms.
+// sections of sections.h 17.3 and 22.6 ms.
 template <class S, int NT, int CB>
 __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 1], bool stopped, TileList<S, NT>& tl, bool inside,
     const S* o, const S* d, S b_first, S b_last, const Candidates& cand)
@@ -1336,8 +1336,8 @@ void launch_march(bool backward, const MarchData<S>& md, const DevCamera<S>& dc,
     const dim3 grid(md.n_tiles), block(TW * TH);
     // float: 32 bins in registers per pass (two waves per SIMD) unless
     // bins_per_chunk asks for 16 (three waves per SIMD, more passes): 200k
-    // Gaussians at 1024^2 take 27.4 / 35.4 ms forward, 24.9 / 34.6 ms read
-    // back from a replay store and 50.2 / 66.9 ms recomputed
+    // Gaussians at 1024^2 take 16.5 / 19.4 ms forward, 24.6 / 30.8 ms read
+    // back from a replay store and 26.0 / 32.8 ms recomputed
     if constexpr (sizeof(S) == 4) {
         const bool chunk16 = ctl.bins_per_chunk == 16;
         if (!backward && ctl.render_mode == 0) {

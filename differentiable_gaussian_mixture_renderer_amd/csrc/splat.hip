@@ -15,6 +15,9 @@
 //      Gaussian id) order, which is the reference's stable order.
 //   6. k_tile_ranges        [first, last) per tile (binary search per tile)
 //   7. k_blend_forward      per tile, LDS-staged batches of Gaussians
+// A view of at most 16 384 Gaussians takes steps 2 and 3 and the bounds in one
+// launch (k_bin_one); the autograd path bins deep views by a prefix of the depth
+// order (k_extend_*).
 // Backward: k_blend_backward (front-to-back replay, transmittance recomputed,
 // wave-reduced atomics) then k_splat_preprocess_backward (per Gaussian).
 #include <algorithm>

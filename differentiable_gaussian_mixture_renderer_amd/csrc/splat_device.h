@@ -558,6 +558,10 @@ __device__ __forceinline__ float gauss_at(const LaneTerms& t, float c_scaled, fl
     return __builtin_amdgcn_exp2f(fmaf(fmaf(c_scaled, dy, t.bdx), dy, t.adx2));
 }
 
+// Bound by VALU issue where the tiles fill the chip.  Which pixels still take
+// Gaussians is kept as wave-uniform masks: with the sign of the transmittance
+// instead, four vector operations a pixel and Gaussian where these are three
+// scalar ones, 39k tiles took 0.325 ms against 0.28 and 8 160 tiles 85 us against 76.
 // Returns whether some pixel of the tile would take more Gaussians than the
 // list holds.
 template <int TW, int TH, int B>
