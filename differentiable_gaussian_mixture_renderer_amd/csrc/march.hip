@@ -173,9 +173,10 @@ struct alignas(16) Staged {
     S mu[3];
     S norm3;  // sqrt(det A) / sqrt((2 pi)^3)
     S mass;
-    S rgb[3];
+    S rgb[3];     // 0 where it is not finite
     S depth;
     uint32_t id;
+    uint32_t odd; // bit c: component c of the colour is infinite or NaN, bit 3 + c: NaN
 };
 
 template <class S>
@@ -253,10 +254,14 @@ template <class S>
 __device__ __forceinline__ void stage_gaussian(Staged<S>* dst, Reach1d* win, uint32_t id, const MarchData<S>& md, const S* o, const TileAxis& ax)
 {
     Staged<S> g;
+    g.odd = 0;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         g.mu[k] = md.means[3 * id + k];
-        g.rgb[k] = md.rgb[3 * id + k];
+        const S c = md.rgb[3 * id + k];
+        const bool odd = !(fabs(c) < S(__builtin_huge_val()));
+        g.rgb[k] = odd ? S(0) : c;
+        g.odd |= odd ? (c != c ? 9u : 1u) << k : 0u;
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k)
@@ -617,13 +622,18 @@ constexpr int kBinGroup = 8;
 // Gaussian reached it, the forward took 52.0 ms on 200k Gaussians at 1024^2 and
 // forward + backward 56.3 ms on 60k at 491x373; with windows, groups and the
 // sections of sections.h 17.3 and 22.6 ms.
-template <class S, int NT, int CB>
+template <bool ODD, class S, int NT, int CB>
 __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 1], bool stopped, TileList<S, NT>& tl, bool inside,
     const S* o, const S* d, S b_first, S b_last, const Candidates& cand)
 {
 #pragma unroll
     for (int k = 0; k < CB; ++k)
         bins[k][0] = bins[k][1] = bins[k][2] = bins[k][3] = 0;
+    // ODD: a colour that is not finite goes only where its mass does (0 times it
+    // is NaN): the bins, as bits per component, that kept mass of such a colour.
+    // The backward needs none of it: the pixel's own colour is not finite.
+    uint32_t odd_bins[3] = { 0, 0, 0 }, odd_nan = 0;
+    static_assert(CB <= 32, "one bit per bin");
     const uint32_t end = __syncthreads_count(!stopped) == 0 ? tl.first : tl.last;
     const float inf = __builtin_inff();
     // no entry meets the empty window of a wave whose pixels have all stopped
@@ -647,6 +657,20 @@ __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 
                 const bool need = deposits_in(r, pass, b_first, b_last, bb[0], bb[CB]);
                 const S lo = need ? r.centre - r.far : S(inf), hi = need ? r.centre + r.far : S(-inf);
                 const S mor = need ? r.mor : S(0);
+                if constexpr (ODD) {
+                    const uint32_t odd = __builtin_amdgcn_readfirstlane(g.odd);
+                    if (odd != 0) {
+                        uint32_t kept = 0;
+                        S c0 = cdf_inv_sd(r.centre, r.inv_sd, bb[0]);
+                        static_for<CB>([&](auto k) {
+                            const S c1 = cdf_inv_sd(r.centre, r.inv_sd, bb[k + 1]);
+                            kept |= (c1 - c0) * mor >= S(0.00001f) ? 1u << k : 0u;
+                            c0 = c1;
+                        });
+                        static_for<3>([&](auto c) { odd_bins[c] |= (odd >> c) & 1u ? kept : 0u; });
+                        odd_nan |= kept ? odd >> 3 : 0u;
+                    }
+                }
                 S c0 = 0;
                 bool have = false;
                 static_for<CB / kBinGroup>([&](auto group) {
@@ -674,6 +698,14 @@ __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 
             }
             cw.store(cand);
         }
+    }
+    if (ODD && __builtin_amdgcn_ballot_w64((odd_bins[0] | odd_bins[1] | odd_bins[2]) != 0) != 0) {
+        static_for<CB>([&](auto k) {
+            static_for<3>([&](auto c) {
+                const S v = (odd_nan >> c) & 1u ? S(__builtin_nan("")) : S(__builtin_huge_val());
+                bins[k][c] = (odd_bins[c] >> k) & 1u ? v : bins[k][c];
+            });
+        });
     }
 }
 
@@ -731,7 +763,7 @@ __global__ __launch_bounds__(TW* TH, sizeof(S) == 4 ? 2 : 1) void k_march_forwar
             for (int k = 1; k <= CB; ++k)
                 bb[k] = (k <= kk) ? walk.next(sec) : bb[k - 1];
             S bins[CB][4];
-            fill_chunk<S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
+            fill_chunk<true, S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
             if (rec) {
                 S* rb = rec + (int64_t(ch * CB) * NT + threadIdx.x) * 4;
                 S* rd = rec + int64_t(NT) * 4 * kBins + int64_t(ch * CB) * NT + threadIdx.x;
@@ -745,12 +777,11 @@ __global__ __launch_bounds__(TW* TH, sizeof(S) == 4 ? 2 : 1) void k_march_forwar
                     rd[int64_t(kk) * NT] = bb[CB];
             }
             // blend, branch-free (branches around the bins cost copies of them):
-            // a stopped pixel's weight is 0, bins past the chunk's end are empty
+            // a stopped pixel takes nothing more, bins past the chunk's end are empty
             static_for<CB>([&](auto k) {
-                const S w = stopped ? S(0) : T;
-                C0 += bins[k][0] * w;
-                C1 += bins[k][1] * w;
-                C2 += bins[k][2] * w;
+                C0 = stopped ? C0 : C0 + bins[k][0] * T;
+                C1 = stopped ? C1 : C1 + bins[k][1] * T;
+                C2 = stopped ? C2 : C2 + bins[k][2] * T;
                 T = stopped ? T : T * dexp(-bins[k][3]);
                 stopped = stopped || T < S(1. / 255.);
             });
@@ -837,7 +868,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_forward_debug(MarchData<S> md,
             if (bins_mode && (target < ch * CB || target >= ch * CB + kk))
                 continue; // only the chunk holding the shown bin
             S bins[CB][4];
-            fill_chunk<S, NT, CB>(bins, bb, done, tl, inside, o, d, b_first, b_last, cand);
+            fill_chunk<true, S, NT, CB>(bins, bb, done, tl, inside, o, d, b_first, b_last, cand);
 #pragma unroll
             for (int k = 0; k < CB; ++k) {
                 if (k < kk) {
@@ -901,10 +932,10 @@ __device__ __forceinline__ S wave_total(S v)
 // Blend adjoint of one chunk (grad/math.h:529-557), front to back from the
 // running transmittance T and remaining colour Cr: bin k's gradient is
 // dL/d(rgb mass) = Tk[k] dL/dC and dL/d(mass) = Gk[k].  Bins past the chunk
-// end or after the pixel stopped get zero.
+// end or after the pixel stopped get zero, and borders that make them empty.
 template <class S, int CB>
-__device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bool& stopped, S& T, S* Cr, S Tf, S gT, const S* gC, S (&Tk)[CB],
-    S (&Gk)[CB])
+__device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], S (&bb)[CB + 1], int kk, bool& stopped, S& T, S* Cr, S Tf, S gT,
+    const S* gC, S (&Tk)[CB], S (&Gk)[CB])
 {
 #pragma unroll
     for (int k = 0; k < CB; ++k) {
@@ -922,6 +953,8 @@ __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bo
             T *= tk;
             if (T < S(1. / 255.))
                 stopped = true;
+        } else {
+            bb[k + 1] = bb[k];
         }
     }
 }
@@ -932,7 +965,9 @@ __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], int kk, bo
 // gradient of the bin's mass is Tk (dL/dC . rgb) + Gk; the rgb gradient is
 // dL/dC times the sum of Tk mass, and the centre and inverse-sd gradients
 // collect the cdf derivatives at both borders of every bin.  Entries, groups of
-// bins and kept bins are fill_chunk's; Tk = Gk = 0 past the pixel's stop.
+// bins and kept bins are fill_chunk's up to the pixel's stop, past which its
+// bins are empty: a pixel adds to the Gaussians it took mass from and to no
+// other, also where its gradient or a colour is infinite or NaN.
 template <class S, int NT, int CB>
 __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candidates& cand, bool active, bool inside, const S* o, const S* d,
     const S (&bb)[CB + 1], S b_first, S b_last, const S (&Tk)[CB], const S (&Gk)[CB], const S* gC, S* __restrict__ render_grads)
@@ -962,7 +997,7 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candida
                 const S gcr = dfma(gC[2], g.rgb[2], dfma(gC[1], g.rgb[1], gC[0] * g.rgb[0]));
                 S c0 = 0, p0 = 0, q0 = 0;
                 S s_d = 0, s_tm = 0, s_c = 0, s_i = 0;
-                bool have = false, any = false;
+                bool have = false, contrib = false;
                 static_for<CB / kBinGroup>([&](auto group) {
                     constexpr int k0 = group * kBinGroup;
                     if (__builtin_amdgcn_ballot_w64(hi > bb[k0] && lo < bb[k0 + kBinGroup]) == 0) {
@@ -971,7 +1006,7 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candida
                     }
                     if (!have)
                         cdf_grad_step(r.centre, r.inv_sd, bb[k0], &c0, &p0, &q0);
-                    have = any = true;
+                    have = true;
                     static_for<kBinGroup>([&](auto bin) {
                         constexpr int k = k0 + bin;
                         S c1, p1, q1;
@@ -979,8 +1014,9 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candida
                         const S delta = c1 - c0;
                         // the bin's mass max(0, m) is kept from 1e-5 on (NaN is not)
                         const bool kept = delta * mor >= S(0.00001f);
+                        contrib = contrib || kept;
                         const S tk = kept ? Tk[k] : S(0);
-                        const S g_m = dfma(tk, gcr, kept ? Gk[k] : S(0));
+                        const S g_m = kept ? dfma(Tk[k], gcr, Gk[k]) : S(0);
                         s_tm = dfma(tk, delta, s_tm);
                         s_d = dfma(g_m, delta, s_d);
                         s_c = dfma(g_m, p1 - p0, s_c);
@@ -990,13 +1026,13 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candida
                         q0 = q1;
                     });
                 });
-                if (!any)
+                if (__builtin_amdgcn_ballot_w64(contrib) == 0)
                     continue;
                 S gr[13];
 #pragma unroll
                 for (int q = 0; q < 13; ++q)
                     gr[q] = 0;
-                if (need) {
+                if (contrib) {
                     S fp, fq;
                     cdf_grad_scale(r.inv_sd, &fp, &fq);
                     // d L / d mass on the ray = s_d; weight = mor / mass
@@ -1120,8 +1156,8 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
             {
                 S bins[CB][4];
                 // pass 2 (identical to the forward)
-                fill_chunk<S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
-                blend_adjoint<S, CB>(bins, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
+                fill_chunk<false, S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
+                blend_adjoint<S, CB>(bins, bb, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
             }
             adjoint_chunk<S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
         }
@@ -1187,7 +1223,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
                     else
                         bins[k][0] = bins[k][1] = bins[k][2] = bins[k][3] = 0;
                 }
-                blend_adjoint<S, CB>(bins, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
+                blend_adjoint<S, CB>(bins, bb, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
             } else {
 #pragma unroll
                 for (int k = 0; k < CB; ++k)

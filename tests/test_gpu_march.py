@@ -528,3 +528,46 @@ def test_entry_windows_at_extreme_shapes(kind):
         got = out["grads"][name].reshape(n, -1)
         ref_g = np.asarray(want[name]).reshape(n, -1)[:, :got.shape[1]]
         assert np.abs(got - ref_g).max() <= 1e-7 * np.abs(ref_g).max(), name
+
+
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_values_that_are_not_finite_stay_where_mass_is(dtype_name, value):
+    """A colour that is not finite shows in the pixels that take mass of its
+    Gaussian, in its component, and nowhere else; a gradient that is not
+    finite at a pixel reaches the Gaussians that the pixel took mass from and
+    no other.  Which pixels and Gaussians those are is read from a colour of
+    1 and of 300 (mass of 1e-5 behind a transmittance of 1/255 moves the pixel
+    by 1e-5, float rounding by 1e-7), and from a gradient of 1."""
+    torch = _torch()
+    dtype = getattr(torch, dtype_name)
+    scene, cam = small_scene(n=2500, w=64, h=48, seed=5)
+    odd = np.arange(0, scene.n, 60)
+    bg = np.array([0.2, 0.3, 0.4])
+    images = []
+    for v in (1.0, 300.0, value):
+        scene.sh[odd] = 0.0
+        scene.sh[odd, 0, 0] = (v - 0.5) / 0.28209479177387814
+        images.append(run_gpu(scene, cam, bg, dtype)["framebuffer"])
+    a, b, got = images
+    untouched = a[0] == b[0]
+    print(f"{dtype_name} {value}: pixels without that colour {untouched.mean():.3f}")
+    assert 0.1 < untouched.mean() < 0.95
+    np.testing.assert_array_equal(got[1:], a[1:])
+    np.testing.assert_array_equal(got[0][untouched], a[0][untouched])
+    assert not np.isfinite(got[0][~untouched]).any()
+
+    scene.sh[odd, 0, 0] = 1.0
+    py, px = np.unravel_index(np.argmin(run_gpu(scene, cam, bg, dtype)["remaining"]), (cam.height, cam.width))
+    for replay in (0, 16):
+        grads = []
+        for v in (1.0, value):
+            g = np.zeros((3, cam.height, cam.width))
+            g[0, py, px] = v
+            grads.append(run_gpu(scene, cam, bg, dtype, grad_fb=g, replay_steps=replay)["grads"])
+        took = sum(np.abs(x.reshape(scene.n, -1)).sum(axis=1) for x in grads[0].values()) > 0
+        assert 3 < took.sum() < scene.n // 2
+        for name, x in grads[1].items():
+            assert np.isfinite(x[~took]).all(), (replay, name)
+            assert not (x[~took] != 0).any(), (replay, name)
+        assert not np.isfinite(grads[1]["opacity"].reshape(-1)[took]).any(), replay
