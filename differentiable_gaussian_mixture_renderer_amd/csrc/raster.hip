@@ -373,7 +373,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
     __shared__ RasterWindow s_win[kThreads];
     __shared__ float s_axis[4];
     __shared__ uint64_t s_seen[kThreads / 64][2][kSeenWords];
-    __shared__ float s_rgb[3][kThreads];
+    __shared__ float s_rgb[3][kThreads];  // 0 where it is not finite
+    __shared__ uint32_t s_odd[kThreads];  // bit c: component c of the colour is infinite (or NaN)
     __shared__ float s_border[kThreads * kBorderStride];
     // the reference returns before rendering when no Gaussian is binned
     // (vol_raster_forward.cu:153-155): the caller's framebuffer stays as it was
@@ -411,11 +412,16 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
         const uint32_t k = first + uint32_t(round) * kThreads + uint32_t(t_id);
         if (k < last) {
             const uint32_t id = a.point_list[k];
+            uint32_t odd = 0;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 s_mu[c][t_id] = a.means[3 * id + c];
-                s_rgb[c][t_id] = a.rgb[3 * id + c];
+                const float v = a.rgb[3 * id + c];
+                const bool finite = fabsf(v) < __builtin_inff();
+                s_rgb[c][t_id] = finite ? v : 0.f;
+                odd |= finite ? 0u : 1u << c;
             }
+            s_odd[t_id] = odd;
             float A[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c)
@@ -511,6 +517,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
         // ------------------------------------------------------------ pass 2
         float result[3] = { 0.f, 0.f, 0.f };
         float transparency = 1.f;
+        uint32_t odd_seen = 0; // components in which the pixel kept mass of a colour that is not finite
         const float max_distance = end_of(kRasterBins - 1);
         const unsigned lane = lane_id();
         uint64_t* rejected = s_seen[t_id / 64][0];
@@ -567,7 +574,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                         const float rgb[3] = { s_rgb[0][j], s_rgb[1][j], s_rgb[2][j] };
                         const float e_scale = -0.72134752044448170f * __builtin_amdgcn_rcpf(var); // exp(-d^2 / (2 var)) = 2^(e_scale d^2)
                         float cdf_start = 0.f;
-                        bool have = false;
+                        bool have = false, kept = false;
                         static_for<kChunk / kGroup>([&](auto group) {
                             constexpr int g0 = group * kGroup;
                             const float x0 = begin_of(k0 + g0);
@@ -586,6 +593,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                                 const float mass = (cdf_end - cdf_start) * wk;
                                 cdf_start = cdf_end;
                                 const bool on = !(mass < 0.0001f) && need;
+                                kept = kept || on;
                                 const float mq = on ? mass : 0.f;
                                 const float d = x - c;
                                 const float e = on ? wk * __builtin_amdgcn_exp2f(d * d * e_scale) : 0.f;
@@ -600,6 +608,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                                 be[q][3] += e;
                             });
                         });
+                        // 0 times such a colour is NaN, so it is kept out of the sums
+                        const uint32_t odd = __builtin_amdgcn_readfirstlane(s_odd[j]);
+                        if (odd != 0)
+                            odd_seen |= kept ? odd : 0u;
                         // the evaluation at the chunk's right border belongs to the
                         // next bin, added when that bin's mass passes (or, after the
                         // last bin, always)
@@ -649,9 +661,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                 }
             });
         }
-        C[0] = result[0];
-        C[1] = result[1];
-        C[2] = result[2];
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch)
+            C[ch] = (odd_seen >> ch) & 1u ? __builtin_nanf("") : result[ch];
     } else if (a.mode == 2) {
         const int bin = int(min(unsigned(a.debug_bin), unsigned(kRasterBins - 1)));
         const float dist = end_of(bin);

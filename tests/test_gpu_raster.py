@@ -140,3 +140,29 @@ def test_raster_empty_view_and_single_gaussian():
     phi = lambda x: 0.5 * (1 + math.erf(x / math.sqrt(2)))
     M = opacity * (scale + f * f) ** 2 / var * (phi(3.0) - phi(-d / math.sqrt(var)))
     np.testing.assert_allclose(got[:, H // 2, W // 2], rgb * (1 - math.exp(-M)) + bg, rtol=0, atol=2e-3)
+
+
+def test_infinite_colours_stay_where_their_mass_is():
+    """An infinite colour makes the pixels that keep mass of its Gaussian NaN
+    (the integrand's segments divide it by itself), in its component, and no
+    other pixel: which those are is read from a colour of 1 and of 300 (a kept
+    mass is at least 1e-4, so the pixel moves by far more than float rounding).
+    A NaN colour never gets here: the clamp at 0 makes it 0."""
+    if not gpu_available():
+        pytest.skip("no GPU")
+    sc, cam = _scene(2500, 21, width=77, height=53)
+    means, scales, rots, opac, sh16, deg = sc
+    odd = np.arange(0, 2500, 60)
+    bg = np.array([0.1, 0.2, 0.3], np.float32)
+    images = []
+    for v in (1.0, 300.0, np.inf):
+        sh = sh16.copy()
+        sh[odd, 0, 0] = (v - 0.5) / SH_C0
+        images.append(_gpu((means, scales, rots, opac, sh, deg), cam, bg)[0])
+    a, b, got = images
+    untouched = a[0] == b[0]
+    print(f"pixels without that colour {untouched.mean():.3f}")
+    assert 0.1 < untouched.mean() < 0.95
+    np.testing.assert_array_equal(got[1:], a[1:])
+    np.testing.assert_array_equal(got[0][untouched], a[0][untouched])
+    assert np.isnan(got[0][~untouched]).all()
