@@ -19,6 +19,7 @@
 #include "device_math.h"
 #include "host_common.h"
 #include "march_device.h"
+#include "raster_terms.h"
 #include "splat_device.h"
 
 namespace dgmr {
@@ -128,7 +129,7 @@ struct BinSizer {
         float tr[L];
         float t = 1.f;
         static_for<L>([&](auto i) {
-            t *= __builtin_amdgcn_exp2f(m[i] * -1.4426950408889634f);
+            t *= slot_transmittance(m[i]);
             tr[i] = t;
         });
         int best = -1;

@@ -1,8 +1,10 @@
 """Builds tests/cpp/_build/libfacade_check.so: the C++ façade check
 (facade_check.cpp over include/dgmr.hpp) that tests/test_gpu_facade.py loads,
 libreach_check.so, the host build of the blends' tile-reach test that
-tests/test_tile_reach.py checks, and libsection_check.so, the host build of the
-marcher's section list that tests/test_section_list.py checks.  Run by __graft_entry__.build() after the
+tests/test_tile_reach.py checks, libsection_check.so, the host build of the
+marcher's section list that tests/test_section_list.py checks, and
+libraster_check.so, the host build of the rasteriser's scalar terms that
+tests/test_raster_terms.py checks.  Run by __graft_entry__.build() after the
 library itself."""
 import os
 import subprocess
@@ -17,6 +19,9 @@ REACH_OUT = os.path.join(HERE, "_build", "libreach_check.so")
 
 
 SECTION_OUT = os.path.join(HERE, "_build", "libsection_check.so")
+
+
+RASTER_OUT = os.path.join(HERE, "_build", "libraster_check.so")
 
 
 def _build_host(source: str, out: str) -> str:
@@ -41,6 +46,11 @@ def build_sections() -> str:
     return _build_host("section_check.cpp", SECTION_OUT)
 
 
+def build_raster() -> str:
+    """The rasteriser's scalar terms, for a CPU check against double."""
+    return _build_host("raster_check.cpp", RASTER_OUT)
+
+
 def build() -> str:
     os.makedirs(os.path.dirname(OUT), exist_ok=True)
     cmd = ["hipcc", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", os.path.join(ROOT, "include"), os.path.join(HERE, "facade_check.cpp"),
@@ -55,4 +65,5 @@ def build() -> str:
 if __name__ == "__main__":
     print(build_reach())
     print(build_sections())
+    print(build_raster())
     print(build())
