@@ -573,7 +573,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                         const float lo = need ? c - far : __builtin_inff(), hi = need ? c + far : -__builtin_inff();
                         const float wk = need ? w : 0.f;
                         const float rgb[3] = { s_rgb[0][j], s_rgb[1][j], s_rgb[2][j] };
-                        const float e_scale = -0.72134752044448170f * __builtin_amdgcn_rcpf(var); // exp(-d^2 / (2 var)) = 2^(e_scale d^2)
+                        const DensityScale e_scale = density_scale(var);
                         float cdf_start = 0.f;
                         bool have = false, kept = false;
                         static_for<kChunk / kGroup>([&](auto group) {
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                                 kept = kept || on;
                                 const float mq = on ? mass : 0.f;
                                 const float d = x - c;
-                                const float e = on ? wk * __builtin_amdgcn_exp2f(d * d * e_scale) : 0.f;
+                                const float e = on ? wk * border_density(e_scale, d) : 0.f;
                                 x = xe;
                                 bm[q][0] = fmaf(rgb[0], mq, bm[q][0]);
                                 bm[q][1] = fmaf(rgb[1], mq, bm[q][1]);
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_raster_render(RasterArgs a)
                             if (!last_chunk)
                                 add_right = next && !((cdf_sd(c, inv_sd, x_end) - cdf_sd(c, inv_sd, x_right)) * wk < 0.0001f);
                             const float d = x_right - c;
-                            const float e = add_right ? wk * __builtin_amdgcn_exp2f(d * d * e_scale) : 0.f;
+                            const float e = add_right ? wk * border_density(e_scale, d) : 0.f;
                             be[kChunk][0] = fmaf(rgb[0], e, be[kChunk][0]);
                             be[kChunk][1] = fmaf(rgb[1], e, be[kChunk][1]);
                             be[kChunk][2] = fmaf(rgb[2], e, be[kChunk][2]);

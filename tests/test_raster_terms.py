@@ -32,3 +32,27 @@ def test_slot_transmittance_holds_float_rounding():
     keep = m <= 86.0
     err = np.abs(out.astype(np.float64) / np.exp(-m.astype(np.float64)) - 1.0)[keep]
     assert err.max() <= 1.5 * 2.0 ** -24 + 2.0 ** -26, err.max()
+
+
+def test_border_density_is_no_further_off_than_the_plain_expression():
+    """exp(-d^2 / (2 var)) from the centre out to 9 standard deviations, over
+    the variances of near and far Gaussians: rms and largest relative error at
+    most those of expf(-d^2 / 2 / var) in float."""
+    rng = np.random.default_rng(2)
+    n = 200_000
+    var = np.exp(rng.normal(-6.0, 2.0, n)).astype(np.float32)
+    d = (rng.uniform(-9.0, 9.0, n) * np.sqrt(var)).astype(np.float32)
+    out, plain = np.empty_like(d), np.empty_like(d)
+    _lib().density_batch(n, _ptr(d), _ptr(var), _ptr(out), _ptr(plain))
+    exact = np.exp(-0.5 * d.astype(np.float64) ** 2 / var.astype(np.float64))
+    e, p = out / exact - 1.0, plain / exact - 1.0
+    rms = lambda x: np.sqrt((x * x).mean())
+    print(f"rms {rms(e):.3g} (plain {rms(p):.3g}), largest {np.abs(e).max():.3g} ({np.abs(p).max():.3g})")
+    assert rms(e) <= rms(p)
+    assert np.abs(e).max() <= np.abs(p).max()
+    # at the centre 1; where the square or the exponent overflows 0, as the plain expression
+    edge = np.array([[0.0, 1e-3], [1e3, 1e-3], [1e20, 1e-3], [1e5, 1e-30], [3e19, 1e30]], np.float32)
+    o, q = np.empty(5, np.float32), np.empty(5, np.float32)
+    _lib().density_batch(5, _ptr(np.ascontiguousarray(edge[:, 0])), _ptr(np.ascontiguousarray(edge[:, 1])), _ptr(o), _ptr(q))
+    np.testing.assert_array_equal(o, [1.0, 0.0, 0.0, 0.0, 0.0])
+    np.testing.assert_array_equal(o, q)
