@@ -21,6 +21,9 @@ DGMR_F32 = 0
 DGMR_F64 = 1
 DGMR_ACT_NONE = 0
 DGMR_ACT_LOG_NORM_SIGMOID = 1
+DGMR_LISTS_WHOLE = 0
+DGMR_LISTS_PREFIX = 1
+DGMR_LISTS_AUTO = 2
 
 c_void_p = ctypes.c_void_p
 
@@ -157,6 +160,8 @@ SIGNATURES = {
     "dgmr_splat_prefix_pairs": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _P(Tiling), ctypes.c_int64, _P(ctypes.c_int64)]),
     "dgmr_splat_forward_prefix": (ctypes.c_int, [_P(Gaussians), _P(Camera), _P(Tiling), _P(SplatGeometry), _P(Binning), c_void_p, c_void_p,
                                                  c_void_p, ctypes.c_size_t, _P(Stats), c_void_p]),
+    "dgmr_splat_forward_lists": (ctypes.c_int, [_P(Gaussians), _P(Camera), _P(Tiling), _P(SplatGeometry), _P(Binning), c_void_p, c_void_p,
+                                                c_void_p, ctypes.c_size_t, ctypes.c_int32, _P(ctypes.c_int64), _P(Stats), c_void_p]),
     "dgmr_splat_backward": (ctypes.c_int, [_P(Gaussians), _P(Camera), _P(Tiling), _P(SplatGeometry), _P(Binning), ctypes.c_int64,
                                            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                            c_void_p]),

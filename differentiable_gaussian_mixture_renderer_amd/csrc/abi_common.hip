@@ -202,7 +202,7 @@ int acquire_count_slot(CountSlot* out)
 }
 } // namespace
 
-int enqueue_count(const uint32_t* dev_count, hipStream_t st, PendingCount* pc)
+int enqueue_count(const uint32_t* dev_count, hipStream_t st, PendingCount* pc, int binned_word)
 {
     if (!t_slot.slot.host) {
         const int rc = acquire_count_slot(&t_slot.slot);
@@ -211,11 +211,12 @@ int enqueue_count(const uint32_t* dev_count, hipStream_t st, PendingCount* pc)
     }
     uint32_t* host = t_slot.slot.host;
     hipEvent_t done = t_slot.slot.done;
-    DGMR_HIP_CHECK(hipMemcpyAsync(host, dev_count, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    DGMR_HIP_CHECK(hipMemcpyAsync(host, dev_count, size_t(binned_word ? binned_word + 2 : 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     DGMR_HIP_CHECK(hipEventRecord(done, st));
     pc->device = dev_count;
     pc->host = host;
     pc->done = done;
+    pc->binned_word = binned_word;
     return DGMR_OK;
 }
 
@@ -228,8 +229,10 @@ int64_t PendingCount::wait()
         return -1;
     }
     const int64_t r = int64_t(*host);
+    binned = int64_t(host[binned_word]);
+    few = binned_word && host[binned_word + 1] != 0;
     for (int k = 0; k < n_slots; ++k)
-        stage_set_bytes(slot[k], per_pair[k] * double(r) + fixed[k]);
+        stage_set_bytes(slot[k], per_pair[k] * double(binned) + fixed[k]);
     return r;
 }
 

@@ -87,7 +87,7 @@ struct PendingCount {
     const uint32_t* device = nullptr; // the count on the device, readable by later kernels
     const volatile uint32_t* host = nullptr;
     hipEvent_t done = nullptr;
-    // stages whose byte model depends on R: bytes = per_pair * R + fixed
+    // stages whose byte model depends on the binned pairs: bytes = per_pair * pairs + fixed
     int slot[4] = { -1, -1, -1, -1 };
     double per_pair[4] = { 0, 0, 0, 0 }, fixed[4] = { 0, 0, 0, 0 };
     int n_slots = 0;
@@ -100,11 +100,15 @@ struct PendingCount {
             ++n_slots;
         }
     }
+    int binned_word = 0;    // words behind the count: the pairs that are binned (0: all), and whether few tiles will be open
+    int64_t binned = 0;     // after wait()
+    bool few = false;
     // R, or -1 when waiting failed; fills the stage byte models
     int64_t wait();
 };
-// queues the copy of *dev_count; returns DGMR_OK or DGMR_ERR_DEVICE
-int enqueue_count(const uint32_t* dev_count, hipStream_t st, PendingCount* pc);
+// queues the copy of *dev_count and, binned_word words behind it, the pairs that
+// are binned (0: all are) with the flag that follows; returns DGMR_OK or DGMR_ERR_DEVICE
+int enqueue_count(const uint32_t* dev_count, hipStream_t st, PendingCount* pc, int binned_word = 0);
 
 // multi-view binning: Gaussian ids span n_views blocks of n_per_view; view v's
 // tiles occupy [views[v].z, views[v].z + views[v].x * views[v].y) of the
@@ -120,21 +124,31 @@ struct BatchBinning {
     int64_t max_view_tiles; // largest grid_x * grid_y over the views
 };
 
-// Prefix binning (single views without tight culling): bins->pair_capacity
-// holds the first pairs of the depth order, and what the extension of the lists
-// needs comes back here, valid until the workspace is used again.
+// Prefix binning (single views without tight culling): the first three are the
+// caller's, the rest comes back, valid until the workspace is used again.
 struct PrefixBinning {
-    const uint32_t* origin; // tile rectangles by position of the depth order
-    const uint32_t* size;
-    const uint32_t* ids;    // Gaussian ids by position of the depth order
+    uint32_t pairs;         // the first pairs of the depth order that are binned when the view has many more
+    bool always;            // without looking at how much they cover
+    const float4* conic_opacity; // by id
+    const uint32_t* ids;    // by position of the depth order, as the tile rectangles
+    uint32_t* origin;
+    uint32_t* size;
+    uint32_t* ids_out;      // the extension's owners
+    uint32_t* flags;        // one word per position
     const uint32_t* n_pairs;
-    uint32_t* used;         // cleared with the tile ranges, as group_noted and groups[0]
-    uint32_t* n_owners;
-    uint32_t* open;         // one word per wave of the blend
+    uint32_t* n_emit;       // the pairs binned
+    uint32_t* few;          // behind it: whether few tiles are expected to be left open
+    uint32_t* n_owners;     // positions of the depth order that own pairs
+    uint32_t* any_open;     // cleared with the tile ranges, as rest, open_tiles, group_noted and groups[0]
+    uint32_t* positions;    // of the depth order that the extension looks at
+    uint32_t* rest;         // pairs of the extended lists
+    uint32_t* units;        // one word per wave of the blend
+    uint32_t* done;         // one word per tile
     uint32_t* group_noted;  // one word per group of 8 x 8 tiles
-    uint32_t* groups;       // the number of open groups, then the groups
-    uint32_t* counts;       // counts_room words
-    int64_t counts_room;
+    uint32_t* groups;       // the number of groups with an open tile, then the groups
+    uint32_t* open_tiles;   // one bit per tile, row_words words per row of tiles
+    int grid_x, row_words;
+    int64_t open_words;
 };
 
 // binning shared by both renderers (implemented with the splatter): depth sort,

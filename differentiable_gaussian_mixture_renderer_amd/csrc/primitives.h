@@ -43,16 +43,25 @@ struct ScanArray {
     uint32_t* total;
     bool inclusive;
 };
-hipError_t scan_u32_arrays(const ScanArray* arrays, int count, int64_t n, void* scratch, hipStream_t stream, bool cleared = false);
+// The length of a scan given on the device, min(n, ceil(*dev / div) * mul); the
+// whole n without dev.  At 0 nothing is written, the total neither.
+struct ScanLength {
+    const uint32_t* dev = nullptr;
+    uint32_t div = 1;
+    int64_t mul = 0;
+};
+hipError_t scan_u32_arrays(const ScanArray* arrays, int count, int64_t n, void* scratch, hipStream_t stream, bool cleared = false,
+    ScanLength length = ScanLength {});
 hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint32_t* total, int64_t n, bool inclusive, void* scratch,
-    hipStream_t stream, bool cleared = false);
+    hipStream_t stream, bool cleared = false, ScanLength length = ScanLength {});
 
 // --- stable LSD radix sort of (uint32 or uint16 key, uint32 value) pairs --
 // Sorts bits [begin_bit, end_bit) in 8-bit digits.  Pass p reads buffer
 // (p % 2 == 0 ? A : B) and writes the other one; the sorted result ends in A
 // when the number of passes is even, in B when it is odd.  n may be given on
 // the device (n_dev != nullptr, capacity n_max; min(*n_dev, n_max) items are
-// sorted) so no host sync is needed.
+// sorted) so no host sync is needed; the launches are sized for n_max, their
+// work follows the items.
 template <class KeyT>
 struct SortBuffersT {
     KeyT* keys_a;

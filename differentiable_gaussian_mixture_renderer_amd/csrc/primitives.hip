@@ -42,10 +42,22 @@ __device__ __forceinline__ uint32_t block_inclusive_scan(uint32_t v, uint32_t* s
     return v + prefix;
 }
 
+__device__ __forceinline__ int64_t scan_length(int64_t n_max, const ScanLength& l)
+{
+    if (!l.dev)
+        return n_max;
+    const uint32_t n = *l.dev;
+    return n == 0 ? 0 : min(n_max, (int64_t((n - 1) / l.div) + 1) * l.mul);
+}
+
 // scans the one tile of a scan of at most 2048 items
-__global__ __launch_bounds__(kScanThreads) void k_scan_tile(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_out, int inclusive)
+__global__ __launch_bounds__(kScanThreads) void k_scan_tile(const uint32_t* in, uint32_t* out, int64_t n_max, uint32_t* total_out, int inclusive,
+    ScanLength length)
 {
     __shared__ uint32_t s_waves[kScanThreads / 64];
+    const int64_t n = scan_length(n_max, length);
+    if (n == 0)
+        return;
     const int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
     uint32_t v[kScanItems];
     uint32_t acc = 0;
@@ -176,15 +188,19 @@ __device__ __forceinline__ void store_items(uint32_t* out, int64_t base, int64_t
 // in ticket order.  Array k's status words are r.status[k * tiles + tile]:
 // both aggregates go out before either look-back, so the two walks overlap.
 template <int ITEMS, int ARRAYS>
-__global__ __launch_bounds__(kScanThreads) void k_scan_onepass(ScanArray a0, ScanArray a1, int64_t n, ScanState r, int vec)
+__global__ __launch_bounds__(kScanThreads) void k_scan_onepass(ScanArray a0, ScanArray a1, int64_t n_max, ScanState r, int vec, ScanLength length)
 {
     constexpr int64_t kTile = int64_t(kScanThreads) * ITEMS;
     __shared__ uint32_t s_waves[kScanThreads / 64];
     __shared__ uint32_t s_tile, s_prefix[ARRAYS];
+    const int64_t n = scan_length(n_max, length);
+    if (int64_t(blockIdx.x) * kTile >= n)
+        return; // the tiles that hold items are as many as the blocks that stay, taken in ticket order
     if (threadIdx.x == 0)
         s_tile = atomicAdd(r.ticket, 1u);
     __syncthreads();
-    const int64_t v = s_tile, tiles = gridDim.x;
+    const int64_t v = s_tile, tiles = gridDim.x; // tiles: the stride of the status words
+    const int64_t last_tile = (n - 1) / kTile;
     const int64_t base = v * kTile + int64_t(threadIdx.x) * ITEMS;
     const ScanArray arr[2] = { a0, a1 };
     uint32_t x[ARRAYS][ITEMS], acc[ARRAYS], incl[ARRAYS], total[ARRAYS];
@@ -207,7 +223,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_onepass(ScanArray a0, Sca
                 if (v > 0)
                     look_publish(r.status + k * tiles + v, kLookPrefix, before + total[k]);
                 s_prefix[k] = before;
-                if (arr[k].total && v == tiles - 1)
+                if (arr[k].total && v == last_tile)
                     *arr[k].total = before + total[k];
             }
         }
@@ -240,7 +256,8 @@ ScanState scan_state(void* scratch, int64_t n, int arrays)
     return r;
 }
 
-hipError_t scan_u32_arrays(const ScanArray* arrays, int count, int64_t n, void* scratch, hipStream_t stream, bool cleared)
+hipError_t scan_u32_arrays(const ScanArray* arrays, int count, int64_t n, void* scratch, hipStream_t stream, bool cleared,
+    ScanLength length)
 {
     if (count < 1 || count > 2)
         return hipErrorInvalidValue;
@@ -255,7 +272,8 @@ hipError_t scan_u32_arrays(const ScanArray* arrays, int count, int64_t n, void* 
     }
     if (n <= kScanTile) {
         for (int k = 0; k < count; ++k)
-            k_scan_tile<<<1, kScanThreads, 0, stream>>>(arrays[k].in, arrays[k].out, n, arrays[k].total, arrays[k].inclusive ? 1 : 0);
+            k_scan_tile<<<1, kScanThreads, 0, stream>>>(arrays[k].in, arrays[k].out, n, arrays[k].total, arrays[k].inclusive ? 1 : 0,
+                length);
         return hipGetLastError();
     }
     const ScanState r = scan_state(scratch, n, count);
@@ -268,21 +286,21 @@ hipError_t scan_u32_arrays(const ScanArray* arrays, int count, int64_t n, void* 
     const unsigned tiles = unsigned(ceil_div(n, scan_tile_items(n)));
     const bool large = n >= kScanLargeFrom;
     if (large && count == 1)
-        k_scan_onepass<kScanItemsLarge, 1><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec);
+        k_scan_onepass<kScanItemsLarge, 1><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec, length);
     else if (large)
-        k_scan_onepass<kScanItemsLarge, 2><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec);
+        k_scan_onepass<kScanItemsLarge, 2><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec, length);
     else if (count == 1)
-        k_scan_onepass<kScanItems, 1><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec);
+        k_scan_onepass<kScanItems, 1><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec, length);
     else
-        k_scan_onepass<kScanItems, 2><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec);
+        k_scan_onepass<kScanItems, 2><<<tiles, kScanThreads, 0, stream>>>(a0, a1, n, r, vec, length);
     return hipGetLastError();
 }
 
 hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint32_t* total, int64_t n, bool inclusive, void* scratch, hipStream_t stream,
-    bool cleared)
+    bool cleared, ScanLength length)
 {
     const ScanArray a { in, out, total, inclusive };
-    return scan_u32_arrays(&a, 1, n, scratch, stream, cleared);
+    return scan_u32_arrays(&a, 1, n, scratch, stream, cleared, length);
 }
 
 // ------------------------------------------------------------------ radix sort
@@ -307,23 +325,30 @@ __device__ __forceinline__ int64_t sort_count(int64_t n_max, const uint32_t* n_d
     return n_dev ? min(int64_t(*n_dev), n_max) : n_max;
 }
 
+// blocks that hold items, of at most n_blocks
+template <int64_t TILE>
+__device__ __forceinline__ int sort_blocks(int64_t n) { return int((n + TILE - 1) / TILE); }
+
 // per-block histogram of the digit (key >> shift) & (2^bits - 1), stored
-// digit-major: hist[digit * n_blocks + block]; also clears the state of the
-// scan over hist that follows
+// digit-major: hist[digit * blocks that hold items + block]; also clears the
+// state of the scan over hist that follows
 template <int ITEMS, class KeyT>
 __global__ __launch_bounds__(kSortThreads) void k_radix_hist(const KeyT* __restrict__ keys, int64_t n_max, const uint32_t* n_dev,
-    int shift, int bits, int n_blocks, uint32_t* __restrict__ hist, ScanState scan, int vec)
+    int shift, int bits, uint32_t* __restrict__ hist, ScanState scan, int vec)
 {
     constexpr int kSortItems = ITEMS, kSortTile = kSortThreads * ITEMS;
     __shared__ uint32_t s_hist[4][kRadixMax];
     scan_clear(scan);
     const int64_t n = sort_count(n_max, n_dev);
     const int64_t base = int64_t(blockIdx.x) * kSortTile;
+    if (base >= n)
+        return;
+    const int n_blocks = sort_blocks<kSortTile>(n);
     const uint32_t mask = (1u << bits) - 1u;
     for (int i = threadIdx.x; i < 4 * kRadixMax; i += kSortThreads)
         (&s_hist[0][0])[i] = 0;
     __syncthreads();
-    if (base < n) {
+    {
         const unsigned wave = threadIdx.x / 64;
         // each thread counts ITEMS consecutive keys (the order of counting
         // does not matter), read with 16-byte loads when they are all in
@@ -380,7 +405,7 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_hist(const KeyT* __restr
 // work to turn the uniform condition into a lane mask and back); 0 reads bits.
 template <int ITEMS, class KeyT, int RADIX, int BITS>
 __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
-    KeyT* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int64_t n_max, const uint32_t* n_dev, int shift, int bits_arg, int n_blocks,
+    KeyT* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int64_t n_max, const uint32_t* n_dev, int shift, int bits_arg,
     const uint32_t* __restrict__ offsets, KeyOut ko)
 {
     const int bits = BITS > 0 ? BITS : bits_arg;
@@ -398,6 +423,7 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const KeyT* __re
     const int64_t base = int64_t(blk) * kSortTile;
     if (base >= n)
         return;
+    const int n_blocks = sort_blocks<kSortTile>(n);
     const int count = int(min<int64_t>(kSortTile, n - base));
     const unsigned lane = lane_id();
     const unsigned wave = threadIdx.x / 64;
@@ -650,22 +676,23 @@ static void radix_pass(int blocks, const KeyT* kin, const uint32_t* vin, KeyT* k
         return;
     }
     const int vec = reinterpret_cast<uintptr_t>(kin) % 16 == 0 ? 1 : 0;
-    k_radix_hist<ITEMS, KeyT><<<blocks, kSortThreads, 0, stream>>>(kin, n_max, n_dev, shift, bits, blocks, hist, scan, vec);
-    *err = scan_u32(hist, hist, nullptr, n_hist, false, scan_scratch, stream, true);
+    k_radix_hist<ITEMS, KeyT><<<blocks, kSortThreads, 0, stream>>>(kin, n_max, n_dev, shift, bits, hist, scan, vec);
+    *err = scan_u32(hist, hist, nullptr, n_hist, false, scan_scratch, stream, true,
+        ScanLength { n_dev, uint32_t(kSortThreads) * ITEMS, int64_t(1) << bits });
     if (*err != hipSuccess)
         return;
     // the digit widths of the binnings (8-bit depth passes, 7 + 6 for tile
     // ids) are compiled in; other widths read theirs at run time
     if (bits == 8)
-        k_radix_scatter<ITEMS, KeyT, 256, 8><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, blocks, hist, ko);
+        k_radix_scatter<ITEMS, KeyT, 256, 8><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, hist, ko);
     else if (bits == 7)
-        k_radix_scatter<ITEMS, KeyT, 128, 7><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, blocks, hist, ko);
+        k_radix_scatter<ITEMS, KeyT, 128, 7><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, hist, ko);
     else if (bits == 6)
-        k_radix_scatter<ITEMS, KeyT, 128, 6><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, blocks, hist, ko);
+        k_radix_scatter<ITEMS, KeyT, 128, 6><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, hist, ko);
     else if (bits <= 7)
-        k_radix_scatter<ITEMS, KeyT, 128, 0><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, blocks, hist, ko);
+        k_radix_scatter<ITEMS, KeyT, 128, 0><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, hist, ko);
     else
-        k_radix_scatter<ITEMS, KeyT, 256, 0><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, blocks, hist, ko);
+        k_radix_scatter<ITEMS, KeyT, 256, 0><<<blocks, kSortThreads, 0, stream>>>(kin, vin, kout, vout, n_max, n_dev, shift, bits, hist, ko);
     *err = hipGetLastError();
 }
 

@@ -77,11 +77,9 @@ constexpr int kEmitWindow = 2048; // owners a block stages in LDS (more take the
 // [offsets[k], offsets[k + 1]) and writes the entries whose pair falls in its
 // range, so each entry is written exactly once and no block searches.
 __device__ __forceinline__ void emit_bounds_of(uint32_t k, uint64_t lo, uint64_t next, uint64_t total, uint32_t capacity, int block_shift,
-    uint32_t* __restrict__ bounds, uint32_t* __restrict__ n_owners)
+    uint32_t* __restrict__ bounds)
 {
     const uint64_t R = min(total, uint64_t(capacity)); // pairs past the capacity are not emitted
-    if (n_owners && lo < total && next == total)
-        *n_owners = k + 1; // the last position that owns pairs
     const uint64_t hi = min(next, R);
     if (lo >= hi)
         return;
@@ -92,13 +90,13 @@ __device__ __forceinline__ void emit_bounds_of(uint32_t k, uint64_t lo, uint64_t
         bounds[(R + up) >> block_shift] = k;
 }
 __global__ void k_emit_bounds(int64_t n, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ n_pairs, uint32_t capacity,
-    int block_shift, uint32_t* __restrict__ bounds, uint32_t* __restrict__ n_owners)
+    const uint32_t* __restrict__ n_emit, int block_shift, uint32_t* __restrict__ bounds)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k >= n)
         return;
     const uint64_t total = *n_pairs;
-    emit_bounds_of(uint32_t(k), offsets[k], k + 1 < n ? uint64_t(offsets[k + 1]) : total, total, capacity, block_shift, bounds, n_owners);
+    emit_bounds_of(uint32_t(k), offsets[k], k + 1 < n ? uint64_t(offsets[k + 1]) : total, total, min(*n_emit, capacity), block_shift, bounds);
 }
 
 // tile rectangle of Gaussian id: first tile and (grid_x << 16 | width); 0 shape when it has no tiles
@@ -126,11 +124,17 @@ __device__ __forceinline__ void owner_rect(uint32_t id, const int32_t* __restric
     *shape = (uint32_t(gx) << 16) | uint32_t(c - a);
 }
 
+// What k_prefix_decide sums up, per cell of the image: sixteenths of a pixel, pairs
+struct DecideSums {
+    unsigned long long alpha[64], rest[64];
+    uint32_t blocks;
+};
 // Tile rectangles by position of the depth order for the lists' extension (null: not
 // wanted): (row << 16 | column) of the first tile, (rows << 16 | columns)
 struct PrefixRects {
     uint32_t* origin;
     uint32_t* size;
+    DecideSums* sums; // to be cleared
 };
 
 // Per position j of the depth order: the pair count of Gaussian ids[j] (for
@@ -146,6 +150,12 @@ __global__ __launch_bounds__(256) void k_gather_owners(int64_t n, const uint32_t
     ScanState scan, PrefixRects prefix)
 {
     scan_clear(scan); // for the scan of counts that follows
+    if (prefix.sums && blockIdx.x == 0) {
+        if (threadIdx.x < 64)
+            prefix.sums->alpha[threadIdx.x] = prefix.sums->rest[threadIdx.x] = 0;
+        if (threadIdx.x == 0)
+            prefix.sums->blocks = 0;
+    }
     const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (j >= n)
         return;
@@ -210,8 +220,6 @@ struct BinOneArgs {
     uint32_t* point_offsets; // by a second workgroup
     uint32_t* n_pairs;
     uint32_t* bounds;
-    uint32_t* n_owners;      // null: not wanted
-    PrefixRects prefix;
 };
 
 // exclusive scan of s[0..n) in place, by the whole workgroup; returns the sum.
@@ -416,11 +424,6 @@ __global__ __launch_bounds__(kBinOneThreads) void k_bin_one(BinOneArgs a)
             a.ids[j] = id[r];
             a.owner_rects[j] = make_uint2(rect[r].x, cols * rows == 0 ? 0u : (a.grid_x << 16) | cols);
             s_key[j] = cols * rows;
-            if (a.prefix.origin) {
-                const uint32_t y = rect[r].x / a.grid_x;
-                a.prefix.origin[j] = (y << 16) | (rect[r].x - y * a.grid_x);
-                a.prefix.size[j] = rect[r].y;
-            }
         }
     }
     __syncthreads();
@@ -430,7 +433,7 @@ __global__ __launch_bounds__(kBinOneThreads) void k_bin_one(BinOneArgs a)
     for (int j = t; j < n; j += kBinOneThreads) {
         const uint32_t first = s_key[j], next = j + 1 < n ? s_key[j + 1] : total;
         a.offsets[j] = first;
-        emit_bounds_of(uint32_t(j), first, next, total, a.capacity, a.block_shift, a.bounds, a.n_owners);
+        emit_bounds_of(uint32_t(j), first, next, total, a.capacity, a.block_shift, a.bounds);
     }
 }
 
@@ -717,6 +720,21 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_pairs(int64_t n, const ui
     }
 }
 
+// What prefix binning (below) notes of the tiles whose lists it leaves open: a
+// bit per tile, words of 32 along the rows; whether there is one (0 or 1); the
+// groups of 8 x 8 tiles that hold one; and for the extension the positions of
+// the depth order that it looks at (0 when there is none) and the pairs it makes
+struct OpenTiles {
+    uint32_t* tiles; // null: whole lists
+    int row_words;
+    int64_t words;
+    uint32_t* any;
+    uint32_t* positions;
+    uint32_t* rest;
+    uint32_t* groups;      // their number, then the groups
+    uint32_t* group_noted; // [groups]
+};
+
 // [first, last) of every tile by binary search over the sorted pairs: one
 // thread per tile, every tile written (an empty tile gets (0, 0)).
 // The sorted order is (view-local tile, view, depth); a pair's view is
@@ -728,16 +746,18 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_pairs(int64_t n, const ui
 template <class KeyT>
 __global__ __launch_bounds__(256) void k_tile_ranges(const KeyT* __restrict__ keys, const uint32_t* __restrict__ vals,
     const uint32_t* __restrict__ n_pairs, uint32_t capacity, const int4* __restrict__ views, int n_views, int64_t n_per_view, int64_t n_tiles,
-    uint32_t* __restrict__ ranges, uint32_t* __restrict__ used, uint32_t* __restrict__ groups, uint32_t* __restrict__ group_noted)
+    uint32_t* __restrict__ ranges, OpenTiles open)
 {
     const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (g >= n_tiles)
         return;
-    if (used) {
-        // for the blend and the extension of the lists (no more groups than tiles)
-        group_noted[g] = 0;
+    if (open.tiles) {
+        // for the blend and the extension of the lists (no more words or groups than tiles)
+        open.group_noted[g] = 0;
+        if (g < open.words)
+            open.tiles[g] = 0;
         if (g == 0)
-            *used = groups[0] = 0;
+            *open.any = *open.rest = open.groups[0] = 0;
     }
     const uint32_t R = min(*n_pairs, capacity);
     uint32_t t0 = uint32_t(g), t1 = uint32_t(g) + 1;
@@ -781,14 +801,17 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const KeyT* __restrict__ ke
     ranges[2 * g + 1] = lo0 < lo1 ? lo1 : 0u;
 }
 
-// prefix binning (below): open notes the tiles whose list ended with an open
-// pixel; the second pass (again) blends only those, when there are any
+// prefix binning (below): the first pass notes which waves' lists ended with an
+// open pixel and keeps those waves' pixels as they stand; the second (again)
+// goes on with them where their lists were left
 struct PrefixPass {
-    uint32_t* open;        // [tiles * waves per tile], null: whole lists
-    uint32_t* groups;      // [0]: number of groups of 8 x 8 tiles with an open one, then their numbers
-    uint32_t* group_noted; // [groups], 0 before the blend
+    uint32_t* units;      // [tiles * waves per tile]: open; null: whole lists
+    OpenTiles open;
+    const uint32_t* done; // per open tile the entries that the first pass walked
     const uint32_t* n_pairs;
+    const uint32_t* n_emit;
     uint32_t pairs;
+    int split;            // waves per tile of the first pass
     bool again;
 };
 
@@ -800,29 +823,34 @@ __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_forward(const uint32
     int n_tiles, float bg0, float bg1, float bg2, float* __restrict__ framebuffer, float* __restrict__ final_T, PrefixPass prefix)
 {
     __shared__ BlendSmem<B> sm_all[kBlendWaves];
-    if (prefix.again && *prefix.n_pairs <= prefix.pairs)
-        return; // the lists were whole the first time
+    if (prefix.again && *prefix.open.any == 0)
+        return;
     const int wave = int(uniform(threadIdx.x / 64));
     const int unit = xcd_tile(blockIdx.x, gridDim.x) * kBlendWaves + wave;
     const int tile = unit / SPLIT, part = unit % SPLIT;
     if (tile >= n_tiles)
         return;
-    if (prefix.again) {
-        uint32_t open = 0;
-        for (int k = 0; k < SPLIT; ++k)
-            open |= prefix.open[tile * SPLIT + k];
-        if (uniform(open) == 0)
-            return; // its list was not extended
-    }
+    if (prefix.again && uniform(prefix.units[tile * prefix.split + part % prefix.split]) == 0)
+        return;
     BlendSmem<B>& sm = sm_all[wave];
-    const uint32_t first = uniform(ranges[2 * tile]), last = uniform(ranges[2 * tile + 1]);
+    uint32_t first = uniform(ranges[2 * tile]);
+    const uint32_t last = uniform(ranges[2 * tile + 1]);
+    if (prefix.again)
+        first = min(first + uniform(prefix.done[tile]), last);
+    // whether the lists are prefixes
+    const BlendResume resume { prefix.again, prefix.units && !prefix.again && *prefix.n_emit == prefix.pairs && *prefix.n_pairs > prefix.pairs };
     const bool open = blend_tile_forward<TW, TH / SPLIT, B>(sm, first, last, (tile % grid_x) * TW, (tile / grid_x) * TH + part * (TH / SPLIT),
-        width, height, bg0, bg1, bg2, point_list, xy, conic_opacity, rgb, framebuffer, final_T);
-    if (prefix.open && !prefix.again && lane_id() == 0) {
-        prefix.open[unit] = open ? 1u : 0u;
-        const int group = (tile / grid_x) / 8 * ((grid_x + 7) / 8) + (tile % grid_x) / 8;
-        if (open && atomicExch(&prefix.group_noted[group], 1u) == 0)
-            prefix.groups[1 + atomicAdd(&prefix.groups[0], 1u)] = uint32_t(group);
+        width, height, bg0, bg1, bg2, point_list, xy, conic_opacity, rgb, framebuffer, final_T, resume);
+    if (resume.keep && lane_id() == 0) {
+        prefix.units[unit] = open ? 1u : 0u;
+        if (open) {
+            const int tx = tile % grid_x, ty = tile / grid_x;
+            const int group = ty / 8 * ((grid_x + 7) / 8) + tx / 8;
+            atomicOr(&prefix.open.tiles[ty * prefix.open.row_words + tx / 32], 1u << (tx % 32));
+            if (atomicExch(&prefix.open.group_noted[group], 1u) == 0)
+                prefix.open.groups[1 + atomicAdd(&prefix.open.groups[0], 1u)] = uint32_t(group);
+            *prefix.open.any = 1u;
+        }
     }
 }
 
@@ -833,22 +861,30 @@ __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_forward(const uint32
 // bandwidth bound and were a fifth of the forward.  With prefix binning only
 // the first pairs of the depth order (kPrefixPerTile per tile of the image) are
 // emitted and sorted, so every tile's list is a prefix of its whole list; the
-// blend notes the tiles whose list ends with a pixel still open, and
-// the extension builds those tiles' whole lists behind the sorted pairs from
-// the depth-ordered rectangles, for a second blend of these tiles.  Nothing
-// waits for the host: both launches leave at once when there is nothing to do.
-// When the lists are whole the four launches of the extension and the second
-// blend find nothing and cost 16 us, as much as the emission and sort of 1.3M
-// pairs: views with fewer pairs to save, by the 16 pairs a Gaussian makes in an
-// ordinary deep view, and those whose pairs are not three times the prefix keep
-// whole lists.
+// blend notes the tiles whose list ends with a pixel still open, and the whole
+// lists of these tiles are built behind the prefixes for a second blend, which
+// goes on where the first one stopped.  The launches of the extension leave at
+// once when no tile is open.
+// Where tiles stay open prefixes cost more than they save, so a view must have
+// kPrefixMin times their pairs, make 1.3M fewer (by the 16 pairs a Gaussian makes
+// in an ordinary deep view) and look covered (k_prefix_decide).  Forward in us,
+// prefixes / whole lists, at 1920x1080 (scales e^-3, cube of side 10 unless noted):
+//   1M, opacities around 1/2      355 / 444   no tile open
+//   3M, the same                  695 / 1026  3 open
+//   1M, around 0.27               440 / 504   23 open
+//   1M, around 0.18               562 / 538   1 004 open (k_prefix_decide: whole)
+//   1M, around 0.007              1004 / 890  all open (whole; 900 with k_prefix_decide)
+//   1M in a cube of side 3        611 / 696   1 838 open at its edges
+//   3M in it, scales e^-4         984 / 976   618 open
 constexpr int64_t kPrefixPerTile = 256;
-constexpr int64_t kPrefixMin = 3;
 constexpr int64_t kPrefixPairsPerGaussian = 16;
 constexpr int64_t kPrefixMinSaved = 1300000;
+constexpr int64_t kPrefixMin = 6;
+static_assert((kPrefixMinSaved + kPrefixPerTile) / kPrefixPairsPerGaussian > kBinOneMax, "small views are binned whole");
 
 // the first pairs that a view of n Gaussians and n_tiles tiles bins with prefix
-// binning, 0 when its whole lists are binned
+// binning when it has kPrefixMin times as many, 0 when its whole lists are
+// binned whatever it has
 static int64_t prefix_pairs(int64_t n, int64_t n_tiles, int64_t pair_capacity)
 {
     const int64_t pairs = kPrefixPerTile * n_tiles, expected = kPrefixPairsPerGaussian * n;
@@ -858,26 +894,275 @@ static int64_t prefix_pairs(int64_t n, int64_t n_tiles, int64_t pair_capacity)
         : 0;
 }
 
-// The extension works on groups of 8 x 8 tiles, a lane per tile, over segments
+// Whether a view's prefixes are worth while, from 4 096 Gaussians of the prefix
+// and as many behind it, at equal steps of the depth order (10 us).  Per cell of
+// an 8 x 8 grid of the image the first give the depth of alpha that the prefix
+// lays over its pixels (a pixel is saturated at 9.2), the second the share of the
+// other pairs: whole lists where more than a sixteenth of these lie in cells
+// below kPrefixAlpha, which separates the scenes of the table above (no pairs at
+// opacities around 0.27, a sixth of them around 0.18).  Few tiles are expected to
+// be open where at most a 64th lies in cells below kFewAlpha.
+constexpr int kDecideThreads = 512, kDecideBlocks = 8; // one CU alone took twice as long over its scattered loads
+constexpr int kDecideSamples = kDecideThreads * kDecideBlocks;
+constexpr int kCells = 8;
+constexpr float kPrefixAlpha = 11.f, kFewAlpha = 12.f;
+struct DecideArgs {
+    int64_t n;
+    const uint32_t* offsets;
+    const uint32_t* n_pairs;
+    uint32_t capacity, prefix;
+    bool always; // the prefix whenever there are kPrefixMin times its pairs
+    const uint32_t* ids;
+    const uint32_t* origin;
+    const uint32_t* size;
+    const float4* conic_opacity;
+    int grid_x, grid_y, tile_pixels;
+    DecideSums* sums; // cleared by the gather
+    uint32_t* n_emit;
+    uint32_t* few; // whether few tiles are expected to be left open
+    uint32_t* n_owners;
+};
+
+// first tile column (row) of a cell column (row): tile t lies in cell t kCells / grid
+__device__ __forceinline__ int cell_edge(int cell, int grid) { return (cell * grid + kCells - 1) / kCells; }
+
+// first position whose offset reaches v (offsets ascend), by a wave
+__device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict__ offsets, uint32_t n, uint32_t v)
+{
+    uint32_t lo = 0, hi = n; // the answer lies in [lo, hi]
+    while (lo < hi) {
+        const uint32_t step = (hi - lo + 63) / 64;
+        const uint32_t at = lo + lane_id() * step;
+        const bool below = at < hi && offsets[at] < v;
+        const uint32_t count = uint32_t(__builtin_popcountll(__builtin_amdgcn_ballot_w64(below))); // lanes in a row from 0
+        if (count == 0)
+            hi = lo;
+        else {
+            hi = min(hi, lo + count * step);
+            lo = lo + (count - 1) * step + 1;
+        }
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(kDecideThreads) void k_prefix_decide(DecideArgs a)
+{
+    __shared__ unsigned long long s_alpha[kCells * kCells], s_rest[kCells * kCells]; // sixteenths of a pixel; pairs
+    __shared__ uint32_t s_at[2];
+    const int t = int(threadIdx.x);
+    const uint32_t total = *a.n_pairs, limit = min(total, a.capacity);
+    const bool deep = total <= a.capacity && total >= uint64_t(kPrefixMin) * a.prefix;
+    if (t < 128 && deep) {
+        const uint32_t at = wave_lower_bound(a.offsets, uint32_t(a.n), t < 64 ? a.prefix : total);
+        if (t % 64 == 0)
+            s_at[t / 64] = at;
+    }
+    if (t < kCells * kCells)
+        s_alpha[t] = s_rest[t] = 0;
+    __syncthreads();
+    const uint32_t owners = s_at[1], front = min(s_at[0], owners);
+    if (!deep || a.always || front == 0 || front == owners) {
+        if (t == 0 && blockIdx.x == 0) {
+            *a.n_emit = deep && front < owners ? a.prefix : limit;
+            *a.few = 0;
+            *a.n_owners = deep ? owners : 0;
+        }
+        return;
+    }
+    const uint64_t i = uint64_t(blockIdx.x) * kDecideThreads + uint64_t(t);
+    const uint32_t pos[2] = { uint32_t(i * front / kDecideSamples), front + uint32_t(i * (owners - front) / kDecideSamples) };
+    const float4 c = a.conic_opacity[a.ids[pos[0]]];
+    // the integral of alpha over the screen, at most its tiles' pixels, and the
+    // pairs: each cell gets its share of the rectangle
+    const float alpha = c.w * 6.2831853f * __builtin_amdgcn_rsqf(c.x * c.z - c.y * c.y);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const uint32_t o = a.origin[pos[q]], sz = a.size[pos[q]], cols = sz & 0xffffu, rows = sz >> 16;
+        const int x0 = int(o & 0xffffu), y0 = int(o >> 16), x1 = x0 + int(cols), y1 = y0 + int(rows);
+        const float each = q == 0 ? fminf(alpha * __builtin_amdgcn_rcpf(float(cols) * float(rows)), float(a.tile_pixels)) : 0.f;
+        for (int cy = y0 * kCells / a.grid_y; cy <= (y1 - 1) * kCells / a.grid_y; ++cy)
+            for (int cx = x0 * kCells / a.grid_x; cx <= (x1 - 1) * kCells / a.grid_x; ++cx) {
+                const int w = min(x1, cell_edge(cx + 1, a.grid_x)) - max(x0, cell_edge(cx, a.grid_x));
+                const int h = min(y1, cell_edge(cy + 1, a.grid_y)) - max(y0, cell_edge(cy, a.grid_y));
+                const float tiles = float(w) * float(h);
+                if (q == 1)
+                    atomicAdd(&s_rest[cy * kCells + cx], static_cast<unsigned long long>(tiles));
+                else if (each > 0.f) // not for NaN
+                    atomicAdd(&s_alpha[cy * kCells + cx], static_cast<unsigned long long>(each * tiles * 16.f));
+            }
+    }
+    __syncthreads();
+    if (t < 64) {
+        static_assert(kCells * kCells == 64, "a lane per cell");
+        atomicAdd(&a.sums->alpha[t], s_alpha[t]);
+        atomicAdd(&a.sums->rest[t], s_rest[t]);
+        __threadfence();
+    }
+    __syncthreads();
+    if (t == 0)
+        s_at[0] = atomicAdd(&a.sums->blocks, 1u);
+    __syncthreads();
+    if (s_at[0] != kDecideBlocks - 1)
+        return;
+    // the last workgroup decides
+    if (t < 64) {
+        const int x = t % kCells, y = t / kCells;
+        const int tiles_x = cell_edge(x + 1, a.grid_x) - cell_edge(x, a.grid_x), tiles_y = cell_edge(y + 1, a.grid_y) - cell_edge(y, a.grid_y);
+        const float pixels = float(max(tiles_x * tiles_y, 1)) * float(a.tile_pixels);
+        const float depth = float(atomicAdd(&a.sums->alpha[t], 0ull)) * (1.f / 16.f) * (float(front) / float(kDecideSamples)) / pixels;
+        float rest = float(atomicAdd(&a.sums->rest[t], 0ull)), open = depth < kPrefixAlpha ? rest : 0.f, thin = depth < kFewAlpha ? rest : 0.f;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            rest += __shfl_xor(rest, d);
+            open += __shfl_xor(open, d);
+            thin += __shfl_xor(thin, d);
+        }
+        if (t == 0) {
+            *a.n_emit = open * 16.f <= rest ? a.prefix : limit;
+            *a.few = thin * 64.f <= rest ? 1u : 0u;
+            *a.n_owners = owners;
+        }
+    }
+}
+
+// The extension elsewhere is the binning's own emission and sort over the
+// Gaussians that hold an open tile.  These, their rectangles
+// shrunk to the open tiles (in place: first tile, columns), so that few open
+// tiles make few pairs.  Four positions per thread: the grid costs when there is
+// nothing to do.  LDS: the open tiles fit (8 192 words: 262 144 tiles and more).
+constexpr int kOpenPer = 4;
+constexpr int kOpenLdsWords = 8192;
+template <bool LDS>
+__global__ __launch_bounds__(256) void k_open_owners(OpenTiles open, int grid_x, const uint32_t* __restrict__ n_owners,
+    uint32_t* __restrict__ origin, uint32_t* __restrict__ size, uint32_t* __restrict__ counts, uint32_t* __restrict__ flags, ScanState scan)
+{
+    extern __shared__ uint32_t s_tiles[];
+    const int64_t owners = *open.any == 0 ? 0 : int64_t(*n_owners);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *open.positions = uint32_t(owners);
+    if (owners == 0)
+        return;
+    scan_clear(scan); // for the scan of counts and flags that follows
+    if (int64_t(blockIdx.x) * kOpenPer * 256 >= owners)
+        return;
+    if (LDS) {
+        for (int i = int(threadIdx.x); i < int(open.words); i += 256)
+            s_tiles[i] = open.tiles[i];
+        __syncthreads();
+    }
+    for (int q = 0; q < kOpenPer; ++q) {
+        const int64_t j = (int64_t(blockIdx.x) * kOpenPer + q) * 256 + threadIdx.x;
+        if (j >= owners)
+            return;
+        uint32_t xa = 0xffffffffu, xb = 0, ya = 0xffffffffu, yb = 0; // the open tiles' columns and rows, ends included
+        {
+            // no Gaussian that owns pairs has an empty rectangle
+            const uint32_t o = origin[j], sz = size[j];
+            const uint32_t x0 = o & 0xffffu, y0 = o >> 16, x1 = x0 + (sz & 0xffffu) - 1, y1 = y0 + (sz >> 16) - 1;
+            for (uint32_t w = x0 / 32; w <= x1 / 32; ++w) {
+                const uint32_t lo = w == x0 / 32 ? x0 % 32 : 0u, hi = w == x1 / 32 ? x1 % 32 : 31u;
+                const uint32_t mask = (0xffffffffu >> (31 - hi)) & (0xffffffffu << lo);
+                uint32_t cols = 0;
+                for (uint32_t y = y0; y <= y1; ++y) {
+                    const uint32_t at = y * uint32_t(open.row_words) + w;
+                    const uint32_t m = (LDS ? s_tiles[at] : open.tiles[at]) & mask;
+                    cols |= m;
+                    ya = m ? min(ya, y) : ya;
+                    yb = m ? max(yb, y) : yb;
+                }
+                if (cols) {
+                    xa = min(xa, 32 * w + uint32_t(__builtin_ctz(cols)));
+                    xb = max(xb, 32 * w + 31u - uint32_t(__builtin_clz(cols)));
+                }
+            }
+        }
+        const uint32_t cols = xa <= xb ? xb - xa + 1 : 0u, rows = xa <= xb ? yb - ya + 1 : 0u;
+        counts[j] = cols * rows;
+        flags[j] = cols ? 1u : 0u;
+        if (cols) {
+            origin[j] = ya * uint32_t(grid_x) + xa;
+            size[j] = cols;
+        }
+    }
+}
+
+// The owners one behind the other (the emission searches the owners of its
+// pairs, and few open tiles leave few of many), and the emission blocks' first ones
+__global__ __launch_bounds__(256) void k_open_bounds(OpenTiles open, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ place,
+    const uint32_t* __restrict__ start, const uint32_t* __restrict__ cols, const uint32_t* __restrict__ ids, int grid_x, uint32_t capacity,
+    int block_shift, uint32_t* __restrict__ offsets_out, uint2* __restrict__ rects_out, uint32_t* __restrict__ ids_out, uint32_t* __restrict__ bounds)
+{
+    if (*open.any == 0)
+        return;
+    const uint64_t total = *open.rest;
+    const int64_t n = *open.positions;
+    for (int q = 0; q < kOpenPer; ++q) {
+        const int64_t j = (int64_t(blockIdx.x) * kOpenPer + q) * 256 + threadIdx.x;
+        if (j >= n)
+            return;
+        const uint32_t lo = offsets[j];
+        const uint64_t next = j + 1 < n ? uint64_t(offsets[j + 1]) : total;
+        if (lo >= next)
+            continue;
+        const uint32_t c = place[j];
+        offsets_out[c] = lo;
+        rects_out[c] = make_uint2(start[j], (uint32_t(grid_x) << 16) | cols[j]);
+        ids_out[c] = ids[j];
+        emit_bounds_of(c, lo, next, total, capacity, block_shift, bounds);
+    }
+}
+
+// ranges of the open tiles in their whole lists (from entry `base` on), and the
+// entries of their prefixes
+template <class KeyT>
+__global__ __launch_bounds__(256) void k_open_ranges(const KeyT* __restrict__ keys, uint32_t capacity, uint32_t base, OpenTiles open, int grid_x,
+    int64_t n_tiles, uint32_t* __restrict__ ranges, uint32_t* __restrict__ done)
+{
+    const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (*open.any == 0 || g >= n_tiles)
+        return;
+    const int tx = int(g % grid_x), ty = int(g / grid_x);
+    if (((open.tiles[ty * open.row_words + tx / 32] >> (tx % 32)) & 1u) == 0)
+        return;
+    const uint32_t R = min(*open.rest, capacity);
+    uint32_t end[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        uint32_t lo = 0, hi = R;
+        while (lo < hi) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            if (int64_t(keys[mid]) >= g + k)
+                hi = mid;
+            else
+                lo = mid + 1;
+        }
+        end[k] = lo;
+    }
+    done[g] = ranges[2 * g + 1] - ranges[2 * g];
+    ranges[2 * g] = end[0] < end[1] ? base + end[0] : 0u;
+    ranges[2 * g + 1] = end[0] < end[1] ? base + end[1] : 0u;
+}
+
+// The extension where few tiles are expected to be open (three launches: 11 us
+// without one, 62 us with 3 of 8 160 at 3M, where k_open_owners and the emission
+// and sort take 32 and 116; all tiles open 600 us at 1M, those 200) works on groups of 8 x 8 tiles, a lane per tile, over segments
 // of the depth order, a wave per (open group, segment): the wave reads 64
 // Gaussians' rectangles at a time and hands each that covers the group to all
 // lanes as a 64-bit tile mask, so a lane counts (k_extend_count) or appends
 // (k_extend_write) its tile's Gaussians in depth order.  In between
 // k_extend_place turns the counts into places.  With few open tiles the
-// segments spread them over the chip.
+// segments spread them over the chip; each open group reads every rectangle.
 struct ExtendArgs {
-    const uint32_t* n_pairs;
     uint32_t prefix;
     uint64_t capacity;     // entries of point_list
     const uint32_t* n_owners;
     const uint32_t* origin;
     const uint32_t* size;
     const uint32_t* ids;
-    const uint32_t* open;  // per wave of the blend
-    const uint32_t* groups; // [0]: number of open groups, then their numbers
+    OpenTiles open;
     uint32_t* counts;      // [groups * segments * 64]
-    uint32_t* used;
-    int split, grid_x, grid_y, segments;
+    uint32_t* done;        // [tiles]
+    int grid_x, grid_y, segments;
 };
 
 constexpr int kExtendBlocks = 1024;
@@ -891,11 +1176,7 @@ __device__ __forceinline__ bool extend_lane_open(const ExtendArgs& a, int g, int
     const int lane = int(lane_id());
     const int tx = *gx0 + lane % 8, ty = *gy0 + lane / 8;
     *tile = ty * a.grid_x + tx;
-    uint32_t any = 0;
-    if (tx < a.grid_x && ty < a.grid_y)
-        for (int k = 0; k < a.split; ++k)
-            any |= a.open[int64_t(*tile) * a.split + k];
-    return any != 0;
+    return tx < a.grid_x && ty < a.grid_y && ((a.open.tiles[ty * a.open.row_words + tx / 32] >> (tx % 32)) & 1u) != 0;
 }
 
 // calls f(id position, this lane's tile is covered) for the positions of segment
@@ -942,13 +1223,13 @@ __device__ __forceinline__ void extend_walk(const ExtendArgs& a, int gx0, int gy
 
 __global__ __launch_bounds__(256) void k_extend_count(ExtendArgs a)
 {
-    if (*a.n_pairs <= a.prefix)
+    if (*a.open.any == 0)
         return;
-    const uint32_t items = a.groups[0] * uint32_t(a.segments);
+    const uint32_t items = a.open.groups[0] * uint32_t(a.segments);
     for (uint32_t i = uniform(blockIdx.x * 4 + threadIdx.x / 64); i < items; i += kExtendBlocks * 4) {
         const int at = int(i / uint32_t(a.segments)), seg = int(i % uint32_t(a.segments));
         int gx0, gy0, tile;
-        const bool open = extend_lane_open(a, int(a.groups[1 + at]), &gx0, &gy0, &tile);
+        const bool open = extend_lane_open(a, int(a.open.groups[1 + at]), &gx0, &gy0, &tile);
         uint32_t count = 0;
         extend_walk(a, gx0, gy0, seg, __builtin_amdgcn_ballot_w64(open), [&](uint32_t, uint32_t covered) { count += covered; });
         a.counts[int64_t(i) * 64 + lane_id()] = count;
@@ -962,13 +1243,13 @@ __global__ __launch_bounds__(64 * kPlaceWaves) void k_extend_place(ExtendArgs a,
 {
     __shared__ uint32_t s_run[kPlaceWaves][64];
     __shared__ uint32_t s_fits;
-    if (*a.n_pairs <= a.prefix)
+    if (*a.open.any == 0)
         return;
     const unsigned lane = lane_id();
     const int wave = int(uniform(threadIdx.x / 64));
     const int per = (a.segments + kPlaceWaves - 1) / kPlaceWaves;
     const int s0 = min(a.segments, wave * per), s1 = min(a.segments, s0 + per);
-    for (uint32_t at = blockIdx.x; at < a.groups[0]; at += gridDim.x) {
+    for (uint32_t at = blockIdx.x; at < a.open.groups[0]; at += gridDim.x) {
         uint32_t* rows = a.counts + int64_t(at) * a.segments * 64 + lane;
         uint32_t sum = 0;
 #pragma unroll 8
@@ -978,7 +1259,7 @@ __global__ __launch_bounds__(64 * kPlaceWaves) void k_extend_place(ExtendArgs a,
         __syncthreads();
         if (wave == 0) {
             int gx0, gy0, tile;
-            const bool open = extend_lane_open(a, int(a.groups[1 + at]), &gx0, &gy0, &tile);
+            const bool open = extend_lane_open(a, int(a.open.groups[1 + at]), &gx0, &gy0, &tile);
             uint32_t total = 0;
             for (int w = 0; w < kPlaceWaves; ++w)
                 total += s_run[w][lane];
@@ -990,11 +1271,12 @@ __global__ __launch_bounds__(64 * kPlaceWaves) void k_extend_place(ExtendArgs a,
             const uint32_t all = __shfl(before, 63);
             uint32_t base = 0;
             if (lane == 0)
-                base = atomicAdd(a.used, all);
+                base = atomicAdd(a.open.rest, all);
             base = a.prefix + __shfl(base, 0);
             const bool fits = uint64_t(base) + all <= a.capacity; // always, unless the pairs exceed the caller's capacity
             uint32_t run = base + (before - total);
             if (open) {
+                a.done[tile] = ranges[2 * tile + 1] - ranges[2 * tile];
                 ranges[2 * tile] = fits && total ? run : 0u;
                 ranges[2 * tile + 1] = fits && total ? run + total : 0u;
             }
@@ -1027,13 +1309,13 @@ __global__ __launch_bounds__(64 * kPlaceWaves) void k_extend_place(ExtendArgs a,
 
 __global__ __launch_bounds__(256) void k_extend_write(ExtendArgs a, uint32_t* __restrict__ point_list)
 {
-    if (*a.n_pairs <= a.prefix)
+    if (*a.open.any == 0)
         return;
-    const uint32_t items = a.groups[0] * uint32_t(a.segments);
+    const uint32_t items = a.open.groups[0] * uint32_t(a.segments);
     for (uint32_t i = uniform(blockIdx.x * 4 + threadIdx.x / 64); i < items; i += kExtendBlocks * 4) {
         const int at = int(i / uint32_t(a.segments)), seg = int(i % uint32_t(a.segments));
         int gx0, gy0, tile;
-        const bool open = extend_lane_open(a, int(a.groups[1 + at]), &gx0, &gy0, &tile);
+        const bool open = extend_lane_open(a, int(a.open.groups[1 + at]), &gx0, &gy0, &tile);
         uint32_t place = a.counts[int64_t(i) * 64 + lane_id()];
         if (uniform(place) == 0xffffffffu)
             continue; // did not fit (the whole group)
@@ -1168,7 +1450,6 @@ struct SplatWorkspace {
     uint32_t* counter;
     void* sort_scratch;
     void* scan_scratch;
-    uint32_t* prefix_open; // prefix binning: [4 tiles] open waves, [tiles] groups noted, [1 + tiles] open groups, counts
 };
 
 static SplatWorkspace carve_splat(Carver& cv, int64_t n, int64_t cap, bool cull)
@@ -1193,9 +1474,6 @@ static SplatWorkspace carve_splat(Carver& cv, int64_t n, int64_t cap, bool cull)
     w.owner_rects = reinterpret_cast<uint2*>(w.owner_reach);
     w.sort_scratch = cv.take<char>(radix_scratch_bytes(std::max(nn, cc)));
     w.scan_scratch = cv.take<char>(scan_scratch_bytes(nn, 2));
-    // the rest of the workspace: a caller of prefix binning has one for at least
-    // kPrefixMin times the pairs that are carved here, 6 words more per pair
-    w.prefix_open = reinterpret_cast<uint32_t*>(cv.base ? cv.base + cv.used : nullptr);
     return w;
 }
 
@@ -1224,8 +1502,9 @@ template <int TW, int TH>
 static void launch_blend_fwd(int batch, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float2* xy,
     const float4* co, const float* rgb, int W, int H, int gx, const double* bg, float* fb, float* T, const PrefixPass& prefix)
 {
+    // the second pass of prefix binning mostly has few tiles to blend
     constexpr int SPLIT = TW * TH / 64;
-    if (SPLIT > 1 && n_tiles <= kFwdSplitTiles)
+    if (SPLIT > 1 && (n_tiles <= kFwdSplitTiles || prefix.again))
         launch_blend_fwd_as<TW, TH, SPLIT>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, prefix);
     else
         launch_blend_fwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, prefix);
@@ -1258,7 +1537,7 @@ static void launch_blend_bwd(int batch, int n_tiles, hipStream_t st, const uint3
         launch_blend_bwd_as<TW, TH, 1>(batch, n_tiles, st, ranges, pl, xy, co, rgb, W, H, gx, bg, fb, T, gfb, sg, prio);
 }
 
-// waves per tile of the forward blend at a tiling and tile count
+// waves per tile of the forward blend (of prefix binning's first pass)
 static int blend_forward_split(const dgmr_tiling& t, int64_t n_tiles) { return n_tiles <= kFwdSplitTiles ? t.tile_w * t.tile_h / 64 : 1; }
 
 void splat_blend_forward(const dgmr_tiling& t, int n_tiles, hipStream_t st, const uint32_t* ranges, const uint32_t* pl, const float* xy,
@@ -1293,6 +1572,8 @@ void splat_blend_backward(const dgmr_tiling& t, int n_tiles, int64_t n_pairs, hi
         launch_blend_bwd<32, 8>(t.batch, n_tiles, st, ranges, pl, xy2, co4, rgb, W, H, gx, bg, fb, T, gfb, sg, prio);
 }
 
+static OpenTiles open_tiles(const PrefixBinning& p) { return OpenTiles { p.open_tiles, p.row_words, p.open_words, p.any_open, p.positions, p.rest, p.groups, p.group_noted }; }
+
 struct EmitArgs {
     int64_t n;
     unsigned blocks_n;
@@ -1309,62 +1590,133 @@ struct EmitArgs {
     bool bounds_written;         // by the small views' binning
 };
 
-static int emit_per(int64_t cap) { return cap >= kEmitLarge ? kEmitPerLarge : kEmitPerSmall; }
+// pairs: the most that are emitted, with prefix binning in its first round
+static int emit_per(int64_t pairs) { return pairs >= kEmitLarge ? kEmitPerLarge : kEmitPerSmall; }
 static int emit_shift(int per) { return __builtin_ctz(unsigned(kEmitThreads * per)); } // log2 of a block's pairs
+
+// the buffer pairs of emission and pair sort, so that the sorted ids end in `list`
+template <class KeyT>
+static SortBuffersT<KeyT> pair_buffers(const SplatWorkspace& w, uint32_t* list, int passes)
+{
+    KeyT* ka = reinterpret_cast<KeyT*>(w.pkeys_a);
+    KeyT* kb = reinterpret_cast<KeyT*>(w.pkeys_b);
+    return passes % 2 == 0 ? SortBuffersT<KeyT> { ka, list, kb, w.pvals_a } : SortBuffersT<KeyT> { ka, w.pvals_a, kb, list };
+}
+
+// emission of *n_emit pairs
+template <class KeyT>
+static int launch_emit(const EmitArgs& a, const SplatWorkspace& w, const uint32_t* n_emit, const uint32_t* offsets, int per,
+    const SortBuffersT<KeyT>& pb, hipStream_t st)
+{
+    const unsigned emit_blocks = unsigned(ceil_div64(a.cap, kEmitThreads * per));
+    if (a.cull && per == kEmitPerLarge)
+        k_emit_reach<KeyT, kEmitPerLarge><<<emit_blocks, kEmitThreads, 0, st>>>(n_emit, a.cap, a.sorted_ids, w.emit_bounds,
+            offsets, w.owner_reach, a.tile_w, a.tile_h, pb.keys_a, pb.vals_a);
+    else if (a.cull)
+        k_emit_reach<KeyT, kEmitPerSmall><<<emit_blocks, kEmitThreads, 0, st>>>(n_emit, a.cap, a.sorted_ids, w.emit_bounds,
+            offsets, w.owner_reach, a.tile_w, a.tile_h, pb.keys_a, pb.vals_a);
+    else if (per == kEmitPerLarge)
+        k_emit_pairs<KeyT, kEmitPerLarge><<<emit_blocks, kEmitThreads, 0, st>>>(a.n, n_emit, a.cap, a.sorted_ids, w.emit_bounds,
+            offsets, w.owner_rects, pb.keys_a, pb.vals_a);
+    else
+        k_emit_pairs<KeyT, kEmitPerSmall><<<emit_blocks, kEmitThreads, 0, st>>>(a.n, n_emit, a.cap, a.sorted_ids, w.emit_bounds,
+            offsets, w.owner_rects, pb.keys_a, pb.vals_a);
+    DGMR_HIP_CHECK(hipGetLastError());
+    return DGMR_OK;
+}
 
 // emission, pair sort on the tile bits, tile ranges; pair keys of type KeyT
 template <class KeyT>
 static int emit_sort_ranges(const EmitArgs& a, const SplatWorkspace& w, dgmr_binning* bins, PendingCount* pending, hipStream_t st)
 {
-    // emit into the buffer pair that leaves the sorted ids in bins->point_list
     const int passes = radix_passes(0, a.tile_bits);
-    KeyT* ka = reinterpret_cast<KeyT*>(w.pkeys_a);
-    KeyT* kb = reinterpret_cast<KeyT*>(w.pkeys_b);
-    SortBuffersT<KeyT> pb;
-    if (passes % 2 == 0)
-        pb = SortBuffersT<KeyT> { ka, bins->point_list, kb, w.pvals_a };
-    else
-        pb = SortBuffersT<KeyT> { ka, w.pvals_a, kb, bins->point_list };
-    const int per = emit_per(a.cap);
-    const uint32_t block_pairs = uint32_t(kEmitThreads * per);
-    const unsigned emit_blocks = unsigned(ceil_div64(a.cap, block_pairs));
+    const SortBuffersT<KeyT> pb = pair_buffers<KeyT>(w, bins->point_list, passes);
+    const uint32_t* n_emit = a.prefix ? a.prefix->n_emit : w.counter;
+    // fewer than kPrefixMin times the prefix are emitted whole
+    const int per = emit_per(a.prefix ? std::min<int64_t>(a.cap, kPrefixMin * a.prefix->pairs) : a.cap);
     {
         StageScope sc("bin.emit", st);
         pending->add_stage(sc.slot, 4.0 + sizeof(KeyT), 28.0 * double(a.n));
         if (!a.bounds_written)
-            k_emit_bounds<<<a.blocks_n, 256, 0, st>>>(a.n, w.pair_offsets, w.counter, a.cap, emit_shift(per), w.emit_bounds,
-                a.prefix ? a.prefix->n_owners : nullptr);
+            k_emit_bounds<<<a.blocks_n, 256, 0, st>>>(a.n, w.pair_offsets, w.counter, a.cap, n_emit, emit_shift(per), w.emit_bounds);
         DGMR_HIP_CHECK(hipGetLastError());
-        if (a.cull && per == kEmitPerLarge)
-            k_emit_reach<KeyT, kEmitPerLarge><<<emit_blocks, kEmitThreads, 0, st>>>(w.counter, a.cap, a.sorted_ids, w.emit_bounds,
-                w.pair_offsets, w.owner_reach, a.tile_w, a.tile_h, pb.keys_a, pb.vals_a);
-        else if (a.cull)
-            k_emit_reach<KeyT, kEmitPerSmall><<<emit_blocks, kEmitThreads, 0, st>>>(w.counter, a.cap, a.sorted_ids, w.emit_bounds,
-                w.pair_offsets, w.owner_reach, a.tile_w, a.tile_h, pb.keys_a, pb.vals_a);
-        else if (per == kEmitPerLarge)
-            k_emit_pairs<KeyT, kEmitPerLarge><<<emit_blocks, kEmitThreads, 0, st>>>(a.n, w.counter, a.cap, a.sorted_ids, w.emit_bounds,
-                w.pair_offsets, w.owner_rects, pb.keys_a, pb.vals_a);
-        else
-            k_emit_pairs<KeyT, kEmitPerSmall><<<emit_blocks, kEmitThreads, 0, st>>>(a.n, w.counter, a.cap, a.sorted_ids, w.emit_bounds,
-                w.pair_offsets, w.owner_rects, pb.keys_a, pb.vals_a);
-        DGMR_HIP_CHECK(hipGetLastError());
+        const int rc = launch_emit<KeyT>(a, w, n_emit, w.pair_offsets, per, pb, st);
+        if (rc != DGMR_OK)
+            return rc;
     }
     {
         StageScope sc("bin.pair_sort", st);
         pending->add_stage(sc.slot, (8.0 + 3.0 * sizeof(KeyT)) * passes, 0.0);
-        DGMR_HIP_CHECK(radix_sort_pairs(pb, a.cap, w.counter, 0, a.tile_bits, w.sort_scratch, st));
+        DGMR_HIP_CHECK(radix_sort_pairs(pb, a.cap, n_emit, 0, a.tile_bits, w.sort_scratch, st));
     }
     const KeyT* sorted_keys = (passes % 2 == 0) ? pb.keys_a : pb.keys_b;
     const uint32_t* sorted_vals = (passes % 2 == 0) ? pb.vals_a : pb.vals_b;
     {
         StageScope sc("bin.ranges", st);
         pending->add_stage(sc.slot, 0.0, 8.0 * double(a.n_tiles));
-        k_tile_ranges<KeyT><<<unsigned(ceil_div64(a.n_tiles, 256)), 256, 0, st>>>(sorted_keys, sorted_vals, w.counter, a.cap, a.views,
-            a.n_views, a.n_per_view, a.n_tiles, bins->ranges, a.prefix ? a.prefix->used : nullptr,
-            a.prefix ? a.prefix->groups : nullptr, a.prefix ? a.prefix->group_noted : nullptr);
+        k_tile_ranges<KeyT><<<unsigned(ceil_div64(a.n_tiles, 256)), 256, 0, st>>>(sorted_keys, sorted_vals, n_emit, a.cap, a.views,
+            a.n_views, a.n_per_view, a.n_tiles, bins->ranges, a.prefix ? open_tiles(*a.prefix) : OpenTiles {});
         DGMR_HIP_CHECK(hipGetLastError());
     }
     return DGMR_OK;
+}
+
+// the whole lists of the open tiles behind the prefixes (nothing when there are none)
+template <class KeyT>
+static int extend_lists_keyed(const EmitArgs& a, const SplatWorkspace& w, dgmr_binning* bins, hipStream_t st)
+{
+    const PrefixBinning& p = *a.prefix;
+    const OpenTiles open = open_tiles(p);
+    const unsigned blocks = unsigned(ceil_div64(a.n, 256 * kOpenPer));
+    const ScanState scan = scan_state(w.scan_scratch, a.n, 2);
+    if (open.words <= kOpenLdsWords)
+        k_open_owners<true><<<blocks, 256, size_t(open.words) * sizeof(uint32_t), st>>>(open, p.grid_x, p.n_owners, p.origin, p.size, w.counts,
+            p.flags, scan);
+    else
+        k_open_owners<false><<<blocks, 256, 0, st>>>(open, p.grid_x, p.n_owners, p.origin, p.size, w.counts, p.flags, scan);
+    DGMR_HIP_CHECK(hipGetLastError());
+    const ScanArray scans[2] = { { w.counts, w.pair_offsets, open.rest, false }, { p.flags, p.flags, nullptr, false } };
+    DGMR_HIP_CHECK(scan_u32_arrays(scans, 2, a.n, w.scan_scratch, st, true, ScanLength { open.positions, 1, 1 }));
+    k_open_bounds<<<blocks, 256, 0, st>>>(open, w.pair_offsets, p.flags, p.origin, p.size, p.ids, p.grid_x, a.cap, emit_shift(kEmitPerSmall),
+        w.counts, w.owner_rects, p.ids_out, w.emit_bounds);
+    DGMR_HIP_CHECK(hipGetLastError());
+    const int passes = radix_passes(0, a.tile_bits);
+    const SortBuffersT<KeyT> pb = pair_buffers<KeyT>(w, bins->point_list + p.pairs, passes);
+    const int rc = launch_emit<KeyT>(a, w, open.rest, w.counts, kEmitPerSmall, pb, st);
+    if (rc != DGMR_OK)
+        return rc;
+    DGMR_HIP_CHECK(radix_sort_pairs(pb, a.cap, open.rest, 0, a.tile_bits, w.sort_scratch, st));
+    k_open_ranges<KeyT><<<unsigned(ceil_div64(a.n_tiles, 256)), 256, 0, st>>>((passes % 2 == 0) ? pb.keys_a : pb.keys_b, a.cap, p.pairs, open,
+        p.grid_x, a.n_tiles, bins->ranges, p.done);
+    DGMR_HIP_CHECK(hipGetLastError());
+    return DGMR_OK;
+}
+
+static int extend_lists(const PrefixBinning& p, bool few, int64_t n, int64_t n_tiles, void* workspace, size_t workspace_bytes, dgmr_binning* bins,
+    hipStream_t st)
+{
+    StageScope sc(few ? "bin.extend_few" : "bin.extend", st);
+    Carver cv(workspace, workspace_bytes);
+    const SplatWorkspace w = carve_splat(cv, n, bins->pair_capacity, false); // as the binning carved it
+    const int64_t cap = std::min<int64_t>(bins->pair_capacity, int64_t(UINT32_MAX));
+    if (few) {
+        // the pair keys are not read again: their buffer holds the counts
+        const int grid_y = int(n_tiles / p.grid_x);
+        const int64_t groups = ceil_div64(p.grid_x, 8) * ceil_div64(grid_y, 8);
+        const int segments = int(std::min<int64_t>(512, cap / (groups * 64)));
+        const ExtendArgs xa { p.pairs, uint64_t(p.pairs + cap), p.n_owners, p.origin, p.size, p.ids, open_tiles(p), w.pkeys_a, p.done, p.grid_x, grid_y,
+            segments };
+        k_extend_count<<<kExtendBlocks, 256, 0, st>>>(xa);
+        DGMR_HIP_CHECK(hipGetLastError());
+        k_extend_place<<<unsigned(std::min<int64_t>(groups, 256)), 64 * kPlaceWaves, 0, st>>>(xa, bins->ranges);
+        DGMR_HIP_CHECK(hipGetLastError());
+        k_extend_write<<<kExtendBlocks, 256, 0, st>>>(xa, bins->point_list);
+        DGMR_HIP_CHECK(hipGetLastError());
+        return DGMR_OK;
+    }
+    const EmitArgs ea { n, unsigned(ceil_div64(n, 256)), uint32_t(cap), n_tiles, int(higher_msb(uint32_t(n_tiles))), p.ids_out, nullptr, 0, 0, 0, 0, false, &p,
+        false };
+    return ea.tile_bits <= 16 ? extend_lists_keyed<uint16_t>(ea, w, bins, st) : extend_lists_keyed<uint32_t>(ea, w, bins, st);
 }
 
 // binning shared by the splatter and the marcher: depth sort, scan, emission,
@@ -1393,7 +1745,7 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
         n_sorted = count;
     }
     const bool multi_view = batch && batch->n_views > 1;
-    const bool one = bin_rects_written && !cull && !batch && n <= kBinOneMax;
+    const bool one = bin_rects_written && !cull && !batch && !prefix && n <= kBinOneMax;
     // with tight culling the culled entries sort last in the view pass, under the key n_views
     const uint32_t culled_view = cull && multi_view ? uint32_t(batch->n_views) : 0xffffffffu;
     if (!one) {
@@ -1418,21 +1770,42 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
     }
     const uint32_t* sorted_ids = V;
     // prefix binning: the sorted depth keys are not read again, their buffers
-    // hold the rectangles
-    PrefixRects rects_out { nullptr, nullptr };
+    // hold the rectangles; nor, once gathered, the records in id order, whose
+    // 2 n words hold what the blend notes (8 per tile and one, and n >= 96 per tile)
+    // and the extension's flags
+    PrefixRects rects_out { nullptr, nullptr, nullptr };
     if (prefix) {
-        rects_out = PrefixRects { K, K2 };
-        const int64_t tiles = int64_t(grid_x) * grid_y;
-        *prefix = PrefixBinning { K, K2, sorted_ids, w.counter, w.counter + 2, w.counter + 3, w.prefix_open, w.prefix_open + 4 * tiles,
-            w.prefix_open + 5 * tiles, w.prefix_open + 6 * tiles + 1, 4 * bins->pair_capacity };
+        static_assert(kPrefixMin * kPrefixPerTile * sizeof(uint32_t) >= sizeof(DecideSums), "the pair keys' buffer holds the sums until the emission");
+        rects_out = PrefixRects { K, K2, reinterpret_cast<DecideSums*>(w.pkeys_a) };
+        const int64_t n_tiles = int64_t(grid_x) * grid_y;
+        uint32_t* words = reinterpret_cast<uint32_t*>(w.bin_rects);
+        prefix->ids = sorted_ids;
+        prefix->ids_out = V2;
+        prefix->origin = K;
+        prefix->size = K2;
+        prefix->n_pairs = w.counter;
+        prefix->n_emit = w.counter + 2;
+        prefix->few = w.counter + 3;
+        prefix->n_owners = w.counter + 4;
+        prefix->any_open = w.counter + 5;
+        prefix->positions = w.counter + 6;
+        prefix->rest = w.counter + 7;
+        prefix->units = words;
+        prefix->done = words + 4 * n_tiles;
+        prefix->open_tiles = words + 5 * n_tiles;
+        prefix->group_noted = words + 6 * n_tiles;
+        prefix->groups = words + 7 * n_tiles;
+        prefix->flags = words + (8 * n_tiles + 1 + 3) / 4 * 4;
+        prefix->grid_x = grid_x;
+        prefix->row_words = int(ceil_div64(grid_x, 32));
+        prefix->open_words = int64_t(prefix->row_words) * grid_y;
     }
     const unsigned blocks_n = unsigned(ceil_div64(n, 256));
     const int64_t cap = std::min<int64_t>(bins->pair_capacity, int64_t(UINT32_MAX));
     if (one) {
         StageScope sc("bin.one", st, 60.0 * double(n));
         k_bin_one<<<bins->point_offsets ? 2 : 1, kBinOneThreads, 0, st>>>(BinOneArgs { int(n), K, w.bin_rects, tiles, uint32_t(grid_x), uint32_t(std::max<int64_t>(cap, 0)),
-            emit_shift(emit_per(cap)), V, w.owner_rects, w.pair_offsets, bins->point_offsets, w.counter, w.emit_bounds,
-            prefix ? prefix->n_owners : nullptr, rects_out });
+            emit_shift(emit_per(cap)), V, w.owner_rects, w.pair_offsets, bins->point_offsets, w.counter, w.emit_bounds });
         DGMR_HIP_CHECK(hipGetLastError());
     } else {
         StageScope sc("bin.scan", st, 44.0 * double(n));
@@ -1458,7 +1831,12 @@ int bin_gaussians(int64_t n, const int32_t* rects, const uint32_t* tiles, const 
         DGMR_HIP_CHECK(scan_u32_arrays(scans, n_scans, n, w.scan_scratch, st, true));
     }
     // R stays on the device: the copy to the host is awaited by the caller
-    const int rc_count = enqueue_count(w.counter, st, pending);
+    if (prefix) {
+        k_prefix_decide<<<kDecideBlocks, kDecideThreads, 0, st>>>(DecideArgs { n, w.pair_offsets, w.counter, uint32_t(cap), prefix->pairs, prefix->always,
+            sorted_ids, prefix->origin, prefix->size, prefix->conic_opacity, grid_x, grid_y, tile_w * tile_h, rects_out.sums, prefix->n_emit, prefix->few, prefix->n_owners });
+        DGMR_HIP_CHECK(hipGetLastError());
+    }
+    const int rc_count = enqueue_count(w.counter, st, pending, prefix ? int(prefix->n_emit - w.counter) : 0);
     if (rc_count != DGMR_OK)
         return rc_count;
     const int64_t n_tiles = batch ? batch->total_tiles : int64_t(grid_x) * grid_y;
@@ -1496,7 +1874,7 @@ using namespace dgmr;
 
 static int splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, dgmr_splat_geometry* geom,
     dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, dgmr_stats* stats,
-    dgmr_stream stream, bool allow_prefix)
+    dgmr_stream stream, int32_t lists, int64_t* n_binned)
 {
     DGMR_ARG_CHECK(g && cam && geom && bins && framebuffer && final_transmittance && workspace, "dgmr_splat_forward: null argument");
     DGMR_ARG_CHECK(g->dtype == DGMR_F32, "dgmr_splat_forward: the splatter computes in float32");
@@ -1516,6 +1894,8 @@ static int splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const 
         stats->n_pairs = 0;
         stats->n_visible = 0;
     }
+    if (n_binned)
+        *n_binned = 0;
     if (n == 0) {
         DGMR_HIP_CHECK(hipMemsetAsync(bins->ranges, 0, size_t(n_tiles) * 2 * sizeof(uint32_t), st));
         splat_blend_forward(*tiling, int(n_tiles), st, bins->ranges, bins->point_list, geom->xy, geom->conic_opacity, geom->rgb, cam->width,
@@ -1535,51 +1915,47 @@ static int splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const 
     }
     Carver cv(workspace, workspace_bytes);
     PendingCount pending;
-    const int64_t prefix = allow_prefix && !cull ? prefix_pairs(n, n_tiles, bins->pair_capacity) : 0;
     PrefixBinning pb {};
-    dgmr_binning first = *bins;
-    if (prefix)
-        first.pair_capacity = prefix;
-    const int rc = bin_gaussians(n, geom->rects, geom->tiles_touched, geom->xy, false, true, cull, dc.grid_x, dc.grid_y, dc.tile_w, dc.tile_h, &first,
+    pb.always = lists == DGMR_LISTS_PREFIX;
+    pb.conic_opacity = reinterpret_cast<const float4*>(geom->conic_opacity);
+    pb.pairs = lists != DGMR_LISTS_WHOLE && !cull ? uint32_t(prefix_pairs(n, n_tiles, bins->pair_capacity)) : 0u;
+    const bool prefix = pb.pairs != 0;
+    const int rc = bin_gaussians(n, geom->rects, geom->tiles_touched, geom->xy, false, true, cull, dc.grid_x, dc.grid_y, dc.tile_w, dc.tile_h, bins,
         cv, &pending, st, nullptr, prefix ? &pb : nullptr);
     if (rc != DGMR_OK)
         return rc;
     int blend_slot = -1;
-    PrefixPass pass { pb.open, pb.groups, pb.group_noted, pb.n_pairs, uint32_t(prefix), false };
+    PrefixPass pass { pb.units, open_tiles(pb), pb.done, pb.n_pairs, pb.n_emit, pb.pairs, blend_forward_split(*tiling, n_tiles), false };
     {
         StageScope sc("splat.blend_forward", st);
         blend_slot = sc.slot;
         splat_blend_forward(*tiling, int(n_tiles), st, bins->ranges, bins->point_list, geom->xy, geom->conic_opacity, geom->rgb, cam->width,
             cam->height, dc.grid_x, cam->background, framebuffer, final_transmittance, pass);
         DGMR_HIP_CHECK(hipGetLastError());
-        if (prefix) {
-            const int64_t groups = ceil_div64(dc.grid_x, 8) * ceil_div64(dc.grid_y, 8);
-            // as many segments as there is room for counts, at most 512
-            const int segments = int(std::min<int64_t>(512, pb.counts_room / (groups * 64)));
-            const ExtendArgs ea { pb.n_pairs, uint32_t(prefix), uint64_t(prefix + bins->pair_capacity), pb.n_owners, pb.origin, pb.size, pb.ids,
-                pb.open, pb.groups, pb.counts, pb.used, blend_forward_split(*tiling, n_tiles), dc.grid_x, dc.grid_y, segments };
-            k_extend_count<<<kExtendBlocks, 256, 0, st>>>(ea);
-            DGMR_HIP_CHECK(hipGetLastError());
-            k_extend_place<<<unsigned(std::min<int64_t>(groups, 256)), 64 * kPlaceWaves, 0, st>>>(ea, bins->ranges);
-            DGMR_HIP_CHECK(hipGetLastError());
-            k_extend_write<<<kExtendBlocks, 256, 0, st>>>(ea, bins->point_list);
-            DGMR_HIP_CHECK(hipGetLastError());
-            pass.again = true;
-            splat_blend_forward(*tiling, int(n_tiles), st, bins->ranges, bins->point_list, geom->xy, geom->conic_opacity, geom->rgb, cam->width,
-                cam->height, dc.grid_x, cam->background, framebuffer, final_transmittance, pass);
-            DGMR_HIP_CHECK(hipGetLastError());
-        }
     }
     pending.add_stage(blend_slot, 40.0, 16.0 * double(plane) + 8.0 * double(n_tiles));
-    // every launch is queued: now wait for the pair count
+    // every launch is queued: now wait for the pair count (the extension, which
+    // needs it, follows while the emission, sort and blend still run)
     const int64_t R = pending.wait();
     if (R < 0)
         return DGMR_ERR_DEVICE;
     if (stats)
         stats->n_pairs = R;
+    if (n_binned)
+        *n_binned = pending.binned;
     if (R > bins->pair_capacity) {
         set_error("pair capacity too small");
         return DGMR_ERR_CAPACITY;
+    }
+    if (prefix && pending.binned < R) {
+        const int rc_ext = extend_lists(pb, pending.few, n, n_tiles, workspace, workspace_bytes, bins, st);
+        if (rc_ext != DGMR_OK)
+            return rc_ext;
+        StageScope sc("splat.blend_open", st);
+        pass.again = true;
+        splat_blend_forward(*tiling, int(n_tiles), st, bins->ranges, bins->point_list, geom->xy, geom->conic_opacity, geom->rgb, cam->width,
+            cam->height, dc.grid_x, cam->background, framebuffer, final_transmittance, pass);
+        DGMR_HIP_CHECK(hipGetLastError());
     }
     return DGMR_OK;
 }
@@ -1597,7 +1973,8 @@ int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dg
     dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, dgmr_stats* stats,
     dgmr_stream stream)
 {
-    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream, false);
+    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream,
+        DGMR_LISTS_WHOLE, nullptr);
 }
 
 int dgmr_splat_prefix_pairs(int64_t n, int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity, int64_t* pairs)
@@ -1613,7 +1990,16 @@ int dgmr_splat_forward_prefix(const dgmr_gaussians* g, const dgmr_camera* cam, c
     dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, dgmr_stats* stats,
     dgmr_stream stream)
 {
-    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream, true);
+    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream,
+        DGMR_LISTS_PREFIX, nullptr);
+}
+
+int dgmr_splat_forward_lists(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, dgmr_splat_geometry* geom,
+    dgmr_binning* bins, float* framebuffer, float* final_transmittance, void* workspace, size_t workspace_bytes, int32_t lists, int64_t* n_binned,
+    dgmr_stats* stats, dgmr_stream stream)
+{
+    DGMR_ARG_CHECK(lists >= DGMR_LISTS_WHOLE && lists <= DGMR_LISTS_AUTO, "dgmr_splat_forward_lists: bad lists");
+    return splat_forward(g, cam, tiling, geom, bins, framebuffer, final_transmittance, workspace, workspace_bytes, stats, stream, lists, n_binned);
 }
 
 int dgmr_splat_backward(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling, const dgmr_splat_geometry* geom,

@@ -536,7 +536,7 @@ __device__ __forceinline__ void wave_lds_sync() { __builtin_amdgcn_wave_barrier(
 
 // lane masks of float comparisons (LLVM predicates), combined with scalar
 // instructions where a wave-uniform decision needs them
-enum : int { kCmpOGE = 3, kCmpOLT = 4 };
+enum : int { kCmpOGT = 2, kCmpOGE = 3, kCmpOLT = 4 };
 template <int PRED>
 __device__ __forceinline__ uint64_t lanes_where(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, PRED); }
 
@@ -563,11 +563,18 @@ __device__ __forceinline__ float gauss_at(const LaneTerms& t, float c_scaled, fl
 // instead, four vector operations a pixel and Gaussian where these are three
 // scalar ones, 39k tiles took 0.325 ms against 0.28 and 8 160 tiles 85 us against 76.
 // Returns whether some pixel of the tile would take more Gaussians than the
-// list holds.
+// list holds.  resume.keep: such a tile's pixels are left as they stand (the
+// colour without the background, the transmittance of a stopped pixel negated)
+// for a later call with resume.load and the rest of the list, which goes on
+// with the same values.
+struct BlendResume {
+    bool load, keep;
+};
 template <int TW, int TH, int B>
 __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t first, uint32_t last, int px0, int py0, int width, int height,
     float bg0, float bg1, float bg2, const uint32_t* __restrict__ point_list, const float2* __restrict__ xy,
-    const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, float* __restrict__ framebuffer, float* __restrict__ final_T)
+    const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, float* __restrict__ framebuffer, float* __restrict__ final_T,
+    BlendResume resume = BlendResume { false, false })
 {
     constexpr int NP = TW * TH / 64;
     constexpr int RS = 64 / TW;
@@ -576,6 +583,7 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
     const float pxf = float(px);
     const float pyf0 = float(py0 + lane / TW);
     const float bx0 = float(px0), bx1 = float(px0 + TW - 1), by0 = float(py0), by1 = float(py0 + TH - 1);
+    const int64_t plane = int64_t(width) * height;
     // the lanes whose pixel k takes more Gaussians, as a wave-uniform mask
     uint64_t live[NP];
     float T[NP], C0[NP], C1[NP], C2[NP];
@@ -585,6 +593,17 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
         live[k] = __builtin_amdgcn_ballot_w64(px < width && py < height);
         T[k] = 1.f;
         C0[k] = C1[k] = C2[k] = 0.f;
+        if (resume.load) {
+            if (px < width && py < height) {
+                const int64_t p = int64_t(py) * width + px;
+                T[k] = final_T[p];
+                C0[k] = framebuffer[p];
+                C1[k] = framebuffer[plane + p];
+                C2[k] = framebuffer[2 * plane + p];
+            }
+            live[k] &= lanes_where<kCmpOGT>(T[k], 0.f);
+            T[k] = fabsf(T[k]);
+        }
     }
     if (first < last) {
         BlendFetch<B> f;
@@ -632,23 +651,23 @@ __device__ __forceinline__ bool blend_tile_forward(BlendSmem<B>& sm, uint32_t fi
             }
         }
     }
-    const int64_t plane = int64_t(width) * height;
+    uint64_t open = 0;
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+        open |= live[k];
+    const bool keep = resume.keep && open != 0;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
         const int py = py0 + lane / TW + RS * k;
         if (px < width && py < height) {
             const int64_t p = int64_t(py) * width + px;
             const float Tk = T[k];
-            framebuffer[p] = fmaf(Tk, bg0, C0[k]);
-            framebuffer[plane + p] = fmaf(Tk, bg1, C1[k]);
-            framebuffer[2 * plane + p] = fmaf(Tk, bg2, C2[k]);
-            final_T[p] = Tk;
+            framebuffer[p] = keep ? C0[k] : fmaf(Tk, bg0, C0[k]);
+            framebuffer[plane + p] = keep ? C1[k] : fmaf(Tk, bg1, C1[k]);
+            framebuffer[2 * plane + p] = keep ? C2[k] : fmaf(Tk, bg2, C2[k]);
+            final_T[p] = keep && !__builtin_amdgcn_inverse_ballot_w64(live[k]) ? -Tk : Tk;
         }
     }
-    uint64_t open = 0;
-#pragma unroll
-    for (int k = 0; k < NP; ++k)
-        open |= live[k];
     return open != 0;
 }
 

@@ -39,13 +39,14 @@ CACHE_FIELDS = ("framebuffer", "rects", "rgb", "rgb_sh_clamped", "depths", "poin
 def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, proj_matrix, cam_position, background,
              render_width: int, render_height: int, tan_fovx: float, tan_fovy: float, sh_degree: int,
              tile=None, batch: int = 0, scale_multiplier: float = 1.0, activation: int = N.DGMR_ACT_NONE, cull=None,
-             whole_lists: bool = True):
+             whole_lists: bool | None = True):
     """cull=True bins each Gaussian only into the tiles where its alpha can
     reach 1/255 (dgmr_tiling.cull): same image, transmittance and gradients,
     fewer pairs; b_point_list and i_ranges then differ from the reference's.
     None: DEFAULT_CULL.  whole_lists=False bins no more of a deep view than its
     tiles can take (dgmr_splat_forward_prefix): same image, transmittance and
-    gradients, but b_point_list holds prefixes of the reference's lists."""
+    gradients, but b_point_list holds prefixes of the reference's lists.  None:
+    that where it pays (dgmr_splat_forward_lists)."""
     cull = DEFAULT_CULL if cull is None else bool(cull)
     tile = tile or DEFAULT_TILING[0]
     batch = batch or DEFAULT_TILING[1]
@@ -75,6 +76,8 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
                                clamped.data_ptr(), depths.data_ptr())
         cap = C.initial_capacity(dev, "splat", n)
         stats = N.Stats()
+        binned = ctypes.c_int64(0)
+        lists = N.DGMR_LISTS_WHOLE if whole_lists else (N.DGMR_LISTS_AUTO if whole_lists is None else N.DGMR_LISTS_PREFIX)
         stream = C.stream_handle(dev)
         for _attempt in range(3):
             prefix = ctypes.c_int64(0)
@@ -83,9 +86,9 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
             point_list = torch.empty((max(cap + prefix.value, 1),), dtype=torch.int32, device=dev)
             bins = N.Binning(offsets.data_ptr(), point_list.data_ptr(), ranges.data_ptr(), cap)
             ws = C.workspace(dev, n, W, H, tiling, cap)
-            forward = lib.dgmr_splat_forward_prefix if prefix.value else lib.dgmr_splat_forward
-            rc = forward(ctypes.byref(g), ctypes.byref(cam), ctypes.byref(tiling), ctypes.byref(geom), ctypes.byref(bins), fb.data_ptr(),
-                         T.data_ptr(), ws.data_ptr(), ws.numel(), ctypes.byref(stats), stream)
+            rc = lib.dgmr_splat_forward_lists(ctypes.byref(g), ctypes.byref(cam), ctypes.byref(tiling), ctypes.byref(geom), ctypes.byref(bins),
+                                              fb.data_ptr(), T.data_ptr(), ws.data_ptr(), ws.numel(), lists, ctypes.byref(binned),
+                                              ctypes.byref(stats), stream)
             if rc == N.DGMR_ERR_CAPACITY:
                 cap = int(stats.n_pairs * 1.25) + 1024
                 C.remember_capacity(dev, "splat", cap)
@@ -94,11 +97,9 @@ def _forward(shs, weights, centroids, cov_scales, cov_rotations, view_matrix, pr
             break
         else:
             raise N.DgmrError(N.DGMR_ERR_CAPACITY, "dgmr_splat_forward", "pair capacity kept growing")
-        R = int(stats.n_pairs)
+        R = int(binned.value)
         C.remember_capacity(dev, "splat", cap)
-    if R > prefix.value > 0:
-        R = prefix.value  # the pairs binned; extended lists lie behind them
-    else:
+    if R == int(stats.n_pairs):  # else extended lists lie behind the binned pairs
         point_list = point_list[:R]
     return [fb, rects, rgb, clamped, depths, xy, conic, tiles, offsets, ranges, point_list, T, torch.tensor([R], dtype=torch.int64)]
 
@@ -148,7 +149,7 @@ class Splatter(torch.autograd.Function):
     def forward(ctx, shs, opacity, means3D, scales, rotations, world_view_transform, full_proj_transform, camera_center, bg_color,
                 image_width: int, image_height: int, tanfovx: float, tanfovy: float, active_sh_degree: int):
         cache = cpp_binding.forward(shs, opacity, means3D, scales, rotations, world_view_transform, full_proj_transform, camera_center,
-                                    bg_color, image_width, image_height, tanfovx, tanfovy, active_sh_degree, whole_lists=False)
+                                    bg_color, image_width, image_height, tanfovx, tanfovy, active_sh_degree, whole_lists=None)
         ctx.scalars = (int(image_width), int(image_height), float(tanfovx), float(tanfovy), int(active_sh_degree))
         ctx.save_for_backward(shs, opacity, means3D, scales, rotations, world_view_transform, full_proj_transform, camera_center,
                               bg_color, *cache)
@@ -181,7 +182,7 @@ class SplatterActivated(torch.autograd.Function):
                 bg_color, image_width: int, image_height: int, tanfovx: float, tanfovy: float, active_sh_degree: int):
         cache = cpp_binding.forward(shs, opacity_logits, means3D, log_scales, rotations, world_view_transform, full_proj_transform,
                                     camera_center, bg_color, image_width, image_height, tanfovx, tanfovy, active_sh_degree,
-                                    activation=N.DGMR_ACT_LOG_NORM_SIGMOID, whole_lists=False)
+                                    activation=N.DGMR_ACT_LOG_NORM_SIGMOID, whole_lists=None)
         ctx.scalars = (int(image_width), int(image_height), float(tanfovx), float(tanfovy), int(active_sh_degree))
         ctx.save_for_backward(shs, opacity_logits, means3D, log_scales, rotations, world_view_transform, full_proj_transform,
                               camera_center, bg_color, *cache)

@@ -133,18 +133,29 @@ int dgmr_splat_forward(const dgmr_gaussians* g, const dgmr_camera* cam, const dg
     void* workspace, size_t workspace_bytes, dgmr_stats* stats, dgmr_stream stream);
 
 /* The same image and transmittance with prefix binning: where the view's pairs
- * are many times what its tiles can take before they saturate, only the first
- * *pairs of the depth order are binned (dgmr_splat_prefix_pairs; 0: the whole
- * lists are, as above), so a tile's list is a prefix of its whole list; tiles
- * with a pixel still open at its end get their whole list behind it.
- * bins->point_list then holds pair_capacity + *pairs entries, and ranges may
- * point anywhere in it; dgmr_splat_backward walks such lists as any other.  No
- * counterpart in the reference, which bins every pair. */
+ * are many times what its tiles can take before they saturate (at least six
+ * times *pairs of dgmr_splat_prefix_pairs; *pairs 0: whole lists whatever the
+ * view has), only the first *pairs of the depth order are binned, so a tile's
+ * list is a prefix of its whole list; tiles with a pixel still open at its end
+ * get their whole list behind the prefixes.  bins->point_list then holds
+ * pair_capacity + *pairs entries, and ranges may point anywhere in it;
+ * dgmr_splat_backward walks such lists as any other.  No counterpart in the
+ * reference, which bins every pair. */
 int dgmr_splat_prefix_pairs(int64_t n, int32_t width, int32_t height, const dgmr_tiling* tiling, int64_t pair_capacity,
     int64_t* pairs);
 int dgmr_splat_forward_prefix(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling,
     dgmr_splat_geometry* geom, dgmr_binning* bins, float* framebuffer, float* final_transmittance,
     void* workspace, size_t workspace_bytes, dgmr_stats* stats, dgmr_stream stream);
+
+/* Either of the two: whole lists (dgmr_splat_forward), prefixes
+ * (dgmr_splat_forward_prefix), or whichever suits the view: prefixes where the
+ * first pairs of the depth order cover the image, by a sample of them, so that
+ * few tiles would be left open.  *n_binned (may be null): the pairs binned, *pairs
+ * of dgmr_splat_prefix_pairs or all of them; buffers as for prefixes. */
+enum { DGMR_LISTS_WHOLE = 0, DGMR_LISTS_PREFIX = 1, DGMR_LISTS_AUTO = 2 };
+int dgmr_splat_forward_lists(const dgmr_gaussians* g, const dgmr_camera* cam, const dgmr_tiling* tiling,
+    dgmr_splat_geometry* geom, dgmr_binning* bins, float* framebuffer, float* final_transmittance,
+    void* workspace, size_t workspace_bytes, int32_t lists, int64_t* n_binned, dgmr_stats* stats, dgmr_stream stream);
 
 /* Splatter backward (no counterpart in the reference, which ships no splat
  * backward; its adjoints are composed from grad/math.h and

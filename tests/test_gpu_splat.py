@@ -391,6 +391,76 @@ def test_prefix_binning_equals_whole_lists(kind, tile, w, h):
         assert float((a - b).norm()) <= 1e-5 * float(a.norm()), name
 
 
+@pytest.mark.parametrize("kind,w,h", [("saturating", 643, 515), ("hole", 643, 515), ("half_open", 643, 515), ("thin", 203, 117), ("open", 203, 117),
+                                      ("shallow", 643, 515)])
+def test_prefix_lists_where_they_pay(kind, w, h):
+    """whole_lists=None bins prefixes where the nearest Gaussians cover the view
+    (with no tile left open, or a few, whose extension is a kernel of its own) and
+    whole lists where much of it stays open (half, Gaussians small for their tiles,
+    low opacities) or the pairs are few.
+    Whatever is binned, image, transmittance and gradients are those of whole
+    lists, and every list is the whole one or a prefix of it."""
+    import ctypes
+    torch = _torch()
+    from differentiable_gaussian_mixture_renderer_amd import _common, _native as N, scenes
+    from differentiable_gaussian_mixture_renderer_amd.python_bindings import splatter
+    n = 150_000
+    scene = scenes.make_scene(n, seed=6, extent=1.0, sh_degree=1)
+    opacity, scales = scene.opacity.copy(), scene.scales.copy()
+    t = math_tan(0.2)  # the scene fills the view
+    off_axis = np.linalg.norm(scene.means[:, :2], axis=1) / (scene.means[:, 2] + 4.0) * h / (2.0 * t)  # pixels
+    if kind in ("saturating", "hole", "half_open"):
+        scales *= 0.7
+        opacity = np.maximum(opacity, 0.95)
+    if kind == "hole":
+        opacity[off_axis < 45.0] *= 0.002
+    elif kind == "half_open":
+        opacity[scene.means[:, 0] > 0.0] *= 0.002
+    elif kind == "open":
+        opacity *= 0.002
+    elif kind == "shallow":
+        scales *= 0.1
+    cam = scenes.look_at_camera([0.0, 0.0, -4.0], [0.0, 0.0, 0.0], w, h, t * w / h, t)
+    dev = torch.device("cuda:0")
+    T = lambda a: torch.tensor(np.ascontiguousarray(a), device=dev)
+    args = [T(scene.sh), T(opacity), T(scene.means), T(scales), T(scene.rotations), T(cam.world_view_transform), T(cam.full_proj_transform),
+            T(cam.camera_center), T(np.array([0.1, 0.6, 0.3], np.float32)), w, h, cam.tan_fovx, cam.tan_fovy, 1]
+    whole = splatter.cpp_binding.forward(*args)
+    tiles, R = whole[9].shape[0], int(whole[12][0])
+    _common.remember_capacity(dev, "splat", max(R, 1600 * tiles))
+    lib = N.load()
+    stages, count = (N.StageTime * 64)(), ctypes.c_int32(0)
+    lib.dgmr_profile_read(stages, 64, ctypes.byref(count))
+    lib.dgmr_profile_enable(1)
+    got = splatter.cpp_binding.forward(*args, whole_lists=None)
+    lib.dgmr_profile_enable(0)
+    lib.dgmr_profile_read(stages, 64, ctypes.byref(count))
+    ran = {stages[k].name.decode() for k in range(count.value)}
+    prefix = 256 * tiles
+    binned = int(got[12][0])
+    rw, rg = whole[9].cpu().numpy(), got[9].cpu().numpy()
+    extended = int((rg[:, 0] >= prefix).sum()) if binned < R else 0
+    print(f"[gpu lists] {kind} {w}x{h}: R {R}, prefix {prefix}, binned {binned}, extended {extended} of {tiles}")
+    if kind in ("saturating", "hole"):
+        assert R >= 6 * prefix and binned == prefix
+        assert (extended > 0) == (kind == "hole")
+        assert kind != "hole" or ("bin.extend_few" in ran and "bin.extend" not in ran)
+    else:
+        assert binned == R and not ran & {"bin.extend", "bin.extend_few"}
+        assert (R >= 6 * prefix) == (kind != "shallow")
+    assert torch.equal(got[0], whole[0]) and torch.equal(got[11], whole[11])
+    pw, pg = whole[10].cpu().numpy(), got[10].cpu().numpy()
+    for k in range(tiles):
+        a, b = pw[rw[k, 0]:rw[k, 1]], pg[rg[k, 0]:rg[k, 1]]
+        assert len(b) <= len(a) and np.array_equal(a[:len(b)], b), k
+        assert len(a) == len(b) or (binned < R and rg[k, 0] < prefix), k
+    grad = torch.randn(3, h, w, device=dev, generator=torch.Generator(device=dev).manual_seed(1))
+    gw = splatter.cpp_binding.backward(*args, grad, whole)
+    gg = splatter.cpp_binding.backward(*args, grad, got)
+    for name, a, b in zip(("sh", "opacity", "means", "scales", "rotations"), gw, gg):
+        assert float((a - b).norm()) <= 1e-5 * float(a.norm()), name
+
+
 def math_tan(v):
     import math
     return math.tan(v)
