@@ -320,9 +320,12 @@ __device__ __forceinline__ uint64_t valid_entries(int j0, int cnt)
     return n >= 64 ? ~uint64_t(0) : ((uint64_t(1) << n) - 1);
 }
 
-// entries of a word whose window meets (wlo, whi): one entry per lane
+// entries of a word whose window meets (wlo, whi): one entry per lane; none meets
+// an empty window, also those without bounds
 __device__ __forceinline__ uint64_t entries_in(const Reach1d* s_win, int j0, int cnt, float wlo, float whi)
 {
+    if (wlo > whi)
+        return 0;
     const Reach1d w = s_win[min(j0 + int(lane_id()), cnt - 1)];
     return __builtin_amdgcn_ballot_w64(!(w.lo > whi) && !(w.hi < wlo)) & valid_entries(j0, cnt);
 }
