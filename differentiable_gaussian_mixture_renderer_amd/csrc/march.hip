@@ -20,7 +20,8 @@
 // store (device memory of about 2.5 KB per pixel and large step), the forward
 // also writes every chunk's bins and borders, and the backward reads them
 // back instead of recomputing sections and bins: only the adjoint walks
-// remain, which makes the backward cost about as much as the forward.
+// remain (200k Gaussians at 1024^2, all steps kept: 11.2 ms against 26.0
+// recomputed and 16.7 forward).
 #include <algorithm>
 #include <utility>
 
@@ -621,7 +622,7 @@ constexpr int kBinGroup = 8;
 // the exact restriction each time and all of a chunk's bins once one pixel's
 // Gaussian reached it, the forward took 52.0 ms on 200k Gaussians at 1024^2 and
 // forward + backward 56.3 ms on 60k at 491x373; with windows, groups and the
-// sections of sections.h 17.3 and 22.6 ms.
+// sections of sections.h 17.7 and 24.0 ms.
 template <bool ODD, class S, int NT, int CB>
 __device__ __forceinline__ void fill_chunk(S (&bins)[CB][4], const S (&bb)[CB + 1], bool stopped, TileList<S, NT>& tl, bool inside,
     const S* o, const S* d, S b_first, S b_last, const Candidates& cand)
@@ -967,8 +968,10 @@ __device__ __forceinline__ void blend_adjoint(const S (&bins)[CB][4], S (&bb)[CB
 // collect the cdf derivatives at both borders of every bin.  Entries, groups of
 // bins and kept bins are fill_chunk's up to the pixel's stop, past which its
 // bins are empty: a pixel adds to the Gaussians it took mass from and to no
-// other, also where its gradient or a colour is infinite or NaN.
-template <class S, int NT, int CB>
+// other, also where its gradient or a colour is infinite or NaN.  RECORD: no
+// deposit pass has visited the chunk's entries, so this one records which are
+// the wave's candidates.
+template <bool RECORD, class S, int NT, int CB>
 __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candidates& cand, bool active, bool inside, const S* o, const S* d,
     const S (&bb)[CB + 1], S b_first, S b_last, const S (&Tk)[CB], const S (&Gk)[CB], const S* gC, S* __restrict__ render_grads)
 {
@@ -982,13 +985,14 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candida
             uint64_t word = entries_in(tl.s_win, j0, cnt, wlo, whi);
             if (word == 0)
                 continue;
-            // the chunk's deposit pass has visited these entries
-            word &= ~CandidateWord(cand, base - tl.first + uint32_t(j0)).rejected;
-            for (; word != 0; word &= word - 1) {
+            CandidateWord cw(cand, base - tl.first + uint32_t(j0));
+            for (word &= ~cw.rejected; word != 0; word &= word - 1) {
                 const int j = __builtin_ctzll(word);
                 const Staged<S>& g = tl.s_g[j0 + j];
                 RayGauss<S> r;
                 const bool pass = ray_gaussian(g, o, d, &r) && active;
+                if (RECORD)
+                    cw.visited(j, inside, r.mor);
                 if (__builtin_amdgcn_ballot_w64(pass && r.centre + r.far > bb[0] && r.centre - r.far < bb[CB]) == 0)
                     continue;
                 const bool need = deposits_in(r, pass, b_first, b_last, bb[0], bb[CB]);
@@ -1069,6 +1073,8 @@ __device__ __forceinline__ void adjoint_chunk(TileList<S, NT>& tl, const Candida
                     }
                 }
             }
+            if (RECORD)
+                cw.store(cand);
         }
     }
 }
@@ -1159,7 +1165,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward(MarchData<S> md, DevC
                 fill_chunk<false, S, NT, CB>(bins, bb, stopped, tl, inside, o, d, b_first, b_last, cand);
                 blend_adjoint<S, CB>(bins, bb, kk, stopped, T, pa.Cr, pa.Tf, pa.gT, pa.gC, Tk, Gk);
             }
-            adjoint_chunk<S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
+            adjoint_chunk<false, S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
         }
         ++steps;
         done = done || sec.size == 0 || T < S(1.f / 255.f) || (ctl.max_large_steps > 0 && steps >= ctl.max_large_steps);
@@ -1229,7 +1235,7 @@ __global__ __launch_bounds__(TW* TH) void k_march_backward_stored(MarchData<S> m
                 for (int k = 0; k < CB; ++k)
                     Tk[k] = Gk[k] = 0;
             }
-            adjoint_chunk<S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
+            adjoint_chunk<true, S, NT, CB>(tl, cand, active, inside, o, d, bb, b_first, b_last, Tk, Gk, pa.gC, render_grads);
         }
     }
 }
@@ -1372,8 +1378,8 @@ void launch_march(bool backward, const MarchData<S>& md, const DevCamera<S>& dc,
     const dim3 grid(md.n_tiles), block(TW * TH);
     // float: 32 bins in registers per pass (two waves per SIMD) unless
     // bins_per_chunk asks for 16 (three waves per SIMD, more passes): 200k
-    // Gaussians at 1024^2 take 16.5 / 19.4 ms forward, 24.6 / 30.8 ms read
-    // back from a replay store and 26.0 / 32.8 ms recomputed
+    // Gaussians at 1024^2 take 16.8 / 19.5 ms forward, 11.2 / 12.8 ms read
+    // back from a replay store and 26.0 / 32.5 ms recomputed
     if constexpr (sizeof(S) == 4) {
         const bool chunk16 = ctl.bins_per_chunk == 16;
         if (!backward && ctl.render_mode == 0) {
