@@ -150,14 +150,15 @@ def main():
     lib.dgmr_profile_enable(0)
     stages = stage_times(lib)
 
-    # pair count of this frame (for the byte model)
+    # pair counts of this frame: all of them, and those the step bins (for the byte model)
     with torch.no_grad():
-        cache = splatter.cpp_binding.forward(sh, torch.sigmoid(logits), means, torch.exp(log_scales),
-                                             torch.nn.functional.normalize(quats, dim=-1), view, proj, campos, bg, W, H, cam.tan_fovx,
-                                             cam.tan_fovy, 3)
+        frame = (sh, torch.sigmoid(logits), means, torch.exp(log_scales), torch.nn.functional.normalize(quats, dim=-1), view, proj, campos, bg,
+                 W, H, cam.tan_fovx, cam.tan_fovy, 3)
+        cache = splatter.cpp_binding.forward(*frame)
+        binned = int(splatter.cpp_binding.forward(*frame, whole_lists=None)[-1][0])
     R = int(cache[-1][0])
     n_visible = int((cache[7] > 0).sum())
-    del cache
+    del cache, frame
 
     tight = None
     if not args.no_tight:
@@ -169,13 +170,13 @@ def main():
     d_avg_ms = d_ms / max(d_launches, 1)
     achieved = (d_bytes / max(d_launches, 1)) / (d_avg_ms * 1e-3) / 1e9
     p_in = 44 + 12 * 16
-    # the shared frame byte model: per pair emission 12, sort 24, ranges 8 and
+    # the shared frame byte model: per binned pair emission 12, sort 24, ranges 8 and
     # both blend reads 40 + 40 (124 B); with 16-bit pair keys (every view here
     # has fewer than 65 536 tiles) the emission and each of the two sort
     # passes move 2 + 6 + 6 bytes less (110 B)
     frame_rest = args.n * (3 * p_in + 160) + 44 * W * H + 8 * ((W + 15) // 16) * ((H + 15) // 16)
-    frame_hbm_frac = (frame_rest + 124 * R) / (ms_per_step * 1e-3) / (HBM_PEAK_GBS * 1e9)
-    frame_hbm_frac_16bit = (frame_rest + 110 * R) / (ms_per_step * 1e-3) / (HBM_PEAK_GBS * 1e9)
+    frame_hbm_frac = (frame_rest + 124 * binned) / (ms_per_step * 1e-3) / (HBM_PEAK_GBS * 1e9)
+    frame_hbm_frac_16bit = (frame_rest + 110 * binned) / (ms_per_step * 1e-3) / (HBM_PEAK_GBS * 1e9)
 
     traffic = None
     tr_path = os.path.join(ROOT, "profiles", "traffic_splat_1M_1080p.json")
@@ -215,7 +216,7 @@ def main():
         "dtype": "f32",
         "data": "synthetic (seeded SplitMix64 scene: means U[-5,5]^3, log-scales N(-3,0.5), SH degree 3; uniform L1 target)",
         "config": {"workload": f"tile splat fwd+bwd, {args.n} Gaussians SH3, {W}x{H}, L1 loss", "tile": f"{tile[0]}x{tile[1]}",
-                   "lds_batch": args.batch, "pairs": R, "visible": n_visible,
+                   "lds_batch": args.batch, "pairs": R, "pairs_binned": binned, "visible": n_visible,
                    "activations": "torch" if args.torch_activations else "fused",
                    "l1_loss": "torch" if args.torch_loss else "fused"},
         "roofline": roofline,
