@@ -166,3 +166,65 @@ def test_infinite_colours_stay_where_their_mass_is():
     np.testing.assert_array_equal(got[1:], a[1:])
     np.testing.assert_array_equal(got[0][untouched], a[0][untouched])
     assert np.isnan(got[0][~untouched]).all()
+
+
+@pytest.mark.parametrize("kind", ["ragged", "needles", "discs", "wide_fov_inside", "opaque_heavy", "long_lists"])
+def test_raster_entry_windows(kind):
+    """The rasterisation visits only the list entries whose window along the rays
+    meets the chunk, and notes for the first 4 096 which no pixel of the wave can
+    take: tiles with pixels outside the image, Gaussians for which the window is
+    widest or gives up (needles and discs up to 1:100 and more, rays more than 90
+    degrees from a Gaussian, slabs whose mass on a ray can pass 100) and lists of
+    several batches, past the notes.  The bars of the other tests: the float
+    restatement on 98 % of the pixels, and the FP64 oracle on the float placement
+    where float32 represents the inverse covariances (not the 1:100 ones)."""
+    if not gpu_available():
+        pytest.skip("no GPU")
+    import oracle as O
+    from differentiable_gaussian_mixture_renderer_amd import scenes
+    rng = np.random.default_rng(11)
+    n, extent, w, h, pos, t = 1500, 1.0, 61, 43, [0.2, -0.1, -4.0], math.tan(math.radians(30))
+    if kind == "wide_fov_inside":
+        extent, pos, t = 2.0, [0.1, 0.2, -0.3], 4.0
+    elif kind == "opaque_heavy":
+        n = 80
+    elif kind == "long_lists":
+        n, w, h, extent = 5200, 16, 16, 0.8
+    scene = scenes.make_scene(n, seed=8, extent=extent, sh_degree=1)
+    s = scene.scales
+    if kind == "needles":
+        s[:, 0] *= 6.0
+        s[:, 1:] *= rng.uniform(0.01, 1.0, (n, 2))
+    elif kind == "discs":
+        s[:, :2] *= 4.0
+        s[:, 2] *= rng.uniform(0.01, 0.3, n)
+    elif kind == "opaque_heavy":
+        s[:, :2] *= 40.0
+        s[:, 2] *= 0.02
+        scene.opacity[:] = 0.999
+    elif kind == "long_lists":
+        s *= 2.0
+        scene.opacity *= 0.05
+    scene.scales = s.astype(np.float32)
+    cam = scenes.look_at_camera(pos, [0.0, 0.0, 0.0], w, h, t * w / h, t)
+    sc = O.scene_arrays(scene)
+    bg = np.array([0.1, 0.2, 0.3], np.float32)
+    print(f"[gpu raster windows] {kind} n={n} {w}x{h}", flush=True)
+    got, cache = _gpu(sc, cam, bg)
+    ranges = cache["i_ranges"].cpu().numpy().view(np.uint32)
+    longest = int((ranges[:, 1].astype(np.int64) - ranges[:, 0]).max())
+    want, n_pairs = O.raster_render(sc, cam, bg)
+    assert n_pairs == cache["n_pairs"] > 0
+    diff = np.abs(got - want).max(axis=0)
+    want64, _, amb = O.raster_render(sc, cam, bg.astype(np.float64), dbl=True)
+    ok = amb == 0
+    err = np.abs(got - want64).max(axis=0)
+    print(f"longest list {longest}, float: {(diff > 1e-3).mean():.4f} over 1e-3, median {np.median(diff):.2g}; "
+          f"FP64: flagged {(~ok).mean():.3f}, max unflagged {err[ok].max():.2g}")
+    if kind == "long_lists":
+        assert longest > 4096
+    assert np.isfinite(got).all()
+    assert (diff <= 1e-3).mean() >= 0.98
+    assert np.median(diff) <= 1e-5
+    if kind not in ("needles", "discs", "opaque_heavy"):
+        assert err[ok].max() <= 1e-4
