@@ -530,6 +530,48 @@ def test_entry_windows_at_extreme_shapes(kind):
         assert np.abs(got - ref_g).max() <= 1e-7 * np.abs(ref_g).max(), name
 
 
+@pytest.mark.parametrize("kind", ["ragged", "wide_fov_inside", "opaque_heavy", "long_lists"])
+def test_entry_windows_in_float(kind):
+    """The float kernels' windows (their own far cut, rounding and queue) where
+    they are widest or give up, as above, with shapes that float32 represents:
+    the float-placed FP64 bars on image, transmittance and gradients, with up to
+    a fifth of the pixels flagged (dense scenes hold each of hundreds of masses
+    per pixel to a threshold)."""
+    torch = _torch()
+    rng = np.random.default_rng(11)
+    n, extent, w, h, pos, t = 700, 1.2, 43, 29, [0.2, -0.1, -5.0], 0.5
+    if kind == "wide_fov_inside":
+        extent, pos, t = 2.0, [0.1, 0.2, -0.3], 4.0
+    if kind == "long_lists":
+        n, w, h, extent = 5200, 16, 16, 0.8
+    from differentiable_gaussian_mixture_renderer_amd import scenes
+    scene = scenes.make_scene(n, seed=8, extent=extent, sh_degree=3)
+    s = scene.scales
+    if kind == "opaque_heavy":
+        s[:, :2] *= 6.0
+        s[:, 2] *= 0.3
+        scene.opacity[:] = 0.999
+    elif kind == "long_lists":
+        s *= 2.0
+        scene.opacity *= 0.02
+    scene.scales = s.astype(np.float32)
+    cam = scenes.look_at_camera(pos, [0.0, 0.0, 0.0], w, h, t * w / h, t)
+    bg = np.array([0.2, 0.3, 0.4], np.float32)
+    ref = O.MarchOracle(O.scene_arrays(scene), cam, dbl=True, float_binning=True)
+    fb, T, _, amb = ref.render(bg, with_ambiguity=True, float_sampling=True)
+    ok = amb == 0
+    grad = rng.normal(size=(3, h, w)).astype(np.float32)
+    grad[:, ~ok] = 0.0
+    out = run_gpu(scene, cam, bg, torch.float32, grad_fb=grad)
+    err = np.abs(out["framebuffer"] - fb).max(axis=0)
+    print(f"{kind}: longest list {np.diff(out['ranges'], axis=1).max()}, flagged {(~ok).mean():.3f}, max (unflagged) {err[ok].max():.3g}")
+    assert (~ok).mean() <= 0.2
+    assert err[ok].max() <= IMG_TOL
+    assert np.abs(out["remaining"] - T)[ok].max() <= IMG_TOL
+    want = ref.backward(bg, fb, T, grad.astype(np.float64), float_sampling=True)
+    _check_grads(out["grads"], want, n, scene.sh.shape[1], kind)
+
+
 @pytest.mark.parametrize("dtype_name", ["float64", "float32"])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 def test_values_that_are_not_finite_stay_where_mass_is(dtype_name, value):
