@@ -1,10 +1,9 @@
-"""Batched multi-view splatting through one persistent launch per stage.
+"""Batched multi-view splatting through one launch per stage.
 
 `BatchSplatter` renders one scene from many cameras of uneven resolution with
 the C ABI's dgmr_splat_batch_forward / dgmr_splat_batch_backward: one
 preprocess launch over all (view, Gaussian) pairs, one binning pass over the
-global tile range, one persistent blend launch pulling tiles of every view from
-a device queue.  The workspace carries geometry and binning from the forward to
+global tile range, one blend launch over the tiles of every view.  The workspace carries geometry and binning from the forward to
 the backward.
 
 `render_plain` is the one-camera-per-launch path (a Splatter call per view)

@@ -236,16 +236,17 @@ __device__ __forceinline__ int find_view(const ViewBlend* views, int n_views, in
 // atomics, 14 ns each, whatever the tiles held (39k tiles of 12 views: forward
 // 0.57 -> 0.33 ms, backward 0.78 -> 0.72 ms; workgroups of four waves, which
 // wait for their longest list, 0.34 and 0.76 ms).  The forward gives each XCD a
-// contiguous band of tiles, the backward takes tile_order[k] in turn.
+// contiguous band of tiles, the backward takes tile_order[k] in turn.  `first`:
+// the tile part of the launch's block 0 (kLaunchParts).
 template <int TW, int TH, int B, int SPLIT, bool BACKWARD>
 __global__ __launch_bounds__(64) void k_batch_blend(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ point_list,
     const float2* __restrict__ xy, const float4* __restrict__ conic_opacity, const float* __restrict__ rgb, const ViewBlend* __restrict__ views,
-    int n_views, float* __restrict__ screen_grads, const uint32_t* __restrict__ tile_order)
+    int n_views, float* __restrict__ screen_grads, const uint32_t* __restrict__ tile_order, int first)
 {
     using Smem = typename std::conditional<BACKWARD, BlendSmemBwd<B>, BlendSmem<B>>::type;
     __shared__ Smem sm;
     constexpr int PH = TH / SPLIT; // rows of a part
-    const int unit = BACKWARD ? int(blockIdx.x) : xcd_tile(int(blockIdx.x), int(gridDim.x));
+    const int unit = first + (BACKWARD ? int(blockIdx.x) : xcd_tile(int(blockIdx.x), int(gridDim.x)));
     const int part = unit % SPLIT;
     int tile = unit / SPLIT;
     if (BACKWARD)
@@ -566,18 +567,22 @@ SplatParams slot_params(const BatchLayout& L, const dgmr_gaussians* g, const dgm
         g->sh_degree, float(g->scale_multiplier), g->activation };
 }
 
+// Most tile parts of one launch of the batched blend.  A launch holds fewer than
+// 2^32 threads, so 2^26 waves, which the tiles of a batch can exceed (16 views of
+// 16 384 x 16 384 in 8x8 tiles): such a batch takes several launches.
+constexpr int64_t kLaunchParts = int64_t(1) << 25;
+
 template <int TW, int TH, int SPLIT>
-void launch_batch_blend(bool backward, int batch, hipStream_t st, const BatchLayout& L, int n_views)
+void launch_batch_blend(bool backward, int batch, hipStream_t st, const BatchLayout& L, int n_views, int first, unsigned grid)
 {
     const auto* xy2 = reinterpret_cast<const float2*>(L.xy);
-    const unsigned grid = unsigned(L.total_tiles * SPLIT);
 #define DGMR_BATCH_BLEND(B)                                                                                                            \
     if (backward)                                                                                                                      \
         k_batch_blend<TW, TH, B, SPLIT, true><<<grid, 64, 0, st>>>(L.ranges, L.point_list, xy2, L.conic_opacity, L.rgb, L.views, n_views, \
-            L.screen_grads, L.tile_order);                                                                                             \
+            L.screen_grads, L.tile_order, first);                                                                                      \
     else                                                                                                                               \
         k_batch_blend<TW, TH, B, SPLIT, false><<<grid, 64, 0, st>>>(L.ranges, L.point_list, xy2, L.conic_opacity, L.rgb, L.views, n_views, \
-            L.screen_grads, nullptr);
+            L.screen_grads, nullptr, first);
     if (batch == 64) {
         DGMR_BATCH_BLEND(64)
     } else if (batch == 128) {
@@ -592,10 +597,12 @@ template <int TW, int TH>
 void launch_batch_blend(bool backward, int batch, hipStream_t st, const BatchLayout& L, int n_views)
 {
     constexpr int SPLIT = TW * TH / 64;
-    if (SPLIT > 1 && L.total_tiles <= (backward ? kBwdSplitTiles : kFwdSplitTiles))
-        launch_batch_blend<TW, TH, SPLIT>(backward, batch, st, L, n_views);
-    else
-        launch_batch_blend<TW, TH, 1>(backward, batch, st, L, n_views);
+    if (SPLIT > 1 && L.total_tiles <= (backward ? kBwdSplitTiles : kFwdSplitTiles)) {
+        launch_batch_blend<TW, TH, SPLIT>(backward, batch, st, L, n_views, 0, unsigned(L.total_tiles * SPLIT));
+    } else {
+        for (int64_t first = 0; first < L.total_tiles; first += kLaunchParts)
+            launch_batch_blend<TW, TH, 1>(backward, batch, st, L, n_views, int(first), unsigned(std::min(kLaunchParts, L.total_tiles - first)));
+    }
 }
 
 void batch_blend(bool backward, const dgmr_tiling& t, hipStream_t st, const BatchLayout& L, int n_views)

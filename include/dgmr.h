@@ -237,8 +237,8 @@ int dgmr_march_backward(const dgmr_gaussians* g, const dgmr_camera* cam, const d
 /* ------------------------------------------------------------ batched views
  * Many cameras of one scene (uneven resolutions) rendered together: one
  * preprocess launch over all (view, Gaussian) pairs, one binning pass over the
- * global tile range of all views, and one persistent blend launch whose
- * workgroups pull tiles of every view from a device queue.  No counterpart in
+ * global tile range of all views, and one blend launch over the tiles of every
+ * view (batches of more than 2^25 tiles take several).  No counterpart in
  * the reference (one camera per call there, vol_marcher.py:19-65).
  * The workspace carries the per-view geometry and binning from the forward to
  * the backward: keep it untouched in between. */

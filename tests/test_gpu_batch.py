@@ -259,3 +259,46 @@ def test_waves_per_tile_of_batches(resolutions):
     for a, b in zip(gb, gp):
         a, b = a.cpu().numpy(), b.cpu().numpy()
         assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b) + 1e-12
+
+
+def test_batch_of_more_tiles_than_one_launch_holds(monkeypatch):
+    """16 views of 16 384 x 16 384 in 8x8 tiles (2^26 tiles, past the threads
+    of one launch; they share one framebuffer, in which all write the same
+    image) and a small view behind them: the large image at its corners and the
+    small view with its gradients as rendered alone."""
+    torch = _torch()
+    if torch.cuda.get_device_properties(0).total_memory < (64 << 30):
+        pytest.skip("needs 64 GB of device memory")
+    from differentiable_gaussian_mixture_renderer_amd import _common, scenes
+    from differentiable_gaussian_mixture_renderer_amd.batching import BatchSplatter, render_plain
+    scene = scenes.make_scene(40, seed=7, extent=5.0, sh_degree=0)
+    large = scenes.sphere_cameras(1, seed=3, resolutions=[(16384, 16384)])[0]
+    small = scenes.sphere_cameras(1, seed=3, resolutions=[(100, 70)])[0]
+    dev = torch.device("cuda:0")
+    t = lambda a: torch.tensor(np.ascontiguousarray(a), device=dev)
+    params = [t(scene.sh), t(scene.opacity), t(scene.means), t(scene.scales), t(scene.rotations)]
+    bg = (0.1, 0.2, 0.3)
+    monkeypatch.setattr(_common, "pairs_per_pixel", lambda device: 0.05)  # the capacity of 4.3 billion pixels; grown if it is short
+    print("[gpu batch] 16 views of 16384x16384 and one of 100x70 in 8x8 tiles", flush=True)
+    bs = BatchSplatter(tile=(8, 8))
+    bs._prepare(*params, [large, small], bg, 0)
+    bs.cameras = [large] * 16 + [small]
+    bs._fbs = [bs._fbs[0]] * 16 + [bs._fbs[1]]
+    bs._Ts = [bs._Ts[0]] * 16 + [bs._Ts[1]]
+    for f in (bs._fbs[0], bs._fbs[16], bs._Ts[0], bs._Ts[16]):
+        f.fill_(-1.0)
+    bs._views = bs._view_array(bs.cameras, bs.bg, bs._fbs, bs._Ts)
+    bs._launch_forward(dev)
+    grad = torch.tensor(np.random.default_rng(1).normal(size=(3, 70, 100)).astype(np.float32), device=dev)
+    gb = bs.backward([None] * 16 + [grad])
+    (img_l,), _ = render_plain(*params, [large], bg=bg, sh_degree=0, tile=(8, 8))
+    (img_s,), gp = render_plain(*params, [small], bg=bg, sh_degree=0, grad_fn=lambda img: grad, tile=(8, 8))
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(bs._fbs[16].cpu().numpy(), img_s.cpu().numpy(), rtol=0, atol=1e-6)
+    for rows in (slice(0, 64), slice(8160, 8224), slice(-64, None)):
+        np.testing.assert_allclose(bs._fbs[0][:, rows].cpu().numpy(), img_l[:, rows].cpu().numpy(), rtol=0, atol=1e-6)
+    for a, b in zip(gb, gp):
+        a, b = a.cpu().numpy(), b.cpu().numpy()
+        assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b) + 1e-12
+    del bs, img_l
+    torch.cuda.empty_cache()
