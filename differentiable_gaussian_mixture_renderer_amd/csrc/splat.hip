@@ -17,7 +17,7 @@
 //   7. k_blend_forward      per tile, LDS-staged batches of Gaussians
 // A view of at most 16 384 Gaussians takes steps 2 and 3 and the bounds in one
 // launch (k_bin_one); the autograd path bins deep views by a prefix of the depth
-// order (k_extend_*).
+// order where that pays (k_prefix_decide, k_extend_*, k_open_*).
 // Backward: k_blend_backward (front-to-back replay, transmittance recomputed,
 // wave-reduced atomics) then k_splat_preprocess_backward (per Gaussian).
 #include <algorithm>
@@ -197,8 +197,9 @@ __global__ __launch_bounds__(256) void k_gather_owners(int64_t n, const uint32_t
 // span few octaves, so the bits that all keys share are not sorted.  Culled
 // Gaussians (key ~0) take the key after the last and stay in order behind.
 // Bound by the latency of its passes on one CU: 12.6 us at 301 Gaussians and 39
-// us at 10 000, against 66 us and 75 us of the launches it replaces; above
-// kBinOneMax the keys no longer fit its registers and LDS and the launches of
+// us at 10 000, against 66 us and 75 us of the launches it replaces; at 16 384 a
+// whole forward call of 256x256 pixels takes 134 us, at 16 385 with the launches
+// 155.  Above kBinOneMax the keys no longer fit its registers and LDS and the launches of
 // the large path fill more CUs (50 000: 12 launches in 60 us).
 constexpr int kBinOneThreads = 1024;
 constexpr int kBinOneItems = 16;
@@ -869,13 +870,13 @@ __global__ __launch_bounds__(64 * kBlendWaves) void k_blend_forward(const uint32
 // kPrefixMin times their pairs, make 1.3M fewer (by the 16 pairs a Gaussian makes
 // in an ordinary deep view) and look covered (k_prefix_decide).  Forward in us,
 // prefixes / whole lists, at 1920x1080 (scales e^-3, cube of side 10 unless noted):
-//   1M, opacities around 1/2      355 / 444   no tile open
-//   3M, the same                  695 / 1026  3 open
-//   1M, around 0.27               440 / 504   23 open
-//   1M, around 0.18               562 / 538   1 004 open (k_prefix_decide: whole)
-//   1M, around 0.007              1004 / 890  all open (whole; 900 with k_prefix_decide)
-//   1M in a cube of side 3        611 / 696   1 838 open at its edges
-//   3M in it, scales e^-4         984 / 976   618 open
+//   1M, opacities around 1/2      352 / 446   no tile open
+//   3M, the same                  696 / 1026  3 open
+//   1M, around 0.27               442 / 505   23 open
+//   1M, around 0.18               562 / 539   1 004 open (whole; 544 with k_prefix_decide)
+//   1M, around 0.007              1004 / 888  all open (whole; 898 with k_prefix_decide)
+//   1M in a cube of side 3        610 / 698   1 838 open at its edges
+//   3M in it, scales e^-4         985 / 975   618 open
 constexpr int64_t kPrefixPerTile = 256;
 constexpr int64_t kPrefixPairsPerGaussian = 16;
 constexpr int64_t kPrefixMinSaved = 1300000;

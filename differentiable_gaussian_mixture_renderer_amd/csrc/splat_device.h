@@ -1,6 +1,6 @@
 // SPDX-License-Identifier: GPL-3.0-or-later
 // Device functions of the tile splatter shared by the single-view kernels and
-// the persistent multi-view kernels (reference: src/dgmr/splat_forward.cu).
+// the multi-view kernels (reference: src/dgmr/splat_forward.cu).
 #pragma once
 
 #include "device_grad.h"

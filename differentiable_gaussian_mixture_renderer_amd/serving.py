@@ -5,8 +5,8 @@ open-loop trace.  A scheduler thread admits waiting requests while the
 estimated HBM footprint of everything in flight stays under a budget, groups
 the admitted requests of one scene into a batch, and hands the batch to the
 next free worker.  Each worker owns a HIP stream and runs the batch through the
-multi-view path (BatchSplatter: one preprocess, one binning, one persistent
-blend launch); workers run concurrently, so batches of different scenes, and
+multi-view path (BatchSplatter: one preprocess, one binning, one blend
+launch); workers run concurrently, so batches of different scenes, and
 new arrivals admitted while others are on the GPU, overlap on the device.
 Latency is completion time minus arrival time.
 
